@@ -20,12 +20,12 @@ constexpr int NV = 5;
 __device__ __forceinline__ float  rcp( float x )  { return __builtin_amdgcn_rcpf( x ); }
 __device__ __forceinline__ double rcp( double x )
 {
-   // hardware estimate + two Newton steps: within 1 ulp of 1/x for normal x
-   double r = __builtin_amdgcn_rcp( x );
-   double e = __builtin_fma( -x, r, 1.0 );
-   r = __builtin_fma( r, e, r );
-   e = __builtin_fma( -x, r, 1.0 );
-   return __builtin_fma( r, e, r );
+   // hardware estimate r = (1 - e)/x and one third-order step r (1 + e + e^2): the estimate's relative error (about
+   // 1e-7) enters cubed, so the result is within 1 ulp of 1/x for normal x, as two Newton steps gave with one
+   // instruction and one link of the dependent chain more
+   const double r = __builtin_amdgcn_rcp( x );
+   const double e = __builtin_fma( -x, r, 1.0 );
+   return __builtin_fma( r, __builtin_fma( e, e, e ), r );
 }
 __device__ __forceinline__ float  vsqrt( float x )  { return __builtin_amdgcn_sqrtf( x ); }
 __device__ __forceinline__ double vsqrt( double x ) { return __builtin_sqrt( x ); }
@@ -48,23 +48,31 @@ __device__ __forceinline__ double rcp_recover( double x )
 
 template <typename R> __device__ __forceinline__ double rcp_pres( double x ) { return sizeof( R ) == 4 ? rcp_recover( x ) : rcp( x ); }
 
+// s = x^1/2 and y = x^-1/2 of a positive x, each within 1 ulp.  FP64: from the hardware reciprocal square root y and
+// its third-order correction 1 + e/2 + 3/8 e^2, e = 1 - x y^2 (the estimate's error enters cubed); FP32: the
+// hardware square root and reciprocal
+__device__ __forceinline__ void sqrt_rsq( double x, double &s, double &y )
+{
+   const double y0 = __builtin_amdgcn_rsq( x ), s0 = x*y0;
+   const double e = __builtin_fma( -s0, y0, 1.0 ), t = __builtin_fma( e, 0.375, 0.5 );
+   s = __builtin_fma( s0*e, t, s0 );
+   y = __builtin_fma( y0*e, t, y0 );
+}
+__device__ __forceinline__ void sqrt_rsq( float x, float &s, float &y ) { s = vsqrt( x );  y = rcp( s ); }
+
 // sound speed (gamma P / rho)^1/2 from gp = gamma P, rho and ir = 1/rho.  Generic form sqrt(gp ir).  FP64:
-// gp (gp rho)^-1/2 from the hardware reciprocal square root and two Newton steps, about 2 ulp, one transcendental
-// and 9 instructions where the reciprocal's Newton steps and the IEEE square root take about 20; gp == 0 gives 0
-// and NaN passes.  The derivative kernels define HYDRO_IEEE_SOUND_SPEED before including this header and keep the
+// gp (gp rho)^-1/2 with sqrt_rsq's third-order step applied to gp y, about 2 ulp, one transcendental and 10 instructions
+// where the reciprocal and the IEEE square root take about 20; gp == 0 gives 0 and NaN passes.  FP32 keeps the
+// generic form: gp rho leaves its range for gases (1e-24 g/cm^3) whose gp/rho does not.  The derivative kernels define HYDRO_IEEE_SOUND_SPEED before including this header and keep the
 // generic form, which their dual-number twins evaluate bit for bit.
 template <typename R> __device__ __forceinline__ R sound_speed( R gp, R rho, R ir ) { (void)rho; return vsqrt( gp*ir ); }
 #ifndef HYDRO_IEEE_SOUND_SPEED
 template <> __device__ __forceinline__ double sound_speed<double>( double gp, double rho, double ir )
 {
    (void)ir;
-   const double a = gp*rho, h = 0.5*a;
-   double y = __builtin_amdgcn_rsq( a );
-   double r = __builtin_fma( -h*y, y, 0.5 );        // y (1.5 - a y^2 / 2) = y + y (0.5 - h y^2)
-   y = __builtin_fma( y, r, y );
-   r = __builtin_fma( -h*y, y, 0.5 );
-   y = __builtin_fma( y, r, y );
-   return ( gp == 0.0 ) ? 0.0 : gp*y;
+   const double a = gp*rho, y = __builtin_amdgcn_rsq( a ), c = gp*y;
+   const double e = __builtin_fma( -( a*y ), y, 1.0 );
+   return ( gp == 0.0 ) ? 0.0 : __builtin_fma( c*e, __builtin_fma( e, 0.375, 0.5 ), c );
 }
 #endif
 
@@ -356,24 +364,6 @@ __device__ __forceinline__ St<R> face_state( const R w[NV], const Prm<R> &P )
    return s;
 }
 
-// face_state<0> or face_state<1> chosen per lane (dy = y-normal face): the same arithmetic, the rotation by select
-template <typename R>
-__device__ __forceinline__ St<R> face_state_xy( const R w[NV], bool dy, const Prm<R> &P )
-{
-   St<R> s;
-   const R vn = dy ? w[2] : w[1], v1 = dy ? w[3] : w[2], v2 = dy ? w[1] : w[3];
-   s.d  = w[0];
-   s.mn = w[0]*vn;
-   s.m1 = w[0]*v1;
-   s.m2 = w[0]*v2;
-   s.u  = vn;
-   s.ir = rcp( w[0] );
-   s.p  = floor_pres( w[4], P.min_pres );
-   s.e  = fmad( (R)0.5*w[0], fmad( w[3], w[3], fmad( w[2], w[2], w[1]*w[1] ) ), w[4]*P.inv_gm1 );
-   s.cs = sound_speed( P.gamma*s.p, s.d, s.ir );
-   return s;
-}
-
 // conserved cell (with its pressure, 1/rho and sound speed) -> interface state rotated to direction D
 template <int D, typename R>
 __device__ __forceinline__ St<R> cell_state( const R c[NV], R p, R ir, R cs )
@@ -386,21 +376,6 @@ __device__ __forceinline__ St<R> cell_state( const R c[NV], R p, R ir, R cs )
    s.e  = c[4];
    s.p  = p;  s.ir = ir;  s.cs = cs;
    s.u  = ir*s.mn;
-   return s;
-}
-
-// cell_state<0> or cell_state<1> chosen per lane (dy = y-normal face) from a cell (conserved, P, 1/rho, c_s)
-template <typename R>
-__device__ __forceinline__ St<R> cell_state_xy( const R q[8], bool dy )
-{
-   St<R> s;
-   s.d  = q[0];
-   s.mn = dy ? q[2] : q[1];
-   s.m1 = dy ? q[3] : q[2];
-   s.m2 = dy ? q[1] : q[3];
-   s.e  = q[4];
-   s.p  = q[5];  s.ir = q[6];  s.cs = q[7];
-   s.u  = s.ir*s.mn;
    return s;
 }
 
@@ -438,23 +413,283 @@ __device__ __forceinline__ void riemann( const St<R> &L, const St<R> &Q, const P
    out[1 + ( D + 2 ) % 3] = f[3];
 }
 
-// riemann<RS, 0> or riemann<RS, 1> chosen per lane (dy = y-normal face)
-template <int RS, typename R>
-__device__ __forceinline__ void riemann_xy( const St<R> &L, const St<R> &Q, const Prm<R> &P, bool dy, R out[NV] )
+// conserved face state -> interface state rotated to direction D, pressure recovered in FP64
+template <int D, typename R>
+__device__ __forceinline__ St<R> cons_state( const R c[NV], const Prm<R> &P )
 {
-   R f[NV];
+   St<R> s;
+   const double eint = (double)c[4] - 0.5*( (double)c[1]*c[1] + (double)c[2]*c[2] + (double)c[3]*c[3] )
+                                      *rcp_pres<R>( (double)c[0] );
+   s.d  = c[0];
+   s.mn = c[1 + D];
+   s.m1 = c[1 + ( D + 1 ) % 3];
+   s.m2 = c[1 + ( D + 2 ) % 3];
+   s.e  = c[4];
+   s.p  = floor_pres( (R)( eint*P.gm1_d ), P.min_pres );
+   s.ir = rcp( c[0] );
+   s.u  = s.ir*s.mn;
+   s.cs = sound_speed( P.gamma*s.p, s.d, s.ir );
+   return s;
+}
+
+// ---------------- interface solves of the marching kernels ----------------
+// One side of an interface: density, normal velocity u, pressure, sound speed, and by kind
+//   KIND 0  an input cell (half step): a, b transverse momenta, e the energy
+//   KIND 1  a primitive face (MHM_RP's full step): a, b transverse velocities, e the internal energy
+//   KIND 2  a conserved face (MHM): mn the normal and a, b the transverse momenta, e the energy
+// The marching kernels solve 35,712 interfaces per patch group, half of their instructions.  Measured per wave64
+// instruction and SIMD, FP32 add, mul and fma issue in 2.2 cycles, min, max, compare and select in 4.8, reciprocals in
+// 9.2 (FP64: 4.8 and 18.5), with two wait states between a compare and its select.  Against rs_hllc() of the
+// derivative and correction kernels (the same HLLC fluxes, CPU_Shared_RiemannSolver_HLLC.cpp:391-655) this form
+//   * takes tl = rho_L (u_L - w_L), tr = rho_R (w_R - u_R) from the wave speeds instead of by selects,
+//   * takes the contact as u_L + x and its pressure as p_L - tl x, x = (p_L - p_R - tr (u_L - u_R))/(tl + tr):
+//     differences come before products, 5 operations instead of 9,
+//   * forms the flux as mass flux times (1, u, a, b, e) plus pressure terms, and, on faces, the energy only of the
+//     side that the contact selects,
+//   * leaves the vs == sp == 0 case to the NaN rescue: HLLE's flux there is the physical flux of the left state.
+// Contraction is off and fused multiply-adds are written out, so that every code path that solves a face gets the
+// same bits.  Roe and HLLE follow the same layout.  With the PLM below and the third-order reciprocals, on 4096 patch
+// groups FP32 HLLC went from 0.696 to 0.654 ms, on 1331 FP64 HLLC from 0.594 to 0.516 ms, on 300 FP64 Roe from 0.445
+// to 0.325 ms, on 1000 FP32 MHM HLLE from 0.264 to 0.257 ms, with the same error against 64 bits.
+template <typename R>
+struct Side { R d, u, a, b, p, cs, e, mn; };
+
+template <int D, typename R>
+__device__ __forceinline__ Side<R> cell_side( const R q[8] )          // (rho, m, E, P, 1/rho, c_s); a, b: momenta
+{
+   Side<R> s;
+   s.d = q[0];  s.u = q[6]*q[1 + D];  s.a = q[1 + ( D + 1 ) % 3];  s.b = q[1 + ( D + 2 ) % 3];
+   s.e = q[4];  s.p = q[5];  s.cs = q[7];
+   return s;
+}
+template <typename R>
+__device__ __forceinline__ Side<R> cell_side_xy( const R q[8], bool dy )
+{
+   Side<R> s;
+   s.d = q[0];  s.u = q[6]*( dy ? q[2] : q[1] );  s.a = dy ? q[3] : q[2];  s.b = dy ? q[1] : q[3];
+   s.e = q[4];  s.p = q[5];  s.cs = q[7];
+   return s;
+}
+
+// pressure floor that lets NaN through, as floor_pres; FP32 in one instruction (gfx950's v_maximum3_f32)
+__device__ __forceinline__ double floor_nan( double p, double pmin ) { return floor_pres( p, pmin ); }
+__device__ __forceinline__ float  floor_nan( float p, float pmin )   { return __builtin_elementwise_maximum( p, pmin ); }
+
+template <typename R>
+__device__ __forceinline__ void face_cs( Side<R> &s, R p, const Prm<R> &P )
+{
+   s.p  = floor_nan( p, P.min_pres );
+   s.cs = sound_speed( P.gamma*s.p, s.d, rcp( s.d ) );
+   s.e  = p*P.inv_gm1;                                                // internal energy of the unfloored pressure
+}
+// conserved face state (MHM's Hancock faces), its pressure recovered in FP64; a, b: momenta
+template <int D, typename R>
+__device__ __forceinline__ Side<R> cons_side( const R c[NV], const Prm<R> &P )
+{
+   const St<R> t = cons_state<D>( c, P );
+   Side<R> s;
+   s.d = t.d;  s.u = t.u;  s.a = t.m1;  s.b = t.m2;  s.p = t.p;  s.cs = t.cs;  s.e = t.e;  s.mn = t.mn;
+   return s;
+}
+template <int D, typename R>
+__device__ __forceinline__ Side<R> face_side( const R w[NV], const Prm<R> &P )   // primitive; a, b: velocities
+{
+   Side<R> s;
+   s.d = w[0];  s.u = w[1 + D];  s.a = w[1 + ( D + 1 ) % 3];  s.b = w[1 + ( D + 2 ) % 3];
+   face_cs( s, w[4], P );
+   return s;
+}
+template <typename R>
+__device__ __forceinline__ Side<R> face_side_xy( const R w[NV], bool dy, const Prm<R> &P )
+{
+   Side<R> s;
+   s.d = w[0];  s.u = dy ? w[2] : w[1];  s.a = dy ? w[3] : w[2];  s.b = dy ? w[1] : w[3];
+   face_cs( s, w[4], P );
+   return s;
+}
+// energy density of a face side (Pri2Con)
+template <typename R>
+__device__ __forceinline__ R face_energy( R d, R u, R a, R b, R eint )
+{
+   return fmad( (R)0.5*d, fmad( b, b, fmad( a, a, u*u ) ), eint );
+}
+
+template <int KIND, typename R>
+__device__ __forceinline__ void hllc_flux( const Side<R> &L, const Side<R> &Q, R pmin, R f[NV] )
+{
+   #pragma clang fp contract(off)
+   const R Z = (R)0;
+   const R wl = vmin( L.u - L.cs, Q.u - Q.cs ), wr = vmax( L.u + L.cs, Q.u + Q.cs );
+   const R tl = L.d*( L.u - wl ), tr = Q.d*( wr - Q.u );
+   const R x  = rcp( tl + tr )*fmad( tr, Q.u - L.u, L.p - Q.p );
+   const R vs = L.u + x;
+   const R ps = vmax( fmad( -tl, x, L.p ), pmin );                    // a NaN here is a NaN in vs too
+   const bool left = ( vs >= Z );
+   const R d = left ? L.d : Q.d, u = left ? L.u : Q.u, a = left ? L.a : Q.a, b = left ? L.b : Q.b,
+           p = left ? L.p : Q.p, e0 = left ? L.e : Q.e, mn = left ? L.mn : Q.mn;
+   const R sp = left ? vmin( wl, Z ) : vmax( wr, Z );
+   const R t  = rcp( vs - sp ), cf = t*vs, m = cf*( u - sp ), cp = cf*p, cs = -( t*sp )*ps, pp = cp + cs;
+   f[0] = KIND == 2 ? cf*fmad( -sp, d, mn ) : m*d;
+   f[1] = KIND == 2 ? fmad( m, mn, pp ) : fmad( f[0], u, pp );
+   f[2] = ( KIND == 1 ? f[0] : m )*a;
+   f[3] = ( KIND == 1 ? f[0] : m )*b;
+   f[4] = fmad( m, KIND == 1 ? face_energy( d, u, a, b, e0 ) : e0, fmad( cp, u, cs*vs ) );
+}
+
+template <int KIND, typename R>
+__device__ __forceinline__ void hlle_flux( const Side<R> &L, const Side<R> &Q, R f[NV] )
+{
+   #pragma clang fp contract(off)
+   const R Z = (R)0;
+   const R sl = vmin( vmin( L.u - L.cs, Q.u - Q.cs ), Z ), sr = vmax( vmax( L.u + L.cs, Q.u + Q.cs ), Z );
+   const bool both0 = ( sl == Z ) && ( sr == Z );
+   const R inv = rcp( sr - sl );
+   const R cl = both0 ? (R)1 : inv*sr, cr = both0 ? Z : -( inv*sl );
+   const R ml = cl*( L.u - sl ), mr = cr*( Q.u - sr );                // mass flux per density of each side
+   const R fl = KIND == 2 ? cl*fmad( -sl, L.d, L.mn ) : ml*L.d, fr = KIND == 2 ? cr*fmad( -sr, Q.d, Q.mn ) : mr*Q.d;
+   const R pl = cl*L.p, pr = cr*Q.p;
+   const R el = KIND == 1 ? face_energy( L.d, L.u, L.a, L.b, L.e ) : L.e, er = KIND == 1 ? face_energy( Q.d, Q.u, Q.a, Q.b, Q.e ) : Q.e;
+   const R al = KIND == 1 ? fl : ml, ar = KIND == 1 ? fr : mr;
+   f[0] = fl + fr;
+   f[1] = KIND == 2 ? fmad( ml, L.mn, fmad( mr, Q.mn, pl + pr ) ) : fmad( fl, L.u, fmad( fr, Q.u, pl + pr ) );
+   f[2] = fmad( al, L.a, ar*Q.a );
+   f[3] = fmad( al, L.b, ar*Q.b );
+   f[4] = fmad( ml, el, fmad( mr, er, fmad( pl, L.u, pr*Q.u ) ) );
+}
+
+// Roe with the intermediate-state check (Roe.cpp:87-711).  Square roots and reciprocals of the densities and of the
+// sound speed come in pairs from one reciprocal square root each; rs_roe() of the derivative kernels takes 3 IEEE
+// square roots and 8 reciprocals.
+template <int KIND, typename R>
+__device__ __forceinline__ void roe_flux( const Side<R> &L, const Side<R> &Q, const Prm<R> &P, R f[NV] )
+{
+   #pragma clang fp contract(off)
+   const R Z = (R)0, HALF = (R)0.5;
+   R sql, sqr, isl, isr;
+   sqrt_rsq( L.d, sql, isl );
+   sqrt_rsq( Q.d, sqr, isr );
+   const R isum = rcp( sql + sqr );
+   const R el = KIND == 1 ? face_energy( L.d, L.u, L.a, L.b, L.e ) : L.e, er = KIND == 1 ? face_energy( Q.d, Q.u, Q.a, Q.b, Q.e ) : Q.e;
+   const R l1 = KIND == 1 ? L.d*L.a : L.a, l2 = KIND == 1 ? L.d*L.b : L.b, r1 = KIND == 1 ? Q.d*Q.a : Q.a, r2 = KIND == 1 ? Q.d*Q.b : Q.b;
+   const R ln = KIND == 2 ? L.mn : L.d*L.u, rn = KIND == 2 ? Q.mn : Q.d*Q.u;
+   const R u = isum*( KIND == 2 ? fmad( isl, ln, isr*rn ) : fmad( sql, L.u, sqr*Q.u ) );
+   const R v = isum*( KIND == 1 ? fmad( sql, L.a, sqr*Q.a ) : fmad( isl, L.a, isr*Q.a ) );
+   const R w = isum*( KIND == 1 ? fmad( sql, L.b, sqr*Q.b ) : fmad( isl, L.b, isr*Q.b ) );
+   const R V2h = HALF*fmad( w, w, fmad( v, v, u*u ) );
+   const R H  = isum*fmad( isl, el + L.p, isr*( er + Q.p ) );
+   // a^2 = (gamma-1)(H - V^2/2), its pressure a^2 rho/gamma floored as the reference does
+   const R g0 = P.gm1*( H - V2h ), irho = isl*isr, gmin = P.gamma*P.min_pres*irho;
+   const R a2 = floor_nan( g0, gmin );
+   R a, ia;
+   sqrt_rsq( a2, a, ia );
+   a = ( a2 == Z ) ? Z : a;
+   const R e0 = u - a, e4 = u + a;
+   if ( e0 >= Z || e4 <= Z )                                          // supersonic: the upwind side's flux
+   {
+      const bool left = ( e0 >= Z );
+      const R un = left ? L.u : Q.u, p = left ? L.p : Q.p;
+      f[0] = left ? ln : rn;
+      f[1] = fmad( f[0], un, p );
+      f[2] = un*( left ? l1 : r1 );
+      f[3] = un*( left ? l2 : r2 );
+      f[4] = un*( ( left ? el : er ) + p );
+      return;
+   }
+   const R j0 = Q.d - L.d, j1 = rn - ln, j2 = r1 - l1, j3 = r2 - l2, j4 = er - el;
+   const R a2_ = fmad( -v, j0, j2 ), a3_ = fmad( -w, j0, j3 );
+   const R a1_ = ( P.gm1*( ia*ia ) )*( fmad( j0, fmad( -u, u, H ), fmad( u, j1, -j4 ) ) + fmad( v, a2_, w*a3_ ) );
+   const R a0_ = ( HALF*ia )*( fmad( j0, e4, -j1 ) - a*a1_ );
+   const R a4_ = j0 - a0_ - a1_;
+   const R ua = u*a, hm = H - ua, hp = H + ua;
+   // intermediate states after the 1st and 4th waves (the degenerate middle waves are skipped)
+   const R d1 = L.d + a0_, m1 = fmad( a0_, e0, ln ), t1 = fmad( a0_, v, l1 ), t2 = fmad( a0_, w, l2 ), n1 = fmad( a0_, hm, el );
+   const R i1 = n1 - HALF*fmad( t2, t2, fmad( t1, t1, m1*m1 ) )*rcp( d1 );
+   const R d4 = d1 + a1_, m4 = fmad( a1_, u, m1 ), s4 = fmad( a1_, v, t1 ) + a2_, r4 = fmad( a1_, w, t2 ) + a3_,
+           n4 = fmad( a1_, V2h, n1 ) + fmad( a2_, v, a3_*w );
+   const R i4 = n4 - HALF*fmad( r4, r4, fmad( s4, s4, m4*m4 ) )*rcp( d4 );
+   if ( ( ( u > e0 ) && ( d1 <= Z || i1*P.gm1 <= Z ) ) || ( ( e4 > u ) && ( d4 <= Z || i4*P.gm1 <= Z ) ) )
+   {
+      hlle_flux<KIND>( L, Q, f );
+      return;
+   }
+   const R A0 = a0_*vabs( e0 ), A1 = a1_*vabs( u ), A2 = a2_*vabs( u ), A3 = a3_*vabs( u ), A4 = a4_*vabs( e4 ), S = A0 + A1 + A4;
+   f[0] = HALF*( ( ln + rn ) - S );
+   f[1] = HALF*( ( fmad( ln, L.u, L.p ) + fmad( rn, Q.u, Q.p ) ) - fmad( A0, e0, fmad( A1, u, A4*e4 ) ) );
+   f[2] = HALF*( fmad( L.u, l1, Q.u*r1 ) - fmad( S, v, A2 ) );
+   f[3] = HALF*( fmad( L.u, l2, Q.u*r2 ) - fmad( S, w, A3 ) );
+   f[4] = HALF*( fmad( L.u, el + L.p, Q.u*( er + Q.p ) ) - fmad( A0, hm, fmad( A1, V2h, fmad( A2, v, fmad( A3, w, A4*hp ) ) ) ) );
+}
+
+template <int RS, int KIND, typename R>
+__device__ __forceinline__ void solve_sides( const Side<R> &L, const Side<R> &Q, const Prm<R> &P, R f[NV] )
+{
    if ( RS == 4 )
    {
-      rs_hllc( L, Q, P.min_pres, f );
-      if ( any_nan5( f ) ) rs_hlle( L, Q, f );
+      hllc_flux<KIND>( L, Q, P.min_pres, f );
+      if ( any_nan5( f ) ) hlle_flux<KIND>( L, Q, f );                // RSOLVER_RESCUE
    }
-   else if ( RS == 3 ) rs_hlle( L, Q, f );
-   else                rs_roe( L, Q, P, f );
-   out[0] = f[0];
-   out[4] = f[4];
-   out[1] = dy ? f[3] : f[1];
-   out[2] = dy ? f[1] : f[2];
-   out[3] = dy ? f[2] : f[3];
+   else if ( RS == 3 ) hlle_flux<KIND>( L, Q, f );
+   else                roe_flux<KIND>( L, Q, P, f );
+}
+// flux across a D-normal interface, and across an x- or y-normal one chosen per lane, in the lab frame
+template <int RS, int D, int KIND, typename R>
+__device__ __forceinline__ void solve( const Side<R> &L, const Side<R> &Q, const Prm<R> &P, R out[NV] )
+{
+   R f[NV];
+   solve_sides<RS, KIND>( L, Q, P, f );
+   out[0] = f[0];  out[1 + D] = f[1];  out[1 + ( D + 1 ) % 3] = f[2];  out[1 + ( D + 2 ) % 3] = f[3];  out[4] = f[4];
+}
+template <int RS, int KIND, typename R>
+__device__ __forceinline__ void solve_xy( const Side<R> &L, const Side<R> &Q, const Prm<R> &P, bool dy, R out[NV] )
+{
+   R f[NV];
+   solve_sides<RS, KIND>( L, Q, P, f );
+   out[0] = f[0];  out[1] = dy ? f[3] : f[1];  out[2] = dy ? f[1] : f[2];  out[3] = dy ? f[2] : f[3];  out[4] = f[4];
+}
+
+// ---------------- PLM of the marching kernels ----------------
+// plm_face for all five fields of a cell.  VL_GMINMOD (LIM == 4) takes half slopes: h = sl sr / |sl + sr|, the limit
+// theta/2 min(|sl|, |sr|) from one min and one mul, and mirrors the left face C - h once, where the reference mirrors
+// it back too (the same up to one rounding); no clamp can act (see plm_face).  12 instructions a pair instead of 17.  The
+// run-time limiter is dispatched once per cell and direction, not per field.
+template <typename R>
+__device__ __forceinline__ void plm_pair4( R L, R C, R Rr, R coeff, R &fL, R &fR )
+{
+   #pragma clang fp contract(off)
+   const R sl = C - L, sr = Rr - C, t = sl + sr;
+   const R h = ( sl*sr )*rcp( vabs( t ) );
+   const R s = vcopysign( gminmod_mag( h, ( (R)0.5*coeff )*vmin( vabs( sl ), vabs( sr ) ) ), t );
+   fL = C - s;
+   fR = fmad( (R)2, C, -fL );
+}
+template <int L_, typename R>
+__device__ __forceinline__ void plm_cell_as( const R L[NV], const R C[NV], const R Rr[NV], R coeff, R fL[NV], R fR[NV] )
+{
+#  pragma unroll
+   for (int v=0; v<NV; v++)
+   {
+      const R s = plm_slope<L_>( C[v] - L[v], Rr[v] - C[v], (R)0, L_, coeff );
+      const R fl = clamp_between( C[v] - (R)0.5*s, C[v], L[v] );
+      fR[v] = clamp_between( (R)2.0*C[v] - fl, C[v], Rr[v] );
+      fL[v] = (R)2.0*C[v] - fR[v];
+   }
+}
+template <int LIM, typename R>
+__device__ __forceinline__ void plm_cell( const R L[NV], const R C[NV], const R Rr[NV], const Prm<R> &P, R fL[NV], R fR[NV] )
+{
+   if constexpr ( LIM == 4 )
+   {
+#     pragma unroll
+      for (int v=0; v<NV; v++) plm_pair4( L[v], C[v], Rr[v], P.coeff, fL[v], fR[v] );
+   }
+   else switch ( P.limiter )
+   {
+      case 1:  plm_cell_as<1>( L, C, Rr, P.coeff, fL, fR );  break;
+      case 2:  plm_cell_as<2>( L, C, Rr, P.coeff, fL, fR );  break;
+      case 3:  plm_cell_as<3>( L, C, Rr, P.coeff, fL, fR );  break;
+      case 4:  plm_cell_as<4>( L, C, Rr, P.coeff, fL, fR );  break;
+      default: plm_cell_as<6>( L, C, Rr, P.coeff, fL, fR );  break;
+   }
 }
 
 template <typename IO> struct IOLim;
@@ -550,25 +785,6 @@ __device__ __forceinline__ void pri2con( const R w[NV], R c[NV], const Prm<R> &P
    c[0] = w[0];
    c[1] = w[0]*w[1];  c[2] = w[0]*w[2];  c[3] = w[0]*w[3];
    c[4] = (R)0.5*( c[1]*c[1] + c[2]*c[2] + c[3]*c[3] )*rcp( w[0] ) + w[4]*P.inv_gm1;
-}
-
-// conserved face state -> interface state rotated to direction D, pressure recovered in FP64
-template <int D, typename R>
-__device__ __forceinline__ St<R> cons_state( const R c[NV], const Prm<R> &P )
-{
-   St<R> s;
-   const double eint = (double)c[4] - 0.5*( (double)c[1]*c[1] + (double)c[2]*c[2] + (double)c[3]*c[3] )
-                                      *rcp_pres<R>( (double)c[0] );
-   s.d  = c[0];
-   s.mn = c[1 + D];
-   s.m1 = c[1 + ( D + 1 ) % 3];
-   s.m2 = c[1 + ( D + 2 ) % 3];
-   s.e  = c[4];
-   s.p  = floor_pres( (R)( eint*P.gm1_d ), P.min_pres );
-   s.ir = rcp( c[0] );
-   s.u  = s.ir*s.mn;
-   s.cs = sound_speed( P.gamma*s.p, s.d, s.ir );
-   return s;
 }
 
 // max_d(|v_d| + c_s) of one cell, pressure recovered in FP64 (CPU_dtSolver_HydroCFL.cpp:104-190)

@@ -66,13 +66,14 @@ __device__ __forceinline__ void recon_cell( const R (*wl)[NC], int c, const R wm
                                             const R u0[NV], const Prm<R> &P, R fc[6][NV] )
 {
    R fp[6][NV];
+   R a[NV], b[NV];
 #  pragma unroll
-   for (int v=0; v<NV; v++)
-   {
-      plm_face<LIM>( wl[v][c - 1],  w0[v], wl[v][c + 1],  P.limiter, P.coeff, fp[0][v], fp[1][v] );
-      plm_face<LIM>( wl[v][c - NX], w0[v], wl[v][c + NX], P.limiter, P.coeff, fp[2][v], fp[3][v] );
-      plm_face<LIM>( wm[v],         w0[v], wp[v],         P.limiter, P.coeff, fp[4][v], fp[5][v] );
-   }
+   for (int v=0; v<NV; v++) { a[v] = wl[v][c - 1];  b[v] = wl[v][c + 1]; }
+   plm_cell<LIM>( a, w0, b, P, fp[0], fp[1] );
+#  pragma unroll
+   for (int v=0; v<NV; v++) { a[v] = wl[v][c - NX];  b[v] = wl[v][c + NX]; }
+   plm_cell<LIM>( a, w0, b, P, fp[2], fp[3] );
+   plm_cell<LIM>( wm, w0, wp, P, fp[4], fp[5] );
 #  pragma unroll
    for (int f=0; f<6; f++) pri2con( fp[f], fc[f], P );
    hancock<R, IO>( fc, fp, u0, P );
@@ -230,7 +231,7 @@ mhm_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restrict_
          R fzn[NV];
          if ( r >= 2 && r <= 18 )
          {
-            riemann<RS, 2>( cons_state<2>( kFzR, Q ), cons_state<2>( kF[4], Q ), Q, fzn );
+            solve<RS, 2, 2>( cons_side<2>( kFzR, Q ), cons_side<2>( kF[4], Q ), Q, fzn );
             if ( flx && ( r - 2 ) % 8 == 0 )
 #              pragma unroll
                for (int v=0; v<NV; v++)
@@ -246,21 +247,21 @@ mhm_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restrict_
             R fx[NV], fy[NV], fo[NV], q[NV];
 #           pragma unroll
             for (int v=0; v<NV; v++) q[v] = S.f[v][kc - 1];
-            riemann<RS, 0>( cons_state<0>( q, Q ), cons_state<0>( kF[0], Q ), Q, fx );
+            solve<RS, 0, 2>( cons_side<0>( q, Q ), cons_side<0>( kF[0], Q ), Q, fx );
 #           pragma unroll
             for (int v=0; v<NV; v++) q[v] = S.f[NV + v][kc - NX];
-            riemann<RS, 1>( cons_state<1>( q, Q ), cons_state<1>( kF[2], Q ), Q, fy );
+            solve<RS, 1, 2>( cons_side<1>( q, Q ), cons_side<1>( kF[2], Q ), Q, fy );
             if ( ofx )
             {
 #              pragma unroll
                for (int v=0; v<NV; v++) q[v] = S.f[v][oc - 1];
-               riemann<RS, 0>( cons_state<0>( q, Q ), cons_state<0>( oF[0], Q ), Q, fo );
+               solve<RS, 0, 2>( cons_side<0>( q, Q ), cons_side<0>( oF[0], Q ), Q, fo );
             }
             if ( ofy )
             {
 #              pragma unroll
                for (int v=0; v<NV; v++) q[v] = S.f[NV + v][oc - NX];
-               riemann<RS, 1>( cons_state<1>( q, Q ), cons_state<1>( oF[2], Q ), Q, fo );
+               solve<RS, 1, 2>( cons_side<1>( q, Q ), cons_side<1>( oF[2], Q ), Q, fo );
             }
 #           pragma unroll
             for (int v=0; v<NV; v++)

@@ -209,27 +209,13 @@ __device__ __forceinline__ void ld_cell( const R (*a)[NC], int c, R q[8] )
 }
 
 template <int D, typename R>
-__device__ __forceinline__ St<R> st_of( const R q[8] ) { return cell_state<D>( q, q[5], q[6], q[7] ); }
+__device__ __forceinline__ Side<R> side_at( const R (*a)[NC], int c ) { R q[8]; ld_cell( a, c, q ); return cell_side<D>( q ); }
 
-template <int D, typename R>
-__device__ __forceinline__ St<R> st_of( const R (*a)[NC], int c ) { R q[8]; ld_cell( a, c, q ); return st_of<D>( q ); }
-
-template <int D, typename R>
-__device__ __forceinline__ St<R> st_face( const R (*a)[NC], int v0, int c, const Prm<R> &P )
+template <int N, typename R>
+__device__ __forceinline__ void ld5( const R (*a)[N], int c, R w[NV] )
 {
-   R w[NV];
 #  pragma unroll
-   for (int v=0; v<NV; v++) w[v] = a[v0 + v][c];
-   return face_state<D>( w, P );
-}
-
-template <typename R>
-__device__ __forceinline__ St<R> st_face_xy( const R (*a)[NC], int v0, int c, bool dy, const Prm<R> &P )
-{
-   R w[NV];
-#  pragma unroll
-   for (int v=0; v<NV; v++) w[v] = a[v0 + v][c];
-   return face_state_xy( w, dy, P );
+   for (int v=0; v<NV; v++) w[v] = a[v][c];
 }
 
 // LDS of one workgroup
@@ -281,7 +267,6 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
    const int  fx_off = ( ( ( K.i - 3 )/8 )*NV*PS*PS + ( K.j - 3 ) )*(int)sizeof( IO );
    const int  fy_off = ( ( 3 + ( K.j - 3 )/8 )*NV*PS*PS + ( K.i - 3 ) )*(int)sizeof( IO );
    const int  fe_off = ( ( e_dy ? 5 : 2 )*NV*PS*PS + ( ( e_dy ? ei : ej ) - 3 ) )*(int)sizeof( IO );
-   const int  lim = P0.limiter;
 
    int base = 0;
    for (int item = 0; ; item++)
@@ -416,7 +401,7 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
             if ( doK && t >= 1 )
             {
                R fz[NV], w[NV];
-               riemann<RS, 2>( st_of<2>( kU1 ), st_of<2>( kU ), Q, fz );
+               solve<RS, 2, 0>( cell_side<2>( kU1 ), cell_side<2>( kU ), Q, fz );
                if ( t >= 2 )
                {
                   half_cell( kU1, kDh, kHz, fz, Q, w );
@@ -429,7 +414,7 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
             if ( arm_z )
             {
                R fz[NV];
-               riemann<RS, 2>( st_of<2>( oU1 ), st_of<2>( oU ), Q, fz );
+               solve<RS, 2, 0>( cell_side<2>( oU1 ), cell_side<2>( oU ), Q, fz );
                if ( t >= 4 ) half_cell( oU1, oDh, oHz, fz, Q, oW );
 #              pragma unroll
                for (int v=0; v<NV; v++) oHz[v] = fz[v];
@@ -439,8 +424,8 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
             R fkx[NV], fox[NV], fky[NV], foy[NV];
             if ( doK && t >= 1 && t <= 20 )
             {
-               riemann<RS, 0>( st_of<0>( S.a, K.c - 1 ), st_of<0>( kU ), Q, fkx );
-               riemann<RS, 1>( st_of<1>( S.a, K.c - NX ), st_of<1>( kU ), Q, fky );
+               solve<RS, 0, 0>( side_at<0>( S.a, K.c - 1 ), cell_side<0>( kU ), Q, fkx );
+               solve<RS, 1, 0>( side_at<1>( S.a, K.c - NX ), cell_side<1>( kU ), Q, fky );
 #              pragma unroll
                for (int v=0; v<NV; v++)
                {
@@ -450,8 +435,8 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
             }
             if ( arm_xy )
             {
-               riemann<RS, 0>( st_of<0>( S.a, O.c - 1 ), st_of<0>( oU ), Q, fox );
-               riemann<RS, 1>( st_of<1>( S.a, O.c - NX ), st_of<1>( oU ), Q, foy );
+               solve<RS, 0, 0>( side_at<0>( S.a, O.c - 1 ), cell_side<0>( oU ), Q, fox );
+               solve<RS, 1, 0>( side_at<1>( S.a, O.c - NX ), cell_side<1>( oU ), Q, foy );
 #              pragma unroll
                for (int v=0; v<NV; v++)
                {
@@ -468,7 +453,7 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
                   R ql[8], qr[8], ff[NV];
                   ld_cell( S.a, fc - ( fdy ? NX : 1 ), ql );
                   ld_cell( S.a, fc, qr );
-                  riemann_xy<RS>( cell_state_xy( ql, fdy ), cell_state_xy( qr, fdy ), Q, fdy, ff );
+                  solve_xy<RS, 0>( cell_side_xy( ql, fdy ), cell_side_xy( qr, fdy ), Q, fdy, ff );
 #                 pragma unroll
                   for (int v=0; v<NV; v++) S.b[( fdy ? NV : 0 ) + v][fc] = ff[v];
                }
@@ -479,27 +464,28 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
             R kFL[3][NV], kFRz[NV], eFL[NV];
             if ( doK && r >= 2 && r <= 19 )
             {
-#              pragma unroll
-               for (int v=0; v<NV; v++) plm_face<LIM>( kW3[v], kW2[v], kW1[v], lim, Q.coeff, kFL[2][v], kFRz[v] );
+               plm_cell<LIM>( kW3, kW2, kW1, Q, kFL[2], kFRz );
                if ( r >= 3 && r <= 18 )
+               {
+                  R a[NV], b[NV], fr[NV];
+                  ld5( S.w, K.c - 1, a );  ld5( S.w, K.c + 1, b );
+                  plm_cell<LIM>( a, kW2, b, Q, kFL[0], fr );
 #                 pragma unroll
-                  for (int v=0; v<NV; v++)
-                  {
-                     R fr;
-                     plm_face<LIM>( S.w[v][K.c - 1], kW2[v], S.w[v][K.c + 1], lim, Q.coeff, kFL[0][v], fr );
-                     S.f[v][K.c] = fr;
-                     plm_face<LIM>( S.w[v][K.c - NX], kW2[v], S.w[v][K.c + NX], lim, Q.coeff, kFL[1][v], fr );
-                     S.f[NV + v][K.c] = fr;
-                  }
+                  for (int v=0; v<NV; v++) S.f[v][K.c] = fr[v];
+                  ld5( S.w, K.c - NX, a );  ld5( S.w, K.c + NX, b );
+                  plm_cell<LIM>( a, kW2, b, Q, kFL[1], fr );
+#                 pragma unroll
+                  for (int v=0; v<NV; v++) S.f[NV + v][K.c] = fr[v];
+               }
             }
             if ( doG && has_e && r >= 3 && r <= 18 )
+            {
+               R a[NV], b[NV], c[NV], fr[NV];
+               ld5( S.w, e_c - e_st, a );  ld5( S.w, e_c, b );  ld5( S.w, e_c + e_st, c );
+               plm_cell<LIM>( a, b, c, Q, eFL, fr );
 #              pragma unroll
-               for (int v=0; v<NV; v++)
-               {
-                  R fr;
-                  plm_face<LIM>( S.w[v][e_c - e_st], S.w[v][e_c], S.w[v][e_c + e_st], lim, Q.coeff, eFL[v], fr );
-                  S.f[e_vo + v][e_c] = fr;
-               }
+               for (int v=0; v<NV; v++) S.f[e_vo + v][e_c] = fr[v];
+            }
             __syncthreads();                        // [H] half-step x/y fluxes visible; S.w plane r no longer read
             __builtin_amdgcn_s_setprio( 0 );
 
@@ -523,7 +509,7 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
             R fzn[NV];
             if ( doK && r >= 3 && r <= 19 )
             {
-               riemann<RS, 2>( face_state<2>( kFzR, Q ), face_state<2>( kFL[2], Q ), Q, fzn );
+               solve<RS, 2, 1>( face_side<2>( kFzR, Q ), face_side<2>( kFL[2], Q ), Q, fzn );
                if ( flx && ( r - 3 ) % 8 == 0 )
 #                 pragma unroll
                   for (int v=0; v<NV; v++)
@@ -539,9 +525,11 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
                __syncthreads();                     // [R] the half-step fluxes in S.b are read
                if constexpr ( doK )
                {
-                  R ffx[NV], ffy[NV];
-                  riemann<RS, 0>( st_face<0>( S.f, 0, K.c - 1, Q ), face_state<0>( kFL[0], Q ), Q, ffx );
-                  riemann<RS, 1>( st_face<1>( S.f, NV, K.c - NX, Q ), face_state<1>( kFL[1], Q ), Q, ffy );
+                  R ffx[NV], ffy[NV], q[NV];
+                  ld5( S.f, K.c - 1, q );
+                  solve<RS, 0, 1>( face_side<0>( q, Q ), face_side<0>( kFL[0], Q ), Q, ffx );
+                  ld5( S.f + NV, K.c - NX, q );
+                  solve<RS, 1, 1>( face_side<1>( q, Q ), face_side<1>( kFL[1], Q ), Q, ffy );
 #                 pragma unroll
                   for (int v=0; v<NV; v++)
                   {
@@ -562,8 +550,9 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
                }
                if ( doG && has_e && e_face )
                {
-                  R fe[NV];
-                  riemann_xy<RS>( st_face_xy( S.f, e_vo, e_c - e_st, e_dy, Q ), face_state_xy( eFL, e_dy, Q ), Q, e_dy, fe );
+                  R fe[NV], q[NV];
+                  ld5( S.f + e_vo, e_c - e_st, q );
+                  solve_xy<RS, 1>( face_side_xy( q, e_dy, Q ), face_side_xy( eFL, e_dy, Q ), Q, e_dy, fe );
 #                 pragma unroll
                   for (int v=0; v<NV; v++) S.b[e_vo + v][e_c] = fe[v];
                   if ( flx )                        // planes x = 16 (2) and y = 16 (5)
