@@ -18,14 +18,11 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-I" + os.path.join(ROOT, "include"), "-I" + CSRC,
 ]
-# per-source additions.  The MHM_RP kernels march z-planes with four barriers per plane; LLVM's iterative ILP
-# scheduler gives the 8-wave kernels a schedule that is 5.1% (FP32) and 9.1% (FP64) faster than the default one
-# and 11% / 4% faster than the max-ILP one (interleaved A/B on the 4096-PG workload).  The MHM file is compiled
-# once per precision: its FP32 kernels run fastest with the max-ILP scheduler (2.3% ahead of iterative ILP), its
-# FP64 kernels with iterative ILP (4.1% ahead of the default).  The adjoint, interpolation and sync sources crash
-# the compiler under these strategies and keep the default.
-EXTRA = {"hydro_mhm_rp.hip": ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
-         "hydro_mhm.hip:32": ["-DMHM_PRECISION=32", "-mllvm", "-amdgpu-sched-strategy=max-ilp"],
+# per-source additions.  The MHM file is compiled once per precision: its FP32 kernels run fastest with LLVM's max-ILP
+# scheduler (2.3% ahead of iterative ILP), its FP64 kernels with iterative ILP (4.1% ahead of the default).  The MHM_RP
+# kernels run fastest with the default scheduler in FP32 (532 against 538 us on 4096 patch groups) and the same with
+# both in FP64; the adjoint, interpolation and sync sources crash the compiler under these strategies.
+EXTRA = {"hydro_mhm.hip:32": ["-DMHM_PRECISION=32", "-mllvm", "-amdgpu-sched-strategy=max-ilp"],
          "hydro_mhm.hip:64": ["-DMHM_PRECISION=64", "-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]}
 
 

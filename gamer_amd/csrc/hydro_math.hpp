@@ -119,13 +119,12 @@ struct Prm {
 // Multi-level batch description: optional per-PG (dt, dh) pairs in device memory (uneven AMR batches, local
 // time steps) and an optional global work-queue counter for the persistent mode (each workgroup pulls tickets of
 // `claim` consecutive patch groups until the queue is exhausted).  pg_dt_dh == nullptr: every PG uses Prm's dt/dh;
-// counter == nullptr: one PG per workgroup.  `waves` selects the MHM_RP kernel's workgroup shape.
+// counter == nullptr: one PG per workgroup.
 struct Batch {
    const double *pg_dt_dh;
    unsigned     *counter;
    double        safety;
    int           claim;
-   int           waves;         // launch shape: 4 or 8 waves per workgroup, 0 = the kernel's default (host side only)
 };
 
 // an interface state rotated to the face normal: conserved fields + derived quantities
@@ -514,26 +513,43 @@ __device__ __forceinline__ R face_energy( R d, R u, R a, R b, R eint )
    return fmad( (R)0.5*d, fmad( b, b, fmad( a, a, u*u ) ), eint );
 }
 
-template <int KIND, typename R>
-__device__ __forceinline__ void hllc_flux( const Side<R> &L, const Side<R> &Q, R pmin, R f[NV] )
+// N interfaces at a time, one operation of all of them after the other: a solve is a chain of about 25 dependent
+// operations of 8 cycles each, and a wave that issues it alone fills half of its issue slots
+template <int KIND, int N, typename R>
+__device__ __forceinline__ void hllc_flux( const Side<R> L[N], const Side<R> Q[N], R pmin, R f[N][NV] )
 {
    #pragma clang fp contract(off)
    const R Z = (R)0;
-   const R wl = vmin( L.u - L.cs, Q.u - Q.cs ), wr = vmax( L.u + L.cs, Q.u + Q.cs );
-   const R tl = L.d*( L.u - wl ), tr = Q.d*( wr - Q.u );
-   const R x  = rcp( tl + tr )*fmad( tr, Q.u - L.u, L.p - Q.p );
-   const R vs = L.u + x;
-   const R ps = vmax( fmad( -tl, x, L.p ), pmin );                    // a NaN here is a NaN in vs too
-   const bool left = ( vs >= Z );
-   const R d = left ? L.d : Q.d, u = left ? L.u : Q.u, a = left ? L.a : Q.a, b = left ? L.b : Q.b,
-           p = left ? L.p : Q.p, e0 = left ? L.e : Q.e, mn = left ? L.mn : Q.mn;
-   const R sp = left ? vmin( wl, Z ) : vmax( wr, Z );
-   const R t  = rcp( vs - sp ), cf = t*vs, m = cf*( u - sp ), cp = cf*p, cs = -( t*sp )*ps, pp = cp + cs;
-   f[0] = KIND == 2 ? cf*fmad( -sp, d, mn ) : m*d;
-   f[1] = KIND == 2 ? fmad( m, mn, pp ) : fmad( f[0], u, pp );
-   f[2] = ( KIND == 1 ? f[0] : m )*a;
-   f[3] = ( KIND == 1 ? f[0] : m )*b;
-   f[4] = fmad( m, KIND == 1 ? face_energy( d, u, a, b, e0 ) : e0, fmad( cp, u, cs*vs ) );
+   R wl[N], wr[N], tl[N], tr[N], x[N], vs[N], ps[N], sp[N], t[N], m[N], cp[N], cs[N];
+   bool left[N];
+#  define GA_N _Pragma( "unroll" ) for (int n=0; n<N; n++)
+   GA_N { wl[n] = vmin( L[n].u - L[n].cs, Q[n].u - Q[n].cs );  wr[n] = vmax( L[n].u + L[n].cs, Q[n].u + Q[n].cs ); }
+   GA_N { tl[n] = L[n].d*( L[n].u - wl[n] );  tr[n] = Q[n].d*( wr[n] - Q[n].u ); }
+   GA_N x[n]  = rcp( tl[n] + tr[n] )*fmad( tr[n], Q[n].u - L[n].u, L[n].p - Q[n].p );
+   GA_N vs[n] = L[n].u + x[n];
+   GA_N ps[n] = vmax( fmad( -tl[n], x[n], L[n].p ), pmin );           // a NaN here is a NaN in vs too
+   GA_N left[n] = ( vs[n] >= Z );
+   GA_N sp[n] = left[n] ? vmin( wl[n], Z ) : vmax( wr[n], Z );
+   GA_N t[n]  = rcp( vs[n] - sp[n] );
+   R d[N], u[N], a[N], b[N], p[N], e[N], mn[N];
+   GA_N
+   {
+      d[n] = left[n] ? L[n].d : Q[n].d;  u[n] = left[n] ? L[n].u : Q[n].u;  a[n] = left[n] ? L[n].a : Q[n].a;
+      b[n] = left[n] ? L[n].b : Q[n].b;  p[n] = left[n] ? L[n].p : Q[n].p;  e[n] = left[n] ? L[n].e : Q[n].e;
+      mn[n] = left[n] ? L[n].mn : Q[n].mn;
+   }
+   GA_N if ( KIND == 1 ) e[n] = face_energy( d[n], u[n], a[n], b[n], e[n] );
+   GA_N { const R cf = t[n]*vs[n];  m[n] = cf*( u[n] - sp[n] );  cp[n] = cf*p[n];  cs[n] = -( t[n]*sp[n] )*ps[n];
+          f[n][0] = KIND == 2 ? cf*fmad( -sp[n], d[n], mn[n] ) : m[n]*d[n]; }
+   GA_N
+   {
+      const R pp = cp[n] + cs[n];
+      f[n][1] = KIND == 2 ? fmad( m[n], mn[n], pp ) : fmad( f[n][0], u[n], pp );
+      f[n][2] = ( KIND == 1 ? f[n][0] : m[n] )*a[n];
+      f[n][3] = ( KIND == 1 ? f[n][0] : m[n] )*b[n];
+      f[n][4] = fmad( m[n], e[n], fmad( cp[n], u[n], cs[n]*vs[n] ) );
+   }
+#  undef GA_N
 }
 
 template <int KIND, typename R>
@@ -620,31 +636,54 @@ __device__ __forceinline__ void roe_flux( const Side<R> &L, const Side<R> &Q, co
    f[4] = HALF*( fmad( L.u, el + L.p, Q.u*( er + Q.p ) ) - fmad( A0, hm, fmad( A1, V2h, fmad( A2, v, fmad( A3, w, A4*hp ) ) ) ) );
 }
 
-template <int RS, int KIND, typename R>
-__device__ __forceinline__ void solve_sides( const Side<R> &L, const Side<R> &Q, const Prm<R> &P, R f[NV] )
+// N solves in the rotated frames; they share one branch to the HLLE rescue of NaN fluxes (RSOLVER_RESCUE), so that
+// nothing separates them for the scheduler
+template <int RS, int KIND, int N, typename R>
+__device__ __forceinline__ void solve_n( const Side<R> L[N], const Side<R> Q[N], const Prm<R> &P, R f[N][NV] )
 {
    if ( RS == 4 )
    {
-      hllc_flux<KIND>( L, Q, P.min_pres, f );
-      if ( any_nan5( f ) ) hlle_flux<KIND>( L, Q, f );                // RSOLVER_RESCUE
+      hllc_flux<KIND, N>( L, Q, P.min_pres, f );
+      bool nan[N], any = false;
+#     pragma unroll
+      for (int n=0; n<N; n++) { nan[n] = any_nan5( f[n] );  any = any || nan[n]; }
+      if ( any )
+#        pragma unroll
+         for (int n=0; n<N; n++) if ( nan[n] ) hlle_flux<KIND>( L[n], Q[n], f[n] );
    }
-   else if ( RS == 3 ) hlle_flux<KIND>( L, Q, f );
-   else                roe_flux<KIND>( L, Q, P, f );
+   else
+#     pragma unroll
+      for (int n=0; n<N; n++)
+         if ( RS == 3 ) hlle_flux<KIND>( L[n], Q[n], f[n] );
+         else           roe_flux<KIND>( L[n], Q[n], P, f[n] );
 }
-// flux across a D-normal interface, and across an x- or y-normal one chosen per lane, in the lab frame
+// rotated flux -> lab frame, of a D-normal face and of an x- or y-normal one chosen per lane
+template <int D, typename R>
+__device__ __forceinline__ void to_lab( const R f[NV], R out[NV] )
+{
+   out[0] = f[0];  out[1 + D] = f[1];  out[1 + ( D + 1 ) % 3] = f[2];  out[1 + ( D + 2 ) % 3] = f[3];  out[4] = f[4];
+}
+template <typename R>
+__device__ __forceinline__ void to_lab_xy( const R f[NV], bool dy, R out[NV] )
+{
+   out[0] = f[0];  out[1] = dy ? f[3] : f[1];  out[2] = dy ? f[1] : f[2];  out[3] = dy ? f[2] : f[3];  out[4] = f[4];
+}
+// flux across a D-normal interface in the lab frame
 template <int RS, int D, int KIND, typename R>
 __device__ __forceinline__ void solve( const Side<R> &L, const Side<R> &Q, const Prm<R> &P, R out[NV] )
 {
-   R f[NV];
-   solve_sides<RS, KIND>( L, Q, P, f );
-   out[0] = f[0];  out[1 + D] = f[1];  out[1 + ( D + 1 ) % 3] = f[2];  out[1 + ( D + 2 ) % 3] = f[3];  out[4] = f[4];
+   const Side<R> l[1] = { L }, q[1] = { Q };
+   R f[1][NV];
+   solve_n<RS, KIND, 1>( l, q, P, f );
+   to_lab<D>( f[0], out );
 }
 template <int RS, int KIND, typename R>
 __device__ __forceinline__ void solve_xy( const Side<R> &L, const Side<R> &Q, const Prm<R> &P, bool dy, R out[NV] )
 {
-   R f[NV];
-   solve_sides<RS, KIND>( L, Q, P, f );
-   out[0] = f[0];  out[1] = dy ? f[3] : f[1];  out[2] = dy ? f[1] : f[2];  out[3] = dy ? f[2] : f[3];  out[4] = f[4];
+   const Side<R> l[1] = { L }, q[1] = { Q };
+   R f[1][NV];
+   solve_n<RS, KIND, 1>( l, q, P, f );
+   to_lab_xy( f[0], dy, out );
 }
 
 // ---------------- PLM of the marching kernels ----------------

@@ -1,37 +1,39 @@
 // MHM_RP (MUSCL-Hancock with Riemann-solver prediction) patch-group kernel for gfx950.
 //
-// One 256-lane workgroup updates one patch group: 22^3 input cells (16^3 interior + 3 ghost zones) ->
+// One 512-lane workgroup updates one patch group: 22^3 input cells (16^3 interior + 3 ghost zones) ->
 // 16^3 output cells + 9 coarse-fine flux planes.  The reference runs the same update as eight global-memory
 // phases over the whole 22^3 block (src/Model_Hydro/CPU_Hydro/CPU_FluidSolver_MHM.cpp:263-589, ~2.9 MB of
 // scratch per patch group in FP64).  Here the workgroup marches along z, one input plane per step, and keeps
 // every intermediate on chip:
 //
-//   * Lane t owns the output column (i,j) = (3 + t%16, 3 + output_row(t)).  Lanes 0-127 (waves 0-1) also own one
-//     "arm" ghost column for the half step (arm_column()), lanes 128-167 (wave 2) one single half-step face per
-//     plane (face_task()); together they update only the half-step cells the reconstruction reads.  Lanes
-//     192-255 (wave 3) each reconstruct one ghost column next to the output block along x or y, and half of them
-//     compute the full-step flux on the face between that column and the block (edge_column()).  Everything that
-//     couples planes along z — the previous input planes, the half-step z-flux, the last three half-step
-//     primitive planes, the lower z-face state and the last full-step z-flux — stays in the owning lane's
-//     registers.
-//   * Only x/y neighbours go through LDS, one plane at a time: the input plane with its pressure, 1/rho and
-//     sound speed, x and y fluxes (half step, then full step), the half-step primitive plane and the upper
-//     x/y face states.  A lane-private LDS ring keeps the input cells of the own output column for the planes
-//     between load and full-step update, so every input value is read from HBM once (148 KB of LDS per
-//     workgroup in FP64, 74 KB in FP32: two workgroups per CU).
+//   * Waves 0-3 (the column waves): lane t owns the output column (i,j) = (3 + t%16, 3 + output_row(t)), with
+//     everything that couples planes along z in its registers: the previous input plane, the half-step z-flux, the
+//     last three half-step primitive planes, the lower z-face state and the last full-step z-flux.  It does the
+//     column's z work, its y work and the updates.
+//   * Waves 4-7 (the side waves): lane g does the x reconstruction and the full-step x face of the column of lane g,
+//     which need no z history.  Besides, side waves 0-1 each own one "arm" ghost column of the half step
+//     (arm_column()); side waves 2-3 do the half-step x faces of two columns a lane; side wave 2 one single half-step
+//     face per plane (face_task()), side wave 3 one reconstructed column next to the block and half of its lanes the
+//     full-step face between the two (edge_column()); all of them stage the input planes.
+//   * x/y neighbours go through LDS, one plane at a time.  A lane-private LDS ring keeps the input cells of the
+//     output column for the planes between load and full-step update, so every input value is read from HBM once.
 //
-// Plane schedule at step t (input plane t just loaded; all indices in input coordinates), with the four
-// barriers of a step:
-//   [A] half-step z-flux at t-1/2, half-step cell update of plane t-1, half-step x/y fluxes of plane t,
-//       PLM reconstruction of plane r = t-2
-//   [H] x/y half-step flux differences of plane t, half-step plane t-1 into LDS
-//   [R] full-step fluxes of plane r (x/y) and at r-1/2 (z)
-//   [F] full-step update and output of plane t-3, input plane t+1 into LDS
-// [A] is the longest interval and waves 0-1 (arm half-step solves) its critical path; they raise their issue
-// priority inside it.  All branches that contain a barrier depend only on t, so every barrier is reached by the
-// whole workgroup.
-
-#include <type_traits>
+// Step t, input plane t staged (planes in input coordinates), with its two barriers:
+//   [A] half-step z-flux at t-1/2 and half-step cell of plane t-1, half-step x/y fluxes of plane t, PLM of plane
+//       r = t-2, x/y flux differences of plane t-3
+//   [H] x/y half-step flux differences of plane t, half-step plane t-1 into LDS, full-step fluxes of plane r (x/y) and
+//       at r-1/2 (z), full-step update and output of plane t-3, input plane t+1 into LDS
+// Every LDS array is written in one interval and read in the other.  All branches around the barriers depend only on
+// t, so every barrier is reached by the whole workgroup.
+//
+// What bounds it: a plane takes about 5,500 cycles (FP32), and a wave's chain of dependent operations (8 cycles each, 128
+// and more for an LDS read) is most of that at any occupancy; the vector units issue half of the time (FP64) or three
+// quarters (FP32).  So the work is split for the longest wave of each interval, by clock readings at the barriers:
+// [A] columns 2,600, arms 2,500, side waves 2-3 2,500; [H] 2,700 to 3,000.  The previous layout, with all x work on the
+// column waves and four barriers a plane, left the side waves waiting.  Nothing may spill in the loops: a reload, also
+// one placed in front of the loop, makes its first use wait for all outstanding prefetches and stores on every plane
+// (the same kernel with 80 instead of 16 bytes of scratch: 563 against 532 us).  On 4096 patch groups FP32 654 -> 528 us
+// (HLLE on 2048: 389 -> 249 before the cheaper solves of both), on 1331 FP64 516 -> 463 us.
 
 #include "hydro_math.hpp"
 #include "hydro_kernels.hpp"
@@ -44,19 +46,9 @@ constexpr int NX  = 22;          // FLU_NXT for MHM_RP
 constexpr int NC  = NX*NX;       // columns per plane
 constexpr int PS  = 16;          // PS2
 constexpr int NK  = 256;         // output columns (lanes of waves 0-3)
-#ifndef WPE32
-#define WPE32 2                  // target waves per SIMD (register budget) of the 4-wave FP32-bulk kernels
-#endif
-#ifndef WPE64
-#define WPE64 1                  // ... and of the 4-wave FP64 kernels
-#endif
-#ifndef WPE32_8
-#define WPE32_8 4                // ... of the 8-wave FP32-bulk kernels (two workgroups per CU)
-#endif
-#ifndef WPE64_8
-#define WPE64_8 2                // ... of the 8-wave FP64 kernels
-#endif
-
+constexpr int NT  = 512;         // lanes per workgroup
+constexpr int FS  = 18;          // LDS row stride of the full-step face arrays: rows 8 apart are 16 banks apart modulo 32
+constexpr int HX  = 20*NX, HY = 21*NX, FX = 16*FS, FY = 17*FS;
 
 // output row (j - 3) of lane t: wave w takes rows w, w+8, w+4, w+12, 16 lanes each.  The neighbour reads of a
 // plane in LDS (row stride NX = 22 words) then put the two rows of each half wave 176 words apart, 16 banks
@@ -70,15 +62,15 @@ __device__ __forceinline__ int output_row( int t )
 // The reconstruction reads half-step cells only in three slabs: the 16^2 output columns over z = 1..20, and the
 // "arm" columns (i or j in {1,2,19,20}, the other in 3..18) over z = 3..18 -- 7,168 of the 8,000 cells the
 // reference updates (CPU_FluidSolver_MHM.cpp:656-666 takes the whole 20^3 block).  Those cells need 22,656 of
-// its 25,200 half-step faces.  The ghost work of waves 0-2 is laid out so that each wave runs one task kind
+// its 25,200 half-step faces.  The ghost work of the side waves is laid out so that each wave runs one task kind
 // over one z range and skips the rest with wave-uniform branches:
-//   wave 0: the 64 arms next to the output block (i or j in {2,19}): half-step cell + low x and y faces
-//   wave 1: the 64 outer arms (i or j in {1,20}): the same
-//   wave 2: 40 single half-step faces (one x or y face per lane, read by an arm or output cell but owned by a
+//   side wave 0: the 64 arms next to the output block (i or j in {2,19}): half-step cell + low x and y faces
+//   side wave 1: the 64 outer arms (i or j in {1,20}): the same
+//   side wave 2: 40 single half-step faces (one x or y face per lane, read by an arm or output cell but owned by a
 //           column that is neither): the low x face of column (21,j) at z = 3..18 and of column (19,j) at the
 //           other planes, where the output cell (18,j) still needs it (and the y analogue); and the low x faces
 //           of (19, {1,2,19,20}) and low y faces of ({1,2,19,20}, 19) at z = 3..18
-// Arm column of lane t (waves 0-1); false = none.
+// Arm column of side lane t (side waves 0-1); false = none.
 __device__ __forceinline__ bool arm_column( int t, int &i, int &j )
 {
    if ( t >= 128 ) { i = j = 0;  return false; }
@@ -89,12 +81,11 @@ __device__ __forceinline__ bool arm_column( int t, int &i, int &j )
    return true;
 }
 
-// single half-step face of lane t (wave 2) at plane z: the column whose low face it is and whether the face is
-// y-normal; false = no face at this plane
-__device__ __forceinline__ bool face_task( int t, int z, int &c, bool &dy )
+// single half-step face of side lane t (side wave 2) at a plane (mid: a plane with arm cells): the column whose low
+// face it is and whether the face is y-normal; false = no face at this plane
+__device__ __forceinline__ bool face_task( int t, bool mid, int &c, bool &dy )
 {
    const int k = t - 128;
-   const bool mid = ( z >= 3 && z <= 18 );
    int i, j;
    dy = false;
    if ( k < 0 || k >= 40 ) return false;
@@ -117,8 +108,8 @@ __device__ __forceinline__ bool face_task( int t, int z, int &c, bool &dy )
    return true;
 }
 
-// ghost column next to the output block reconstructed by lane t of wave 3 (along y if dy), and whether the
-// lane also owns the full-step flux on the face between that column and the block (columns 19 only)
+// column next to the output block reconstructed by side lane t of side wave 3 (along y if dy): the columns 2 give the
+// left states of the block's first faces; the columns 19 own the full-step flux on the block's last face (face)
 __device__ __forceinline__ bool edge_column( int t, int &i, int &j, bool &dy, bool &face )
 {
    const int k = t - 192;
@@ -129,34 +120,6 @@ __device__ __forceinline__ bool edge_column( int t, int &i, int &j, bool &dy, bo
    i = dy ? b : a;
    j = dy ? a : b;
    return ( k >= 0 && k < 64 );
-}
-
-// roles of a column (i,j) of the 22x22 footprint
-struct Col {
-   int  c;                   // i + 22 j
-   bool w;                   // half-step cell (1..20)^2, owns the half-step z-face below it
-   bool hx, hy;              // owns the half-step x (y) face on its low side
-   bool rx, ry;              // needs x (y) reconstruction
-   bool fx, fy;              // owns the full-step x (y) face on its low side
-   bool core;                // output column (3..18)^2
-   int  i, j;
-};
-
-__device__ __forceinline__ Col make_col( int i, int j )
-{
-   Col k;
-   k.i = i;  k.j = j;  k.c = i + NX*j;
-   const bool ii = ( i >= 1 && i <= 20 ), jj = ( j >= 1 && j <= 20 );
-   k.w  = ii && jj;
-   k.hx = ( i >= 1 && i <= 21 ) && jj;
-   k.hy = ( j >= 1 && j <= 21 ) && ii;
-   const bool ci = ( i >= 3 && i <= 18 ), cj = ( j >= 3 && j <= 18 );
-   k.rx = ( i >= 2 && i <= 19 ) && cj;
-   k.ry = ( j >= 2 && j <= 19 ) && ci;
-   k.fx = ( i >= 3 && i <= 19 ) && cj;
-   k.fy = ( j >= 3 && j <= 19 ) && ci;
-   k.core = ci && cj;
-   return k;
 }
 
 // cell quantities of one input cell: conserved + pressure (recovered in FP64), 1/rho, sound speed
@@ -217,56 +180,50 @@ __device__ __forceinline__ void ld5( const R (*a)[N], int c, R w[NV] )
 #  pragma unroll
    for (int v=0; v<NV; v++) w[v] = a[v][c];
 }
+template <int N, typename R>
+__device__ __forceinline__ void st5( R (*a)[N], int c, const R w[NV] )
+{
+#  pragma unroll
+   for (int v=0; v<NV; v++) a[v][c] = w[v];
+}
 
-// LDS of one workgroup
+// LDS of one workgroup: 81,584 B (FP32, two workgroups per CU) or 163,160 B (FP64, one)
 template <typename R>
 struct SmemRP {
    R a[8][NC];                  // input plane (rho,mx,my,mz,E,P,1/rho,c_s)
-   R f[2*NV][NC];               // upper x (0-4) and y (5-9) face states of the reconstructed plane
-   R b[2*NV][NC];               // half-step or full-step x (0-4) and y (5-9) fluxes
-   R w[NV][NC];                 // half-step primitive plane read by the reconstruction
+   // x and y arrays of a field next to each other, so that a lane that does either adds one offset
+   R h[NV][HX + HY];            // half-step fluxes of the low x (from HX: y) face of column (i,j) at i + NX (j-1)
+   R l[NV][FX + FY];            // left states of the full-step x (from FX: y) faces: low face of column (i,j) at i-3 + FS (j-3)
+   R g[NV][FX + FY];            // full-step fluxes of those faces
+   R w[NV][HX];                 // half-step primitive plane read by the reconstruction, cell (i,j) at i + NX (j-1)
    R u3[3][NV][NK];             // lane-private ring: input cells of the own output column, planes t-3 .. t-1
    int fail, next;
-   R cfl[8][4];       // fused CFL: per-patch maxima of the 4 waves (R is the I/O type)
+   R cfl[8][4];                 // fused CFL: per-patch maxima of the 4 column waves (R is the I/O type)
 };
 
-// NW = 4: every lane owns an output column and one ghost role (waves 0-1 arms, wave 2 single faces, wave 3 edge
-// columns), both marched in one loop.  NW = 8: waves 0-3 own the output columns only and waves 4-7 the ghost
-// roles only (in the same wave order), each half in a loop of its own, so a lane keeps only its own half's z
-// history in registers and two waves share each SIMD.  Both layouts run the same per-cell arithmetic in the
-// same order, so their results are bitwise equal.
-template <typename R, typename IO, int RS, int LIM, bool PERSIST, int NW>
-__global__ void __launch_bounds__( 64*NW )
-__attribute__(( amdgpu_waves_per_eu( NW == 8 ? ( sizeof(R) == 4 ? WPE32_8 : WPE64_8 ) : ( sizeof(R) == 4 ? WPE32 : WPE64 ) ) ))
+template <typename R, typename IO, int RS, int LIM, bool PERSIST>
+__global__ void __launch_bounds__( NT ) __attribute__(( amdgpu_waves_per_eu( sizeof(R) == 4 ? 4 : 2 ) ))
 mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restrict__ g_flux,
                int npg, int store_flux, int minmod_maxiter, R minmod_coeff, Prm<R> P0,
                IO *__restrict__ g_dt, double dh_safety0, Batch B )
 {
    static_assert( sizeof( R ) == sizeof( IO ), "the input ring holds IO values in R storage" );
-   static_assert( NW == 4 || NW == 8, "4 or 8 waves per workgroup" );
    __shared__ SmemRP<R> S;
+   static_assert( sizeof( S ) <= ( sizeof( R ) == 4 ? 81920 : 163840 ), "two FP32 workgroups or one FP64 workgroup per CU" );
 
    const int tid  = threadIdx.x;
    const int wave = __builtin_amdgcn_readfirstlane( tid >> 6 );   // wave-uniform role switch
-   const int g    = ( NW == 4 ) ? tid : tid - 256;                // ghost-role index (0..255 on the ghost waves)
-   const int gw   = ( NW == 4 ) ? wave : wave - 4;                // ghost wave: 0-1 arms, 2 single faces, 3 edges
+   const int g    = tid - NK;                                     // side lane (0..255 on waves 4-7)
+   const int gw   = wave - 4;                                     // side wave: 0-1 arms, 2 single faces, 3 edges
 
-   const Col K = make_col( 3 + tid % PS, 3 + output_row( tid ) );
-   int oi, oj;
-   arm_column( g, oi, oj );
-   const Col O = make_col( oi, oj );
-   int ei, ej;
-   bool e_dy, e_face;
-   const bool has_e = edge_column( g, ei, ej, e_dy, e_face );
-   const int  e_c  = ei + NX*ej;
-   const int  e_st = e_dy ? NX : 1;             // neighbour stride of the edge column's direction
-   const int  e_vo = e_dy ? NV : 0;             // its face states / fluxes in S.f / S.b
+   // the lane's output column: column lane tid, or the one whose x work side lane g does
+   const int ki = 3 + ( tid & 15 ), kj = 3 + output_row( tid & ( NK - 1 ) );
+   const int kc = ki + NX*kj, kh = kc - NX, kq = ( ki - 3 ) + FS*( kj - 3 );   // in S.a, in S.h and S.w, in S.l and S.g
    // lane-constant byte offsets of the global stores: output column in a 16^2 plane, and the coarse-fine flux
-   // planes x = 0/8 (ffx), y = 0/8 (ffy) and x or y = 16 (edge lanes) at row K.j, K.i or the edge column
-   const int  kxy    = ( K.i - 3 ) + PS*( K.j - 3 );
-   const int  fx_off = ( ( ( K.i - 3 )/8 )*NV*PS*PS + ( K.j - 3 ) )*(int)sizeof( IO );
-   const int  fy_off = ( ( 3 + ( K.j - 3 )/8 )*NV*PS*PS + ( K.i - 3 ) )*(int)sizeof( IO );
-   const int  fe_off = ( ( e_dy ? 5 : 2 )*NV*PS*PS + ( ( e_dy ? ei : ej ) - 3 ) )*(int)sizeof( IO );
+   // planes x = 0/8 (fx), y = 0/8 (fy) and x or y = 16 (edge lanes) at row kj, ki or the edge column
+   const int  kxy    = ( ki - 3 ) + PS*( kj - 3 );
+   const int  fx_off = ( ( ( ki - 3 )/8 )*NV*PS*PS + ( kj - 3 ) )*(int)sizeof( IO );
+   const int  fy_off = ( ( 3 + ( kj - 3 )/8 )*NV*PS*PS + ( ki - 3 ) )*(int)sizeof( IO );
 
    int base = 0;
    for (int item = 0; ; item++)
@@ -308,6 +265,7 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
       const double dt = B.pg_dt_dh[2*pg], dh = B.pg_dt_dh[2*pg + 1];
       P.dt_dh2 = 0.5*dt/dh;  P.dt_dh = dt/dh;  dh_safety = B.safety*dh;
    }
+   constexpr int t0 = 0, t1 = NX - 1;          // first and last input plane of the march
 
    for (int iter = 0; ; iter++)
    {
@@ -318,26 +276,146 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
       }
       if ( tid == 0 ) S.fail = 0;
       IO cfl[2] = { (IO)0, (IO)0 };            // fused CFL: max(|v_d|+c_s) of this column in patches z=0,1
+      __syncthreads();                         // the previous patch group / iteration is done with the LDS arrays
 
-      // the z-march; DK: this lane runs its output column, DG: its ghost role (both compile-time)
-      auto march = [&]( auto DK, auto DG )
+      auto march_columns = [&]()
       {
-         constexpr bool doK = decltype( DK )::value, doG = decltype( DG )::value;
-         // lane state carried along z (output column K, half-step arm column O)
          R kU[8], kU1[8];                            // input cell of planes t and t-1 (+ pressure, 1/rho, c_s)
          R kHz[NV], kDh[NV];                         // half-step z-flux at t-3/2 ; half-step dFx+dFy of plane t-1
          R kW1[NV], kW2[NV], kW3[NV];                // half-step primitives of planes t-1, t-2, t-3
-         R kFzR[NV], kFz[NV], kDf[NV];               // upper z face of plane r-1 ; full z-flux at r-3/2 ; full dFx+dFy of plane r-1
-         R oU[8], oU1[8], oHz[NV], oDh[NV], oW[NV];  // arm column
+         R kFzR[NV], kFz[NV];                        // upper z face of plane r-1 ; full z-flux at r-3/2
 
-         // prefetch of the next input plane by the ghost-role lanes (two cells per lane, coalesced)
+         // two steps per iteration would rename the plane-to-plane register hand-offs instead of copying them, but spill
+         // (FP64 HLLC on 1331 patch groups 564 us, rolled 511)
+#        pragma unroll 1
+         for (int t = t0; t <= t1; t++)
+         {
+            const int o = t - 3;                     // output plane of this step
+            const int r = t - 2;                     // reconstructed plane of this step
+            __syncthreads();                         // [A] input plane t and the full-step fluxes of plane t-3 visible
+
+#           pragma unroll
+            for (int v=0; v<8; v++) kU1[v] = kU[v];
+            ld_cell( S.a, kc, kU );
+#           pragma unroll
+            for (int v=0; v<NV; v++) S.u3[( t + 2 ) % 3][v][tid] = kU1[v];     // plane t-1, read back at step t+2
+
+            R df[NV];                                // full-step dFx+dFy of plane o
+            if ( o >= t0 + 3 && o <= t1 - 3 )
+#              pragma unroll
+               for (int v=0; v<NV; v++) df[v] = ( S.g[v][kq + 1] - S.g[v][kq] ) + ( S.g[v][FX + kq + FS] - S.g[v][FX + kq] );
+
+            // half-step z-flux at t-1/2 and half-step cell of plane t-1
+            if ( t >= t0 + 1 )
+            {
+               R fz[NV], w[NV];
+               solve<RS, 2, 0>( cell_side<2>( kU1 ), cell_side<2>( kU ), Q, fz );
+               if ( t >= t0 + 2 )
+               {
+                  half_cell( kU1, kDh, kHz, fz, Q, w );
+#                 pragma unroll
+                  for (int v=0; v<NV; v++) { kW3[v] = kW2[v];  kW2[v] = kW1[v];  kW1[v] = w[v]; }
+               }
+#              pragma unroll
+               for (int v=0; v<NV; v++) kHz[v] = fz[v];
+            }
+            // half-step y flux of plane t
+            if ( t >= t0 + 1 && t <= t1 - 1 )
+            {
+               R f[NV];
+               solve<RS, 1, 0>( side_at<1>( S.a, kc - NX ), cell_side<1>( kU ), Q, f );
+               st5( S.h, HX + kh, f );
+            }
+            // PLM of plane r along z and y; the y neighbours come from the half-step plane r in S.w
+            R zL[NV], zR[NV], yL[NV];
+            if ( r >= t0 + 2 && r <= t1 - 2 )
+            {
+               plm_cell<LIM>( kW3, kW2, kW1, Q, zL, zR );
+               if ( r >= t0 + 3 && r <= t1 - 3 )
+               {
+                  R a[NV], b[NV], fr[NV];
+                  ld5( S.w, kh - NX, a );  ld5( S.w, kh + NX, b );
+                  plm_cell<LIM>( a, kW2, b, Q, yL, fr );
+                  st5( S.l, FX + kq + FS, fr );
+               }
+            }
+            __syncthreads();                         // [H] half-step fluxes and left states of plane r visible
+
+
+            if ( t >= t0 + 1 && t <= t1 - 1 )
+#              pragma unroll
+               for (int v=0; v<NV; v++) kDh[v] = ( S.h[v][kh + 1] - S.h[v][kh] ) + ( S.h[v][HX + kh + NX] - S.h[v][HX + kh] );
+            if ( t >= t0 + 2 ) st5( S.w, kh, kW1 );  // plane t-1 replaces plane t-2 for the next reconstruction
+
+            // full-step z-flux at r-1/2
+            R fz[NV];
+            if ( r >= t0 + 3 && r <= t1 - 2 )
+            {
+               solve<RS, 2, 1>( face_side<2>( kFzR, Q ), face_side<2>( zL, Q ), Q, fz );
+               if ( flx && ( r - 3 ) % 8 == 0 )
+#                 pragma unroll
+                  for (int v=0; v<NV; v++)
+                     buf_store( (IO)fz[v], b_flx, kxy*SZ, ( ( 6 + ( r - 3 )/8 )*NV + v )*PS*PS*SZ );
+            }
+            if ( r >= t0 + 2 )
+#              pragma unroll
+               for (int v=0; v<NV; v++) kFzR[v] = zR[v];
+            // full-step y-flux of plane r
+            if ( r >= t0 + 3 && r <= t1 - 3 )
+            {
+               R f[NV], q[NV];
+               ld5( S.l, FX + kq, q );
+               solve<RS, 1, 1>( face_side<1>( q, Q ), face_side<1>( yL, Q ), Q, f );
+               st5( S.g, FX + kq, f );
+               if ( flx && ( kj - 3 ) % 8 == 0 )
+#                 pragma unroll
+                  for (int v=0; v<NV; v++) buf_store( (IO)f[v], b_flx, fy_off, ( v*PS*PS + PS*( r - 3 ) )*SZ );
+            }
+            // full-step update and output of plane o
+            if ( o >= t0 + 3 && o <= t1 - 3 )
+            {
+               IO res[NV], uo[NV];
+               ld5( S.u3[t % 3], tid, uo );
+               const bool bad = full_cell( uo, df, kFz, fz, Q, res );
+#              pragma unroll
+               for (int v=0; v<NV; v++) buf_store( res[v], b_out, kxy*SZ, ( v*PS*PS*PS + PS*PS*( o - 3 ) )*SZ );
+               if ( bad ) S.fail = 1;
+               if ( g_dt ) cfl[ ( o - 3 )/8 ] = vmax( cfl[ ( o - 3 )/8 ], cell_cfl( res, (double)Q.gamma, Q.gm1_d, Q.min_pres_d ) );
+            }
+            if ( r >= t0 + 3 && r <= t1 - 2 )
+#              pragma unroll
+               for (int v=0; v<NV; v++) kFz[v] = fz[v];
+         }
+      };
+      auto march_sides = [&]()
+      {
+         int oi, oj, ei, ej;
+         bool e_dy, e_face;
+         arm_column( g, oi, oj );
+         const int  oc = oi + NX*oj, oh = oc - NX;
+         const bool has_e = edge_column( g, ei, ej, e_dy, e_face );
+         const int  eh = ei + NX*( ej - 1 );             // in S.w
+         const int  e_st = e_dy ? NX : 1;                // neighbour stride of the edge column's direction
+         // the edge column's face in S.l / S.g: the low face of a column 19, the high face of a column 2
+         const int  eq = e_dy ? FX + ( ei - 3 ) + FS*( e_face ? 16 : 0 ) : ( e_face ? 16 : 0 ) + FS*( ej - 3 );
+         const int  fe_off = ( ( e_dy ? 5 : 2 )*NV*PS*PS + ( ( e_dy ? ei : ej ) - 3 ) )*(int)sizeof( IO );
+         // single half-step face of the lane at the planes with arm cells (tm) and at the others (tn), -1 = none
+         int tm_c = -1, tn_c = -1;
+         bool t_dy = false, t_d2;
+         if ( !face_task( g, true, tm_c, t_dy ) ) tm_c = -1;
+         if ( !face_task( g, false, tn_c, t_d2 ) ) tn_c = -1;
+         // column of side waves 0-1 whose half-step x face this lane of side waves 2-3 does
+         const int k2 = ki + NX*( 3 + output_row( ( g & 63 ) + ( gw & 1 )*64 ) );
+         R oU[8], oU1[8], oHz[NV], oDh[NV], oW[NV];      // arm column: input cell of planes t, t-1, and as the output column
+
+         // prefetch of the next input plane, two cells per lane (coalesced)
          IO pf[2][NV];
          auto issue = [&]( int t )
          {
 #           pragma unroll
             for (int k=0; k<2; k++)
             {
-               const int c = g + k*256;
+               const int c = g + k*NK;
                if ( c < NC )
 #                 pragma unroll
                   for (int v=0; v<NV; v++) buf_load( b_in, c*SZ, ( v*NC*NX + t*NC )*SZ, pf[k][v] );
@@ -349,7 +427,7 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
 #           pragma unroll
             for (int k=0; k<2; k++)
             {
-               const int c = g + k*256;
+               const int c = g + k*NK;
                if ( c < NC )
                {
                   R q[8];
@@ -359,250 +437,117 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
                }
             }
          };
-         __syncthreads();                            // the previous patch group / iteration is done with S.a
-         if constexpr ( doG ) { issue( 0 );  stage();  issue( 1 ); }
+         issue( t0 );
+         stage();
+         issue( t0 + 1 );
 
-         // two steps per iteration let the compiler rename the plane-to-plane register hand-offs (kU1 = kU, the
-         // z-flux and face carries) instead of copying them; the Roe kernels stay rolled, their code is twice as large,
-         // and so does the 8-wave FP32-bulk kernel, whose 128-register budget the unrolled schedule exceeds more
-#        pragma unroll ( RS != 2 && ( NW == 4 || sizeof( R ) == 8 ) ? 2 : 1 )
-         for (int t = 0; t < NX; t++)
+#        pragma unroll 1
+         for (int t = t0; t <= t1; t++)
          {
-            const int o = t - 3;                    // output plane of this step
-            const int r = t - 2;                    // reconstructed plane of this step
-            const int ring = t % 3;                 // u3 slot of input plane t-3 (read at the update); plane t-1
-                                                    // goes into slot (t+2) % 3 as soon as it leaves S.a
-            __syncthreads();                        // [A] input plane t visible
-            // the longest work of this interval issues first: with 4 waves the arm waves 0-1 (output column and
-            // arm half step), with 8 the output-column waves 0-3; the others issue behind them
-            if ( NW == 4 ? wave < 2 : wave < 4 ) __builtin_amdgcn_s_setprio( 3 ); else __builtin_amdgcn_s_setprio( 1 );
-            // arm half step: cells of planes 3..18 (updated at steps 4..19), their z faces (steps 3..19) and their
-            // low x/y faces (planes 3..18)
-            const bool arm_ld = doG && ( gw < 2 ) && t >= 2 && t <= 19;
-            const bool arm_z  = doG && ( gw < 2 ) && t >= 3 && t <= 19;
-            const bool arm_xy = doG && ( gw < 2 ) && t >= 3 && t <= 18;
-
-            if constexpr ( doK )
-            {
-#              pragma unroll
-               for (int v=0; v<8; v++) kU1[v] = kU[v];
-               ld_cell( S.a, K.c, kU );
-#              pragma unroll
-               for (int v=0; v<NV; v++) S.u3[( t + 2 ) % 3][v][tid] = kU1[v];     // read back at step t+2
-            }
-            if constexpr ( doG )
-            {
-#              pragma unroll
-               for (int v=0; v<8; v++) oU1[v] = oU[v];
-               if ( arm_ld ) ld_cell( S.a, O.c, oU );
-            }
-
-            // ---- half-step z-flux at t-1/2 and half-step cell update of plane t-1
-            if ( doK && t >= 1 )
-            {
-               R fz[NV], w[NV];
-               solve<RS, 2, 0>( cell_side<2>( kU1 ), cell_side<2>( kU ), Q, fz );
-               if ( t >= 2 )
-               {
-                  half_cell( kU1, kDh, kHz, fz, Q, w );
-#                 pragma unroll
-                  for (int v=0; v<NV; v++) { kW3[v] = kW2[v];  kW2[v] = kW1[v];  kW1[v] = w[v]; }
-               }
-#              pragma unroll
-               for (int v=0; v<NV; v++) kHz[v] = fz[v];
-            }
+            const int r = t - 2;
+            __syncthreads();                         // [A]
+            // arm half step: cells of planes t0+3 .. t1-3 (updated one step later), their z faces and low x/y faces
+            const bool arm_ld = ( gw < 2 ) && t >= t0 + 2 && t <= t1 - 2;
+            const bool arm_z  = ( gw < 2 ) && t >= t0 + 3 && t <= t1 - 2;
+            const bool arm_xy = ( gw < 2 ) && t >= t0 + 3 && t <= t1 - 3;
+#           pragma unroll
+            for (int v=0; v<8; v++) oU1[v] = oU[v];
+            if ( arm_ld ) ld_cell( S.a, oc, oU );
             if ( arm_z )
             {
                R fz[NV];
                solve<RS, 2, 0>( cell_side<2>( oU1 ), cell_side<2>( oU ), Q, fz );
-               if ( t >= 4 ) half_cell( oU1, oDh, oHz, fz, Q, oW );
+               if ( t >= t0 + 4 ) half_cell( oU1, oDh, oHz, fz, Q, oW );
 #              pragma unroll
                for (int v=0; v<NV; v++) oHz[v] = fz[v];
             }
-
-            // ---- half-step x and y fluxes of plane t (low face owned by each column)
-            R fkx[NV], fox[NV], fky[NV], foy[NV];
-            if ( doK && t >= 1 && t <= 20 )
-            {
-               solve<RS, 0, 0>( side_at<0>( S.a, K.c - 1 ), cell_side<0>( kU ), Q, fkx );
-               solve<RS, 1, 0>( side_at<1>( S.a, K.c - NX ), cell_side<1>( kU ), Q, fky );
-#              pragma unroll
-               for (int v=0; v<NV; v++)
-               {
-                  S.b[v][K.c] = fkx[v];
-                  S.b[NV + v][K.c] = fky[v];
-               }
-            }
             if ( arm_xy )
             {
-               solve<RS, 0, 0>( side_at<0>( S.a, O.c - 1 ), cell_side<0>( oU ), Q, fox );
-               solve<RS, 1, 0>( side_at<1>( S.a, O.c - NX ), cell_side<1>( oU ), Q, foy );
-#              pragma unroll
-               for (int v=0; v<NV; v++)
-               {
-                  S.b[v][O.c] = fox[v];
-                  S.b[NV + v][O.c] = foy[v];
-               }
+               const Side<R> l[2] = { side_at<0>( S.a, oc - 1 ), side_at<1>( S.a, oc - NX ) }, q[2] = { cell_side<0>( oU ), cell_side<1>( oU ) };
+               R f[2][NV], ox[NV], oy[NV];
+               solve_n<RS, 0, 2>( l, q, Q, f );
+               to_lab<0>( f[0], ox );  to_lab<1>( f[1], oy );
+               st5( S.h, oh, ox );
+               st5( S.h, HX + oh, oy );
             }
-            if ( doG && gw == 2 && t >= 1 && t <= 20 )
+            if ( gw == 2 && t >= t0 + 1 && t <= t1 - 1 )
             {
-               int fc;
-               bool fdy;
-               if ( face_task( g, t, fc, fdy ) )
+               const bool fdy = t_dy;
+               const int  fc = ( t >= t0 + 3 && t <= t1 - 3 ) ? tm_c : tn_c;
+               if ( fc >= 0 )
                {
-                  R ql[8], qr[8], ff[NV];
+                  R ql[8], qr[8], f[NV];
                   ld_cell( S.a, fc - ( fdy ? NX : 1 ), ql );
                   ld_cell( S.a, fc, qr );
-                  solve_xy<RS, 0>( cell_side_xy( ql, fdy ), cell_side_xy( qr, fdy ), Q, fdy, ff );
-#                 pragma unroll
-                  for (int v=0; v<NV; v++) S.b[( fdy ? NV : 0 ) + v][fc] = ff[v];
+                  solve_xy<RS, 0>( cell_side_xy( ql, fdy ), cell_side_xy( qr, fdy ), Q, fdy, f );
+                  st5( S.h, ( fdy ? HX - NX : -NX ) + fc, f );
                }
             }
-
-            // ---- PLM reconstruction of plane r (x/y upper faces to LDS, z faces stay in the lane); the x/y
-            //      neighbours come from the half-step plane r in S.w
-            R kFL[3][NV], kFRz[NV], eFL[NV];
-            if ( doK && r >= 2 && r <= 19 )
+            // half-step x fluxes of plane t
+            if ( gw >= 2 && t >= t0 + 1 && t <= t1 - 1 )
             {
-               plm_cell<LIM>( kW3, kW2, kW1, Q, kFL[2], kFRz );
-               if ( r >= 3 && r <= 18 )
-               {
-                  R a[NV], b[NV], fr[NV];
-                  ld5( S.w, K.c - 1, a );  ld5( S.w, K.c + 1, b );
-                  plm_cell<LIM>( a, kW2, b, Q, kFL[0], fr );
-#                 pragma unroll
-                  for (int v=0; v<NV; v++) S.f[v][K.c] = fr[v];
-                  ld5( S.w, K.c - NX, a );  ld5( S.w, K.c + NX, b );
-                  plm_cell<LIM>( a, kW2, b, Q, kFL[1], fr );
-#                 pragma unroll
-                  for (int v=0; v<NV; v++) S.f[NV + v][K.c] = fr[v];
-               }
+               const Side<R> l[2] = { side_at<0>( S.a, kc - 1 ), side_at<0>( S.a, k2 - 1 ) }, q[2] = { side_at<0>( S.a, kc ), side_at<0>( S.a, k2 ) };
+               R f[2][NV], fx[NV], f2[NV];
+               solve_n<RS, 0, 2>( l, q, Q, f );
+               to_lab<0>( f[0], fx );  to_lab<0>( f[1], f2 );
+               st5( S.h, kh, fx );
+               st5( S.h, k2 - NX, f2 );
             }
-            if ( doG && has_e && r >= 3 && r <= 18 )
+            // PLM of plane r along x, and of the edge column
+            R xL[NV], eL[NV];
+            if ( r >= t0 + 3 && r <= t1 - 3 )
             {
                R a[NV], b[NV], c[NV], fr[NV];
-               ld5( S.w, e_c - e_st, a );  ld5( S.w, e_c, b );  ld5( S.w, e_c + e_st, c );
-               plm_cell<LIM>( a, b, c, Q, eFL, fr );
-#              pragma unroll
-               for (int v=0; v<NV; v++) S.f[e_vo + v][e_c] = fr[v];
-            }
-            __syncthreads();                        // [H] half-step x/y fluxes visible; S.w plane r no longer read
-            __builtin_amdgcn_s_setprio( 0 );
-
-            // flux differences; the lane's own low-face fluxes are read back from LDS rather than held in registers
-            // across the reconstruction (the stored values, so both launch shapes round alike)
-            if ( doK && t >= 1 && t <= 20 )
-#              pragma unroll
-               for (int v=0; v<NV; v++) kDh[v] = ( S.b[v][K.c + 1] - S.b[v][K.c] ) + ( S.b[NV + v][K.c + NX] - S.b[NV + v][K.c] );
-            if ( arm_xy )
-#              pragma unroll
-               for (int v=0; v<NV; v++) oDh[v] = ( S.b[v][O.c + 1] - S.b[v][O.c] ) + ( S.b[NV + v][O.c + NX] - S.b[NV + v][O.c] );
-            // the half-step plane t-1 replaces plane t-2 in LDS for the next reconstruction
-            if ( doK && t >= 2 )
-#              pragma unroll
-               for (int v=0; v<NV; v++) S.w[v][K.c] = kW1[v];
-            if ( arm_z && t >= 4 )
-#              pragma unroll
-               for (int v=0; v<NV; v++) S.w[v][O.c] = oW[v];
-
-            // ---- full-step fluxes: z at r-1/2 (lane-local), x and y of plane r through LDS
-            R fzn[NV];
-            if ( doK && r >= 3 && r <= 19 )
-            {
-               solve<RS, 2, 1>( face_side<2>( kFzR, Q ), face_side<2>( kFL[2], Q ), Q, fzn );
-               if ( flx && ( r - 3 ) % 8 == 0 )
-#                 pragma unroll
-                  for (int v=0; v<NV; v++)
-                     buf_store( (IO)fzn[v], b_flx, kxy*SZ, ( ( 6 + ( r - 3 )/8 )*NV + v )*PS*PS*SZ );
-            }
-            if ( doK && r >= 2 )
-#              pragma unroll
-               for (int v=0; v<NV; v++) kFzR[v] = kFRz[v];
-
-            R dfn[NV];
-            if ( r >= 3 && r <= 18 )
-            {
-               __syncthreads();                     // [R] the half-step fluxes in S.b are read
-               if constexpr ( doK )
+               ld5( S.w, kh - 1, a );  ld5( S.w, kh, b );  ld5( S.w, kh + 1, c );
+               plm_cell<LIM>( a, b, c, Q, xL, fr );
+               st5( S.l, kq + 1, fr );
+               if ( has_e )
                {
-                  R ffx[NV], ffy[NV], q[NV];
-                  ld5( S.f, K.c - 1, q );
-                  solve<RS, 0, 1>( face_side<0>( q, Q ), face_side<0>( kFL[0], Q ), Q, ffx );
-                  ld5( S.f + NV, K.c - NX, q );
-                  solve<RS, 1, 1>( face_side<1>( q, Q ), face_side<1>( kFL[1], Q ), Q, ffy );
-#                 pragma unroll
-                  for (int v=0; v<NV; v++)
-                  {
-                     S.b[v][K.c] = ffx[v];
-                     S.b[NV + v][K.c] = ffy[v];
-                  }
-                  if ( flx )
-                  {
-                     if ( ( K.i - 3 ) % 8 == 0 )
-#                       pragma unroll
-                        for (int v=0; v<NV; v++)
-                           buf_store( (IO)ffx[v], b_flx, fx_off, ( v*PS*PS + PS*( r - 3 ) )*SZ );
-                     if ( ( K.j - 3 ) % 8 == 0 )
-#                       pragma unroll
-                        for (int v=0; v<NV; v++)
-                           buf_store( (IO)ffy[v], b_flx, fy_off, ( v*PS*PS + PS*( r - 3 ) )*SZ );
-                  }
+                  ld5( S.w, eh - e_st, a );  ld5( S.w, eh, b );  ld5( S.w, eh + e_st, c );
+                  plm_cell<LIM>( a, b, c, Q, eL, fr );
+                  if ( !e_face ) st5( S.l, eq, fr );
                }
-               if ( doG && has_e && e_face )
-               {
-                  R fe[NV], q[NV];
-                  ld5( S.f + e_vo, e_c - e_st, q );
-                  solve_xy<RS, 1>( face_side_xy( q, e_dy, Q ), face_side_xy( eFL, e_dy, Q ), Q, e_dy, fe );
-#                 pragma unroll
-                  for (int v=0; v<NV; v++) S.b[e_vo + v][e_c] = fe[v];
-                  if ( flx )                        // planes x = 16 (2) and y = 16 (5)
-#                    pragma unroll
-                     for (int v=0; v<NV; v++)
-                        buf_store( (IO)fe[v], b_flx, fe_off, ( v*PS*PS + PS*( r - 3 ) )*SZ );
-               }
-               __syncthreads();                     // [F] full-step fluxes visible
-               if constexpr ( doK )                 // own fluxes read back, as for the half step
-#                 pragma unroll
-                  for (int v=0; v<NV; v++) dfn[v] = ( S.b[v][K.c + 1] - S.b[v][K.c] ) + ( S.b[NV + v][K.c + NX] - S.b[NV + v][K.c] );
             }
+            __syncthreads();                         // [H]
 
-            if constexpr ( doK )
-            {
-               // ---- full-step update and output of plane o = t-3
-               if ( o >= 3 && o <= 18 )
-               {
-                  IO res[NV], uo[NV];
-#                 pragma unroll
-                  for (int v=0; v<NV; v++) uo[v] = S.u3[ring][v][tid];
-                  const bool bad = full_cell( uo, kDf, kFz, fzn, Q, res );
-#                 pragma unroll
-                  for (int v=0; v<NV; v++) buf_store( res[v], b_out, kxy*SZ, ( v*PS*PS*PS + PS*PS*( o - 3 ) )*SZ );
-                  if ( bad ) S.fail = 1;
-                  if ( g_dt ) cfl[ ( o - 3 )/8 ] = vmax( cfl[ ( o - 3 )/8 ], cell_cfl( res, (double)Q.gamma, Q.gm1_d, Q.min_pres_d ) );
-               }
-               if ( r >= 3 && r <= 19 )
-#                 pragma unroll
-                  for (int v=0; v<NV; v++) kFz[v] = fzn[v];
-               if ( r >= 3 && r <= 18 )
-#                 pragma unroll
-                  for (int v=0; v<NV; v++) kDf[v] = dfn[v];
-            }
 
-            // ---- input plane t+1 into LDS: every read of S.a of this step came before barrier [H]
-            if ( doG && t + 1 < NX )
+            // input plane t+1 into LDS: every read of S.a of this step came before barrier [H].  First, as the wait for its
+            // loads would also wait for the flux stores below
+            if ( t + 1 <= t1 )
             {
                stage();
-               if ( t + 2 < NX ) issue( t + 2 );
+               if ( t + 2 <= t1 ) issue( t + 2 );
             }
-         } // for t
-      };
-      using T_ = std::integral_constant<bool, true>;
-      using F_ = std::integral_constant<bool, false>;
-      if constexpr ( NW == 4 ) march( T_(), T_() );
-      else if ( wave < 4 )     march( T_(), F_() );
-      else                     march( F_(), T_() );
+            if ( arm_xy )
+#              pragma unroll
+               for (int v=0; v<NV; v++) oDh[v] = ( S.h[v][oh + 1] - S.h[v][oh] ) + ( S.h[v][HX + oh + NX] - S.h[v][HX + oh] );
+            if ( arm_z && t >= t0 + 4 ) st5( S.w, oh, oW );
 
-      if ( g_dt ) fused_dt( cfl, ( K.i - 3 )/8 + 2*( ( K.j - 3 )/8 ), S.cfl, g_dt + (size_t)pg*8, dh_safety );
+            // full-step x-flux of plane r, and the faces x = 16 and y = 16 of the block
+            if ( r >= t0 + 3 && r <= t1 - 3 )
+            {
+               R f[NV], q[NV];
+               ld5( S.l, kq, q );
+               solve<RS, 0, 1>( face_side<0>( q, Q ), face_side<0>( xL, Q ), Q, f );
+               st5( S.g, kq, f );
+               if ( flx && ( ki - 3 ) % 8 == 0 )
+#                 pragma unroll
+                  for (int v=0; v<NV; v++) buf_store( (IO)f[v], b_flx, fx_off, ( v*PS*PS + PS*( r - 3 ) )*SZ );
+               if ( has_e && e_face )
+               {
+                  ld5( S.l, eq, q );
+                  solve_xy<RS, 1>( face_side_xy( q, e_dy, Q ), face_side_xy( eL, e_dy, Q ), Q, e_dy, f );
+                  st5( S.g, eq, f );
+                  if ( flx )                         // planes x = 16 (2) and y = 16 (5)
+#                    pragma unroll
+                     for (int v=0; v<NV; v++) buf_store( (IO)f[v], b_flx, fe_off, ( v*PS*PS + PS*( r - 3 ) )*SZ );
+               }
+            }
+         }
+      };
+      if ( wave < 4 ) march_columns(); else march_sides();
+
+      if ( g_dt ) fused_dt( cfl, ( ki - 3 )/8 + 2*( ( kj - 3 )/8 ), S.cfl, g_dt + (size_t)pg*8, dh_safety );
       __syncthreads();
       const bool redo = ( S.fail != 0 ) && ( iter + 1 <= minmod_maxiter );
       __syncthreads();
@@ -617,15 +562,12 @@ template <typename R, typename IO, int RS>
 static void launch_rs( const IO *in, IO *out, IO *flux, int npg, int store_flux, int minmod_maxiter,
                        double minmod_coeff, const Prm<R> &P, IO *dt, double dh_safety, const Batch &B, int grid_blocks, hipStream_t stream )
 {
-   const int nw = ( B.waves == 4 ) ? 4 : 8;
-   const dim3 grid( grid_blocks > 0 ? grid_blocks : npg ), block( 64*nw );
+   const dim3 grid( grid_blocks > 0 ? grid_blocks : npg ), block( NT );
    const bool pers = ( B.counter != nullptr );
-#  define GA_LAUNCH( LIM_, PERS_, NW_ ) hipLaunchKernelGGL( ( mhm_rp_kernel<R, IO, RS, LIM_, PERS_, NW_> ), grid, block, 0, stream, \
-                                                           in, out, flux, npg, store_flux, minmod_maxiter, (R)minmod_coeff, P, dt, dh_safety, B )
-#  define GA_SHAPE( LIM_, PERS_ ) { if ( nw == 4 ) GA_LAUNCH( LIM_, PERS_, 4 ); else GA_LAUNCH( LIM_, PERS_, 8 ); }
-   if ( kernel_limiter( P.limiter, minmod_coeff ) == 4 ) { if ( pers ) GA_SHAPE( 4, true ) else GA_SHAPE( 4, false ) }
-   else                  { if ( pers ) GA_SHAPE( 0, true ) else GA_SHAPE( 0, false ) }
-#  undef GA_SHAPE
+#  define GA_LAUNCH( LIM_, PERS_ ) hipLaunchKernelGGL( ( mhm_rp_kernel<R, IO, RS, LIM_, PERS_> ), grid, block, 0, stream, \
+                                                      in, out, flux, npg, store_flux, minmod_maxiter, (R)minmod_coeff, P, dt, dh_safety, B )
+   if ( kernel_limiter( P.limiter, minmod_coeff ) == 4 ) { if ( pers ) GA_LAUNCH( 4, true ); else GA_LAUNCH( 4, false ); }
+   else                  { if ( pers ) GA_LAUNCH( 0, true ); else GA_LAUNCH( 0, false ); }
 #  undef GA_LAUNCH
 }
 

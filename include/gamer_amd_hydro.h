@@ -57,9 +57,9 @@ typedef struct HydroSolveArgs {
    void  *dt_patch;        /* optional device pointer [npg][8]: fused CFL dt of the updated patches
                               (index px + 2 py + 4 pz within the PG); NULL = not computed */
    double safety;          /* CFL safety factor of the fused dt (DT__FLUID) */
-   int    waves_per_group; /* launch shape of the MHM_RP kernel: 0 = default (8), 4 or 8 waves per workgroup
-                              (results are bitwise equal); MHM accepts 0 or 4.  No counterpart in the reference,
-                              whose block size is a compile-time constant (include/CUFLU.h:302-371). */
+   int    waves_per_group; /* requested launch shape: 0, 4 or 8 for MHM_RP, 0 or 4 for MHM.  Each scheme has one shape
+                              (MHM_RP 8 waves per workgroup, MHM 4), which every accepted value runs.  No counterpart in
+                              the reference, whose block size is a compile-time constant (include/CUFLU.h:302-371). */
 } HydroSolveArgs;
 
 /* Select the HIP device (replaces CUAPI_SetDevice, src/GPU_API/CUAPI_SetDevice.cu). */
