@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstring>
 #include <cstdarg>
+#include <atomic>
 #include <vector>
 #include <mutex>
 
@@ -125,7 +126,7 @@ Prm<R> make_prm( const HydroSolveArgs *a )
 int enqueue( const HydroSolveArgs *a, const void *in, void *out, void *flux, void *dt, int npg, hipStream_t s,
              const Batch *batch = nullptr, int grid_blocks = 0 )
 {
-   Batch B;
+   Batch B = {};
    if ( batch ) B = *batch;
    else { B.pg_dt_dh = nullptr;  B.counter = nullptr;  B.safety = 0.0;  B.claim = 1; }
    int rc;
@@ -162,6 +163,22 @@ void free_buffers()
 }
 
 } // namespace
+
+namespace gamer_amd {
+
+// compute units of the current device (a constant of the device, looked up once)
+int device_cus()
+{
+   static std::atomic<int> cus[MAX_DEVICES];
+   int dev = 0, n = 0;
+   if ( hipGetDevice( &dev ) != hipSuccess || dev < 0 || dev >= MAX_DEVICES ) return 0;
+   n = cus[dev].load( std::memory_order_relaxed );
+   if ( n == 0 && hipDeviceGetAttribute( &n, hipDeviceAttributeMultiprocessorCount, dev ) == hipSuccess )
+      cus[dev].store( n, std::memory_order_relaxed );
+   return n;
+}
+
+} // namespace gamer_amd
 
 extern "C" {
 
@@ -459,7 +476,7 @@ int hydro_mhm_solve_batch_async( const HydroSolveArgs *a, const double *pg_dt_dh
 {
    int rc = check_args( a );
    if ( rc != HYDRO_OK ) return rc;
-   Batch B;
+   Batch B = {};
    B.pg_dt_dh = pg_dt_dh;
    B.counter  = queue_counter;
    B.safety   = a->safety;

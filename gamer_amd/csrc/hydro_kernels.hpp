@@ -20,6 +20,35 @@ __device__ __forceinline__ long xcd_block()
    return ( ( x < r ) ? x*( q + 1 ) : r*( q + 1 ) + ( x - r )*q ) + i;
 }
 
+// How a launch of npg patch groups is split over workgroups: B.whole patch groups run one per workgroup, the others in
+// B.slabs z slabs of 16/slabs output planes, one workgroup per slab, which marches `halo` more input planes than it
+// updates.  The planes are sequential, so a launch that does not fill the chip takes one patch group's march however few
+// patch groups it has, and one of k full rounds and a rest takes k + 1: whole rounds (per_cu workgroups per compute unit)
+// run whole, and the rest takes the slab count with the fewest planes in sequence, rounds x (16/slabs + halo); two FP32
+// workgroups on one unit take 1.28 times as long as one (8 patch groups 51.5 us, 512 66 us).  A slab's planes are
+// computed exactly as in the whole march, so the results are bitwise equal.  Not split: the MinMod retry (maxiter > 0),
+// which is decided over the whole patch group; with the fused dt only into halves, whose patches do not straddle slabs.
+// Measured (us, whole -> split), MHM_RP: FP32 8 patch groups 51.7 -> 14.5, 32 with dt 54.7 -> 35.5, 100 53 -> 31.7, 256
+// 53.7 -> 46.3; FP64 16 73 -> 20, 64 73.8 -> 33.4, 700 224 -> 222.6, 1331 464 -> 433; FP64 Roe 300 264 -> 192.
+int device_cus();                    // compute units of the current device, 0 if unknown
+inline void slab_split( int npg, int halo, int per_cu, int minmod_maxiter, bool with_dt, Batch &B )
+{
+   B.whole = npg;
+   B.slabs = 1;
+   const int cus = device_cus(), slots = cus*per_cu;
+   if ( slots <= 0 || minmod_maxiter > 0 ) return;
+   const int rest = npg % slots;
+   double best = 0.0;
+   for (int s = 1; s <= ( with_dt ? 2 : 16 ); s *= 2)
+   {
+      const int blocks = rest*s;
+      const double rounds = ( blocks <= cus ) ? ( per_cu == 2 ? 0.78 : 1.0 ) : ( blocks + slots - 1 )/slots;
+      const double cost = rounds*( 16/s + halo );
+      if ( s == 1 || cost < best ) { best = cost;  B.slabs = s; }
+   }
+   if ( B.slabs > 1 ) B.whole = npg - rest;
+}
+
 // MHM_RP patch-group update: in[npg][5][22^3] -> out[npg][5][16^3] (+ flux[npg][9][5][16^2] if store_flux)
 template <typename R, typename IO>
 int launch_mhm_rp( const IO *in, IO *out, IO *flux, int npg, int rsolver, int store_flux, int minmod_maxiter,

@@ -119,12 +119,14 @@ struct Prm {
 // Multi-level batch description: optional per-PG (dt, dh) pairs in device memory (uneven AMR batches, local
 // time steps) and an optional global work-queue counter for the persistent mode (each workgroup pulls tickets of
 // `claim` consecutive patch groups until the queue is exhausted).  pg_dt_dh == nullptr: every PG uses Prm's dt/dh;
-// counter == nullptr: one PG per workgroup.
+// counter == nullptr: the patch groups from `whole` on are split into `slabs` z slabs, one workgroup each, the others
+// run one per workgroup (slab_split() in hydro_kernels.hpp).
 struct Batch {
    const double *pg_dt_dh;
    unsigned     *counter;
    double        safety;
    int           claim;
+   int           whole, slabs;
 };
 
 // an interface state rotated to the face normal: conserved fields + derived quantities
@@ -741,14 +743,15 @@ template <typename R, typename IO>
 __device__ __forceinline__ bool full_cell( const IO u[NV], const R dfxy[NV], const R fzl[NV], const R fzu[NV],
                                            const Prm<R> &P, IO o[NV] )
 {
+   #pragma clang fp contract(off)      // fused where written: every launch mode rounds alike
 #  pragma unroll
    for (int v=0; v<NV; v++)
-      o[v] = (IO)( (double)u[v] - P.dt_dh*( (double)dfxy[v] + ( (double)fzu[v] - (double)fzl[v] ) ) );
+      o[v] = (IO)fmad( -P.dt_dh, (double)dfxy[v] + ( (double)fzu[v] - (double)fzl[v] ), (double)u[v] );
    // each test is one ordered compare, false for NaN: "not finite-and-in-range" covers the NaN test too
    const IO huge = IOLim<IO>::huge, Z = (IO)0;
    bool ok = ( vabs( o[1] ) <= huge ) && ( vabs( o[2] ) <= huge ) && ( vabs( o[3] ) <= huge );
    ok = ok && ( o[0] > Z && o[0] <= huge ) && ( o[4] > Z && o[4] <= huge );
-   const IO ei = o[4] - (IO)0.5*( o[1]*o[1] + o[2]*o[2] + o[3]*o[3] )*rcp( o[0] );
+   const IO ei = fmad( (IO)-0.5*fmad( o[3], o[3], fmad( o[2], o[2], o[1]*o[1] ) ), rcp( o[0] ), o[4] );
    ok = ok && ( ei >= (IO)-3.0*o[4]*IOLim<IO>::eps && ei <= huge );
    return !ok;
 }
@@ -842,9 +845,10 @@ __device__ __forceinline__ IO cell_cfl( const IO u[NV], double gamma, double gm1
 // Fused CFL of one patch group: each lane holds the maxima of its output column in the two z-halves; the 8
 // patches (px + 2 py + 4 pz, x fastest) are reduced with wave64 butterflies and LDS across the 4 waves, in the
 // I/O type (the reference computes dt in `real`, CPU_dtSolver_HydroCFL.cpp:62-209).
-// Called by every lane of the workgroup (waves 0-3 hold the output columns); writes dt[8] = dh_safety / max.
+// Called by every lane of the workgroup (waves 0-3 hold the output columns); writes dt[8] = dh_safety / max, or only
+// the four patches of z half `half` if that is 0 or 1.
 template <typename IO>
-__device__ __forceinline__ void fused_dt( const IO cfl[2], int pxy, IO (*red)[4], IO *dt, double dh_safety )
+__device__ __forceinline__ void fused_dt( const IO cfl[2], int pxy, IO (*red)[4], IO *dt, double dh_safety, int half )
 {
    const int tid = threadIdx.x, w = tid >> 6;
    if ( w < 4 )                      // the output columns live on waves 0-3; further waves hold ghost columns
@@ -859,7 +863,7 @@ __device__ __forceinline__ void fused_dt( const IO cfl[2], int pxy, IO (*red)[4]
          if ( ( tid & 63 ) == 0 ) red[q + 4*pz][w] = m;
       }
    __syncthreads();
-   if ( tid < 8 )
+   if ( tid < 8 && ( half < 0 || ( tid >> 2 ) == half ) )
    {
       const IO m = vmax( vmax( red[tid][0], red[tid][1] ), vmax( red[tid][2], red[tid][3] ) );
       dt[tid] = (IO)( dh_safety / (double)m );

@@ -313,7 +313,7 @@ mhm_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restrict_
             for (int v=0; v<NV; v++) kDf[v] = dfn[v];
       } // for t
 
-      if ( g_dt ) fused_dt( cfl, ( ki - 2 )/8 + 2*( ( kj - 2 )/8 ), S.cfl, g_dt + (size_t)pg*8, dh_safety );
+      if ( g_dt ) fused_dt( cfl, ( ki - 2 )/8 + 2*( ( kj - 2 )/8 ), S.cfl, g_dt + (size_t)pg*8, dh_safety, -1 );
       __syncthreads();
       const bool redo = ( S.fail != 0 ) && ( iter + 1 <= minmod_maxiter );
       __syncthreads();

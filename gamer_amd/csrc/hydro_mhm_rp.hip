@@ -126,8 +126,9 @@ __device__ __forceinline__ bool edge_column( int t, int &i, int &j, bool &dy, bo
 template <typename R, typename IO>
 __device__ __forceinline__ void derive_cell( const IO u[NV], R q[8], const Prm<R> &P )
 {
+   #pragma clang fp contract(off)      // fused where written: every launch mode rounds alike
    const double d = (double)u[0], mx = (double)u[1], my = (double)u[2], mz = (double)u[3], e = (double)u[4];
-   const double eint = e - 0.5*( mx*mx + my*my + mz*mz )*rcp_pres<R>( d );
+   const double eint = fmad( -0.5*fmad( mz, mz, fmad( my, my, mx*mx ) ), rcp_pres<R>( d ), e );
    const R p = floor_pres( (R)( eint*P.gm1_d ), P.min_pres );
    const R ir = rcp( (R)u[0] );
 #  pragma unroll
@@ -144,17 +145,18 @@ template <typename R>
 __device__ __forceinline__ void half_cell( const R u[NV], const R dfxy[NV], const R hzl[NV], const R hzu[NV],
                                            const Prm<R> &P, R w[NV] )
 {
+   #pragma clang fp contract(off)
    R c[NV];
    const R k = (R)P.dt_dh2;
 #  pragma unroll
-   for (int v=0; v<NV; v++) c[v] = u[v] - k*( dfxy[v] + ( hzu[v] - hzl[v] ) );
+   for (int v=0; v<NV; v++) c[v] = fmad( -k, dfxy[v] + ( hzu[v] - hzl[v] ), u[v] );
    c[0] = vmax( c[0], P.min_dens );
    const double d = (double)c[0], m1 = (double)c[1], m2 = (double)c[2], m3 = (double)c[3];
-   const double ke = 0.5*( m1*m1 + m2*m2 + m3*m3 )*rcp_pres<R>( d );
+   const double q = -0.5*fmad( m3, m3, fmad( m2, m2, m1*m1 ) ), rd = rcp_pres<R>( d );
    double e = (double)c[4];
-   double ein = e - ke;
+   double ein = fmad( q, rd, e );
    const double eout = ( ein == ein ) ? __builtin_fmax( ein, P.min_eint_d ) : ein;
-   if ( ein != eout ) { e = e - ein + eout;  ein = e - ke; }
+   if ( ein != eout ) { e = e - ein + eout;  ein = fmad( q, rd, e ); }
    const R r = rcp( c[0] );
    w[0] = c[0];
    w[1] = c[1]*r;
@@ -201,7 +203,8 @@ struct SmemRP {
    R cfl[8][4];                 // fused CFL: per-patch maxima of the 4 column waves (R is the I/O type)
 };
 
-template <typename R, typename IO, int RS, int LIM, bool PERSIST>
+// MODE 0: one patch group per workgroup; 1: persistent work queue; 2: the last patch groups in z slabs (slab_split())
+template <typename R, typename IO, int RS, int LIM, int MODE>
 __global__ void __launch_bounds__( NT ) __attribute__(( amdgpu_waves_per_eu( sizeof(R) == 4 ? 4 : 2 ) ))
 mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restrict__ g_flux,
                int npg, int store_flux, int minmod_maxiter, R minmod_coeff, Prm<R> P0,
@@ -228,11 +231,11 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
    int base = 0;
    for (int item = 0; ; item++)
    {
-   // next patch group: blockIdx.x, or the next PG of this workgroup's ticket of the persistent work queue (a ticket
-   // covers B.claim consecutive PGs; the barrier before every PG also keeps the previous PG's LDS reads ahead of
-   // the next PG's writes)
-   int pg;
-   if ( PERSIST )
+   // next patch group: blockIdx.x (of the last ones, a z slab: slab_split()), or the next PG of this workgroup's ticket of
+   // the persistent work queue (a ticket covers B.claim consecutive PGs; the barrier before every PG also keeps the
+   // previous PG's LDS reads ahead of the next PG's writes)
+   int pg, slab_z = 0, slab_h = PS, half = -1;        // first output plane and output planes of the march; z half whose dt it writes
+   if ( MODE == 1 )
    {
       const int sub = item % B.claim;
       __syncthreads();
@@ -248,6 +251,14 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
    {
       if ( item > 0 ) break;
       pg = blockIdx.x;
+      if ( MODE == 2 && pg >= B.whole )
+      {
+         const int e = pg - B.whole, k = e % B.slabs;
+         pg = B.whole + e / B.slabs;
+         slab_h  = PS / B.slabs;
+         slab_z = k*slab_h;
+         half = ( B.slabs == 2 ) ? k : -1;
+      }
    }
    if ( pg >= npg ) break;
 
@@ -255,9 +266,12 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
    const IO *in  = g_in  + (size_t)pg*NV*NC*NX;
    IO       *out = g_out + (size_t)pg*NV*PS*PS*PS;
    IO       *flx = store_flux ? g_flux + (size_t)pg*9*NV*PS*PS : nullptr;
-   const __amdgpu_buffer_rsrc_t b_in  = make_buf( in,  NV*NC*NX*SZ );
-   const __amdgpu_buffer_rsrc_t b_out = make_buf( out, NV*PS*PS*PS*SZ );
-   const __amdgpu_buffer_rsrc_t b_flx = make_buf( flx, flx ? 9*NV*PS*PS*SZ : 0 );
+   const int z0 = ( MODE == 2 ) ? slab_z : 0;
+   // the march counts its planes from 0: the descriptors start at the slab's first plane (the x and y flux planes at its
+   // first row)
+   const __amdgpu_buffer_rsrc_t b_in  = make_buf( in + z0*NC,     ( NV*NC*NX - z0*NC )*SZ );
+   const __amdgpu_buffer_rsrc_t b_out = make_buf( out + z0*PS*PS, ( NV*PS*PS*PS - z0*PS*PS )*SZ );
+   const __amdgpu_buffer_rsrc_t b_flx = make_buf( flx ? flx + z0*PS : nullptr, flx ? ( 9*NV*PS*PS - z0*PS )*SZ : 0 );
    Prm<R> P = P0;
    double dh_safety = dh_safety0;
    if ( B.pg_dt_dh )
@@ -265,7 +279,6 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
       const double dt = B.pg_dt_dh[2*pg], dh = B.pg_dt_dh[2*pg + 1];
       P.dt_dh2 = 0.5*dt/dh;  P.dt_dh = dt/dh;  dh_safety = B.safety*dh;
    }
-   constexpr int t0 = 0, t1 = NX - 1;          // first and last input plane of the march
 
    for (int iter = 0; ; iter++)
    {
@@ -280,6 +293,7 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
 
       auto march_columns = [&]()
       {
+         const int z0 = ( MODE == 2 ) ? slab_z : 0, t1 = ( MODE == 2 ) ? slab_h + 5 : NX - 1;     // t1: last input plane
          R kU[8], kU1[8];                            // input cell of planes t and t-1 (+ pressure, 1/rho, c_s)
          R kHz[NV], kDh[NV];                         // half-step z-flux at t-3/2 ; half-step dFx+dFy of plane t-1
          R kW1[NV], kW2[NV], kW3[NV];                // half-step primitives of planes t-1, t-2, t-3
@@ -288,7 +302,7 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
          // two steps per iteration would rename the plane-to-plane register hand-offs instead of copying them, but spill
          // (FP64 HLLC on 1331 patch groups 564 us, rolled 511)
 #        pragma unroll 1
-         for (int t = t0; t <= t1; t++)
+         for (int t = 0; t <= t1; t++)
          {
             const int o = t - 3;                     // output plane of this step
             const int r = t - 2;                     // reconstructed plane of this step
@@ -301,16 +315,16 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
             for (int v=0; v<NV; v++) S.u3[( t + 2 ) % 3][v][tid] = kU1[v];     // plane t-1, read back at step t+2
 
             R df[NV];                                // full-step dFx+dFy of plane o
-            if ( o >= t0 + 3 && o <= t1 - 3 )
+            if ( o >= 3 && o <= t1 - 3 )
 #              pragma unroll
                for (int v=0; v<NV; v++) df[v] = ( S.g[v][kq + 1] - S.g[v][kq] ) + ( S.g[v][FX + kq + FS] - S.g[v][FX + kq] );
 
             // half-step z-flux at t-1/2 and half-step cell of plane t-1
-            if ( t >= t0 + 1 )
+            if ( t >= 1 )
             {
                R fz[NV], w[NV];
                solve<RS, 2, 0>( cell_side<2>( kU1 ), cell_side<2>( kU ), Q, fz );
-               if ( t >= t0 + 2 )
+               if ( t >= 2 )
                {
                   half_cell( kU1, kDh, kHz, fz, Q, w );
 #                 pragma unroll
@@ -320,7 +334,7 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
                for (int v=0; v<NV; v++) kHz[v] = fz[v];
             }
             // half-step y flux of plane t
-            if ( t >= t0 + 1 && t <= t1 - 1 )
+            if ( t >= 1 && t <= t1 - 1 )
             {
                R f[NV];
                solve<RS, 1, 0>( side_at<1>( S.a, kc - NX ), cell_side<1>( kU ), Q, f );
@@ -328,10 +342,10 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
             }
             // PLM of plane r along z and y; the y neighbours come from the half-step plane r in S.w
             R zL[NV], zR[NV], yL[NV];
-            if ( r >= t0 + 2 && r <= t1 - 2 )
+            if ( r >= 2 && r <= t1 - 2 )
             {
                plm_cell<LIM>( kW3, kW2, kW1, Q, zL, zR );
-               if ( r >= t0 + 3 && r <= t1 - 3 )
+               if ( r >= 3 && r <= t1 - 3 )
                {
                   R a[NV], b[NV], fr[NV];
                   ld5( S.w, kh - NX, a );  ld5( S.w, kh + NX, b );
@@ -342,26 +356,26 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
             __syncthreads();                         // [H] half-step fluxes and left states of plane r visible
 
 
-            if ( t >= t0 + 1 && t <= t1 - 1 )
+            if ( t >= 1 && t <= t1 - 1 )
 #              pragma unroll
                for (int v=0; v<NV; v++) kDh[v] = ( S.h[v][kh + 1] - S.h[v][kh] ) + ( S.h[v][HX + kh + NX] - S.h[v][HX + kh] );
-            if ( t >= t0 + 2 ) st5( S.w, kh, kW1 );  // plane t-1 replaces plane t-2 for the next reconstruction
+            if ( t >= 2 ) st5( S.w, kh, kW1 );  // plane t-1 replaces plane t-2 for the next reconstruction
 
             // full-step z-flux at r-1/2
             R fz[NV];
-            if ( r >= t0 + 3 && r <= t1 - 2 )
+            if ( r >= 3 && r <= t1 - 2 )
             {
                solve<RS, 2, 1>( face_side<2>( kFzR, Q ), face_side<2>( zL, Q ), Q, fz );
-               if ( flx && ( r - 3 ) % 8 == 0 )
+               if ( flx && ( z0 + r - 3 ) % 8 == 0 && ( r < t1 - 2 || z0 + r == 19 ) )    // the next slab stores the face between
 #                 pragma unroll
                   for (int v=0; v<NV; v++)
-                     buf_store( (IO)fz[v], b_flx, kxy*SZ, ( ( 6 + ( r - 3 )/8 )*NV + v )*PS*PS*SZ );
+                     buf_store( (IO)fz[v], b_flx, kxy*SZ, ( ( ( 6 + ( z0 + r - 3 )/8 )*NV + v )*PS*PS - z0*PS )*SZ );
             }
-            if ( r >= t0 + 2 )
+            if ( r >= 2 )
 #              pragma unroll
                for (int v=0; v<NV; v++) kFzR[v] = zR[v];
             // full-step y-flux of plane r
-            if ( r >= t0 + 3 && r <= t1 - 3 )
+            if ( r >= 3 && r <= t1 - 3 )
             {
                R f[NV], q[NV];
                ld5( S.l, FX + kq, q );
@@ -372,7 +386,7 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
                   for (int v=0; v<NV; v++) buf_store( (IO)f[v], b_flx, fy_off, ( v*PS*PS + PS*( r - 3 ) )*SZ );
             }
             // full-step update and output of plane o
-            if ( o >= t0 + 3 && o <= t1 - 3 )
+            if ( o >= 3 && o <= t1 - 3 )
             {
                IO res[NV], uo[NV];
                ld5( S.u3[t % 3], tid, uo );
@@ -380,15 +394,16 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
 #              pragma unroll
                for (int v=0; v<NV; v++) buf_store( res[v], b_out, kxy*SZ, ( v*PS*PS*PS + PS*PS*( o - 3 ) )*SZ );
                if ( bad ) S.fail = 1;
-               if ( g_dt ) cfl[ ( o - 3 )/8 ] = vmax( cfl[ ( o - 3 )/8 ], cell_cfl( res, (double)Q.gamma, Q.gm1_d, Q.min_pres_d ) );
+               if ( g_dt ) cfl[ ( z0 + o - 3 )/8 ] = vmax( cfl[ ( z0 + o - 3 )/8 ], cell_cfl( res, (double)Q.gamma, Q.gm1_d, Q.min_pres_d ) );
             }
-            if ( r >= t0 + 3 && r <= t1 - 2 )
+            if ( r >= 3 && r <= t1 - 2 )
 #              pragma unroll
                for (int v=0; v<NV; v++) kFz[v] = fz[v];
          }
       };
       auto march_sides = [&]()
       {
+         const int t1 = ( MODE == 2 ) ? slab_h + 5 : NX - 1;     // t1: last input plane
          int oi, oj, ei, ej;
          bool e_dy, e_face;
          arm_column( g, oi, oj );
@@ -437,19 +452,19 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
                }
             }
          };
-         issue( t0 );
+         issue( 0 );
          stage();
-         issue( t0 + 1 );
+         issue( 1 );
 
 #        pragma unroll 1
-         for (int t = t0; t <= t1; t++)
+         for (int t = 0; t <= t1; t++)
          {
             const int r = t - 2;
             __syncthreads();                         // [A]
-            // arm half step: cells of planes t0+3 .. t1-3 (updated one step later), their z faces and low x/y faces
-            const bool arm_ld = ( gw < 2 ) && t >= t0 + 2 && t <= t1 - 2;
-            const bool arm_z  = ( gw < 2 ) && t >= t0 + 3 && t <= t1 - 2;
-            const bool arm_xy = ( gw < 2 ) && t >= t0 + 3 && t <= t1 - 3;
+            // arm half step: cells of planes 3 .. t1-3 (updated one step later), their z faces and low x/y faces
+            const bool arm_ld = ( gw < 2 ) && t >= 2 && t <= t1 - 2;
+            const bool arm_z  = ( gw < 2 ) && t >= 3 && t <= t1 - 2;
+            const bool arm_xy = ( gw < 2 ) && t >= 3 && t <= t1 - 3;
 #           pragma unroll
             for (int v=0; v<8; v++) oU1[v] = oU[v];
             if ( arm_ld ) ld_cell( S.a, oc, oU );
@@ -457,7 +472,7 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
             {
                R fz[NV];
                solve<RS, 2, 0>( cell_side<2>( oU1 ), cell_side<2>( oU ), Q, fz );
-               if ( t >= t0 + 4 ) half_cell( oU1, oDh, oHz, fz, Q, oW );
+               if ( t >= 4 ) half_cell( oU1, oDh, oHz, fz, Q, oW );
 #              pragma unroll
                for (int v=0; v<NV; v++) oHz[v] = fz[v];
             }
@@ -470,10 +485,10 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
                st5( S.h, oh, ox );
                st5( S.h, HX + oh, oy );
             }
-            if ( gw == 2 && t >= t0 + 1 && t <= t1 - 1 )
+            if ( gw == 2 && t >= 1 && t <= t1 - 1 )
             {
                const bool fdy = t_dy;
-               const int  fc = ( t >= t0 + 3 && t <= t1 - 3 ) ? tm_c : tn_c;
+               const int  fc = ( t >= 3 && t <= t1 - 3 ) ? tm_c : tn_c;
                if ( fc >= 0 )
                {
                   R ql[8], qr[8], f[NV];
@@ -484,7 +499,7 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
                }
             }
             // half-step x fluxes of plane t
-            if ( gw >= 2 && t >= t0 + 1 && t <= t1 - 1 )
+            if ( gw >= 2 && t >= 1 && t <= t1 - 1 )
             {
                const Side<R> l[2] = { side_at<0>( S.a, kc - 1 ), side_at<0>( S.a, k2 - 1 ) }, q[2] = { side_at<0>( S.a, kc ), side_at<0>( S.a, k2 ) };
                R f[2][NV], fx[NV], f2[NV];
@@ -495,7 +510,7 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
             }
             // PLM of plane r along x, and of the edge column
             R xL[NV], eL[NV];
-            if ( r >= t0 + 3 && r <= t1 - 3 )
+            if ( r >= 3 && r <= t1 - 3 )
             {
                R a[NV], b[NV], c[NV], fr[NV];
                ld5( S.w, kh - 1, a );  ld5( S.w, kh, b );  ld5( S.w, kh + 1, c );
@@ -521,10 +536,10 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
             if ( arm_xy )
 #              pragma unroll
                for (int v=0; v<NV; v++) oDh[v] = ( S.h[v][oh + 1] - S.h[v][oh] ) + ( S.h[v][HX + oh + NX] - S.h[v][HX + oh] );
-            if ( arm_z && t >= t0 + 4 ) st5( S.w, oh, oW );
+            if ( arm_z && t >= 4 ) st5( S.w, oh, oW );
 
             // full-step x-flux of plane r, and the faces x = 16 and y = 16 of the block
-            if ( r >= t0 + 3 && r <= t1 - 3 )
+            if ( r >= 3 && r <= t1 - 3 )
             {
                R f[NV], q[NV];
                ld5( S.l, kq, q );
@@ -547,7 +562,7 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
       };
       if ( wave < 4 ) march_columns(); else march_sides();
 
-      if ( g_dt ) fused_dt( cfl, ( ki - 3 )/8 + 2*( ( kj - 3 )/8 ), S.cfl, g_dt + (size_t)pg*8, dh_safety );
+      if ( g_dt ) fused_dt( cfl, ( ki - 3 )/8 + 2*( ( kj - 3 )/8 ), S.cfl, g_dt + (size_t)pg*8, dh_safety, half );
       __syncthreads();
       const bool redo = ( S.fail != 0 ) && ( iter + 1 <= minmod_maxiter );
       __syncthreads();
@@ -560,14 +575,17 @@ mhm_rp_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restri
 
 template <typename R, typename IO, int RS>
 static void launch_rs( const IO *in, IO *out, IO *flux, int npg, int store_flux, int minmod_maxiter,
-                       double minmod_coeff, const Prm<R> &P, IO *dt, double dh_safety, const Batch &B, int grid_blocks, hipStream_t stream )
+                       double minmod_coeff, const Prm<R> &P, IO *dt, double dh_safety, Batch B, int grid_blocks, hipStream_t stream )
 {
-   const dim3 grid( grid_blocks > 0 ? grid_blocks : npg ), block( NT );
    const bool pers = ( B.counter != nullptr );
-#  define GA_LAUNCH( LIM_, PERS_ ) hipLaunchKernelGGL( ( mhm_rp_kernel<R, IO, RS, LIM_, PERS_> ), grid, block, 0, stream, \
+   if ( !pers ) slab_split( npg, NX - PS, sizeof( R ) == 4 ? 2 : 1, minmod_maxiter, dt != nullptr, B );
+   const dim3 grid( pers ? ( grid_blocks > 0 ? grid_blocks : npg ) : B.whole + ( npg - B.whole )*B.slabs ), block( NT );
+   const int mode = pers ? 1 : ( B.slabs > 1 ) ? 2 : 0;
+#  define GA_LAUNCH( LIM_, MODE_ ) hipLaunchKernelGGL( ( mhm_rp_kernel<R, IO, RS, LIM_, MODE_> ), grid, block, 0, stream, \
                                                       in, out, flux, npg, store_flux, minmod_maxiter, (R)minmod_coeff, P, dt, dh_safety, B )
-   if ( kernel_limiter( P.limiter, minmod_coeff ) == 4 ) { if ( pers ) GA_LAUNCH( 4, true ); else GA_LAUNCH( 4, false ); }
-   else                  { if ( pers ) GA_LAUNCH( 0, true ); else GA_LAUNCH( 0, false ); }
+#  define GA_MODE( LIM_ ) { if ( mode == 0 ) GA_LAUNCH( LIM_, 0 ); else if ( mode == 1 ) GA_LAUNCH( LIM_, 1 ); else GA_LAUNCH( LIM_, 2 ); }
+   if ( kernel_limiter( P.limiter, minmod_coeff ) == 4 ) GA_MODE( 4 ) else GA_MODE( 0 )
+#  undef GA_MODE
 #  undef GA_LAUNCH
 }
 
