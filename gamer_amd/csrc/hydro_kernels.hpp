@@ -38,6 +38,7 @@ inline void slab_split( int npg, int halo, int per_cu, int minmod_maxiter, bool 
    const int cus = device_cus(), slots = cus*per_cu;
    if ( slots <= 0 || minmod_maxiter > 0 ) return;
    const int rest = npg % slots;
+   if ( rest == 0 ) return;
    double best = 0.0;
    for (int s = 1; s <= ( with_dt ? 2 : 16 ); s *= 2)
    {
