@@ -4,7 +4,7 @@
 //
 //   interpolate_kernel   Interpolate() with Interpolate_Iterate (Interpolate.cpp:90-330) for INT_MINMOD3D, INT_MINMOD1D,
 //                        INT_VANLEER, INT_CQUAD, INT_QUAD, INT_CQUAR and INT_QUAR (src/Interpolation/Int_*.cpp): one
-//                        workgroup per coarse box, one lane per coarse cell producing its 2x2x2 fine cells.  For the
+//                        workgroup per coarse box, one lane per asked-for coarse cell producing its 2x2x2 fine cells.  For the
 //                        tensor-product schemes (all but INT_MINMOD1D) the lane evaluates the x pass on the
 //                        (2G+1)x(2G+1) coarse (y,z) neighbourhood (G = 1, or 2 for the quartic schemes), then the y
 //                        pass, then the z pass: the same operations in the same order as the reference's split
@@ -28,7 +28,8 @@ namespace gamer_amd {
 namespace {
 
 constexpr int PS = 16, H = 8, P3 = H*H*H;
-constexpr int NT = 256;
+// Lanes of an interpolation block: the wide stencils need more registers than 512 lanes leave.
+template <typename T> constexpr int interp_lanes( int scheme ) { return ( scheme == 7 || ( sizeof( T ) == 8 && scheme >= 5 ) ) ? 256 : 512; }
 
 template <typename T> __device__ __forceinline__ T sgn( T a ) { return ( a < (T)0 ) ? (T)-1 : (T)+1; }
 
@@ -39,17 +40,10 @@ __device__ __forceinline__ T cquad_slope( T L, T C, T R, bool mono, T coeff, boo
    T s = (T)0.125*( R - L );
    if ( mono )
    {
-      T l = (T)0.25*( C - L ), r = (T)0.25*( R - C );
-      if ( l*r > (T)0 )
-      {
-         const T sg = sgn( l );
-         s *= sg;  l *= sg;  r *= sg;
-         if ( l < r ) l *= coeff; else r *= coeff;
-         s = vmin( l, s );
-         s = vmin( r, s );
-         s *= sg;
-      }
-      else s = (T)0;
+      const T l = (T)0.25*( C - L ), r = (T)0.25*( R - C );
+      // of one sign where it matters, so that R - L has it too: the smallest magnitude, the smaller side scaled
+      const T m = vmin( vmin( vmin( vabs( l ), vabs( r ) )*coeff, vmax( vabs( l ), vabs( r ) ) ), vabs( s ) );
+      s = ( l*r > (T)0 ) ? __builtin_copysign( m, l ) : (T)0;
    }
    if ( opp0 && L*R < (T)0 ) s = (T)0;
    return s;
@@ -277,35 +271,23 @@ __device__ __forceinline__ bool store_fine( T f[NV][8], bool iterate, bool prim,
    return true;
 }
 
-// x pass of the rows y-1, y, y+1 of coarse plane z' around index q, then the y pass: Y[y-lo/hi][x-lo/hi] of that
-// plane, exactly as interp_cell computes its Y[a] (3-point schemes)
-template <typename T, int SCHEME>
-__device__ __forceinline__ void xy_pass( const T *__restrict__ c, int q, int dy, bool mono, T coeff, bool opp0, T Y[2][2] )
-{
-   #pragma clang fp contract(off)
-   T X[3][2], u[5];
-#  pragma unroll
-   for (int b=0; b<3; b++)
-   {
-      const int qq = q + ( b - 1 )*dy;
-      u[0] = (T)0;  u[1] = c[qq - 1];  u[2] = c[qq];  u[3] = c[qq + 1];  u[4] = (T)0;
-      pass1d<T, SCHEME>( u, mono, coeff, opp0, X[b][0], X[b][1] );
-   }
-#  pragma unroll
-   for (int x=0; x<2; x++)
-   {
-      u[0] = (T)0;  u[1] = X[0][x];  u[2] = X[1][x];  u[3] = X[2][x];  u[4] = (T)0;
-      pass1d<T, SCHEME>( u, mono, coeff, opp0, Y[0][x], Y[1][x] );
-   }
-}
-
-template <typename T, int SCHEME>
-__global__ void __launch_bounds__( NT )
+// One lane per asked-for coarse cell, from a list: a box next to a patch of its own level needs two layers of its 12^3 cells,
+// and a lane's chain of 95 one-dimensional passes (19 a field) is the time, so the lanes must all have cells.  PLAIN: all
+// fields monotonic and no clipping across 0 (the default); with these as run-time bits every pass had branches of its own,
+// which kept the passes from overlapping.  512 boxes of the AMR step (216 ask for nothing, most others for 288 cells), CQUAD:
+// FP32 118 -> 34 us, FP64 155 -> 48; every cell asked for 130 -> 65 and 217 -> 150; one box 95 -> 26.  The first form marched
+// a lane per column through the box: 9 passes a cell and field in place of 19, but 24 lanes of 144 at work beside an x face,
+// twelve planes in sequence; the list with the branches took 90.
+template <typename T, int SCHEME, bool PLAIN>
+__global__ void __launch_bounds__( interp_lanes<T>( SCHEME ) )
 interpolate_kernel( T *__restrict__ g_c, T *__restrict__ g_f, int nbox, InterpPrm p, int *__restrict__ nfail )
 {
    #pragma clang fp contract(off)
+   constexpr int NT = interp_lanes<T>( SCHEME );
    __shared__ int s_fail;
+   __shared__ int s_n;
    __shared__ unsigned char s_done[INTERP_MAX_CELLS];
+   __shared__ unsigned short s_todo[INTERP_MAX_CELLS];
    const int q = blockIdx.x, tid = threadIdx.x;
    if ( q >= nbox ) return;
    const int dy = p.cs[0], dz = p.cs[0]*p.cs[1], C3 = dz*p.cs[2];
@@ -316,7 +298,23 @@ interpolate_kernel( T *__restrict__ g_c, T *__restrict__ g_f, int nbox, InterpPr
    const bool iterate = p.int_prim || p.reduce;
    const int mono_max = p.reduce ? p.mono_max_iter : 0, max_iter = p.int_prim ? mono_max + 1 : mono_max;
 
-   for (int c = tid; c < ncell; c += NT) s_done[c] = p.need ? !p.need[ (size_t)q*ncell + c ] : 0;
+   // the cells that are asked for, listed (in any order: they are independent)
+   if ( tid == 0 ) s_n = 0;
+   __syncthreads();
+   for (int c = tid; c < ncell; c += NT)
+   {
+      const bool todo = !p.need || p.need[ (size_t)q*ncell + c ];
+      s_done[c] = !todo;
+      const unsigned long long m = __ballot( todo );
+      const int lane = tid & 63, first = __ffsll( (long long)__ballot( true ) ) - 1;
+      int at = 0;
+      if ( lane == first ) at = atomicAdd( &s_n, __popcll( m ) );
+      at = __shfl( at, first, 64 );
+      if ( todo ) s_todo[ at + __popcll( m & ( ( 1ULL << lane ) - 1 ) ) ] = (unsigned short)c;
+   }
+   __syncthreads();
+   const int ntodo = s_n;
+   if ( ntodo == 0 ) return;
    T coeff = (T)p.mono_coeff;
    bool prim = false;
    for (int it = 0; ; it++)
@@ -349,69 +347,15 @@ interpolate_kernel( T *__restrict__ g_c, T *__restrict__ g_f, int nbox, InterpPr
       if ( tid == 0 ) s_fail = 0;
       __syncthreads();
 
-      constexpr bool MARCH = ( SCHEME == 1 || SCHEME == 3 || SCHEME == 4 || SCHEME == 5 );
-      if ( MARCH && it == 0 )
+      for (int k = tid; k < ntodo; k += NT)
       {
-         // first pass of a 3-point tensor-product scheme: one lane per (x, y) column of the coarse range, marching
-         // along z with the y-pass results of planes z-1, z, z+1 in registers, so each plane's x and y passes run
-         // once per column instead of once per cell that reads them (9 pass1d per cell and field instead of 19).
-         // The operations and their order are interp_cell's, so the values are bitwise the same.
-         const int ncol = p.cr[0]*p.cr[1], cz = p.cr[0]*p.cr[1];
-         for (int col = tid; col < ncol; col += NT)
-         {
-            const int x = col % p.cr[0], y = col / p.cr[0];
-            bool todo = false;
-            for (int z = 0; z < p.cr[2]; z++) todo |= !s_done[ col + z*cz ];
-            if ( !todo ) continue;
-            const int q0 = p.c0[2]*dz + ( p.c0[1] + y )*dy + p.c0[0] + x;      // coarse index of (x, y, z = 0)
-            T Yw[NV][3][2][2];
-#           pragma unroll
-            for (int v=0; v<NV; v++)
-            {
-               xy_pass<T, SCHEME>( C + (size_t)v*C3, q0 - dz, dy, ( p.mono >> v ) & 1, coeff, p.opp0, Yw[v][0] );
-               xy_pass<T, SCHEME>( C + (size_t)v*C3, q0,      dy, ( p.mono >> v ) & 1, coeff, p.opp0, Yw[v][1] );
-            }
-            for (int z = 0; z < p.cr[2]; z++)
-            {
-               T f[NV][8], u[5];
-#              pragma unroll
-               for (int v=0; v<NV; v++)
-               {
-                  xy_pass<T, SCHEME>( C + (size_t)v*C3, q0 + ( z + 1 )*dz, dy, ( p.mono >> v ) & 1, coeff, p.opp0, Yw[v][2] );
-#                 pragma unroll
-                  for (int yy=0; yy<2; yy++)
-#                    pragma unroll
-                     for (int xx=0; xx<2; xx++)
-                     {
-                        u[0] = (T)0;  u[1] = Yw[v][0][yy][xx];  u[2] = Yw[v][1][yy][xx];  u[3] = Yw[v][2][yy][xx];  u[4] = (T)0;
-                        pass1d<T, SCHEME>( u, ( p.mono >> v ) & 1, coeff, p.opp0, f[v][( 0*2 + yy )*2 + xx],
-                                           f[v][( 1*2 + yy )*2 + xx] );
-                     }
-               }
-               const int c = col + z*cz;
-               if ( !s_done[c] )
-               {
-                  const int fo = ( p.f0[2] + 2*z )*fdz + ( p.f0[1] + 2*y )*fdy + p.f0[0] + 2*x;
-                  if ( store_fine( f, iterate, prim, p, F, F3, fo, fdy, fdz ) ) s_done[c] = 1; else s_fail = 1;
-               }
-#              pragma unroll
-               for (int v=0; v<NV; v++)
-#                 pragma unroll
-                  for (int yy=0; yy<2; yy++)
-#                    pragma unroll
-                     for (int xx=0; xx<2; xx++) { Yw[v][0][yy][xx] = Yw[v][1][yy][xx];  Yw[v][1][yy][xx] = Yw[v][2][yy][xx]; }
-            }
-         }
-      }
-      else
-      for (int c = tid; c < ncell; c += NT)
-      {
+         const int c = s_todo[k];
          if ( s_done[c] ) continue;
          const int x = c % p.cr[0], y = ( c/p.cr[0] ) % p.cr[1], z = c/( p.cr[0]*p.cr[1] );
          const int ic = ( p.c0[2] + z )*dz + ( p.c0[1] + y )*dy + p.c0[0] + x;
          T f[NV][8];
 #        pragma unroll
-         for (int v=0; v<NV; v++) interp_cell<T, SCHEME>( C + (size_t)v*C3, ic, dy, dz, ( p.mono >> v ) & 1, coeff, p.opp0, f[v] );
+         for (int v=0; v<NV; v++) interp_cell<T, SCHEME>( C + (size_t)v*C3, ic, dy, dz, PLAIN || ( ( p.mono >> v ) & 1 ), coeff, !PLAIN && p.opp0, f[v] );
          const int fo = ( p.f0[2] + 2*z )*fdz + ( p.f0[1] + 2*y )*fdy + p.f0[0] + 2*x;
          if ( store_fine( f, iterate, prim, p, F, F3, fo, fdy, fdz ) ) s_done[c] = 1; else s_fail = 1;
       }
@@ -427,96 +371,87 @@ interpolate_kernel( T *__restrict__ g_c, T *__restrict__ g_f, int nbox, InterpPr
    }
 }
 
-// Coarse boxes of general size: one block per (box, field, z plane), its 256 threads over the plane's cells in linear
-// order (one division per cell for (x, y)).  A 32 x 8 thread grid over (x, y) left most lanes idle on the ~14^2
-// planes of a refined patch group's coarse box; the linear layout made the two-level AMR step 1.2% faster.
-constexpr int CPX = 32, CPY = 8;
-
-// patch-group input window (N = 16 + 2 ghost <= 32 per axis, N even): cell (x,y,z) from the patch
-// slot[pg][Z/8][Y/8][X/8], (X,Y,Z) = (x,y,z) - ghost + 8; slot -1: from the fine box fbox at (x,y,z) + fb.origin, or
-// kept if fbox == NULL.  Each thread copies EPT consecutive cells of the linear window index e = x + N (y + N z) of
-// one (PG, field): every lane is busy, the EPT loads are independent, and the store is one aligned vector (N^3 is a
-// multiple of 8, so a group never straddles two windows; an unaligned destination takes scalar stores).  (x,y,z)
-// of the first cell come from a float reciprocal: after the +0.5 shift, e/N^2 and r/N sit at least 1/(2 N^2) away
-// from an integer, far above the float error for N <= 32.  Measured against a 32 x 8-thread (x, y) block layout
-// and a lane-contiguous layout (each instruction over 64 consecutive cells), this one was the fastest.
-constexpr int EPT = 4;
-template <typename IO> struct Vec4;
-template <> struct Vec4<float>  { typedef float  type __attribute__(( ext_vector_type( 4 ) )); };
-template <> struct Vec4<double> { typedef double type __attribute__(( ext_vector_type( 4 ) )); };
-
+// Patch-group input window (N = 16 + 2 ghost <= 32 per axis): cell (x,y,z) from the patch slot[pg][Z/8][Y/8][X/8],
+// (X,Y,Z) = (x,y,z) - ghost + 8; slot -1: from the fine box fbox at (x,y,z) + fb.origin, or kept if fbox == NULL.  Block
+// (patch group, field, PREP_N cells of the window in linear order), a thread copies the cells t, t + 512, ...: every store
+// instruction covers 64 consecutive cells and every load pieces of patch rows that lie side by side, and PREP_Q loads are in
+// flight per lane.  (x,y,z) come from a float reciprocal: after the +0.5 shift, e/N^2 and r/N sit at least 1/(2 N^2) away
+// from an integer, far above the float error for N <= 32.  The slot table goes through LDS, so that a cell's patch lookup is
+// no second dependent global load.  Bound by memory.
+// 512 patch groups with ghost 3 at a refinement boundary (218 MB FP32): 62 us within an AMR step, 48 alone; four consecutive
+// cells a lane and one vector store 78 and 53.  FP64 alone 156 -> 100, without fine boxes 80 -> 73 (FP32 40 -> 44: what the
+// caches hold); XCD-major blocks 89, 256 lanes with 6 cells 98, 21 cells 90.
+constexpr int PREP_NT = 512, PREP_Q = 11, PREP_N = PREP_NT*PREP_Q;
 template <typename IO>
-__global__ void __launch_bounds__( NT )
+__global__ void __launch_bounds__( PREP_NT )
 prepare_patches_kernel( const IO *__restrict__ patch, const IO *__restrict__ fbox, IO *__restrict__ pg_in,
                         const int *__restrict__ slot, int ghost, BoxGeom fb )
 {
-   const int p = blockIdx.x, v = blockIdx.y, n = PS + 2*ghost, n2 = n*n, n3 = n2*n;
-   // the patch group's 4^3 slot table in LDS: each cell's patch lookup is then an LDS read, not a second
-   // dependent global load in front of the data load
+   const int n = PS + 2*ghost, n2 = n*n, n3 = n2*n;
+   const int p = blockIdx.x, v = blockIdx.y, bz = blockIdx.z;
    __shared__ int sl[64];
    if ( threadIdx.x < 64 ) sl[ threadIdx.x ] = slot[ (size_t)p*64 + threadIdx.x ];
    __syncthreads();
-   const int e0 = ( blockIdx.z*NT + threadIdx.x )*EPT;
-   if ( e0 >= n3 ) return;
-   int z = (int)( ( (float)e0 + 0.5f )*( 1.0f/(float)n2 ) );
-   const int r = e0 - z*n2;
-   int y = (int)( ( (float)r + 0.5f )*( 1.0f/(float)n ) );
-   int x = r - y*n;
-   const IO  *pv = patch + (size_t)v*P3;
-   const IO  *fv = fbox ? fbox + ( (size_t)p*NV + v )*fb.size[2]*fb.size[1]*fb.size[0] : nullptr;
-   IO   val[EPT];
-   bool put[EPT];
+   const float rn = 1.0f/(float)n, rn2 = 1.0f/(float)n2;
+   const int sx = fb.size[0], sxy = fb.size[1]*fb.size[0];
+   const IO *pv = patch + (size_t)v*P3;
+   const IO *fv = fbox ? fbox + ( (size_t)p*NV + v )*fb.size[2]*sxy + ( (size_t)fb.origin[2]*sxy + fb.origin[1]*sx + fb.origin[0] )
+                       : nullptr;
+   IO *dst = pg_in + ( (size_t)p*NV + v )*n3;
+   IO   val[PREP_Q];
+   bool put[PREP_Q];
 #  pragma unroll
-   for (int k = 0; k < EPT; k++)
+   for (int q=0; q<PREP_Q; q++)
    {
+      const int e = bz*PREP_N + q*PREP_NT + (int)threadIdx.x;
+      put[q] = false;
+      if ( e >= n3 ) continue;
+      const int z = (int)( ( (float)e + 0.5f )*rn2 ), r = e - z*n2, y = (int)( ( (float)r + 0.5f )*rn ), x = r - y*n;
       const int X = x - ghost + H, Y = y - ghost + H, Z = z - ghost + H;
       const int s = sl[ ( Z >> 3 )*16 + ( Y >> 3 )*4 + ( X >> 3 ) ];
-      put[k] = true;
-      if ( s >= 0 )  val[k] = pv[ (size_t)s*NV*P3 + ( Z & 7 )*H*H + ( Y & 7 )*H + ( X & 7 ) ];
-      else if ( fv ) val[k] = fv[ ( (size_t)( z + fb.origin[2] )*fb.size[1] + y + fb.origin[1] )*fb.size[0] + x + fb.origin[0] ];
-      else           put[k] = false;
-      // next cell of the window
-      x++;
-      const bool wx = ( x == n );
-      x = wx ? 0 : x;
-      y = wx ? y + 1 : y;
-      const bool wy = ( y == n );
-      y = wy ? 0 : y;
-      z = wy ? z + 1 : z;
+      const IO *src = ( s >= 0 ) ? pv + ( (size_t)s*NV*P3 + ( Z & 7 )*H*H + ( Y & 7 )*H + ( X & 7 ) )
+                                 : fv + ( (size_t)z*sxy + y*sx + x );
+      put[q] = ( s >= 0 ) || fv;
+      if ( put[q] ) val[q] = *src;
    }
-   IO *dst = pg_in + ( (size_t)p*NV + v )*n3 + e0;
-   const bool aligned = ( reinterpret_cast<size_t>( dst ) % sizeof( typename Vec4<IO>::type ) ) == 0;
-   if ( aligned && put[0] && put[1] && put[2] && put[3] )
-   {
-      typename Vec4<IO>::type q;
-      q.x = val[0];  q.y = val[1];  q.z = val[2];  q.w = val[3];
-      *reinterpret_cast<typename Vec4<IO>::type*>( dst ) = q;
-   }
-   else
-   {
-#     pragma unroll
-      for (int k = 0; k < EPT; k++) if ( put[k] ) dst[k] = val[k];
-   }
+#  pragma unroll
+   for (int q=0; q<PREP_Q; q++)
+      if ( put[q] ) dst[ bz*PREP_N + q*PREP_NT + (int)threadIdx.x ] = val[q];
 }
 
 // box[q][v][z][y][x] (size) = patch[ slot[q][Z/8][Y/8][X/8] ][v][Z%8][Y%8][X%8], (X,Y,Z) = origin + (x,y,z);
-// slot -1 keeps the box value
+// slot -1 keeps the box value.  Block (box, field, GB_N cells of the box in linear order), as above; the sizes are general,
+// so the cell's coordinates take two integer divisions. 
+// 512 boxes of 14^3 FP32 cells: 22 us, one block per plane 24.
+constexpr int GB_NT = 256, GB_Q = 6, GB_N = GB_NT*GB_Q;
 template <typename IO>
-__global__ void __launch_bounds__( CPX*CPY )
-gather_boxes_kernel( const IO *__restrict__ patch, IO *__restrict__ box, BoxGeom g, const int *__restrict__ slot )
+__global__ void __launch_bounds__( GB_NT )
+gather_boxes_kernel( const IO *__restrict__ patch, IO *__restrict__ box, BoxGeom g, const int *__restrict__ slot, unsigned chunks )
 {
-   const int q = blockIdx.x, v = blockIdx.y, z = blockIdx.z;
-   const int Z = z + g.origin[2];
-   const int *sl = slot + (size_t)q*g.tdim[0]*g.tdim[1]*g.tdim[2] + ( Z >> 3 )*g.tdim[1]*g.tdim[0];
-   IO *dst = box + ( ( (size_t)q*NV + v )*g.size[2] + z )*g.size[1]*g.size[0];
-   const int nxy = g.size[0]*g.size[1];
-   for (int e = threadIdx.x + CPX*threadIdx.y; e < nxy; e += CPX*CPY)
+   const long lb = xcd_block();
+   const long w = lb / chunks, q = w / NV, v = w - q*NV;                          // chunk fastest, then field, then box
+   const unsigned nx = g.size[0], nxy = nx*g.size[1];
+   const long n = (long)nxy*g.size[2], e0 = ( lb - w*chunks )*GB_N + threadIdx.x;
+   const int *sl = slot + (size_t)q*g.tdim[0]*g.tdim[1]*g.tdim[2];
+   const IO *pv = patch + (size_t)v*P3;
+   IO *dst = box + w*n;
+   const IO *src[GB_Q];
+#  pragma unroll
+   for (int k=0; k<GB_Q; k++)
    {
-      const int y = e / g.size[0], x = e - y*g.size[0];
-      const int X = x + g.origin[0], Y = y + g.origin[1];
-      const int s = sl[ ( Y >> 3 )*g.tdim[0] + ( X >> 3 ) ];
-      if ( s >= 0 ) dst[ e ] = patch[ ( ( (size_t)s*NV + v )*H + ( Z & 7 ) )*H*H + ( Y & 7 )*H + ( X & 7 ) ];
+      const long e = e0 + k*GB_NT;
+      src[k] = nullptr;
+      if ( e >= n ) continue;
+      const unsigned z = ( n >> 32 ) ? (unsigned)( e / nxy ) : (unsigned)e / nxy, r = (unsigned)( e - (long)z*nxy ), y = r / nx, x = r - y*nx;
+      const int X = (int)x + g.origin[0], Y = (int)y + g.origin[1], Z = (int)z + g.origin[2];
+      const int s = sl[ ( (size_t)( Z >> 3 )*g.tdim[1] + ( Y >> 3 ) )*g.tdim[0] + ( X >> 3 ) ];
+      if ( s >= 0 ) src[k] = pv + ( (size_t)s*NV*P3 + ( Z & 7 )*H*H + ( Y & 7 )*H + ( X & 7 ) );
    }
+   IO val[GB_Q];
+#  pragma unroll
+   for (int k=0; k<GB_Q; k++) if ( src[k] ) val[k] = *src[k];
+#  pragma unroll
+   for (int k=0; k<GB_Q; k++) if ( src[k] ) dst[ e0 + k*GB_NT ] = val[k];
 }
 
 } // namespace
@@ -525,7 +460,10 @@ template <typename T>
 int launch_interpolate( T *cdata, T *fdata, int nbox, const InterpPrm &p, int *nfail, hipStream_t stream )
 {
    if ( nbox <= 0 ) return 0;
-#  define GA_INT( S ) hipLaunchKernelGGL( ( interpolate_kernel<T, S> ), dim3( nbox ), dim3( NT ), 0, stream, cdata, fdata, nbox, p, nfail )
+   const bool plain = ( p.mono & 0x1F ) == 0x1F && !p.opp0;
+#  define GA_INT( S ) { if ( plain ) GA_LAUNCH( S, true ); else GA_LAUNCH( S, false ); }
+#  define GA_LAUNCH( S, PLAIN_ ) hipLaunchKernelGGL( ( interpolate_kernel<T, S, PLAIN_> ), dim3( nbox ), dim3( interp_lanes<T>( S ) ), 0, stream, \
+                                                    cdata, fdata, nbox, p, nfail )
    switch ( p.scheme )
    {
       case 1: GA_INT( 1 ); break;
@@ -538,6 +476,7 @@ int launch_interpolate( T *cdata, T *fdata, int nbox, const InterpPrm &p, int *n
       default: return -1;
    }
 #  undef GA_INT
+#  undef GA_LAUNCH
    return ( hipGetLastError() == hipSuccess ) ? 0 : -2;
 }
 
@@ -551,7 +490,9 @@ template <typename IO>
 int launch_gather_boxes( const IO *patch, IO *box, int nbox, const BoxGeom &g, const int *slot, hipStream_t stream )
 {
    if ( nbox <= 0 ) return 0;
-   hipLaunchKernelGGL( gather_boxes_kernel<IO>, dim3( nbox, NV, g.size[2] ), dim3( CPX, CPY ), 0, stream, patch, box, g, slot );
+   const long n = (long)g.size[0]*g.size[1]*g.size[2], chunks = ( n + GB_N - 1 )/GB_N;
+   hipLaunchKernelGGL( gather_boxes_kernel<IO>, dim3( nbox, NV, (unsigned)chunks ), dim3( GB_NT ), 0, stream, patch, box, g, slot,
+                       (unsigned)chunks );
    return ( hipGetLastError() == hipSuccess ) ? 0 : -2;
 }
 
@@ -560,9 +501,9 @@ int launch_assemble( const IO *patch, const IO *fbox, IO *pg_in, int npg, const 
                      hipStream_t stream )
 {
    if ( npg <= 0 ) return 0;
-   const int n = PS + 2*ghost, per = NT*EPT;
-   hipLaunchKernelGGL( prepare_patches_kernel<IO>, dim3( npg, NV, ( n*n*n + per - 1 )/per ), dim3( NT ), 0, stream, patch, fbox,
-                       pg_in, slot, ghost, fb );
+   const int n = PS + 2*ghost;
+   hipLaunchKernelGGL( prepare_patches_kernel<IO>, dim3( npg, NV, ( n*n*n + PREP_N - 1 )/PREP_N ), dim3( PREP_NT ), 0, stream,
+                       patch, fbox, pg_in, slot, ghost, fb );
    return ( hipGetLastError() == hipSuccess ) ? 0 : -2;
 }
 
