@@ -105,68 +105,48 @@ constexpr Box HALF_CELLS = { 1, 1, 1, 20, 20, 20 }, CORE_CELLS = { 3, 3, 3, 16, 
 
 // ---------------- pieces of the step, generic in the arithmetic type ----------------
 // cell-centred interface state of the half step (pressure recovery + floor, 1/rho, sound speed)
-template <int D, typename T>
-__device__ __forceinline__ St<T> cell_st( const T u[NV], const Prm<T> &P )
+template <typename T>
+__device__ __forceinline__ St<T> cell_st( int d, const T u[NV], const Prm<T> &P )
 {
    const T ir = rcp( u[0] );
    const T eint = u[4] - (T)0.5*( u[1]*u[1] + u[2]*u[2] + u[3]*u[3] )*ir;
    const T p = floor_pres( eint*P.gm1, P.min_pres );
-   return cell_state<D>( u, p, ir, vsqrt( P.gamma*p*ir ) );
+   return cell_state( d, u, p, ir, vsqrt( P.gamma*p*ir ) );
 }
 
 template <int RS, typename T>
 __device__ __forceinline__ void half_flux( int d, const T uL[NV], const T uR[NV], const Prm<T> &P, T f[NV] )
 {
-   if      ( d == 0 ) riemann<RS, 0>( cell_st<0>( uL, P ), cell_st<0>( uR, P ), P, f );
-   else if ( d == 1 ) riemann<RS, 1>( cell_st<1>( uL, P ), cell_st<1>( uR, P ), P, f );
-   else               riemann<RS, 2>( cell_st<2>( uL, P ), cell_st<2>( uR, P ), P, f );
+   riemann<RS>( d, cell_st( d, uL, P ), cell_st( d, uR, P ), P, f );
 }
 
 template <int RS, typename T>
 __device__ __forceinline__ void full_flux( int d, const T wL[NV], const T wR[NV], const Prm<T> &P, T f[NV] )
 {
-   if      ( d == 0 ) riemann<RS, 0>( face_state<0>( wL, P ), face_state<0>( wR, P ), P, f );
-   else if ( d == 1 ) riemann<RS, 1>( face_state<1>( wL, P ), face_state<1>( wR, P ), P, f );
-   else               riemann<RS, 2>( face_state<2>( wL, P ), face_state<2>( wR, P ), P, f );
+   riemann<RS>( d, face_state( d, wL, P ), face_state( d, wR, P ), P, f );
 }
 
 // reverse sweeps of half_flux / full_flux: bL, bR = (d flux / d input side)^T bf, one pass
-template <int RS, int D>
-__device__ __forceinline__ void half_flux_rev_d( const double uL[NV], const double uR[NV], const Prm<double> &P,
-                                                 const double bf[NV], double bL[NV], double bR[NV] )
-{
-   const StD L = cell_st<D>( uL, P ), Q = cell_st<D>( uR, P );
-   StD sL, sQ;
-   riemann_rev<RS, D>( L, Q, P, bf, sL, sQ );
-   cell_st_rev<D>( uL, L, sL, P, bL );
-   cell_st_rev<D>( uR, Q, sQ, P, bR );
-}
 template <int RS>
 __device__ __forceinline__ void half_flux_rev( int d, const double uL[NV], const double uR[NV], const Prm<double> &P,
                                                const double bf[NV], double bL[NV], double bR[NV] )
 {
-   if      ( d == 0 ) half_flux_rev_d<RS, 0>( uL, uR, P, bf, bL, bR );
-   else if ( d == 1 ) half_flux_rev_d<RS, 1>( uL, uR, P, bf, bL, bR );
-   else               half_flux_rev_d<RS, 2>( uL, uR, P, bf, bL, bR );
+   const StD L = cell_st( d, uL, P ), Q = cell_st( d, uR, P );
+   StD sL, sQ;
+   riemann_rev<RS>( d, L, Q, P, bf, sL, sQ );
+   cell_st_rev( d, uL, L, sL, P, bL );
+   cell_st_rev( d, uR, Q, sQ, P, bR );
 }
 
-template <int RS, int D>
-__device__ __forceinline__ void full_flux_rev_d( const double wL[NV], const double wR[NV], const Prm<double> &P,
-                                                 const double bf[NV], double bL[NV], double bR[NV] )
-{
-   const StD L = face_state<D>( wL, P ), Q = face_state<D>( wR, P );
-   StD sL, sQ;
-   riemann_rev<RS, D>( L, Q, P, bf, sL, sQ );
-   face_state_rev<D>( wL, L, sL, P, bL );
-   face_state_rev<D>( wR, Q, sQ, P, bR );
-}
 template <int RS>
 __device__ __forceinline__ void full_flux_rev( int d, const double wL[NV], const double wR[NV], const Prm<double> &P,
                                                const double bf[NV], double bL[NV], double bR[NV] )
 {
-   if      ( d == 0 ) full_flux_rev_d<RS, 0>( wL, wR, P, bf, bL, bR );
-   else if ( d == 1 ) full_flux_rev_d<RS, 1>( wL, wR, P, bf, bL, bR );
-   else               full_flux_rev_d<RS, 2>( wL, wR, P, bf, bL, bR );
+   const StD L = face_state( d, wL, P ), Q = face_state( d, wR, P );
+   StD sL, sQ;
+   riemann_rev<RS>( d, L, Q, P, bf, sL, sQ );
+   face_state_rev( d, wL, L, sL, P, bL );
+   face_state_rev( d, wR, Q, sQ, P, bR );
 }
 
 // half-step conserved state -> density floor, internal-energy floor, primitive variables with pressure floor

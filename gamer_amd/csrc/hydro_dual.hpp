@@ -71,6 +71,14 @@ struct Dual {
    friend __device__ __forceinline__ bool operator!=( const Dual &a, const Dual &b ) { return a.v != b.v; }
 };
 
+template <int N> __device__ __forceinline__ Dual<N> sel( bool c, const Dual<N> &a, const Dual<N> &b )
+{
+   Dual<N> r;  r.v = c ? a.v : b.v;
+#  pragma unroll
+   for (int k=0; k<N; k++) r.d[k] = c ? a.d[k] : b.d[k];
+   return r;
+}
+
 // a*b + c with the value rounded once, as the plain-type fmad
 template <int N> __device__ __forceinline__ Dual<N> fmad( const Dual<N> &a, const Dual<N> &b, const Dual<N> &c )
 {
@@ -98,14 +106,14 @@ template <int N> __device__ __forceinline__ Dual<N> vsqrt( const Dual<N> &a )
 }
 // fmax/fmin semantics: a NaN operand loses
 template <int N> __device__ __forceinline__ Dual<N> vmax( const Dual<N> &a, const Dual<N> &b )
-{ return ( b.v != b.v || a.v >= b.v ) ? a : b; }
+{ return sel( b.v != b.v || a.v >= b.v, a, b ); }
 template <int N> __device__ __forceinline__ Dual<N> vmin( const Dual<N> &a, const Dual<N> &b )
-{ return ( b.v != b.v || a.v <= b.v ) ? a : b; }
-template <int N> __device__ __forceinline__ Dual<N> vabs( const Dual<N> &a ) { return __builtin_signbit( a.v ) ? -a : a; }
+{ return sel( b.v != b.v || a.v <= b.v, a, b ); }
+template <int N> __device__ __forceinline__ Dual<N> vabs( const Dual<N> &a ) { return sel( __builtin_signbit( a.v ), -a, a ); }
 template <int N> __device__ __forceinline__ Dual<N> vcopysign( const Dual<N> &m, const Dual<N> &s )
 {
    const Dual<N> am = vabs( m );
-   return __builtin_signbit( s.v ) ? -am : am;
+   return sel( __builtin_signbit( s.v ), -am, am );
 }
 template <int N> __device__ __forceinline__ Dual<N> clamp_between( const Dual<N> &x, const Dual<N> &a, const Dual<N> &b )
 { return vmin( vmax( x, vmin( a, b ) ), vmax( a, b ) ); }

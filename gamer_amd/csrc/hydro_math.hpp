@@ -129,6 +129,30 @@ struct Batch {
    int           whole, slabs;
 };
 
+// c ? a : b as a select of values; of dual numbers, part by part (hydro_dual.hpp)
+template <typename R> __device__ __forceinline__ R sel( bool c, R a, R b ) { return c ? a : b; }
+
+// vector components of the axes (x, y, z) <-> those of a d-normal face (normal, two tangential ones).  d is a run-time
+// value: one solve serves all three directions.  With a copy of the solve per direction, lanes of different directions
+// ran them one after the other, and the compiler merged the copies' ends through scratch memory.
+// FP64 derivative kernels, with the reverse sweeps and dual numbers in selects of values, copies -> run time: half-step
+// reverse faces of 512 patch groups 674 -> 528 us, half-step fluxes 316 -> 264; dual numbers on 125: 157 -> 129 and full-step
+// faces 124 -> 103.  Same bits.
+template <typename R>
+__device__ __forceinline__ void to_face( int d, R x, R y, R z, R &n, R &a, R &b )
+{
+   n = sel( d == 0, x, sel( d == 1, y, z ) );
+   a = sel( d == 0, y, sel( d == 1, z, x ) );
+   b = sel( d == 0, z, sel( d == 1, x, y ) );
+}
+template <typename R>
+__device__ __forceinline__ void from_face( int d, R n, R a, R b, R &x, R &y, R &z )
+{
+   x = sel( d == 0, n, sel( d == 1, b, a ) );
+   y = sel( d == 0, a, sel( d == 1, n, b ) );
+   z = sel( d == 0, b, sel( d == 1, a, n ) );
+}
+
 // an interface state rotated to the face normal: conserved fields + derived quantities
 template <typename R>
 struct St { R d, mn, m1, m2, e, p, ir, cs, u; };
@@ -171,7 +195,7 @@ __device__ __forceinline__ void rs_hlle( const St<R> &L, const St<R> &Q, R f[NV]
    const bool both0 = ( sl == Z ) && ( sr == Z );
    const R inv = rcp( sr - sl );
 #  pragma unroll
-   for (int v=0; v<NV; v++) f[v] = both0 ? fl[v] : inv*( sr*fl[v] - sl*fr[v] );
+   for (int v=0; v<NV; v++) f[v] = sel( both0, fl[v], inv*( sr*fl[v] - sl*fr[v] ) );
 }
 
 template <typename R>
@@ -181,8 +205,8 @@ __device__ __forceinline__ void rs_hllc( const St<R> &L, const St<R> &Q, R pmin,
    const R wl1 = L.u - L.cs, wl2 = Q.u - Q.cs, wr1 = L.u + L.cs, wr2 = Q.u + Q.cs;
    const R wl = vmin( wl1, wl2 ), wr = vmax( wr1, wr2 );
    const R du = L.u - Q.u;
-   const R tl =  L.d*( ( wl1 < wl2 ) ? L.cs : du + Q.cs );
-   const R tr = -Q.d*( ( wr2 > wr1 ) ? Q.cs : du + L.cs );
+   const R tl =  L.d*sel( wl1 < wl2, L.cs, du + Q.cs );
+   const R tr = -Q.d*sel( wr2 > wr1, Q.cs, du + L.cs );
    const R t2 = rcp( tl - tr );
    const R vs = t2*( L.p - Q.p + tl*L.u - tr*Q.u );
    R ps = t2*( tl*( Q.p + tr*Q.u ) - tr*( L.p + tl*L.u ) );
@@ -190,16 +214,16 @@ __device__ __forceinline__ void rs_hllc( const St<R> &L, const St<R> &Q, R pmin,
 
    const bool left = ( vs >= Z );
    St<R> s;
-   s.d  = left ? L.d  : Q.d;   s.mn = left ? L.mn : Q.mn;  s.m1 = left ? L.m1 : Q.m1;
-   s.m2 = left ? L.m2 : Q.m2;  s.e  = left ? L.e  : Q.e;   s.p  = left ? L.p  : Q.p;
-   s.u  = left ? L.u  : Q.u;
-   const R sp = left ? vmin( wl, Z ) : vmax( wr, Z );
+   s.d  = sel( left, L.d,  Q.d );   s.mn = sel( left, L.mn, Q.mn );  s.m1 = sel( left, L.m1, Q.m1 );
+   s.m2 = sel( left, L.m2, Q.m2 );  s.e  = sel( left, L.e,  Q.e );   s.p  = sel( left, L.p,  Q.p );
+   s.u  = sel( left, L.u,  Q.u );
+   const R sp = sel( left, vmin( wl, Z ), vmax( wr, Z ) );
    R F[NV];
    xflux_minus( s, sp, F );
    const bool deg = left && ( vs == Z ) && ( sp == Z );
    const R t4 = rcp( vs - sp );
-   const R cf = deg ? ONE : t4*vs;
-   const R cs = deg ? Z   : -t4*sp*ps;
+   const R cf = sel( deg, ONE, t4*vs );
+   const R cs = sel( deg, Z, -t4*sp*ps );
    f[0] = cf*F[0];
    f[1] = cf*F[1] + cs;
    f[2] = cf*F[2];
@@ -345,14 +369,15 @@ __device__ __forceinline__ void plm_face( R L, R C, R Rr, int lim, R coeff, R &f
    fR = fr;
 }
 
-// primitive face state (rho, vx, vy, vz, P) -> interface state rotated to direction D
+// primitive face state (rho, vx, vy, vz, P) -> interface state rotated to direction d
 // (Pri2Con, FluUtility.cpp:343-420; the solver takes the face pressure and velocity directly instead of
 // recovering them from the conserved face state)
-template <int D, typename R>
-__device__ __forceinline__ St<R> face_state( const R w[NV], const Prm<R> &P )
+template <typename R>
+__device__ __forceinline__ St<R> face_state( int d, const R w[NV], const Prm<R> &P )
 {
    St<R> s;
-   const R vn = w[1 + D], v1 = w[1 + ( D + 1 ) % 3], v2 = w[1 + ( D + 2 ) % 3];
+   R vn, v1, v2;
+   to_face( d, w[1], w[2], w[3], vn, v1, v2 );
    s.d  = w[0];
    s.mn = w[0]*vn;
    s.m1 = w[0]*v1;
@@ -365,15 +390,13 @@ __device__ __forceinline__ St<R> face_state( const R w[NV], const Prm<R> &P )
    return s;
 }
 
-// conserved cell (with its pressure, 1/rho and sound speed) -> interface state rotated to direction D
-template <int D, typename R>
-__device__ __forceinline__ St<R> cell_state( const R c[NV], R p, R ir, R cs )
+// conserved cell (with its pressure, 1/rho and sound speed) -> interface state rotated to direction d
+template <typename R>
+__device__ __forceinline__ St<R> cell_state( int d, const R c[NV], R p, R ir, R cs )
 {
    St<R> s;
    s.d  = c[0];
-   s.mn = c[1 + D];
-   s.m1 = c[1 + ( D + 1 ) % 3];
-   s.m2 = c[1 + ( D + 2 ) % 3];
+   to_face( d, c[1], c[2], c[3], s.mn, s.m1, s.m2 );
    s.e  = c[4];
    s.p  = p;  s.ir = ir;  s.cs = cs;
    s.u  = ir*s.mn;
@@ -394,10 +417,10 @@ __device__ __forceinline__ bool any_nan5( const float f[NV] )
    return m != m;
 }
 
-// Riemann solve across a D-normal face; flux returned in the lab frame.  HLLC falls back to HLLE when a flux
+// Riemann solve across a d-normal face; flux returned in the lab frame.  HLLC falls back to HLLE when a flux
 // component is NaN (RSOLVER_RESCUE, CPU_FluidSolver_MHM.cpp:737-786, ComputeFlux.cpp:313-362).
-template <int RS, int D, typename R>
-__device__ __forceinline__ void riemann( const St<R> &L, const St<R> &Q, const Prm<R> &P, R out[NV] )
+template <int RS, typename R>
+__device__ __forceinline__ void riemann( int d, const St<R> &L, const St<R> &Q, const Prm<R> &P, R out[NV] )
 {
    R f[NV];
    if ( RS == 4 )
@@ -409,9 +432,7 @@ __device__ __forceinline__ void riemann( const St<R> &L, const St<R> &Q, const P
    else                rs_roe( L, Q, P, f );
    out[0] = f[0];
    out[4] = f[4];
-   out[1 + D]             = f[1];
-   out[1 + ( D + 1 ) % 3] = f[2];
-   out[1 + ( D + 2 ) % 3] = f[3];
+   from_face( d, f[1], f[2], f[3], out[1], out[2], out[3] );
 }
 
 // conserved face state -> interface state rotated to direction D, pressure recovered in FP64

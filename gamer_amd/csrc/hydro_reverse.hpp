@@ -42,9 +42,20 @@ __device__ __forceinline__ void xflux_minus_rev( const StD &s, double sp, const 
    bsp   -= s.d*bF[0] + s.mn*bF[1] + s.m1*bF[2] + s.m2*bF[3] + s.e*bF[4];
 }
 
-__device__ __forceinline__ void add_upwind( StD &b, const StD &bs )
+// The branches of the sweeps are selects of values, never of references (which would put the states in scratch memory)
+// and never jumps (which would cut the chains of both sides apart): add_if adds x where c holds.
+__device__ __forceinline__ void add_if( bool c, double &b, double x ) { const double t = b + x;  b = c ? t : b; }
+__device__ __forceinline__ void add_side( bool c, StD &b, const StD &bs )
 {
-   b.d += bs.d;  b.mn += bs.mn;  b.m1 += bs.m1;  b.m2 += bs.m2;  b.e += bs.e;  b.p += bs.p;  b.u += bs.u;
+   add_if( c, b.d, bs.d );    add_if( c, b.mn, bs.mn );  add_if( c, b.m1, bs.m1 );  add_if( c, b.m2, bs.m2 );
+   add_if( c, b.e, bs.e );    add_if( c, b.p, bs.p );    add_if( c, b.u, bs.u );
+}
+__device__ __forceinline__ StD pick( bool c, const StD &a, const StD &b )
+{
+   StD s;
+   s.d  = c ? a.d  : b.d;   s.mn = c ? a.mn : b.mn;  s.m1 = c ? a.m1 : b.m1;  s.m2 = c ? a.m2 : b.m2;  s.e = c ? a.e : b.e;
+   s.p  = c ? a.p  : b.p;   s.ir = c ? a.ir : b.ir;  s.cs = c ? a.cs : b.cs;  s.u  = c ? a.u  : b.u;
+   return s;
 }
 
 // HLLE: sl = min(min(uL-cL, uR-cR), 0), sr = max(max(uL+cL, uR+cR), 0),
@@ -85,8 +96,8 @@ __device__ __forceinline__ void rs_hlle_rev( const StD &L, const StD &Q, const d
    xflux_minus_rev( L, sl, bfl, bL, bsl );
    xflux_minus_rev( Q, sr, bfr, bQ, bsr );
    const double bslr = kl ? bsl : 0.0, bsrr = kr ? bsr : 0.0;
-   if ( k1 ) { bL.u += bslr;  bL.cs -= bslr; } else { bQ.u += bslr;  bQ.cs -= bslr; }
-   if ( k2 ) { bL.u += bsrr;  bL.cs += bsrr; } else { bQ.u += bsrr;  bQ.cs += bsrr; }
+   add_if( k1, bL.u, bslr );  add_if( k1, bL.cs, -bslr );  add_if( !k1, bQ.u, bslr );  add_if( !k1, bQ.cs, -bslr );
+   add_if( k2, bL.u, bsrr );  add_if( k2, bL.cs,  bsrr );  add_if( !k2, bQ.u, bsrr );  add_if( !k2, bQ.cs,  bsrr );
 }
 
 // HLLC (rs_hllc).  Returns false, with nothing accumulated, when the forward flux has a NaN component: the
@@ -108,7 +119,7 @@ __device__ __forceinline__ bool rs_hllc_rev( const StD &L, const StD &Q, double 
    const bool   pk = !( psr < pmin );
    const double ps = pk ? psr : pmin;
    const bool   left = ( vs >= 0.0 );
-   const StD   &s = left ? L : Q;
+   const StD    s = pick( left, L, Q );
    const bool   spk = left ? min_first( wl, 0.0 ) : max_first( wr, 0.0 );
    const double sp = spk ? ( left ? wl : wr ) : 0.0;
    double F[NV];
@@ -132,21 +143,20 @@ __device__ __forceinline__ bool rs_hllc_rev( const StD &L, const StD &Q, double 
    for (int v=0; v<NV; v++) { bF[v] = cf*bf[v];  bcf += bf[v]*F[v]; }
    const double bcs = bf[1] + bf[4]*vs;
    double bvs = bf[4]*cs, bsp = 0.0, bps = 0.0;
-   if ( !deg )
    {
       // cf = t4 vs, cs = (-t4) sp ps, t4 = 1/(vs - sp)
       const double bt4 = bcf*vs - bcs*sp*ps;
-      bvs += bcf*t4;
-      bsp -= bcs*t4*ps;
-      bps -= bcs*t4*sp;
       const double bdf = -t4*t4*bt4;
-      bvs += bdf;
-      bsp -= bdf;
+      const double v1 = ( bvs + bcf*t4 ) + bdf, p1 = ( bsp - bcs*t4*ps ) - bdf, s1 = bps - bcs*t4*sp;
+      bvs = deg ? bvs : v1;
+      bsp = deg ? bsp : p1;
+      bps = deg ? bps : s1;
    }
    StD bs;
    st_zero( bs );
    xflux_minus_rev( s, sp, bF, bs, bsp );
-   add_upwind( left ? bL : bQ, bs );
+   add_side(  left, bL, bs );
+   add_side( !left, bQ, bs );
    const double bwl = ( spk &&  left ) ? bsp : 0.0;
    const double bwr = ( spk && !left ) ? bsp : 0.0;
 
@@ -172,13 +182,13 @@ __device__ __forceinline__ bool rs_hllc_rev( const StD &L, const StD &Q, double 
    bQ.d -= btr*XR;
    const double bXL = btl*L.d, bXR = -btr*Q.d;
    double bdu = 0.0;
-   if ( cl ) bL.cs += bXL; else { bdu += bXL;  bQ.cs += bXL; }
-   if ( cr ) bQ.cs += bXR; else { bdu += bXR;  bL.cs += bXR; }
+   add_if( cl, bL.cs, bXL );  add_if( !cl, bdu, bXL );  add_if( !cl, bQ.cs, bXL );
+   add_if( cr, bQ.cs, bXR );  add_if( !cr, bdu, bXR );  add_if( !cr, bL.cs, bXR );
    bL.u += bdu;
    bQ.u -= bdu;
    // wl = min(wl1, wl2), wr = max(wr1, wr2)
-   if ( kl ) { bL.u += bwl;  bL.cs -= bwl; } else { bQ.u += bwl;  bQ.cs -= bwl; }
-   if ( kr ) { bL.u += bwr;  bL.cs += bwr; } else { bQ.u += bwr;  bQ.cs += bwr; }
+   add_if( kl, bL.u, bwl );  add_if( kl, bL.cs, -bwl );  add_if( !kl, bQ.u, bwl );  add_if( !kl, bQ.cs, -bwl );
+   add_if( kr, bL.u, bwr );  add_if( kr, bL.cs,  bwr );  add_if( !kr, bQ.u, bwr );  add_if( !kr, bQ.cs,  bwr );
    return true;
 }
 
@@ -209,8 +219,10 @@ __device__ __forceinline__ void rs_roe_rev( const StD &L, const StD &Q, const Pr
    if ( e0 >= 0.0 || e4 <= 0.0 )                 // supersonic: the upwind physical flux
    {
       st_zero( bs );
-      xflux_minus_rev( ( e0 >= 0.0 ) ? L : Q, 0.0, bf, bs, bsp );
-      add_upwind( ( e0 >= 0.0 ) ? bL : bQ, bs );
+      const bool left = ( e0 >= 0.0 );
+      xflux_minus_rev( pick( left, L, Q ), 0.0, bf, bs, bsp );
+      add_side(  left, bL, bs );
+      add_side( !left, bQ, bs );
       return;
    }
    const double j0 = Q.d - L.d, j1 = Q.mn - L.mn, j2 = Q.m1 - L.m1, j3 = Q.m2 - L.m2, j4 = Q.e - L.e;
@@ -238,10 +250,10 @@ __device__ __forceinline__ void rs_roe_rev( const StD &L, const StD &Q, const Pr
    for (int k=0; k<NV; k++) bh[k] = HALF*bf[k];
    st_zero( bs );
    xflux_minus_rev( L, 0.0, bh, bs, bsp );
-   add_upwind( bL, bs );
+   add_side( true, bL, bs );
    st_zero( bs );
    xflux_minus_rev( Q, 0.0, bh, bs, bsp );
-   add_upwind( bQ, bs );
+   add_side( true, bQ, bs );
    const double bA0 = -( bh[0] + bh[1]*e0 + bh[2]*v + bh[3]*w + bh[4]*( H - u*a ) );
    const double bA1 = -( bh[0] + bh[1]*u  + bh[2]*v + bh[3]*w + bh[4]*( HALF*V2 ) );
    const double bA2 = -( bh[2] + bh[4]*v );
@@ -321,17 +333,15 @@ __device__ __forceinline__ void rs_roe_rev( const StD &L, const StD &Q, const Pr
    bQ.ir += bhr*( Q.e + Q.p );  bQ.e += bhr*Q.ir;  bQ.p += bhr*Q.ir;
 }
 
-// riemann<RS, D> (HLLC with the HLLE rescue, HLLE, or Roe): bout is the adjoint of the lab-frame flux
-template <int RS, int D>
-__device__ __forceinline__ void riemann_rev( const StD &L, const StD &Q, const Prm<double> &P, const double bout[NV],
+// riemann<RS> across a d-normal face (HLLC with the HLLE rescue, HLLE, or Roe): bout is the adjoint of the lab-frame flux
+template <int RS>
+__device__ __forceinline__ void riemann_rev( int d, const StD &L, const StD &Q, const Prm<double> &P, const double bout[NV],
                                              StD &bL, StD &bQ )
 {
    static_assert( RS == 2 || RS == 3 || RS == 4, "reverse sweeps exist for Roe, HLLE and HLLC" );
    double bf[NV];
    bf[0] = bout[0];
-   bf[1] = bout[1 + D];
-   bf[2] = bout[1 + ( D + 1 ) % 3];
-   bf[3] = bout[1 + ( D + 2 ) % 3];
+   to_face( d, bout[1], bout[2], bout[3], bf[1], bf[2], bf[3] );
    bf[4] = bout[4];
    st_zero( bL );
    st_zero( bQ );
@@ -340,12 +350,13 @@ __device__ __forceinline__ void riemann_rev( const StD &L, const StD &Q, const P
    rs_hlle_rev( L, Q, bf, bL, bQ );
 }
 
-// face_state<D>: primitive face (rho, vx, vy, vz, P) -> interface state; bw accumulates
-template <int D>
-__device__ __forceinline__ void face_state_rev( const double w[NV], const StD &s, const StD &bs, const Prm<double> &P,
+// face_state: primitive face (rho, vx, vy, vz, P) -> interface state; bw accumulates
+__device__ __forceinline__ void face_state_rev( int d, const double w[NV], const StD &s, const StD &bs, const Prm<double> &P,
                                                 double bw[NV] )
 {
-   constexpr int IN = 1 + D, I1 = 1 + ( D + 1 ) % 3, I2 = 1 + ( D + 2 ) % 3;
+   double wn, w1, w2, x, y, z;
+   to_face( d, w[1], w[2], w[3], wn, w1, w2 );
+   from_face( d, bs.mn*w[0] + bs.u, bs.m1*w[0], bs.m2*w[0], x, y, z );
    const double K = fmad( w[3], w[3], fmad( w[2], w[2], w[1]*w[1] ) );
    // cs = sqrt(gamma p ir)
    const double bx = bs.cs*( 0.5/s.cs );
@@ -353,10 +364,10 @@ __device__ __forceinline__ void face_state_rev( const double w[NV], const StD &s
    const double bir = bs.ir + bx*P.gamma*s.p;
    // e = (0.5 rho) K + P/(gamma-1)
    const double bK = bs.e*0.5*w[0];
-   bw[0]  += bs.d + bs.mn*w[IN] + bs.m1*w[I1] + bs.m2*w[I2] + bs.e*0.5*K - s.ir*s.ir*bir;
-   bw[IN] += bs.mn*w[0] + bs.u;
-   bw[I1] += bs.m1*w[0];
-   bw[I2] += bs.m2*w[0];
+   bw[0]  += bs.d + bs.mn*wn + bs.m1*w1 + bs.m2*w2 + bs.e*0.5*K - s.ir*s.ir*bir;
+   bw[1]  += x;
+   bw[2]  += y;
+   bw[3]  += z;
    bw[1]  += 2.0*bK*w[1];
    bw[2]  += 2.0*bK*w[2];
    bw[3]  += 2.0*bK*w[3];
@@ -365,11 +376,11 @@ __device__ __forceinline__ void face_state_rev( const double w[NV], const StD &s
 
 // conserved cell -> interface state: ir = 1/rho, p = max((gamma-1)(E - |m|^2 ir/2), MinPres),
 // cs = sqrt(gamma p ir), u = ir m_n; bu accumulates
-template <int D>
-__device__ __forceinline__ void cell_st_rev( const double u[NV], const StD &s, const StD &bs, const Prm<double> &P,
+__device__ __forceinline__ void cell_st_rev( int d, const double u[NV], const StD &s, const StD &bs, const Prm<double> &P,
                                              double bu[NV] )
 {
-   constexpr int IN = 1 + D, I1 = 1 + ( D + 1 ) % 3, I2 = 1 + ( D + 2 ) % 3;
+   double x, y, z;
+   from_face( d, bs.mn + bs.u*s.ir, bs.m1, bs.m2, x, y, z );
    const double S = 0.5*( u[1]*u[1] + u[2]*u[2] + u[3]*u[3] );
    const double eint = u[4] - S*s.ir;
    const double bx = bs.cs*( 0.5/s.cs );
@@ -379,9 +390,9 @@ __device__ __forceinline__ void cell_st_rev( const double u[NV], const StD &s, c
    const double bS = -beint*s.ir;
    bir -= beint*S;
    bu[0]  += bs.d - s.ir*s.ir*bir;
-   bu[IN] += bs.mn + bs.u*s.ir;
-   bu[I1] += bs.m1;
-   bu[I2] += bs.m2;
+   bu[1]  += x;
+   bu[2]  += y;
+   bu[3]  += z;
    bu[1]  += bS*u[1];
    bu[2]  += bS*u[2];
    bu[3]  += bS*u[3];
@@ -396,8 +407,7 @@ __device__ __forceinline__ int clamp_pick( double x, double a, double b )
    const double lo = lo_a ? a : b, hi = hi_a ? a : b;
    const bool   x1_x = max_first( x, lo );
    const double x1 = x1_x ? x : lo;
-   if ( min_first( x1, hi ) ) return x1_x ? 0 : ( lo_a ? 1 : 2 );
-   return hi_a ? 1 : 2;
+   return min_first( x1, hi ) ? ( x1_x ? 0 : ( lo_a ? 1 : 2 ) ) : ( hi_a ? 1 : 2 );
 }
 
 // plm_face<LIM>: faces fL, fR of the centre C from (L, C, R).  Given their adjoints (bfL, bfR), accumulate the
@@ -420,11 +430,13 @@ __device__ __forceinline__ void plm_face_rev( double L, double C, double Rr, int
    // reverse
    const double bfr = bfR - bfL;
    double bc = 2.0*bfL, bl = 0.0, br = 0.0;
-   double bx2 = 0.0, bx1 = 0.0;
-   if ( p2 == 0 ) bx2 = bfr; else if ( p2 == 1 ) bc += bfr; else br += bfr;
+   const double bx2 = ( p2 == 0 ) ? bfr : 0.0;
+   add_if( p2 == 1, bc, bfr );
+   add_if( p2 == 2, br, bfr );
    bc += 2.0*bx2;
-   const double bfl = -bx2;
-   if ( p1 == 0 ) bx1 = bfl; else if ( p1 == 1 ) bc += bfl; else bl += bfl;
+   const double bfl = -bx2, bx1 = ( p1 == 0 ) ? bfl : 0.0;
+   add_if( p1 == 1, bc, bfl );
+   add_if( p1 == 2, bl, bfl );
    bc += bx1;
    const double bs = -0.5*bx1;
    const double bsl = bs*s.d[0], bsr = bs*s.d[1];
