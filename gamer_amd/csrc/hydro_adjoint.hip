@@ -5,19 +5,18 @@
 // Explicit phases over a per-PG global workspace, each phase one kernel over all patch groups with one face or
 // cell per lane:
 //
-//   forward   F1 + F2, one z plane per workgroup: half-step fluxes (Hydro_RiemannPredict_Flux) in LDS, then the
-//                half-step update, floors and primitive W (Hydro_RiemannPredict) -> ws
+//   forward   F1 + F2, z plane by z plane: half-step fluxes (Hydro_RiemannPredict_Flux) in LDS, then the half-step
+//                update, floors and primitive W (Hydro_RiemannPredict) -> ws
 //             F4 (tangent / plain forward only) PLM faces (Hydro_DataReconstruction) and the full-step flux of
 //                each face, then the update of the 16^3 output cells
 //   reverse   R4 lambda_F of each full-step face from lambda_out (transpose of Hydro_FullStepUpdate),
 //                lambda_FC = J_RS^T lambda_F (transpose of Hydro_ComputeFlux), with the two PLM faces of the
 //                face recomputed from W
-//             R3 lambda_W = sum over the three stencil cells of J_PLM^T lambda_FC (transpose of the limiter,
-//                face clamp and mirror), one line march per direction
-//             R2 lambda_U_half = J_Con2Pri^T lambda_W (transpose of the floors and primitive conversion)
-//             R1 + R0, one z plane per workgroup: lambda of every half-step face, J_RS^T of the cell-centred
-//                half-step solve per side, and lambda_in = lambda_out (core) + lambda_U_half + the half-step face
-//                contributions (the z faces' upper sides added by a second, small kernel)
+//             R3 + R2, z plane by z plane: lambda_W = sum over the three stencil cells of J_PLM^T lambda_FC
+//                (transpose of the limiter, face clamp and mirror) in LDS, then lambda_U_half = J_Con2Pri^T lambda_W
+//                (transpose of the floors and primitive conversion) -> ws
+//             R1 + R0, z plane by z plane: lambda of every half-step face, J_RS^T of the cell-centred half-step
+//                solve per side, and lambda_in = lambda_out (core) + lambda_U_half + the half-step face contributions
 //
 // The reverse sweep is written out by hand.  The Riemann solves (HLLC, HLLE and Roe) run backwards as hand-written
 // reverse-mode sweeps (hydro_reverse.hpp: solver + interface-state builders, one pass per face for all ten
@@ -58,14 +57,22 @@ constexpr int STRIDE[3] = { 1, NX, N2 };
 
 // workspace layout per patch group, in units of N3 doubles.  Written / last read by:
 constexpr int WS_W   = 0;            // [5]       half-step primitives (cells 1..20)            F1+F2 / R3
-constexpr int WS_LFC = 5;            // [3][2][5] lambda of the full-step faces                 R4 / R3
-constexpr int WS_LW  = 35;           // [5]       lambda_W                                      R3 / R2
+constexpr int WS_LFC = 5;            // [3][2][5][NLC] lambda of the full-step faces, dense     R4 / R3
 constexpr int WS_LU  = 40;           // [5]       lambda of the half-step conserved state       R2 / R0
 constexpr int WS_H   = 45;           // [5]       half-step conserved state                     F1+F2 / R2
-constexpr int WS_ZGR = 0;            // [5]       upper-side contributions of the half-step z faces  R1 / R0
-                                     //           (over W, dead after R3)
 constexpr int WS_ADJ = 50;
-static_assert( WS_LFC + 30 <= WS_LW && WS_H + NV <= WS_ADJ, "workspace slots overlap" );
+// lambda of the full-step faces, per direction, side and field a dense block over the reconstruction's centres (normal 2..19,
+// tangential 3..18) with x fastest, so that rows are whole cache lines: as rows of 16 out of 22 cells,
+// R4 on 512 patch groups took 357 us, this takes 273.
+constexpr int NLC = 18*16*16;
+constexpr int LFC0 = ( WS_LFC*N3 + 15 )/16*16;           // its first element, on a cache line
+static_assert( LFC0 + 30*NLC <= WS_LU*N3 && WS_H + NV <= WS_ADJ, "workspace slots overlap" );
+__device__ __forceinline__ int lfc_cell( int d, int i, int j, int k )
+{
+   return ( d == 0 ) ? ( i - 2 ) + 18*( ( j - 3 ) + 16*( k - 3 ) )
+        : ( d == 1 ) ? ( i - 3 ) + 16*( ( j - 2 ) + 18*( k - 3 ) )
+        :              ( i - 3 ) + 16*( ( j - 3 ) + 16*( k - 2 ) );
+}
 
 __device__ __forceinline__ void coords( int c, int &i, int &j, int &k ) { i = c % NX;  j = ( c / NX ) % NX;  k = c / N2; }
 __device__ __forceinline__ bool in_rng( int x, int lo, int hi ) { return x >= lo && x <= hi; }
@@ -101,7 +108,7 @@ __device__ __forceinline__ Box face_box( int d, int n0, int nn, int t0, int nt )
 }
 constexpr int NHF = 21*20*20;        // half-step faces per direction: normal 0..20, tangential 1..20
 constexpr int NFF = 17*16*16;        // full-step faces per direction: normal 2..18, tangential 3..18
-constexpr Box HALF_CELLS = { 1, 1, 1, 20, 20, 20 }, CORE_CELLS = { 3, 3, 3, 16, 16, 16 };
+constexpr Box CORE_CELLS = { 3, 3, 3, 16, 16, 16 };
 
 // ---------------- pieces of the step, generic in the arithmetic type ----------------
 // cell-centred interface state of the half step (pressure recovery + floor, 1/rho, sound speed)
@@ -215,7 +222,7 @@ template <> struct Load< Dual<1> >
 // marching through all phases of its patch group kept only 4 waves per patch group busy; spread over the grid,
 // a phase keeps as many patch groups' workspace traffic in flight as the registers of its own kernel allow.
 constexpr int bpp( int count ) { return ( count + NT - 1 ) / NT; }
-constexpr int N_F4 = PS*PS*PS, N_R4 = 3*NFF, N_R2 = 8000;
+constexpr int N_F4 = PS*PS*PS, N_R4 = 3*NFF;
 
 // Consecutive logical blocks of a phase share data (the planes k-1..k+1 of a plane-per-workgroup phase, the W
 // stencils of neighbouring face blocks), so every phase takes its block index from xcd_block() (hydro_kernels.hpp).
@@ -246,68 +253,83 @@ template <> struct Store< Dual<1> >
 
 constexpr size_t NIN = (size_t)NV*N3, NOUT = (size_t)NV*PS*PS*PS;
 
-// F1 + F2 for one z plane k per workgroup: the half-step fluxes of the plane's x and y faces and of the z faces
-// below and above it (Hydro_RiemannPredict_Flux) go to LDS, then the plane's 20^2 cells take the half-step update
-// (x and y flux differences, then z, as the production kernel), the floors and the primitive conversion
-// (Hydro_RiemannPredict).  The fluxes never reach memory; the price is that each interior z face is solved by
-// both planes it separates (32,800 solves per PG instead of 25,200).  h_off >= 0 (FP64 only): the half-step
-// state h is stored too, for R2.
-constexpr int F12_NT = 512, F12_NXF = 21*20, F12_NZF = 20*20, F12_NF = 2*F12_NXF + 2*F12_NZF;
+// F1 + F2: a workgroup takes F12_JR rows (y) of F12_KS planes (z), plane by plane.  The half-step fluxes of the plane's x
+// and y faces and of the z faces above it (Hydro_RiemannPredict_Flux) go to LDS, where the z faces below it are from the
+// plane before (solved first for the first plane), then the cells take the half-step update (x and y flux differences,
+// then z, as the production kernel), the floors and the primitive conversion (Hydro_RiemannPredict).  The fluxes never
+// reach memory; the price is that faces between workgroups are solved by both.  h_off >= 0 (FP64 only): the half-step state h
+// is stored too, for R2.  With one whole plane per workgroup every z face was solved twice: 512 patch groups 264 us, this
+// takes 238; half as many rows 240, five planes 242.  What the cell contributes to its six faces (pressure, 1/rho, sound
+// speed) kept in LDS instead of recomputed took 265: the solves wait, the vector units do not bound it.
+constexpr int F12_JR = 10, F12_KS = 4, F12_NT = 256;
+constexpr int F12_RB = 20/F12_JR, F12_KB = 20/F12_KS, F12_BPP = F12_RB*F12_KB;
+constexpr int F12_NXF = 21*F12_JR, F12_NYF = 20*( F12_JR + 1 ), F12_NZF = 20*F12_JR;
+static_assert( 20 % F12_JR == 0 && 20 % F12_KS == 0, "the blocks must tile the 20 x 20 half-step rows and planes" );
+
 template <int RS, typename T>
 __global__ void __launch_bounds__( F12_NT )
 f12_kernel( const double *__restrict__ g_in, const double *__restrict__ g_tin, double *__restrict__ g_ws, int h_off,
             Prm<double> P0, double minmod_coeff )
 {
-   __shared__ double s_raw[NV*F12_NF*( sizeof( T )/sizeof( double ) )];
-   T *sF = reinterpret_cast<T*>( s_raw );                    // [v][face]
-   const int tid = threadIdx.x, lb = (int)xcd_block(), pg = lb / 20, k = 1 + lb % 20;
+   __shared__ double s_raw[NV*( F12_NXF + F12_NYF + 2*F12_NZF )*( sizeof( T )/sizeof( double ) )];
+   T *sX = reinterpret_cast<T*>( s_raw ), *sY = sX + NV*F12_NXF, *sZ = sY + NV*F12_NYF;      // [v][face]; sZ [k % 2][v][face]
+   const int tid = threadIdx.x, lb = (int)xcd_block(), rb = lb % F12_RB, kb = ( lb / F12_RB ) % F12_KB, pg = lb / F12_BPP;
+   const int j0 = rb*F12_JR, ka = 1 + kb*F12_KS;                 // rows j0 + 1 .. j0 + F12_JR, planes ka .. ka + F12_KS - 1
    const Prm<T> P = phase_prm<T>( P0, minmod_coeff );
    const double *in = g_in + pg*NIN, *tin = g_tin ? g_tin + pg*NIN : nullptr;
    Fwd<T> F( reinterpret_cast<T*>( g_ws + (size_t)pg*WS_ADJ*N3 ) );
-   // faces, stored at their low cell: x (normal i = 0..20, j = 1..20), y (i = 1..20, j = 0..20), then the z
-   // faces with low cell in plane k - 1 and in plane k (i, j = 1..20); lanes run along x
-   for (int f = tid; f < F12_NF; f += F12_NT)
+#  pragma unroll 1
+   for (int k = ka - 1; k < ka + F12_KS; k++)
    {
-      int d, c;
-      if ( f < F12_NXF )        { d = 0;  c = f % 21 + NX*( 1 + f / 21 ) + N2*k; }
-      else if ( f < 2*F12_NXF ) { d = 1;  const int r = f - F12_NXF;  c = 1 + r % 20 + NX*( r / 20 ) + N2*k; }
-      else
+      // faces, stored at their low cell: x (normal i = 0..20), y (normal j0 .. j0 + F12_JR), then the z faces with low cell
+      // in plane k; lanes run along x
+      const int f0 = ( k < ka ) ? F12_NXF + F12_NYF : 0;
+      for (int f = f0 + tid; f < F12_NXF + F12_NYF + F12_NZF; f += F12_NT)
       {
-         d = 2;
-         const int r = f - 2*F12_NXF, zz = r / F12_NZF, q = r - zz*F12_NZF;
-         c = 1 + q % 20 + NX*( 1 + q / 20 ) + N2*( k - 1 + zz );
-      }
-      T uL[NV], uR[NV], fl[NV];
-      Load<T>::cell( in, tin, c, uL );
-      Load<T>::cell( in, tin, c + STRIDE[d], uR );
-      half_flux<RS>( d, uL, uR, P, fl );
-#     pragma unroll
-      for (int v=0; v<NV; v++) sF[ v*F12_NF + f ] = fl[v];
-   }
-   __syncthreads();
-   for (int e = tid; e < F12_NZF; e += F12_NT)
-   {
-      const int i = 1 + e % 20, j = 1 + e / 20, c = i + NX*j + N2*k;
-      const int xh = i + 21*( j - 1 ), yh = F12_NXF + ( i - 1 ) + 20*j, zh = 2*F12_NXF + F12_NZF + ( i - 1 ) + 20*( j - 1 );
-      T u[NV], h[NV], w[NV];
-      Load<T>::cell( in, tin, c, u );
-#     pragma unroll
-      for (int v=0; v<NV; v++)
-      {
-         const T *fv = sF + v*F12_NF;
-         const T dxy = ( fv[xh] - fv[xh - 1] ) + ( fv[yh] - fv[yh - 20] );
-         h[v] = u[v] - P.dt_dh2*( dxy + ( fv[zh] - fv[zh - F12_NZF] ) );
-      }
-      con2pri_floor( h, P, w );
-#     pragma unroll
-      for (int v=0; v<NV; v++) F.w( v, c ) = w[v];
-      if constexpr ( std::is_same<T, double>::value )
-         if ( h_off >= 0 )
+         int d, i, j, r = f, n = F12_NXF;
+         T *dst = sX;
+         if ( f < F12_NXF )                 { d = 0;  i = r % 21;  j = j0 + 1 + r / 21; }
+         else if ( f < F12_NXF + F12_NYF )  { d = 1;  r = f - F12_NXF;  i = 1 + r % 20;  j = j0 + r / 20;  dst = sY;  n = F12_NYF; }
+         else
          {
-            double *H = g_ws + (size_t)pg*WS_ADJ*N3 + (size_t)h_off*N3;
-#           pragma unroll
-            for (int v=0; v<NV; v++) H[ v*N3 + c ] = h[v];
+            d = 2;  r = f - F12_NXF - F12_NYF;  i = 1 + r % 20;  j = j0 + 1 + r / 20;  dst = sZ + ( k & 1 )*NV*F12_NZF;  n = F12_NZF;
          }
+         const int c = i + NX*j + N2*k;
+         T uL[NV], uR[NV], fl[NV];
+         Load<T>::cell( in, tin, c, uL );
+         Load<T>::cell( in, tin, c + ( d == 0 ? 1 : d == 1 ? NX : N2 ), uR );
+         half_flux<RS>( d, uL, uR, P, fl );
+#        pragma unroll
+         for (int v=0; v<NV; v++) dst[ v*n + r ] = fl[v];
+      }
+      __syncthreads();
+      if ( k >= ka )
+      for (int e = tid; e < F12_NZF; e += F12_NT)
+      {
+         const int i = 1 + e % 20, jr = e / 20, c = i + NX*( j0 + 1 + jr ) + N2*k;
+         const int xh = i + 21*jr, yh = ( i - 1 ) + 20*( jr + 1 );
+         const T *zu = sZ + ( k & 1 )*NV*F12_NZF + e, *zl = sZ + ( ( k - 1 ) & 1 )*NV*F12_NZF + e;
+         T u[NV], h[NV], w[NV];
+         Load<T>::cell( in, tin, c, u );
+#        pragma unroll
+         for (int v=0; v<NV; v++)
+         {
+            const T *fx = sX + v*F12_NXF + xh, *fy = sY + v*F12_NYF + yh;
+            const T dxy = ( fx[0] - fx[-1] ) + ( fy[0] - fy[-20] );
+            h[v] = u[v] - P.dt_dh2*( dxy + ( zu[v*F12_NZF] - zl[v*F12_NZF] ) );
+         }
+         con2pri_floor( h, P, w );
+#        pragma unroll
+         for (int v=0; v<NV; v++) F.w( v, c ) = w[v];
+         if constexpr ( std::is_same<T, double>::value )
+            if ( h_off >= 0 )
+            {
+               double *H = g_ws + (size_t)pg*WS_ADJ*N3 + (size_t)h_off*N3;
+#              pragma unroll
+               for (int v=0; v<NV; v++) H[ v*N3 + c ] = h[v];
+            }
+      }
+      __syncthreads();
    }
 }
 
@@ -385,11 +407,10 @@ f4_update_kernel( const double *__restrict__ g_in, const double *__restrict__ g_
 
 // ---------------- reverse phases ----------------
 struct Adj {
-   double *LW, *LU, *LFC;
-   __device__ Adj( double *base ) : LW( base + WS_LW*N3 ), LU( base + WS_LU*N3 ), LFC( base + WS_LFC*N3 ) {}
-   __device__ double &lw( int v, int c )                { return LW[ v*N3 + c ]; }
+   double *LU, *LFC;
+   __device__ Adj( double *base ) : LU( base + WS_LU*N3 ), LFC( base + LFC0 ) {}
    __device__ double &lu( int v, int c )                { return LU[ v*N3 + c ]; }
-   __device__ double &lfc( int d, int s, int v, int c ) { return LFC[ ( ( d*2 + s )*NV + v )*N3 + c ]; }
+   __device__ double &lfc( int d, int s, int v, int e ) { return LFC[ ( ( d*2 + s )*NV + v )*NLC + e ]; }     // e: lfc_cell()
 };
 
 typedef Dual<1> D1;
@@ -435,170 +456,143 @@ r4_kernel( const double *__restrict__ g_lout, double *__restrict__ g_ws, Prm<dou
    // one reverse sweep for both sides
    double gl[NV] = { 0.0, 0.0, 0.0, 0.0, 0.0 }, gr[NV] = { 0.0, 0.0, 0.0, 0.0, 0.0 };
    full_flux_rev<RS>( d, wl, wr, P, lf, gl, gr );
+   const int e = lfc_cell( d, i, j, k ), es = ( d == 0 ) ? 1 : ( d == 1 ) ? 16 : 256;
 #  pragma unroll
-   for (int v=0; v<NV; v++) { A.lfc( d, 1, v, c ) = gl[v];  A.lfc( d, 0, v, c + s ) = gr[v]; }
+   for (int v=0; v<NV; v++) { A.lfc( d, 1, v, e ) = gl[v];  A.lfc( d, 0, v, e + es ) = gr[v]; }
 }
 
-// R3 along y (d = 1) and z (d = 2), after r3x_kernel has written lambda_W along x: one launch per direction.
-// Task (v, line): the lane marches the line through the reconstruction stencils (centres 2..19) of field v and
-// reverses each one (plm_face_rev), keeping a window of the three cell adjoints the stencil touches, and adds each
-// cell's adjoint to lambda_W once the stencil above it is done.  Only the 16^2 lines with both tangential
-// coordinates in 3..18 carry face adjoints (the L face of a centre at normal coordinate 3..19, the R face at
-// 2..18); lanes run along x, so the loads of a march step are coalesced.
-constexpr int R3_LINES = 16*16;
-template <int LIM>
-__global__ void __launch_bounds__( NT )
-r3_kernel( double *__restrict__ g_ws, Prm<double> P0, double minmod_coeff, int d )
-{
-   const Elem x = elem( NV*R3_LINES );
-   if ( x.e >= NV*R3_LINES ) return;
-   const Prm<double> P = phase_prm<double>( P0, minmod_coeff );
-   double *ws = g_ws + (size_t)x.pg*WS_ADJ*N3;
-   Fwd<double> F( ws );
-   Adj A( ws );
-   const int s = STRIDE[d], v = x.e / R3_LINES, ln = x.e - v*R3_LINES;
-   const int a = 3 + ln % 16, b = 3 + ln / 16;                                  // i, and k (d = 1) or j (d = 2)
-   const int c0 = ( d == 1 ) ? a + N2*b : a + NX*b;                             // n = 0 of the line
-   double wm = F.w( v, c0 + s ), w0 = F.w( v, c0 + 2*s ), am = 0.0, a0 = 0.0;
-   for (int n=2; n<=19; n++)
-   {
-      const int    cc = c0 + n*s;
-      const double wp = F.w( v, cc + s );
-      const double gl = ( n >= 3 )  ? A.lfc( d, 0, v, cc ) : 0.0;
-      const double gr = ( n <= 18 ) ? A.lfc( d, 1, v, cc ) : 0.0;
-      double br = 0.0;
-      plm_face_rev<LIM>( wm, w0, wp, P.limiter, P.coeff, gl, gr, am, a0, br );
-      A.lw( v, cc - s ) += am;
-      am = a0;  a0 = br;  wm = w0;  w0 = wp;
-   }
-   A.lw( v, c0 + 19*s ) += am;
-   A.lw( v, c0 + 20*s ) += a0;
-}
-
-// R3 along x (d = 0) with the lines staged through LDS.  The x lines of one (z, field) pair are the 20 rows
-// j = 1..20 of one z plane, 440 consecutive doubles of each workspace array, so a workgroup loads W and the two
-// face-adjoint arrays of R3X_PAIRS pairs coalesced, lane t marches row 1 + t % 20 of pair t / 20 in LDS (the
-// adjoint of row cell n - 1 replaces its W, which the march has passed), and the rows go back coalesced.
-// Marching lanes over x lines directly puts 64 different rows under every load instruction.
-constexpr int R3X_PAIRS = 6, R3X_NT = 128, R3X_RL = 23, R3X_PAIR = 20*R3X_RL, R3X_NPAIR = 20*NV;
-constexpr int R3X_BPP = ( R3X_NPAIR + R3X_PAIRS - 1 )/R3X_PAIRS;
-static_assert( R3X_PAIRS*20 <= R3X_NT, "one lane per staged row" );
+// R3 + R2: a workgroup takes R32_KS planes of the half-step cells.  Step n: every lane reverses reconstruction stencils
+// (plm_face_rev) of all fields, those along z with centre plane n and those along x and y in plane n - 1, whose z neighbours
+// are done by then.  The stencils along x and y leave the adjoints of their three cells in LDS; those along z march, a lane
+// per (field, column), with the two cell adjoints still open in registers, and leave the one that is complete.  Then each
+// cell of plane n - 1 sums x, y and z in this order (each from the lower centre up) and takes lambda of the half-step
+// conserved state: J_Con2Pri^T lambda_W (floors included), at the state F2 stored.  lambda_W never reaches memory.
+// Only the 16^2 lines with both tangential coordinates in 3..18 carry face adjoints (the L face of a centre at normal
+// coordinate 3..19, the R face at 2..18).  Bound by the workspace's traffic (860 MB for 512 patch groups, 174 us at the
+// card's copy rate) and the stencils' chains: 380 us, where the phases one by one (x lines, y lines, z lines, conversion),
+// with lambda_W through memory between them, took 288 + 157 + 157 + 150.  Two planes a workgroup: 64 patch groups 187 us
+// for the whole adjoint against 199 with four; the recomputed z stencils cost nothing on 512 (383 against 377).
+constexpr int R32_KS = 2, R32_NT = 512, R32_BPP = 20/R32_KS;
+constexpr int R32_XY = 18*16, R32_Z = 16*16, R32_ZT = ( NV*R32_Z + R32_NT - 1 )/R32_NT;
+static_assert( 20 % R32_KS == 0, "the blocks must tile the 20 half-step planes" );
 
 template <int LIM>
-__global__ void __launch_bounds__( R3X_NT )
-r3x_kernel( double *__restrict__ g_ws, Prm<double> P0, double minmod_coeff )
+__global__ void __launch_bounds__( R32_NT )
+r32_kernel( double *__restrict__ g_ws, Prm<double> P0, double minmod_coeff )
 {
-   __shared__ double sW[R3X_PAIRS*R3X_PAIR], sG0[R3X_PAIRS*R3X_PAIR], sG1[R3X_PAIRS*R3X_PAIR];
-   const int tid = threadIdx.x, lb = (int)xcd_block(), pg = lb / R3X_BPP, q0 = ( lb % R3X_BPP )*R3X_PAIRS;
-   const int np = min( R3X_PAIRS, R3X_NPAIR - q0 );
-   const Prm<double> P = phase_prm<double>( P0, minmod_coeff );
-   double *ws = g_ws + (size_t)pg*WS_ADJ*N3;
-   Fwd<double> F( ws );
-   Adj A( ws );
-   // pair q: field q / 20, z = 1 + q % 20; its rows j = 1..20 start at cell NX + N2 z, a 16-byte aligned offset
-   // (NX and N2 are even), so the block moves as 220 double2 per array, R3X_LD of them per lane in flight
-   constexpr int U = 20*NX/2, R3X_LD = 4;
-   const int nu = np*U;
-   for (int u0 = tid; u0 < nu; u0 += R3X_LD*R3X_NT)
-   {
-      double2 a[R3X_LD], b[R3X_LD], g[R3X_LD];
-#     pragma unroll
-      for (int t=0; t<R3X_LD; t++)
-      {
-         const int u = u0 + t*R3X_NT;
-         if ( u >= nu ) continue;
-         const int p = u / U, q = q0 + p, v = q / 20, c = NX + N2*( 1 + q % 20 ) + 2*( u - p*U );
-         a[t] = *reinterpret_cast<const double2*>( &F.w( v, c ) );
-         b[t] = *reinterpret_cast<const double2*>( &A.lfc( 0, 0, v, c ) );
-         g[t] = *reinterpret_cast<const double2*>( &A.lfc( 0, 1, v, c ) );
-      }
-#     pragma unroll
-      for (int t=0; t<R3X_LD; t++)
-      {
-         const int u = u0 + t*R3X_NT;
-         if ( u >= nu ) continue;
-         const int p = u / U, r = 2*( u - p*U ), l = p*R3X_PAIR + ( r / NX )*R3X_RL + r % NX;   // r, r + 1: one row
-         sW[l] = a[t].x;   sW[l + 1] = a[t].y;
-         sG0[l] = b[t].x;  sG0[l + 1] = b[t].y;
-         sG1[l] = g[t].x;  sG1[l + 1] = g[t].y;
-      }
-   }
-   __syncthreads();
-   if ( tid < np*20 )
-   {
-      const int p = tid / 20, j = 1 + tid % 20, k = 1 + ( q0 + p ) % 20;
-      double *row = sW + p*R3X_PAIR + ( j - 1 )*R3X_RL;
-      const double *g0 = sG0 + p*R3X_PAIR + ( j - 1 )*R3X_RL, *g1 = sG1 + p*R3X_PAIR + ( j - 1 )*R3X_RL;
-      if ( !( in_rng( j, 3, 18 ) && in_rng( k, 3, 18 ) ) )
-      {
-         for (int n=1; n<=20; n++) row[n] = 0.0;
-      }
-      else
-      {
-         double wm = row[1], w0 = row[2], am = 0.0, a0 = 0.0;
-         for (int n=2; n<=19; n++)
-         {
-            const double wp = row[n + 1];
-            const double gl = ( n >= 3 )  ? g0[n] : 0.0;
-            const double gr = ( n <= 18 ) ? g1[n] : 0.0;
-            double br = 0.0;
-            plm_face_rev<LIM>( wm, w0, wp, P.limiter, P.coeff, gl, gr, am, a0, br );
-            row[n - 1] = am;
-            am = a0;  a0 = br;  wm = w0;  w0 = wp;
-         }
-         row[19] = am;  row[20] = a0;
-      }
-   }
-   __syncthreads();
-   for (int e = tid; e < np*400; e += R3X_NT)
-   {
-      const int p = e / 400, r = e - p*400, q = q0 + p, v = q / 20, j = 1 + r / 20, n = 1 + r % 20;
-      A.lw( v, n + NX*j + N2*( 1 + q % 20 ) ) = sW[ p*R3X_PAIR + ( j - 1 )*R3X_RL + n ];
-   }
-}
-
-// R2 lambda of the half-step conserved state: J_Con2Pri^T lambda_W (floors included), at the state F2 stored
-__global__ void __launch_bounds__( NT )
-r2_kernel( double *__restrict__ g_ws, Prm<double> P0, double minmod_coeff )
-{
-   const Elem x = elem( N_R2 );
-   if ( x.e >= N_R2 ) return;
+   __shared__ double sX[3][NV][R32_XY], sY[3][NV][R32_XY], sZ[NV][R32_Z];      // x, y: [lower cell, centre, upper cell][v][stencil]
+   const int tid = threadIdx.x, lb = (int)xcd_block(), pg = lb / R32_BPP, ka = 1 + ( lb % R32_BPP )*R32_KS, ke = ka + R32_KS;
    const Prm<double> P = phase_prm<double>( P0, minmod_coeff );
    const Prm<D1> PD = prm_as<D1>( P );
-   double *ws = g_ws + (size_t)x.pg*WS_ADJ*N3;
+   double *ws = g_ws + (size_t)pg*WS_ADJ*N3;
    const double *H = ws + (size_t)WS_H*N3;
+   Fwd<double> F( ws );
    Adj A( ws );
-   int i, j, k;
-   const int c = box_cell( HALF_CELLS, x.e, i, j, k );
-   double h[NV], lw[NV];
+   double wm[R32_ZT], w0[R32_ZT], am[R32_ZT], a0[R32_ZT];
 #  pragma unroll
-   for (int v=0; v<NV; v++)
+   for (int t=0; t<R32_ZT; t++)
    {
-      h[v]  = H[ v*N3 + c ];
-      lw[v] = A.lw( v, c );
+      const int x = tid + t*R32_NT, v = x / R32_Z, ln = x - v*R32_Z, c = ( 3 + ln % 16 ) + NX*( 3 + ln / 16 );
+      const int n = ( ka - 1 < 2 ) ? 2 : ka - 1;                               // first centre
+      am[t] = a0[t] = wm[t] = w0[t] = 0.0;
+      if ( x < NV*R32_Z ) { wm[t] = F.w( v, c + N2*( n - 1 ) );  w0[t] = F.w( v, c + N2*n ); }
    }
-   for (int q=0; q<NV; q++)
+#  pragma unroll 1
+   for (int n = ka - 1; n <= ke; n++)
    {
-      D1 hd[NV], w[NV];
+      const int q = n - 1;                                                     // plane that is completed
 #     pragma unroll
-      for (int v=0; v<NV; v++) { hd[v] = D1( h[v] );  hd[v].d[0] = ( q == v ) ? 1.0 : 0.0; }
-      con2pri_floor( hd, PD, w );
-      double g = 0.0;
-#     pragma unroll
-      for (int v=0; v<NV; v++) g += lw[v]*w[v].d[0];
-      A.lu( q, c ) = g;
+      for (int t=0; t<R32_ZT; t++)
+      {
+         const int x = tid + t*R32_NT, v = x / R32_Z, ln = x - v*R32_Z;
+         if ( x >= NV*R32_Z ) continue;
+         double br = 0.0;
+         if ( n >= 2 && n <= 19 )
+         {
+            const int c = ( 3 + ln % 16 ) + NX*( 3 + ln / 16 ) + N2*n, e = ln + 256*( n - 2 );
+            const double wp = F.w( v, c + N2 );
+            const double gl = ( n >= 3 )  ? A.lfc( 2, 0, v, e ) : 0.0;
+            const double gr = ( n <= 18 ) ? A.lfc( 2, 1, v, e ) : 0.0;
+            plm_face_rev<LIM>( wm[t], w0[t], wp, P.limiter, P.coeff, gl, gr, am[t], a0[t], br );
+            wm[t] = w0[t];
+            w0[t] = wp;
+         }
+         sZ[v][ln] = am[t];
+         am[t] = a0[t];
+         a0[t] = br;
+      }
+      if ( q >= ka && q >= 3 && q <= 18 )
+         for (int x = tid; x < 2*NV*R32_XY; x += R32_NT)
+         {
+            const int d = x / ( NV*R32_XY ), y = x - d*NV*R32_XY, v = y / R32_XY, r = y - v*R32_XY;
+            const int m = d ? 2 + r / 16 : 2 + r % 18;                         // centre along d
+            const int i = d ? 3 + r % 16 : m, j = d ? m : 3 + r / 18, c = i + NX*j + N2*q, s = d ? NX : 1;
+            const int e = d*2*NV*NLC + v*NLC + R32_XY*( q - 3 ) + r;
+            const double gl = ( m >= 3 )  ? A.LFC[ e ] : 0.0;
+            const double gr = ( m <= 18 ) ? A.LFC[ e + NV*NLC ] : 0.0;
+            double bl = 0.0, bc = 0.0, br = 0.0;
+            plm_face_rev<LIM>( F.w( v, c - s ), F.w( v, c ), F.w( v, c + s ), P.limiter, P.coeff, gl, gr, bl, bc, br );
+            double *o = ( d ? &sY[0][0][0] : &sX[0][0][0] ) + v*R32_XY + r;
+            o[0] = bl;  o[NV*R32_XY] = bc;  o[2*NV*R32_XY] = br;
+         }
+      __syncthreads();
+      if ( q >= ka )
+         for (int x = tid; x < 400; x += R32_NT)
+         {
+            const int i = 1 + x % 20, j = 1 + x / 20, c = i + NX*j + N2*q;
+            const bool ci = in_rng( i, 3, 18 ), cj = in_rng( j, 3, 18 ), ck = in_rng( q, 3, 18 );
+            double h[NV], lw[NV];
+#           pragma unroll
+            for (int v=0; v<NV; v++)
+            {
+               h[v] = H[ v*N3 + c ];
+               double lx = 0.0, ly = 0.0;
+               if ( cj && ck )
+               {
+                  const int r = 18*( j - 3 ) + i - 2;                          // stencil centred here
+                  if ( i >= 3 )           lx += sX[2][v][r - 1];
+                  if ( i >= 2 && i <= 19 ) lx += sX[1][v][r];
+                  if ( i <= 18 )          lx += sX[0][v][r + 1];
+               }
+               if ( ci && ck )
+               {
+                  const int r = 16*( j - 2 ) + i - 3;
+                  if ( j >= 3 )           ly += sY[2][v][r - 16];
+                  if ( j >= 2 && j <= 19 ) ly += sY[1][v][r];
+                  if ( j <= 18 )          ly += sY[0][v][r + 16];
+               }
+               lw[v] = lx + ly;
+               if ( ci && cj ) lw[v] += sZ[v][ 16*( j - 3 ) + i - 3 ];
+            }
+            for (int u=0; u<NV; u++)
+            {
+               D1 hd[NV], w[NV];
+#              pragma unroll
+               for (int v=0; v<NV; v++) { hd[v] = D1( h[v] );  hd[v].d[0] = ( u == v ) ? 1.0 : 0.0; }
+               con2pri_floor( hd, PD, w );
+               double g = 0.0;
+#              pragma unroll
+               for (int v=0; v<NV; v++) g = fmad( lw[v], w[v].d[0], g );
+               A.lu( u, c ) = g;
+            }
+         }
+      __syncthreads();
    }
 }
 
-// R1 + R0, one z plane k = 0..21 per workgroup.  R1: lambda_Fh = dt/(2dh) (lambda_U(c+e_d) - lambda_U(c)) of
-// every half-step face, then J_RS^T per side; the plane's x and y faces and the z face above it (normal k)
-// leave their side contributions in LDS, the z face's upper-side one goes to the workspace (zgr).  R0: lambda_in of the plane's cells = lambda_out (output cells) +
-// lambda_U_half (half-step cells) + the face contributions in the order x low, x high, y low, y high, z low;
-// r0z_kernel then adds the z high contribution.  Each face is solved once.
-// 768 lanes (3 waves per SIMD, <= 170 VGPRs); Roe's reverse solve needs about 210, so it runs 512
-constexpr int R10_NXF = 21*20, R10_NZF = 20*20, R10_NF = 2*R10_NXF + R10_NZF;
-constexpr int N_R0Z = 21*R10_NZF;
-constexpr int r10_nt( int rs ) { return rs == 2 ? 512 : 768; }
+// R1 + R0: a workgroup takes R10_JR rows (y) of about 22/R10_KB planes (z), plane by plane.  R1: lambda_Fh = dt/(2dh)
+// (lambda_U(c+e_d) - lambda_U(c)) of every half-step face, then J_RS^T per side; the side contributions of the plane's x
+// and y faces and of the z face above it (normal k) stay in LDS.  R0: lambda_in of the plane's cells = lambda_out (output
+// cells) + lambda_U_half (half-step cells) + the face contributions in the order x low, x high, y low, y high, z low, z high,
+// the last one from the plane before (solved first for the first plane).  Faces between workgroups are solved by both.
+// 3 waves per SIMD (<= 170 VGPRs); Roe's reverse solve needs about 230, 2 waves.  512 patch groups 514 us; one whole plane of
+// 768 lanes, with the z faces' high sides added by a kernel of their own through memory, 525 + 95.  192 lanes against 256
+// (610) and 128 (608); Roe 128 lanes against 256: 1724 and 1917 us for the whole adjoint.
+constexpr int R10_JR = 5, R10_KB = 4;
+constexpr int r10_nt( int rs ) { return rs == 2 ? 128 : 192; }
+constexpr int R10_RB = 20/R10_JR, R10_BPP = R10_RB*R10_KB;
+constexpr int R10_NXF = 21*R10_JR, R10_NYF = 20*( R10_JR + 1 ), R10_NZF = 20*R10_JR;
+static_assert( 20 % R10_JR == 0, "the blocks must tile the 20 half-step rows" );
 
 template <int RS>
 __global__ void __launch_bounds__( r10_nt( RS ) )
@@ -606,78 +600,68 @@ r10_kernel( const double *__restrict__ g_in, const double *__restrict__ g_lout, 
             double *__restrict__ g_ws, Prm<double> P0, double minmod_coeff )
 {
    constexpr int R10_NT = r10_nt( RS );
-   __shared__ double sX[2][NV][R10_NXF], sY[2][NV][R10_NXF], sZ[NV][R10_NZF];     // [low/high side][v][face]
-   const int tid = threadIdx.x, lb = (int)xcd_block(), pg = lb / 22, k = lb % 22;
+   // [low/high side][v][face]; sZh [k % 2][v][face]: the z faces' high sides, read one plane later
+   __shared__ double sX[2][NV][R10_NXF], sY[2][NV][R10_NYF], sZ[NV][R10_NZF], sZh[2][NV][R10_NZF];
+   const int tid = threadIdx.x, lb = (int)xcd_block(), rb = lb % R10_RB, kb = ( lb / R10_RB ) % R10_KB, pg = lb / R10_BPP;
+   const int j0 = rb*R10_JR, ka = 22*kb/R10_KB, ke = 22*( kb + 1 )/R10_KB;      // half-step rows j0 + 1 .. j0 + R10_JR, planes [ka, ke)
+   const int ja = ( rb == 0 ) ? 0 : j0 + 1, je = ( rb == R10_RB - 1 ) ? NX : j0 + R10_JR + 1;      // rows of lambda_in [ja, je)
    const Prm<double> P = phase_prm<double>( P0, minmod_coeff );
    const double *in = g_in + pg*NIN, *lout = g_lout + pg*NOUT;
-   double *lin = g_lin + pg*NIN, *ws = g_ws + (size_t)pg*WS_ADJ*N3, *zgr = ws + (size_t)WS_ZGR*N3;
-   Adj A( ws );
-   // faces with low cell in plane k: x (normal i = 0..20, j = 1..20), y (i = 1..20, j = 0..20), z (i, j = 1..20);
-   // plane 0 has only its z faces, plane 21 none
-   const int nf = ( k >= 1 && k <= 20 ) ? R10_NF : ( k == 0 ) ? R10_NZF : 0, f0 = ( k == 0 ) ? 2*R10_NXF : 0;
-   for (int t = tid; t < nf; t += R10_NT)
+   double *lin = g_lin + pg*NIN;
+   Adj A( g_ws + (size_t)pg*WS_ADJ*N3 );
+#  pragma unroll 1
+   for (int k = ( ka > 0 ) ? ka - 1 : 0; k < ke; k++)
    {
-      const int f = f0 + t;
-      int d, c, r;
-      if ( f < R10_NXF )        { d = 0;  r = f;                c = f % 21 + NX*( 1 + f / 21 ) + N2*k; }
-      else if ( f < 2*R10_NXF ) { d = 1;  r = f - R10_NXF;      c = 1 + r % 20 + NX*( r / 20 ) + N2*k; }
-      else                      { d = 2;  r = f - 2*R10_NXF;    c = 1 + r % 20 + NX*( 1 + r / 20 ) + N2*k; }
-      int i, j, kk, n, a, b;
-      coords( c, i, j, kk );
-      split( d, i, j, kk, n, a, b );
-      const int s = STRIDE[d];
-      const bool lo = in_rng( n, 1, 20 ), hi = in_rng( n + 1, 1, 20 );   // tangential range is 1..20 already
-      double lf[NV];
-#     pragma unroll
-      for (int v=0; v<NV; v++) lf[v] = P.dt_dh2*( ( hi ? A.lu( v, c + s ) : 0.0 ) - ( lo ? A.lu( v, c ) : 0.0 ) );
-      double uL[NV], uR[NV];
-#     pragma unroll
-      for (int v=0; v<NV; v++) { uL[v] = in[ v*N3 + c ];  uR[v] = in[ v*N3 + c + s ]; }
-      double gl[NV] = { 0.0, 0.0, 0.0, 0.0, 0.0 }, gr[NV] = { 0.0, 0.0, 0.0, 0.0, 0.0 };
-      half_flux_rev<RS>( d, uL, uR, P, lf, gl, gr );
-#     pragma unroll
-      for (int v=0; v<NV; v++)
+      // faces with low cell in plane k: x (normal i = 0..20), y (normal j0 .. j0 + R10_JR), z; plane 0 and the plane
+      // before the first have only their z faces, plane 21 none
+      const int f0 = ( k == 0 || k < ka ) ? R10_NXF + R10_NYF : 0, f1 = ( k <= 20 ) ? R10_NXF + R10_NYF + R10_NZF : 0;
+      for (int f = f0 + tid; f < f1; f += R10_NT)
       {
-         if      ( d == 0 ) { sX[0][v][r] = gl[v];  sX[1][v][r] = gr[v]; }
-         else if ( d == 1 ) { sY[0][v][r] = gl[v];  sY[1][v][r] = gr[v]; }
-         else               { sZ[v][r] = gl[v];  zgr[ v*N3 + k*R10_NZF + r ] = gr[v]; }
+         int d, i, j, r = f, n;
+         if ( f < R10_NXF )                 { d = 0;  i = r % 21;  j = j0 + 1 + r / 21;  n = i; }
+         else if ( f < R10_NXF + R10_NYF )  { d = 1;  r = f - R10_NXF;  i = 1 + r % 20;  j = j0 + r / 20;  n = j; }
+         else                               { d = 2;  r = f - R10_NXF - R10_NYF;  i = 1 + r % 20;  j = j0 + 1 + r / 20;  n = k; }
+         const int c = i + NX*j + N2*k, s = ( d == 0 ? 1 : d == 1 ? NX : N2 );
+         const bool lo = in_rng( n, 1, 20 ), hi = in_rng( n + 1, 1, 20 );   // tangential range is 1..20 already
+         double lf[NV];
+#        pragma unroll
+         for (int v=0; v<NV; v++) lf[v] = P.dt_dh2*( ( hi ? A.lu( v, c + s ) : 0.0 ) - ( lo ? A.lu( v, c ) : 0.0 ) );
+         double uL[NV], uR[NV];
+#        pragma unroll
+         for (int v=0; v<NV; v++) { uL[v] = in[ v*N3 + c ];  uR[v] = in[ v*N3 + c + s ]; }
+         double gl[NV] = { 0.0, 0.0, 0.0, 0.0, 0.0 }, gr[NV] = { 0.0, 0.0, 0.0, 0.0, 0.0 };
+         half_flux_rev<RS>( d, uL, uR, P, lf, gl, gr );
+         double *pl = ( d == 0 ) ? &sX[0][0][r] : ( d == 1 ) ? &sY[0][0][r] : &sZ[0][r];
+         double *ph = ( d == 0 ) ? &sX[1][0][r] : ( d == 1 ) ? &sY[1][0][r] : &sZh[k & 1][0][r];
+         const int m = ( d == 0 ) ? R10_NXF : ( d == 1 ) ? R10_NYF : R10_NZF;
+#        pragma unroll
+         for (int v=0; v<NV; v++) { pl[ v*m ] = gl[v];  ph[ v*m ] = gr[v]; }
       }
-   }
-   __syncthreads();
-   for (int e = tid; e < NX*NX; e += R10_NT)
-   {
-      const int i = e % NX, j = e / NX, c = i + NX*j + N2*k;
-      const bool core = core3( i, j, k ), half = in_rng( i, 1, 20 ) && in_rng( j, 1, 20 ) && in_rng( k, 1, 20 );
-      const bool xl = half_face( i, j, k ), xh = half_face( i - 1, j, k ), yl = half_face( j, i, k ),
-                 yh = half_face( j - 1, i, k ), zl = half_face( k, i, j );
-      const int rx = i + 21*( j - 1 ), ry = ( i - 1 ) + 20*j, rz = ( i - 1 ) + 20*( j - 1 );
-#     pragma unroll
-      for (int v=0; v<NV; v++)
+      __syncthreads();
+      if ( k >= ka )
+      for (int e = ja*NX + tid; e < je*NX; e += R10_NT)
       {
-         double acc = core ? lout[ (size_t)v*PS*PS*PS + out_index( i, j, k ) ] : 0.0;
-         if ( half ) acc += A.lu( v, c );
-         if ( xl ) acc += sX[0][v][rx];
-         if ( xh ) acc += sX[1][v][rx - 1];
-         if ( yl ) acc += sY[0][v][ry];
-         if ( yh ) acc += sY[1][v][ry - 20];
-         if ( zl ) acc += sZ[v][rz];
-         lin[ v*N3 + c ] = acc;
+         const int i = e % NX, j = e / NX, c = i + NX*j + N2*k;
+         const bool core = core3( i, j, k ), half = in_rng( i, 1, 20 ) && in_rng( j, 1, 20 ) && in_rng( k, 1, 20 );
+         const bool xl = half_face( i, j, k ), xh = half_face( i - 1, j, k ), yl = half_face( j, i, k ),
+                    yh = half_face( j - 1, i, k ), zl = half_face( k, i, j ), zh = half_face( k - 1, i, j );
+         const int rx = i + 21*( j - j0 - 1 ), ry = ( i - 1 ) + 20*( j - j0 ), rz = ( i - 1 ) + 20*( j - j0 - 1 );
+#        pragma unroll
+         for (int v=0; v<NV; v++)
+         {
+            double acc = core ? lout[ (size_t)v*PS*PS*PS + out_index( i, j, k ) ] : 0.0;
+            if ( half ) acc += A.lu( v, c );
+            if ( xl ) acc += sX[0][v][rx];
+            if ( xh ) acc += sX[1][v][rx - 1];
+            if ( yl ) acc += sY[0][v][ry];
+            if ( yh ) acc += sY[1][v][ry - 20];
+            if ( zl ) acc += sZ[v][rz];
+            if ( zh ) acc += sZh[( k - 1 ) & 1][v][rz];
+            lin[ v*N3 + c ] = acc;
+         }
       }
+      __syncthreads();
    }
-}
-
-// the z high contribution: cell (i, j, k), k = 1..21, i, j = 1..20, is the upper side of z face k - 1/2
-__global__ void __launch_bounds__( NT )
-r0z_kernel( double *__restrict__ g_lin, const double *__restrict__ g_ws )
-{
-   const Elem x = elem( N_R0Z );
-   if ( x.e >= N_R0Z ) return;
-   double *lin = g_lin + x.pg*NIN;
-   const double *zgr = g_ws + (size_t)x.pg*WS_ADJ*N3 + (size_t)WS_ZGR*N3;
-   const int n = x.e / R10_NZF, q = x.e - n*R10_NZF;                  // face normal n = 0..20
-   const int c = 1 + q % 20 + NX*( 1 + q / 20 ) + N2*( n + 1 );
-#  pragma unroll
-   for (int v=0; v<NV; v++) lin[ v*N3 + c ] += zgr[ v*N3 + n*R10_NZF + q ];
 }
 
 // ---------------- transpose of the periodic ghost-zone preparation ----------------
@@ -742,8 +726,9 @@ namespace {
 
 // one flat grid of bpp(count) workgroups per patch group
 void phase_grid( int npg, int count, dim3 &grid ) { grid = dim3( (unsigned)( (long)npg*bpp( count ) ) ); }
-// whether every phase's grid of npg patch groups fits one launch (the per-plane R1 + R0 kernel has the most lanes)
-bool grids_fit( int npg ) { return (long)npg*22*r10_nt( 4 ) < ( 1L << 32 ) && (long)npg*bpp( N_R4 )*NT < ( 1L << 32 ); }
+// whether every phase's grid of npg patch groups fits one launch (R4 has the most lanes)
+bool grids_fit( int npg ) { return (long)npg*bpp( N_R4 )*NT < ( 1L << 32 ); }
+static_assert( F12_BPP*F12_NT <= bpp( N_R4 )*NT && R10_BPP*r10_nt( 4 ) <= bpp( N_R4 )*NT && R32_BPP*R32_NT <= bpp( N_R4 )*NT, "R4 has the most lanes" );
 
 template <int RS, int LIM>
 int adjoint_phases( const double *in, const double *lam_out, double *lam_in, double *ws, int npg, double minmod_coeff,
@@ -753,21 +738,12 @@ int adjoint_phases( const double *in, const double *lam_out, double *lam_in, dou
    dim3 g;
    // forward: F1 + F2 (the PLM faces are recomputed where they are needed instead of stored)
    if ( !grids_fit( npg ) ) return -3;
-   hipLaunchKernelGGL( ( f12_kernel<RS, double> ), dim3( (unsigned)( 20*npg ) ), dim3( F12_NT ), 0, stream, in, nullptr, ws, WS_H, P, minmod_coeff );
-   // reverse: R4, R3 (x staged through LDS, then y and z), R2, R1 + R0 per z plane, the z faces' upper sides
+   hipLaunchKernelGGL( ( f12_kernel<RS, double> ), dim3( (unsigned)( F12_BPP*npg ) ), dim3( F12_NT ), 0, stream, in, nullptr, ws, WS_H, P, minmod_coeff );
+   // reverse: R4, R3 + R2, R1 + R0
    phase_grid( npg, N_R4, g );
    hipLaunchKernelGGL( ( r4_kernel<RS, LIM> ), g, block, 0, stream, lam_out, ws, P, minmod_coeff );
-   hipLaunchKernelGGL( ( r3x_kernel<LIM> ), dim3( (unsigned)( npg*R3X_BPP ) ), dim3( R3X_NT ), 0, stream, ws, P, minmod_coeff );
-   for (int d=1; d<3; d++)
-   {
-      phase_grid( npg, NV*R3_LINES, g );
-      hipLaunchKernelGGL( ( r3_kernel<LIM> ), g, block, 0, stream, ws, P, minmod_coeff, d );
-   }
-   phase_grid( npg, N_R2, g );
-   hipLaunchKernelGGL( r2_kernel, g, block, 0, stream, ws, P, minmod_coeff );
-   hipLaunchKernelGGL( ( r10_kernel<RS> ), dim3( (unsigned)( 22*npg ) ), dim3( r10_nt( RS ) ), 0, stream, in, lam_out, lam_in, ws, P, minmod_coeff );
-   phase_grid( npg, N_R0Z, g );
-   hipLaunchKernelGGL( r0z_kernel, g, block, 0, stream, lam_in, ws );
+   hipLaunchKernelGGL( ( r32_kernel<LIM> ), dim3( (unsigned)( npg*R32_BPP ) ), dim3( R32_NT ), 0, stream, ws, P, minmod_coeff );
+   hipLaunchKernelGGL( ( r10_kernel<RS> ), dim3( (unsigned)( R10_BPP*npg ) ), dim3( r10_nt( RS ) ), 0, stream, in, lam_out, lam_in, ws, P, minmod_coeff );
    return ( hipGetLastError() == hipSuccess ) ? 0 : -2;
 }
 
@@ -778,7 +754,7 @@ int tangent_phases( const double *in, const double *tin, double *out, double *to
    const dim3 block( NT );
    dim3 g;
    if ( !grids_fit( npg ) ) return -3;
-   hipLaunchKernelGGL( ( f12_kernel<RS, T> ), dim3( (unsigned)( 20*npg ) ), dim3( F12_NT ), 0, stream, in, tin, ws, -1, P, minmod_coeff );
+   hipLaunchKernelGGL( ( f12_kernel<RS, T> ), dim3( (unsigned)( F12_BPP*npg ) ), dim3( F12_NT ), 0, stream, in, tin, ws, -1, P, minmod_coeff );
    phase_grid( npg, 3*NFF, g );
    hipLaunchKernelGGL( ( f4_face_kernel<RS, LIM, T> ), g, block, 0, stream, ws, P, minmod_coeff );
    phase_grid( npg, N_F4, g );

@@ -8,7 +8,8 @@
 // Branches: every min / max / select / floor takes the branch of the forward evaluation, with the tie rules
 // of the dual numbers (a tie of min or max goes to the first operand, a NaN second operand loses), so this
 // adjoint and the dual-number tangent agree at the kinks too (Davis speeds, HLLC upwind side, pressure
-// floors, the HLLE rescue of a NaN HLLC flux).
+// floors, the HLLE rescue of a NaN HLLC flux).  The recomputed forward values are rounded as the forward sweep's, without
+// contraction; the adjoints themselves, on which nothing branches, are accumulated with fused multiply-adds.
 //
 // Forward definitions being reversed:
 //   rs_hllc, rs_hlle, rs_roe, riemann, face_state  hydro_math.hpp (CPU_Shared_RiemannSolver_HLLC.cpp:391-655,
@@ -31,6 +32,7 @@ __device__ __forceinline__ bool max_first( double a, double b ) { return b != b 
 // F = x-flux(s) - sp*U(s)  (xflux_minus)
 __device__ __forceinline__ void xflux_minus_rev( const StD &s, double sp, const double bF[NV], StD &bs, double &bsp )
 {
+   #pragma clang fp contract(on)
    const double us = s.u - sp;
    bs.d  -= sp*bF[0];
    bs.mn += bF[0] + us*bF[1];
@@ -77,6 +79,7 @@ __device__ __forceinline__ void rs_hlle_rev( const StD &L, const StD &Q, const d
    }
    else
    {
+      #pragma clang fp contract(on)
       const double inv = rcp( sr - sl );
       double binv = 0.0;
 #     pragma unroll
@@ -138,6 +141,8 @@ __device__ __forceinline__ bool rs_hllc_rev( const StD &L, const StD &Q, double 
    if ( nan ) return false;
 
    // reverse: f_k = cf F_k (+ cs, + cs vs)
+   {
+   #pragma clang fp contract(on)
    double bF[NV], bcf = 0.0;
 #  pragma unroll
    for (int v=0; v<NV; v++) { bF[v] = cf*bf[v];  bcf += bf[v]*F[v]; }
@@ -189,6 +194,7 @@ __device__ __forceinline__ bool rs_hllc_rev( const StD &L, const StD &Q, double 
    // wl = min(wl1, wl2), wr = max(wr1, wr2)
    add_if( kl, bL.u, bwl );  add_if( kl, bL.cs, -bwl );  add_if( !kl, bQ.u, bwl );  add_if( !kl, bQ.cs, -bwl );
    add_if( kr, bL.u, bwr );  add_if( kr, bL.cs,  bwr );  add_if( !kr, bQ.u, bwr );  add_if( !kr, bQ.cs,  bwr );
+   }
    return true;
 }
 
@@ -245,6 +251,8 @@ __device__ __forceinline__ void rs_roe_rev( const StD &L, const StD &Q, const Pr
    const double A0 = a0_*( s0*e0 ), A1 = a1_*( su*u ), A2 = a2_*( su*u ), A3 = a3_*( su*u ), A4 = a4_*( s4*e4 );
 
    // reverse: f = (F_L + F_R - sum_k A_k R_k) / 2
+   {
+   #pragma clang fp contract(on)
    double bh[NV];
 #  pragma unroll
    for (int k=0; k<NV; k++) bh[k] = HALF*bf[k];
@@ -331,6 +339,7 @@ __device__ __forceinline__ void rs_roe_rev( const StD &L, const StD &Q, const Pr
    bQ.d += bsqr*( 0.5/sqr );
    bL.ir += bhl*( L.e + L.p );  bL.e += bhl*L.ir;  bL.p += bhl*L.ir;
    bQ.ir += bhr*( Q.e + Q.p );  bQ.e += bhr*Q.ir;  bQ.p += bhr*Q.ir;
+   }
 }
 
 // riemann<RS> across a d-normal face (HLLC with the HLLE rescue, HLLE, or Roe): bout is the adjoint of the lab-frame flux
@@ -354,6 +363,7 @@ __device__ __forceinline__ void riemann_rev( int d, const StD &L, const StD &Q, 
 __device__ __forceinline__ void face_state_rev( int d, const double w[NV], const StD &s, const StD &bs, const Prm<double> &P,
                                                 double bw[NV] )
 {
+   #pragma clang fp contract(on)
    double wn, w1, w2, x, y, z;
    to_face( d, w[1], w[2], w[3], wn, w1, w2 );
    from_face( d, bs.mn*w[0] + bs.u, bs.m1*w[0], bs.m2*w[0], x, y, z );
@@ -379,14 +389,17 @@ __device__ __forceinline__ void face_state_rev( int d, const double w[NV], const
 __device__ __forceinline__ void cell_st_rev( int d, const double u[NV], const StD &s, const StD &bs, const Prm<double> &P,
                                              double bu[NV] )
 {
-   double x, y, z;
-   from_face( d, bs.mn + bs.u*s.ir, bs.m1, bs.m2, x, y, z );
    const double S = 0.5*( u[1]*u[1] + u[2]*u[2] + u[3]*u[3] );
    const double eint = u[4] - S*s.ir;
+   const bool   floored = ( eint*P.gm1 < P.min_pres );
+   {
+   #pragma clang fp contract(on)
+   double x, y, z;
+   from_face( d, bs.mn + bs.u*s.ir, bs.m1, bs.m2, x, y, z );
    const double bx = bs.cs*( 0.5/s.cs );
    const double bp = bs.p + bx*P.gamma*s.ir;
    double bir = bs.ir + bx*P.gamma*s.p + bs.u*s.mn;
-   const double beint = ( eint*P.gm1 < P.min_pres ) ? 0.0 : bp*P.gm1;
+   const double beint = floored ? 0.0 : bp*P.gm1;
    const double bS = -beint*s.ir;
    bir -= beint*S;
    bu[0]  += bs.d - s.ir*s.ir*bir;
@@ -397,6 +410,7 @@ __device__ __forceinline__ void cell_st_rev( int d, const double u[NV], const St
    bu[2]  += bS*u[2];
    bu[3]  += bS*u[3];
    bu[4]  += bs.e + beint;
+   }
 }
 
 // clamp_between(x, a, b) = min(max(x, min(a, b)), max(a, b)) under the dual tie rules: which operand the result
@@ -410,13 +424,48 @@ __device__ __forceinline__ int clamp_pick( double x, double a, double b )
    return min_first( x1, hi ) ? ( x1_x ? 0 : ( lo_a ? 1 : 2 ) ) : ( hi_a ? 1 : 2 );
 }
 
+// Partials of slope_vl_gminmod by (sl, sr), as the two-direction dual evaluation gives them
+__device__ __forceinline__ double slope_vl_gminmod_d( double sl, double sr, double coeff, double &d0, double &d1 )
+{
+   const double t = sl + sr, p2 = 2.0*( sl*sr ), r = rcp( vabs( t ) );
+   const double rr = -r*r, w = p2*( __builtin_signbit( t ) ? -rr : rr ), h = p2*r;
+   const double h0 = fmad( 2.0*sr, r, w ), h1 = fmad( 2.0*sl, r, w );
+   const double g1 = vabs( sl )*coeff, g2 = vabs( sr )*coeff;
+   const bool   k = min_first( g1, g2 ), kh = ( h >= 0.0 );
+   const double x = k ? g1 : g2, hp = kh ? h : 0.0;
+   const bool   kx = ( x <= hp );
+   const double m  = kx ? x : hp;
+   const double m0 = kx ? ( k ? __builtin_copysign( coeff, sl ) : 0.0 ) : ( kh ? h0 : 0.0 );
+   const double m1 = kx ? ( k ? 0.0 : __builtin_copysign( coeff, sr ) ) : ( kh ? h1 : 0.0 );
+   const bool   neg = ( __builtin_signbit( m ) != 0 ) != ( __builtin_signbit( t ) != 0 );
+   d0 = neg ? -m0 : m0;
+   d1 = neg ? -m1 : m1;
+   return __builtin_copysign( m, t );
+}
+
 // plm_face<LIM>: faces fL, fR of the centre C from (L, C, R).  Given their adjoints (bfL, bfR), accumulate the
 // adjoints of L, C, R.  The face clamps and the mirror fL = 2C - fR are reversed here; the limited slope's two
-// partials come from a two-direction dual evaluation of the same slope function.
+// partials come from a two-direction dual evaluation of the same slope function, for LIM == 4 written out.  Its clamps
+// do not act on finite faces (plm_face), so they are left to the cells whose faces are not.
 template <int LIM>
 __device__ __forceinline__ void plm_face_rev( double L, double C, double Rr, int lim, double coeff,
                                               double bfL, double bfR, double &bL, double &bC, double &bR )
 {
+   if constexpr ( LIM == 4 )
+   {
+      double d0, d1;
+      const double sv = slope_vl_gminmod_d( C - L, Rr - C, coeff, d0, d1 );
+      const double x2 = 2.0*C - ( C - 0.5*sv );
+      if ( vabs( x2 ) <= 1.7976931348623157e308 )
+      {
+         const double bfr = bfR - bfL, bc = ( 2.0*bfL + 2.0*bfr ) - bfr, bs = 0.5*bfr;
+         const double bsl = bs*d0, bsr = bs*d1;
+         bL -= bsl;
+         bC += bc + bsl - bsr;
+         bR += bsr;
+         return;
+      }
+   }
    Dual<2> sl( C - L ), sr( Rr - C );
    sl.d[0] = 1.0;
    sr.d[1] = 1.0;
