@@ -29,7 +29,8 @@ __device__ __forceinline__ long xcd_block()
 // computed exactly as in the whole march, so the results are bitwise equal.  Not split: the MinMod retry (maxiter > 0),
 // which is decided over the whole patch group; with the fused dt only into halves, whose patches do not straddle slabs.
 // Measured (us, whole -> split), MHM_RP: FP32 8 patch groups 51.7 -> 14.5, 32 with dt 54.7 -> 35.5, 100 53 -> 31.7, 256
-// 53.7 -> 46.3; FP64 16 73 -> 20, 64 73.8 -> 33.4, 700 224 -> 222.6, 1331 464 -> 433; FP64 Roe 300 264 -> 192.
+// 53.7 -> 46.3; FP64 16 73 -> 20, 64 73.8 -> 33.4, 700 224 -> 222.6, 1331 464 -> 433; FP64 Roe 300 264 -> 192.  MHM:
+// FP32 8 103 -> 17, 64 102 -> 31, 200 with dt 106 -> 81; FP64 8 122 -> 20, 64 123 -> 44, Roe 300 338 -> 219.
 int device_cus();                    // compute units of the current device, 0 if unknown
 inline void slab_split( int npg, int halo, int per_cu, int minmod_maxiter, bool with_dt, Batch &B )
 {

@@ -79,7 +79,8 @@ __device__ __forceinline__ void recon_cell( const R (*wl)[NC], int c, const R wm
    hancock<R, IO>( fc, fp, u0, P );
 }
 
-template <typename R, typename IO, int RS, int LIM, bool PERSIST>
+// MODE 0: one patch group per workgroup; 1: persistent work queue; 2: the last patch groups in z slabs (slab_split())
+template <typename R, typename IO, int RS, int LIM, int MODE>
 __global__ void __launch_bounds__( NT ) __attribute__(( amdgpu_waves_per_eu( sizeof(R) == 4 ? 2 : 1 ) ))
 mhm_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restrict__ g_flux,
             int npg, int store_flux, int minmod_maxiter, R minmod_coeff, Prm<R> P0,
@@ -110,11 +111,11 @@ mhm_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restrict_
    int base = 0;
    for (int item = 0; ; item++)
    {
-   // next patch group: blockIdx.x, or the next PG of this workgroup's ticket of the persistent work queue (a ticket
-   // covers B.claim consecutive PGs; the barrier before every PG also keeps the previous PG's LDS reads ahead of
-   // the next PG's writes)
-   int pg;
-   if ( PERSIST )
+   // next patch group: blockIdx.x (of the last ones, a z slab: slab_split()), or the next PG of this workgroup's ticket of
+   // the persistent work queue (a ticket covers B.claim consecutive PGs; the barrier before every PG also keeps the
+   // previous PG's LDS reads ahead of the next PG's writes)
+   int pg, slab_z = 0, slab_h = PS, half = -1; // first output plane and output planes of the march; z half whose dt it writes
+   if ( MODE == 1 )
    {
       const int sub = item % B.claim;
       __syncthreads();
@@ -130,16 +131,27 @@ mhm_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restrict_
    {
       if ( item > 0 ) break;
       pg = blockIdx.x;
+      if ( MODE == 2 && pg >= B.whole )
+      {
+         const int e = pg - B.whole, k = e % B.slabs;
+         pg = B.whole + e / B.slabs;
+         slab_h = PS / B.slabs;
+         slab_z = k*slab_h;
+         half = ( B.slabs == 2 ) ? k : -1;
+      }
    }
    if ( pg >= npg ) break;
+   const int z0 = ( MODE == 2 ) ? slab_z : 0, t1 = ( MODE == 2 ) ? slab_h + 3 : NX - 1;     // t1: last input plane
 
    constexpr int SZ = sizeof( IO );
    const IO *in  = g_in  + (size_t)pg*NV*NC*NX;
    IO       *out = g_out + (size_t)pg*NV*PS*PS*PS;
    IO       *flx = store_flux ? g_flux + (size_t)pg*9*NV*PS*PS : nullptr;
-   const __amdgpu_buffer_rsrc_t b_in  = make_buf( in,  NV*NC*NX*SZ );
-   const __amdgpu_buffer_rsrc_t b_out = make_buf( out, NV*PS*PS*PS*SZ );
-   const __amdgpu_buffer_rsrc_t b_flx = make_buf( flx, flx ? 9*NV*PS*PS*SZ : 0 );
+   // the march counts its planes from 0: the descriptors start at the slab's first plane (the x and y flux planes at its
+   // first row)
+   const __amdgpu_buffer_rsrc_t b_in  = make_buf( in + z0*NC,     ( NV*NC*NX - z0*NC )*SZ );
+   const __amdgpu_buffer_rsrc_t b_out = make_buf( out + z0*PS*PS, ( NV*PS*PS*PS - z0*PS*PS )*SZ );
+   const __amdgpu_buffer_rsrc_t b_flx = make_buf( flx ? flx + z0*PS : nullptr, flx ? ( 9*NV*PS*PS - z0*PS )*SZ : 0 );
    Prm<R> P = P0;
    double dh_safety = dh_safety0;
    if ( B.pg_dt_dh )
@@ -179,7 +191,7 @@ mhm_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restrict_
       // two steps per iteration: the LDS slot (t & 1) becomes a constant and the plane-to-plane register hand-offs
       // are renamed instead of copied; the Roe kernels stay rolled, their code is twice as large
 #     pragma unroll ( RS != 2 ? 2 : 1 )
-      for (int t = 0; t < NX; t++)
+      for (int t = 0; t <= t1; t++)
       {
          const int slot = t & 1;
          // ---- plane t -> primitive plane in LDS; own columns' conserved and primitive values to registers
@@ -196,7 +208,7 @@ mhm_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restrict_
                for (int v=0; v<NV; v++) { S.w[slot][v][c] = w[v];  S.u[v][c] = (R)pf[k][v]; }
             }
          }
-         if ( t + 1 < NX ) issue( t + 1 );
+         if ( t < t1 ) issue( t + 1 );
          const int o = t - 2;
 #        pragma unroll
          for (int v=0; v<NV; v++) S.u2[v][tid] = kU0[v];          // input plane t-2 of the own column
@@ -213,12 +225,12 @@ mhm_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restrict_
          // ---- PLM + Hancock of plane r = t-1
          const int r = t - 1;
          R kF[6][NV], oF[6][NV];
-         if ( r >= 1 && r <= 18 )
+         if ( r >= 1 && r <= t1 - 1 )
          {
             recon_cell<LIM, R, IO>( S.w[slot ^ 1], kc, kWm, kW0, kWp, kU0, Q, kF );
 #           pragma unroll
             for (int v=0; v<NV; v++) { S.f[v][kc] = kF[1][v];  S.f[NV + v][kc] = kF[3][v]; }
-            if ( has_o && r >= 2 && r <= 17 )
+            if ( has_o && r >= 2 && r <= t1 - 2 )
             {
                recon_cell<LIM, R, IO>( S.w[slot ^ 1], oc, oWm, oW0, oWp, oU0, Q, oF );
 #              pragma unroll
@@ -229,20 +241,20 @@ mhm_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restrict_
 
          // ---- full-step fluxes: z at r-1/2 (lane-local), x and y of plane r through LDS
          R fzn[NV];
-         if ( r >= 2 && r <= 18 )
+         if ( r >= 2 && r <= t1 - 1 )
          {
             solve<RS, 2, 2>( cons_side<2>( kFzR, Q ), cons_side<2>( kF[4], Q ), Q, fzn );
-            if ( flx && ( r - 2 ) % 8 == 0 )
+            if ( flx && ( z0 + r - 2 ) % 8 == 0 && ( r < t1 - 1 || z0 + r == 18 ) )    // the next slab stores the face between
 #              pragma unroll
                for (int v=0; v<NV; v++)
-                  buf_store( (IO)fzn[v], b_flx, kxy*SZ, ( ( 6 + ( r - 2 )/8 )*NV + v )*PS*PS*SZ );
+                  buf_store( (IO)fzn[v], b_flx, kxy*SZ, ( ( ( 6 + ( z0 + r - 2 )/8 )*NV + v )*PS*PS - z0*PS )*SZ );
          }
          if ( r >= 1 )
 #           pragma unroll
             for (int v=0; v<NV; v++) kFzR[v] = kF[5][v];
 
          R dfn[NV];
-         if ( r >= 2 && r <= 17 )
+         if ( r >= 2 && r <= t1 - 2 )
          {
             R fx[NV], fy[NV], fo[NV], q[NV];
 #           pragma unroll
@@ -294,7 +306,7 @@ mhm_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restrict_
          }
 
          // ---- full-step update and output of plane o = t-2
-         if ( o >= 2 && o <= 17 )
+         if ( o >= 2 && o <= t1 - 2 )
          {
             IO res[NV], uo[NV];
 #           pragma unroll
@@ -303,17 +315,17 @@ mhm_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restrict_
 #           pragma unroll
             for (int v=0; v<NV; v++) buf_store( res[v], b_out, kxy*SZ, ( v*PS*PS*PS + PS*PS*( o - 2 ) )*SZ );
             if ( bad ) S.fail = 1;
-            if ( g_dt ) cfl[ ( o - 2 )/8 ] = vmax( cfl[ ( o - 2 )/8 ], cell_cfl( res, (double)Q.gamma, Q.gm1_d, Q.min_pres_d ) );
+            if ( g_dt ) cfl[ ( z0 + o - 2 )/8 ] = vmax( cfl[ ( z0 + o - 2 )/8 ], cell_cfl( res, (double)Q.gamma, Q.gm1_d, Q.min_pres_d ) );
          }
-         if ( r >= 2 && r <= 18 )
+         if ( r >= 2 && r <= t1 - 1 )
 #           pragma unroll
             for (int v=0; v<NV; v++) kFz[v] = fzn[v];
-         if ( r >= 2 && r <= 17 )
+         if ( r >= 2 && r <= t1 - 2 )
 #           pragma unroll
             for (int v=0; v<NV; v++) kDf[v] = dfn[v];
       } // for t
 
-      if ( g_dt ) fused_dt( cfl, ( ki - 2 )/8 + 2*( ( kj - 2 )/8 ), S.cfl, g_dt + (size_t)pg*8, dh_safety, -1 );
+      if ( g_dt ) fused_dt( cfl, ( ki - 2 )/8 + 2*( ( kj - 2 )/8 ), S.cfl, g_dt + (size_t)pg*8, dh_safety, half );
       __syncthreads();
       const bool redo = ( S.fail != 0 ) && ( iter + 1 <= minmod_maxiter );
       __syncthreads();
@@ -324,14 +336,17 @@ mhm_kernel( const IO *__restrict__ g_in, IO *__restrict__ g_out, IO *__restrict_
 
 template <typename R, typename IO, int RS>
 void launch_rs( const IO *in, IO *out, IO *flux, int npg, int store_flux, int minmod_maxiter, double minmod_coeff,
-                const Prm<R> &P, IO *dt, double dh_safety, const Batch &B, int grid_blocks, hipStream_t stream )
+                const Prm<R> &P, IO *dt, double dh_safety, Batch B, int grid_blocks, hipStream_t stream )
 {
-   const dim3 grid( grid_blocks > 0 ? grid_blocks : npg ), block( NT );
    const bool pers = ( B.counter != nullptr );
-#  define GA_LAUNCH( LIM_, PERS_ ) hipLaunchKernelGGL( ( mhm_kernel<R, IO, RS, LIM_, PERS_> ), grid, block, 0, stream, \
+   if ( !pers ) slab_split( npg, NX - PS, sizeof( R ) == 4 ? 2 : 1, minmod_maxiter, dt != nullptr, B );
+   const dim3 grid( pers ? ( grid_blocks > 0 ? grid_blocks : npg ) : B.whole + ( npg - B.whole )*B.slabs ), block( NT );
+   const int mode = pers ? 1 : ( B.slabs > 1 ) ? 2 : 0;
+#  define GA_LAUNCH( LIM_, MODE_ ) hipLaunchKernelGGL( ( mhm_kernel<R, IO, RS, LIM_, MODE_> ), grid, block, 0, stream, \
                                                       in, out, flux, npg, store_flux, minmod_maxiter, (R)minmod_coeff, P, dt, dh_safety, B )
-   if ( kernel_limiter( P.limiter, minmod_coeff ) == 4 ) { if ( pers ) GA_LAUNCH( 4, true ); else GA_LAUNCH( 4, false ); }
-   else                  { if ( pers ) GA_LAUNCH( 0, true ); else GA_LAUNCH( 0, false ); }
+#  define GA_MODE( LIM_ ) { if ( mode == 0 ) GA_LAUNCH( LIM_, 0 ); else if ( mode == 1 ) GA_LAUNCH( LIM_, 1 ); else GA_LAUNCH( LIM_, 2 ); }
+   if ( kernel_limiter( P.limiter, minmod_coeff ) == 4 ) GA_MODE( 4 ) else GA_MODE( 0 )
+#  undef GA_MODE
 #  undef GA_LAUNCH
 }
 

@@ -42,21 +42,22 @@ def _random_groups(npg, n, dtype):
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
 @pytest.mark.parametrize("rsolver,limiter,store_flux,with_dt", [
     ("HLLC", "VL_GMINMOD", True, False), ("ROE", "VANLEER", True, True), ("HLLE", "GMINMOD", False, True)])
-def test_slabs_equal_whole_groups(rsolver, limiter, store_flux, with_dt, prec):
+@pytest.mark.parametrize("scheme", ["MHM_RP", "MHM"])
+def test_slabs_equal_whole_groups(scheme, rsolver, limiter, store_flux, with_dt, prec):
     """The launch splits what does not fill the chip into z slabs.  1024 patch groups fill it with whole ones on 256 compute
     units (one or two groups each); every smaller call has to give the same bits, fluxes and time steps included, and the
     work queue, which never splits, too."""
     from gamer_amd import hydro
-    print(f"[gpu] slabs {rsolver} {limiter} flux {store_flux} dt {with_dt} {prec}", flush=True)
+    print(f"[gpu] slabs {scheme} {rsolver} {limiter} flux {store_flux} dt {with_dt} {prec}", flush=True)
     dtype = torch.float64 if prec == "fp64" else torch.float32
-    u = _random_groups(1024, 22, dtype)
+    u = _random_groups(1024, hydro.NX[scheme], dtype)
     g = torch.Generator(device=DEV).manual_seed(21)
     dtdh = torch.rand((1024, 2), dtype=torch.float64, device=DEV, generator=g) * 1e-4 + 1e-4
     dtdh[:, 1] = 1.0 / 64
 
     def solve(n, **kw):
         dtp = torch.full((n, 8), -1.0, dtype=dtype, device=DEV) if with_dt else None
-        out, flux = hydro.solve_batch(u[:n], dtdh[:n], rsolver=rsolver, limiter=limiter, store_flux=store_flux,
+        out, flux = hydro.solve_batch(u[:n], dtdh[:n], scheme=scheme, rsolver=rsolver, limiter=limiter, store_flux=store_flux,
                                       dt_patch=dtp, **kw)
         return [x for x in (out, flux, dtp) if x is not None]
 
