@@ -428,8 +428,8 @@ int hydro_prepare_patches_async( const void *patch, void *pg_in, int npg, const 
    return rc == 0 ? HYDRO_OK : fail( HYDRO_E_DEVICE, "prepare_patches launch failed" );
 }
 
-int hydro_gather_boxes_async( const void *patch, void *box, int nbox, const int size[3], const int origin[3],
-                              const int *slot, const int tdim[3], int precision, void *stream )
+static int gather_boxes( const void *patch, const void *patch2, void *box, int nbox, const int size[3], const int origin[3],
+                         const int *slot, const int tdim[3], int precision, void *stream )
 {
    if ( nbox < 0 || size == nullptr || origin == nullptr || tdim == nullptr ||
         ( nbox > 0 && ( patch == nullptr || box == nullptr || slot == nullptr ) ) )
@@ -443,10 +443,23 @@ int hydro_gather_boxes_async( const void *patch, void *box, int nbox, const int 
       g.size[d] = size[d];  g.origin[d] = origin[d];  g.tdim[d] = tdim[d];
    }
    int rc;
-   if      ( precision == HYDRO_FP64 )      rc = launch_gather_boxes<double>( (const double*)patch, (double*)box, nbox, g, slot, (hipStream_t)stream );
-   else if ( precision == HYDRO_FP32_BULK ) rc = launch_gather_boxes<float> ( (const float*)patch,  (float*)box,  nbox, g, slot, (hipStream_t)stream );
+   if      ( precision == HYDRO_FP64 )      rc = launch_gather_boxes<double>( (const double*)patch, (const double*)patch2, (double*)box, nbox, g, slot, (hipStream_t)stream );
+   else if ( precision == HYDRO_FP32_BULK ) rc = launch_gather_boxes<float> ( (const float*)patch,  (const float*)patch2,  (float*)box,  nbox, g, slot, (hipStream_t)stream );
    else return fail( HYDRO_E_ARG, "unsupported precision %d", precision );
    return rc == 0 ? HYDRO_OK : fail( HYDRO_E_DEVICE, "gather_boxes launch failed" );
+}
+
+int hydro_gather_boxes_async( const void *patch, void *box, int nbox, const int size[3], const int origin[3],
+                              const int *slot, const int tdim[3], int precision, void *stream )
+{
+   return gather_boxes( patch, nullptr, box, nbox, size, origin, slot, tdim, precision, stream );
+}
+
+int hydro_gather_boxes_mean_async( const void *patch_a, const void *patch_b, void *box, int nbox, const int size[3],
+                                   const int origin[3], const int *slot, const int tdim[3], int precision, void *stream )
+{
+   if ( nbox > 0 && patch_b == nullptr ) return fail( HYDRO_E_ARG, "gather_boxes: bad pointers/size" );
+   return gather_boxes( patch_a, patch_b, box, nbox, size, origin, slot, tdim, precision, stream );
 }
 
 int hydro_assemble_patch_groups_async( const void *patch, const void *fbox, void *pg_in, int npg, const int *slot,

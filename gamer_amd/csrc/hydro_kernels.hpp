@@ -118,10 +118,11 @@ int launch_interpolate( T *cdata, T *fdata, int nbox, const InterpPrm &p, int *n
 // same-level part of the patch-group input preparation: slot[npg][4][4][4] of patch indices (-1 = keep)
 template <typename IO>
 int launch_prepare_patches( const IO *patch, IO *pg_in, int npg, const int *slot, int ghost, hipStream_t stream );
-// a box of `size` cells at `origin` inside a tdim[0] x tdim[1] x tdim[2] table of 8^3 patches
+// a box of `size` cells at `origin` inside a tdim[0] x tdim[1] x tdim[2] table of 8^3 patches; patch2 (or NULL): half the sum of
+// patch and patch2
 struct BoxGeom { int size[3], origin[3], tdim[3]; };
 template <typename IO>
-int launch_gather_boxes( const IO *patch, IO *box, int nbox, const BoxGeom &g, const int *slot, hipStream_t stream );
+int launch_gather_boxes( const IO *patch, const IO *patch2, IO *box, int nbox, const BoxGeom &g, const int *slot, hipStream_t stream );
 template <typename IO>
 int launch_assemble( const IO *patch, const IO *fbox, IO *pg_in, int npg, const int *slot, int ghost, const BoxGeom &fb,
                      hipStream_t stream );

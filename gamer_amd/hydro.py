@@ -37,7 +37,8 @@ EXPORTS = ("hydro_init", "hydro_mhm_solve_async", "hydro_synchronize", "hydro_la
            "hydro_mhm_tangent_async", "hydro_prepare_uniform_adjoint_async", "hydro_correct_unphysical_async",
            "hydro_store_flux_async", "hydro_correct_flux_async", "hydro_fixup_flux_async",
            "hydro_fixup_restrict_async", "hydro_close_patches_async", "hydro_interpolate_async",
-           "hydro_prepare_patches_async", "hydro_gather_boxes_async", "hydro_assemble_patch_groups_async",
+           "hydro_prepare_patches_async", "hydro_gather_boxes_async", "hydro_gather_boxes_mean_async",
+           "hydro_assemble_patch_groups_async",
            "hydro_host_dt_buffers", "hydro_asyn_dt_solver", "hydro_device_info", "hydro_mhm_solve_batch_noalloc")
 
 
@@ -152,6 +153,8 @@ def lib():
         I3p = ctypes.POINTER(ctypes.c_int * 3)
         L.hydro_gather_boxes_async.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, I3p, I3p,
                                                ctypes.c_void_p, I3p, ctypes.c_int, ctypes.c_void_p]
+        L.hydro_gather_boxes_mean_async.argtypes = [ctypes.c_void_p] * 3 + [ctypes.c_int, I3p, I3p, ctypes.c_void_p, I3p,
+                                                    ctypes.c_int, ctypes.c_void_p]
         L.hydro_assemble_patch_groups_async.argtypes = [ctypes.c_void_p] * 3 + [ctypes.c_int, ctypes.c_void_p,
                                                         ctypes.c_int, I3p, I3p, ctypes.c_int, ctypes.c_void_p]
         _lib = L
@@ -535,9 +538,10 @@ def prepare_patches(patch, pg_in, slot, ghost, stream=None):
     return pg_in
 
 
-def gather_boxes(patch, box, slot, origin, stream=None):
+def gather_boxes(patch, box, slot, origin, stream=None, mean_with=None):
     """Coarse boxes (nbox, 5, sz, sy, sx) from patches (npatch, 5, 8, 8, 8), in place: box cell (x,y,z) comes from the
-    patch covering cell origin + (x,y,z) of the box's slot table slot (nbox, tz, ty, tx) (-1 = keep).  (x,y,z) tuples."""
+    patch covering cell origin + (x,y,z) of the box's slot table slot (nbox, tz, ty, tx) (-1 = keep).  (x,y,z) tuples.
+    ``mean_with``: patches like ``patch``; the boxes then hold (patch + mean_with) * 0.5."""
     nbox = box.shape[0]
     tdim = tuple(reversed(slot.shape[1:]))
     _int_table(slot, (nbox,) + tuple(slot.shape[1:]), "slot")
@@ -545,10 +549,16 @@ def gather_boxes(patch, box, slot, origin, stream=None):
         raise HydroError("gather_boxes: slot must be (nbox, tz, ty, tx)")
     I3 = ctypes.c_int * 3
     patch = patch.contiguous()
-    _check(lib().hydro_gather_boxes_async(patch.data_ptr(), box.data_ptr(), nbox,
-                                          ctypes.byref(I3(*reversed(box.shape[2:]))), ctypes.byref(I3(*origin)),
-                                          slot.data_ptr(), ctypes.byref(I3(*tdim)), _prec(box),
-                                          _stream(box.device, stream, patch, box, slot)))
+    rest = (box.data_ptr(), nbox, ctypes.byref(I3(*reversed(box.shape[2:]))), ctypes.byref(I3(*origin)), slot.data_ptr(),
+            ctypes.byref(I3(*tdim)), _prec(box))
+    if mean_with is None:
+        _check(lib().hydro_gather_boxes_async(patch.data_ptr(), *rest, _stream(box.device, stream, patch, box, slot)))
+        return box
+    if mean_with.shape != patch.shape or mean_with.dtype != patch.dtype or mean_with.device != patch.device:
+        raise HydroError("gather_boxes: mean_with must be like patch")
+    other = mean_with.contiguous()
+    _check(lib().hydro_gather_boxes_mean_async(patch.data_ptr(), other.data_ptr(), *rest,
+                                               _stream(box.device, stream, patch, other, box, slot)))
     return box
 
 
@@ -570,13 +580,14 @@ def assemble_patch_groups(patch, fbox, pg_in, slot, ghost, fb_origin, stream=Non
 
 
 def prepare_refined_patch_groups(coarse_patch, fine_patch, coarse_slot, fine_slot, pg_in, ghost=3, scheme="CQUAD",
-                                 need=None, stream=None, nfail=None, **interp_kw):
+                                 need=None, stream=None, nfail=None, coarse_mean_with=None, **interp_kw):
     """Prepare_PatchData for fine patch groups at a refinement boundary, on the device: the coarse box of each patch
     group (father patch + 26 siblings: coarse_slot (npg, 3, 3, 3)) -> Interpolate() over coarse cells -2..9 around the
     father (the 22^3 window of ghost 3 plus one fine cell) -> same-level fine patches (fine_slot (npg, 4, 4, 4)) and
     the interpolated cells into pg_in (npg, 5, 16+2g, ...).  ``need`` (npg, 12, 12, 12) uint8, optional: the coarse
     cells whose fine cells have no same-level patch (gamer_amd.amr.refined_interp_need); only those are
-    interpolated.  Returns the interpolation failure counter (``nfail``, when given, is added to and returned)."""
+    interpolated.  Returns the interpolation failure counter (``nfail``, when given, is added to and returned).
+    ``coarse_mean_with``: the coarse data are (coarse_patch + coarse_mean_with) * 0.5."""
     import torch
     if ghost != 3:
         raise HydroError("prepare_refined_patch_groups: ghost 3 (the MHM_RP window) only")
@@ -584,7 +595,7 @@ def prepare_refined_patch_groups(coarse_patch, fine_patch, coarse_slot, fine_slo
     npg = pg_in.shape[0]
     n = 12 + 2 * g
     cbox = torch.empty((npg, 5, n, n, n), dtype=pg_in.dtype, device=pg_in.device)
-    gather_boxes(coarse_patch, cbox, coarse_slot, (6 - g,) * 3, stream=stream)
+    gather_boxes(coarse_patch, cbox, coarse_slot, (6 - g,) * 3, stream=stream, mean_with=coarse_mean_with)
     fbox = torch.empty((npg, 5, 24, 24, 24), dtype=pg_in.dtype, device=pg_in.device)
     nfail = interpolate(cbox, fbox, (g,) * 3, (12, 12, 12), scheme=scheme, need=need, stream=stream, nfail=nfail,
                         **interp_kw)

@@ -213,6 +213,10 @@ int hydro_prepare_patches_async( const void *patch, void *pg_in, int npg, const 
    scheme's coarse ghost width. */
 int hydro_gather_boxes_async( const void *patch, void *box, int nbox, const int size[3], const int origin[3],
                               const int *slot, const int tdim[3], int precision, void *stream );
+/* The same from half the sum of two patch arrays: coarse data halfway between two times
+   (src/Main/Prepare_PatchData.cpp:2282-2283 with both weights 1/2). */
+int hydro_gather_boxes_mean_async( const void *patch_a, const void *patch_b, void *box, int nbox, const int size[3],
+                                   const int origin[3], const int *slot, const int tdim[3], int precision, void *stream );
 
 /* Patch-group inputs at a refinement boundary (Prepare_PatchData, src/Main/Prepare_PatchData.cpp:166): cells
    with a same-level patch in slot[npg][4][4][4] copy it, as hydro_prepare_patches_async; the others take the

@@ -80,3 +80,7 @@ def test_windows_and_boxes(ghost, dtype):
         dst = T(box)
         hydro.gather_boxes(T(patch), dst, T(bs), origin)
         np.testing.assert_array_equal(dst.cpu().numpy(), oracle.gather_boxes(patch, box, bs, origin))
+        late = rng.standard_normal(patch.shape).astype(dtype)
+        dst = T(box)
+        hydro.gather_boxes(T(patch), dst, T(bs), origin, mean_with=T(late))
+        np.testing.assert_array_equal(dst.cpu().numpy(), oracle.gather_boxes((patch + late) * dtype(0.5), box, bs, origin))
