@@ -31,6 +31,10 @@ int fail( int code, const char *fmt, ... )
    do { hipError_t e_ = ( call );                                                                \
         if ( e_ != hipSuccess ) return fail( HYDRO_E_DEVICE, "%s: %s", #call, hipGetErrorString( e_ ) ); } while (0)
 
+// pieces of a large call of the host-array solver, and the input from which a call is large (solve_duplex())
+constexpr int    HOST_PIECES       = 3;
+constexpr size_t HOST_DUPLEX_BYTES = 20000000;
+
 // GPU_API state: device buffers sized once for flu_npg patch groups, pinned host double buffers, streams
 // (the module globals of src/GPU_API/CUAPI_MemAllocate_Fluid.cu:211-334)
 struct FluidBuffers {
@@ -43,6 +47,12 @@ struct FluidBuffers {
    void  *d_flu_t = nullptr, *d_dt = nullptr;
    void  *h_flu_t[2] = { nullptr, nullptr }, *h_dt[2] = { nullptr, nullptr };
    std::vector<hipStream_t> streams;
+   // large calls of the fluid solver: streams of the copies in, the copies out and the kernels, created one after the other
+   // so that they get hardware queues of their own; a piece's input there, solved; all results out
+   hipStream_t up = nullptr, down = nullptr, mid = nullptr;
+   hipEvent_t  here[HOST_PIECES] = {}, done[HOST_PIECES] = {}, out = nullptr, left = nullptr;
+   // per stream: holds work of a small call that no large one has waited for; has not yet waited for the last large call
+   std::vector<char> small_work, large_ahead;
 };
 FluidBuffers g_buf;
 std::mutex   g_mtx;
@@ -159,6 +169,16 @@ void free_buffers()
       if ( g_buf.h_dt[k] )    (void)hipHostFree( g_buf.h_dt[k] );
    }
    for (hipStream_t s : g_buf.streams) (void)hipStreamDestroy( s );
+   if ( g_buf.up )   (void)hipStreamDestroy( g_buf.up );
+   if ( g_buf.down ) (void)hipStreamDestroy( g_buf.down );
+   if ( g_buf.mid )  (void)hipStreamDestroy( g_buf.mid );
+   if ( g_buf.out )  (void)hipEventDestroy( g_buf.out );
+   if ( g_buf.left ) (void)hipEventDestroy( g_buf.left );
+   for (int c=0; c<HOST_PIECES; c++)
+   {
+      if ( g_buf.here[c] ) (void)hipEventDestroy( g_buf.here[c] );
+      if ( g_buf.done[c] ) (void)hipEventDestroy( g_buf.done[c] );
+   }
    g_buf = FluidBuffers();
 }
 
@@ -561,6 +581,19 @@ int hydro_mem_allocate_fluid( int flu_npg, int nstream, int scheme, int precisio
       free_buffers();
       return fail( HYDRO_E_NOMEM, "allocation of %d patch groups x %d streams failed", flu_npg, nstream );
    }
+   ok = hipStreamCreateWithFlags( &g_buf.up, hipStreamNonBlocking ) == hipSuccess &&
+        hipStreamCreateWithFlags( &g_buf.down, hipStreamNonBlocking ) == hipSuccess &&
+        hipStreamCreateWithFlags( &g_buf.mid, hipStreamNonBlocking ) == hipSuccess &&
+        hipEventCreateWithFlags( &g_buf.out, hipEventDisableTiming ) == hipSuccess &&
+        hipEventCreateWithFlags( &g_buf.left, hipEventDisableTiming ) == hipSuccess;
+   for (int c=0; c<HOST_PIECES && ok; c++)
+      ok = hipEventCreateWithFlags( &g_buf.here[c], hipEventDisableTiming ) == hipSuccess &&
+           hipEventCreateWithFlags( &g_buf.done[c], hipEventDisableTiming ) == hipSuccess;
+   if ( !ok )
+   {
+      free_buffers();
+      return fail( HYDRO_E_DEVICE, "stream creation failed" );
+   }
    g_buf.streams.resize( nstream );
    for (int s=0; s<nstream; s++)
       if ( hipStreamCreateWithFlags( &g_buf.streams[s], hipStreamNonBlocking ) != hipSuccess )
@@ -569,6 +602,8 @@ int hydro_mem_allocate_fluid( int flu_npg, int nstream, int scheme, int precisio
          free_buffers();
          return fail( HYDRO_E_DEVICE, "stream creation failed" );
       }
+   g_buf.small_work.assign( nstream, 0 );
+   g_buf.large_ahead.assign( nstream, 0 );
    g_buf.npg_max = flu_npg;  g_buf.nstream = nstream;  g_buf.scheme = scheme;  g_buf.precision = precision;
    return HYDRO_OK;
 }
@@ -655,6 +690,49 @@ int hydro_device_info( HydroDeviceInfo *info )
    info->concurrent_kernels    = p.concurrentKernels;
    return HYDRO_OK;
 }
+// Large calls: all copies in on one stream, all kernels on another, all copies out on a third, in HOST_PIECES pieces joined
+// by events.  With each piece's copy in, kernel and copy out on one of several streams, the copies of both directions came
+// one after the other (512 FP32 MHM_RP patch groups, 109 MB in and 66 MB out: 3150 us = the sum of both at 56 GB/s), where
+// the link takes both at once (115 MB each way 2.39 ms, alone 2.02).  These
+// take 2452 us; 128 FP32 patch groups 788 -> 698, 512 FP64 6218 -> 4794.  Four pieces 2497, 721 and 4857; 14 MB of input
+// 421 -> 406, 7 MB 223 -> 260, where the events cost more than the overlap gives.
+static int solve_duplex( const HydroSolveArgs &a, const void *h_in, void *h_out, void *h_flux, size_t in_pg, size_t out_pg, size_t fl_pg )
+{
+   hipStream_t st = g_buf.mid;
+   HIP_TRY( hipStreamWaitEvent( g_buf.up, g_buf.done[HOST_PIECES - 1], 0 ) );     // the last call's kernels have read d_in
+   HIP_TRY( hipStreamWaitEvent( st, g_buf.out, 0 ) );                             // its results have left d_out and d_flux
+   for (int s=0; s<g_buf.nstream; s++)                                            // and the small calls before are through
+   {
+      g_buf.large_ahead[s] = 1;
+      if ( !g_buf.small_work[s] ) continue;
+      g_buf.small_work[s] = 0;
+      HIP_TRY( hipEventRecord( g_buf.left, g_buf.streams[s] ) );
+      HIP_TRY( hipStreamWaitEvent( g_buf.up, g_buf.left, 0 ) );
+      HIP_TRY( hipStreamWaitEvent( st, g_buf.left, 0 ) );
+   }
+   for (int c=0; c<HOST_PIECES; c++)
+   {
+      const size_t off = (size_t)a.npg*c/HOST_PIECES, n = (size_t)a.npg*( c + 1 )/HOST_PIECES - off;
+      char *din = (char*)g_buf.d_in + off*in_pg, *dout = (char*)g_buf.d_out + off*out_pg, *dfl = (char*)g_buf.d_flux + off*fl_pg;
+      HIP_TRY( hipMemcpyAsync( din, (const char*)h_in + off*in_pg, n*in_pg, hipMemcpyHostToDevice, g_buf.up ) );
+      HIP_TRY( hipEventRecord( g_buf.here[c], g_buf.up ) );
+      HIP_TRY( hipStreamWaitEvent( st, g_buf.here[c], 0 ) );
+      const int rc = enqueue( &a, din, dout, dfl, nullptr, (int)n, st );
+      if ( rc != HYDRO_OK ) return rc;
+      HIP_TRY( hipEventRecord( g_buf.done[c], st ) );
+   }
+   for (int c=0; c<HOST_PIECES; c++)
+   {
+      const size_t off = (size_t)a.npg*c/HOST_PIECES, n = (size_t)a.npg*( c + 1 )/HOST_PIECES - off;
+      HIP_TRY( hipStreamWaitEvent( g_buf.down, g_buf.done[c], 0 ) );
+      HIP_TRY( hipMemcpyAsync( (char*)h_out + off*out_pg, (char*)g_buf.d_out + off*out_pg, n*out_pg, hipMemcpyDeviceToHost, g_buf.down ) );
+      if ( a.store_flux )
+         HIP_TRY( hipMemcpyAsync( (char*)h_flux + off*fl_pg, (char*)g_buf.d_flux + off*fl_pg, n*fl_pg, hipMemcpyDeviceToHost, g_buf.down ) );
+   }
+   HIP_TRY( hipEventRecord( g_buf.out, g_buf.down ) );
+   return HYDRO_OK;
+}
+
 int hydro_asyn_fluid_solver( const void *h_in, void *h_out, void *h_flux, const HydroSolveArgs *args, int gpu_nstream )
 {
    // call order first: without buffers no argument can be valid
@@ -672,6 +750,7 @@ int hydro_asyn_fluid_solver( const void *h_in, void *h_out, void *h_flux, const 
 
    const int nx = nx_of( a.scheme );
    const size_t in_pg = (size_t)5*nx*nx*nx*g_buf.elem, out_pg = (size_t)5*4096*g_buf.elem, fl_pg = (size_t)9*5*256*g_buf.elem;
+   if ( a.npg*in_pg >= HOST_DUPLEX_BYTES ) return solve_duplex( a, h_in, h_out, h_flux, in_pg, out_pg, fl_pg );
    // NPG/NStream per stream, remainder to the last stream (CUAPI_Asyn_FluidSolver.cu:433-445)
    const int base = a.npg / gpu_nstream;
    int off = 0;
@@ -681,6 +760,13 @@ int hydro_asyn_fluid_solver( const void *h_in, void *h_out, void *h_flux, const 
       if ( n <= 0 ) continue;
       hipStream_t st = g_buf.streams[s];
       char *din = (char*)g_buf.d_in + off*in_pg, *dout = (char*)g_buf.d_out + off*out_pg, *dfl = (char*)g_buf.d_flux + off*fl_pg;
+      if ( g_buf.large_ahead[s] )
+      {
+         g_buf.large_ahead[s] = 0;
+         HIP_TRY( hipStreamWaitEvent( st, g_buf.done[HOST_PIECES - 1], 0 ) );
+         HIP_TRY( hipStreamWaitEvent( st, g_buf.out, 0 ) );
+      }
+      g_buf.small_work[s] = 1;
       HIP_TRY( hipMemcpyAsync( din, (const char*)h_in + off*in_pg, n*in_pg, hipMemcpyHostToDevice, st ) );
       rc = enqueue( &a, din, dout, dfl, nullptr, n, st );
       if ( rc != HYDRO_OK ) return rc;
