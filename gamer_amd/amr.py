@@ -142,9 +142,8 @@ def autotune(torch, batch: LevelBatch, groups=(1, 2, 3, 4), tickets=(1, 2, 4), w
 
     Configurations: one workgroup per patch group ("grid:w"), and the persistent work queue ("persistent:g:k:w")
     with g workgroups per compute unit for g in ``groups``, each taking k consecutive patch groups per queue
-    ticket for k in ``tickets`` (fewer queue atomics and barriers against a coarser tail); each in every workgroup
-    shape w of ``waves`` (MHM_RP: 4 waves, every lane marching an output column and a ghost role, or 8 waves, the
-    two on separate waves; MHM: 4 only).  The configurations are timed in ``rounds`` interleaved rounds of
+    ticket for k in ``tickets`` (fewer queue atomics and barriers against a coarser tail); each with every value w of
+    ``waves`` as ``waves_per_group`` (accepted values; each scheme has one workgroup shape).  The configurations are timed in ``rounds`` interleaved rounds of
     ``reps`` launches and each keeps its best round, so that a clock or thermal drift during the sweep does not
     pick the winner.  Results are cached in ``cache`` (a JSON path) keyed by the batch shape and precision when
     given."""
