@@ -423,9 +423,12 @@ prepare_patches_kernel( const IO *__restrict__ patch, const IO *__restrict__ fbo
 // slot -1 keeps the box value.  Block (box, field, GB_N cells of the box in linear order), as above; the sizes are general,
 // so the cell's coordinates take two integer divisions.  With patch2, half the sum of the cells of both: coarse data halfway
 // between two times, where two passes over the whole level made them first (20 + 23 us of a two-level step of 4096 patches). 
-// 512 boxes of 14^3 FP32 cells: 22 us, one block per plane 24.
-constexpr int GB_NT = 256, GB_Q = 6, GB_N = GB_NT*GB_Q;
-template <typename IO>
+// One block per plane took 24 us where the same with divisions takes 22.
+// SMALL: boxes of at most GB_SMALL cells take the coordinates from float reciprocals instead, which is most of the instructions
+// otherwise: (e + 0.5)/nxy lies at least 1/(2 nxy) from an integer and its float error is below nz/2^22, less than that for
+// nxy*nz < 2^21.  512 boxes of 14^3 FP32 cells: 18 us with them, 23 with the divisions (the half sum 24.6 and 27.5).
+constexpr int GB_NT = 512, GB_Q = 6, GB_N = GB_NT*GB_Q, GB_SMALL = 1 << 20;
+template <typename IO, bool SMALL>
 __global__ void __launch_bounds__( GB_NT )
 gather_boxes_kernel( const IO *__restrict__ patch, const IO *__restrict__ patch2, IO *__restrict__ box, BoxGeom g,
                      const int *__restrict__ slot, unsigned chunks )
@@ -439,13 +442,25 @@ gather_boxes_kernel( const IO *__restrict__ patch, const IO *__restrict__ patch2
    IO *dst = box + w*n;
    const IO *src[GB_Q];
    const ptrdiff_t other = patch2 ? patch2 - patch : 0;
+   const float rx = 1.0f/(float)nx, rxy = 1.0f/(float)nxy;
 #  pragma unroll
    for (int k=0; k<GB_Q; k++)
    {
       const long e = e0 + k*GB_NT;
       src[k] = nullptr;
       if ( e >= n ) continue;
-      const unsigned z = ( n >> 32 ) ? (unsigned)( e / nxy ) : (unsigned)e / nxy, r = (unsigned)( e - (long)z*nxy ), y = r / nx, x = r - y*nx;
+      unsigned z, r, y;
+      if ( SMALL )
+      {
+         z = (unsigned)( ( (float)(int)e + 0.5f )*rxy );  r = (unsigned)e - z*nxy;
+         y = (unsigned)( ( (float)(int)r + 0.5f )*rx );
+      }
+      else
+      {
+         z = ( n >> 32 ) ? (unsigned)( e / nxy ) : (unsigned)e / nxy;  r = (unsigned)( e - (long)z*nxy );
+         y = r / nx;
+      }
+      const unsigned x = r - y*nx;
       const int X = (int)x + g.origin[0], Y = (int)y + g.origin[1], Z = (int)z + g.origin[2];
       const int s = sl[ ( (size_t)( Z >> 3 )*g.tdim[1] + ( Y >> 3 ) )*g.tdim[0] + ( X >> 3 ) ];
       if ( s >= 0 ) src[k] = pv + ( (size_t)s*NV*P3 + ( Z & 7 )*H*H + ( Y & 7 )*H + ( X & 7 ) );
@@ -497,8 +512,10 @@ int launch_gather_boxes( const IO *patch, const IO *patch2, IO *box, int nbox, c
 {
    if ( nbox <= 0 ) return 0;
    const long n = (long)g.size[0]*g.size[1]*g.size[2], chunks = ( n + GB_N - 1 )/GB_N;
-   hipLaunchKernelGGL( gather_boxes_kernel<IO>, dim3( nbox, NV, (unsigned)chunks ), dim3( GB_NT ), 0, stream, patch, patch2, box, g, slot,
-                       (unsigned)chunks );
+#  define GA_GB( SMALL_ ) hipLaunchKernelGGL( ( gather_boxes_kernel<IO, SMALL_> ), dim3( nbox, NV, (unsigned)chunks ), dim3( GB_NT ), 0, \
+                                              stream, patch, patch2, box, g, slot, (unsigned)chunks )
+   if ( n <= GB_SMALL ) GA_GB( true ); else GA_GB( false );
+#  undef GA_GB
    return ( hipGetLastError() == hipSuccess ) ? 0 : -2;
 }
 

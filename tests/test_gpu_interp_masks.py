@@ -74,7 +74,8 @@ def test_windows_and_boxes(ghost, dtype):
         hydro.assemble_patch_groups(T(patch), T(fb), dst, T(slot), ghost, (1, 2, 3))
         np.testing.assert_array_equal(dst.cpu().numpy(), oracle.assemble_patch_groups(patch, fb, pg, slot, ghost, (1, 2, 3)))
     for size, origin, tdim in (((1, 1, 1), (0, 0, 0), (1, 1, 1)), ((14, 14, 14), (5, 5, 5), (3, 3, 3)),
-                               ((33, 7, 19), (6, 1, 4), (5, 1, 3)), ((16, 16, 6), (0, 0, 10), (2, 2, 2))):
+                               ((33, 7, 19), (6, 1, 4), (5, 1, 3)), ((16, 16, 6), (0, 0, 10), (2, 2, 2)),
+                               ((128, 64, 128), (0, 3, 5), (16, 9, 17)), ((101, 103, 101), (1, 0, 2), (13, 13, 13))):
         bs = rng.integers(-4, npatch, (npg,) + tdim[::-1]).clip(-1).astype(np.int32)
         box = np.full((npg, 5) + size[::-1], -6.0, dtype=dtype)
         dst = T(box)
