@@ -303,6 +303,7 @@ int hydro_device_info( HydroDeviceInfo *info );
 
 /* Asynchronous solve over host arrays: per stream H2D copy, kernel, D2H copy of out (and flux), the
    NPG/NStream split with the remainder on the last stream (src/GPU_API/CUAPI_Asyn_FluidSolver.cu:433-722).
+   Calls with 20 MB of input or more run in three pieces with a stream of the library's own for each copy direction.
    Host arrays should be the pinned buffers from hydro_host_buffers.  Returns before the GPU finishes.  As in
    GAMER (src/Main/InvokeSolver.cpp:227-267), one call is in flight at a time: both host buffers share the device
    arrays, so call hydro_synchronize before the next call; the other host buffer can be filled or read meanwhile. */
