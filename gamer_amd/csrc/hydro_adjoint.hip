@@ -2,8 +2,7 @@
 //
 // The step is the map U_in (22^3 x 5 per patch group) -> U_out (16^3 x 5) of the forward kernel
 // (src/Model_Hydro/CPU_Hydro/CPU_FluidSolver_MHM.cpp:263-589 with the half-step prediction of :615-949).
-// Explicit phases over a per-PG global workspace, each phase one kernel over all patch groups with one face or
-// cell per lane:
+// Explicit phases over a per-PG global workspace, one kernel for one or two phases over all patch groups:
 //
 //   forward   F1 + F2, z plane by z plane: half-step fluxes (Hydro_RiemannPredict_Flux) in LDS, then the half-step
 //                update, floors and primitive W (Hydro_RiemannPredict) -> ws
@@ -21,7 +20,7 @@
 // The reverse sweep is written out by hand.  The Riemann solves (HLLC, HLLE and Roe) run backwards as hand-written
 // reverse-mode sweeps (hydro_reverse.hpp: solver + interface-state builders, one pass per face for all ten
 // inputs).  The PLM reconstruction (face clamps and mirror) is reversed by hand for every
-// limiter, with the limited slope's two partials from a two-direction dual evaluation.  The half-step conversion
+// limiter, with the limited slope's two partials from a two-direction dual evaluation (written out for VL_GMINMOD).  The half-step conversion
 // with floors takes its local Jacobian from forward-mode dual numbers (hydro_dual.hpp) pushed through the same
 // templated device function, one input direction at a time.  All forms take exactly the branches of the forward
 // evaluation.
@@ -216,11 +215,11 @@ template <> struct Load< Dual<1> >
 };
 
 // ---------------- phases: one kernel each, one element per lane ----------------
-// Every phase is a gather over the faces or cells of each patch group that reads only what earlier phases
-// wrote, so the phases run as separate kernels in stream order, each over a flat grid of bpp(count) workgroups
-// per patch group: element e of patch group pg is lane e % NT of workgroup pg*bpp + e / NT.  One workgroup
-// marching through all phases of its patch group kept only 4 waves per patch group busy; spread over the grid,
-// a phase keeps as many patch groups' workspace traffic in flight as the registers of its own kernel allow.
+// Every phase is a gather over the faces or cells of each patch group that reads only what earlier phases wrote, so the
+// phases run as separate kernels in stream order, each over many workgroups per patch group: R4 and F4 over flat grids of
+// bpp(count) workgroups (element e of patch group pg is lane e % NT of workgroup pg*bpp + e / NT), the others over blocks of
+// rows and planes.  One workgroup marching through all phases of its patch group kept only 4 waves per patch group busy;
+// spread over the grid, a phase keeps as many patch groups' workspace traffic in flight as its registers allow.
 constexpr int bpp( int count ) { return ( count + NT - 1 ) / NT; }
 constexpr int N_F4 = PS*PS*PS, N_R4 = 3*NFF;
 
