@@ -464,8 +464,11 @@ __device__ __forceinline__ St<R> cons_state( const R c[NV], const Prm<R> &P )
 // 9.2 (FP64: 4.8 and 18.5), with two wait states between a compare and its select.  Against rs_hllc() of the
 // derivative and correction kernels (the same HLLC fluxes, CPU_Shared_RiemannSolver_HLLC.cpp:391-655) this form
 //   * takes tl = rho_L (u_L - w_L), tr = rho_R (w_R - u_R) from the wave speeds instead of by selects,
-//   * takes the contact as u_L + x and its pressure as p_L - tl x, x = (p_L - p_R - tr (u_L - u_R))/(tl + tr):
-//     differences come before products, 5 operations instead of 9,
+//   * takes the contact's speed and pressure as means of both sides with the weights tl and tr, the pressure's velocity
+//     term from the difference: (tl (p_R + tr (u_L - u_R)) + tr p_L)/(tl + tr).  Where one side is much denser, neither
+//     may be formed from a value of one side and a step: the step cancels the heavy side's pressure or the fast side's
+//     velocity, and its rounding stays (p_L - tl x, x = (p_L - p_R - tr (u_L - u_R))/(tl + tr), was off by 6e-3 in the
+//     light gas at a density contrast of 1e6 in FP32).  tl tr alone leaves the FP32 range for gases of 1e-24 g/cm^3,
 //   * forms the flux as mass flux times (1, u, a, b, e) plus pressure terms, and, on faces, the energy only of the
 //     side that the contact selects,
 //   * leaves the vs == sp == 0 case to the NaN rescue: HLLE's flux there is the physical flux of the left state.
@@ -543,14 +546,14 @@ __device__ __forceinline__ void hllc_flux( const Side<R> L[N], const Side<R> Q[N
 {
    #pragma clang fp contract(off)
    const R Z = (R)0;
-   R wl[N], wr[N], tl[N], tr[N], x[N], vs[N], ps[N], sp[N], t[N], m[N], cp[N], cs[N];
+   R wl[N], wr[N], tl[N], tr[N], r[N], vs[N], ps[N], sp[N], t[N], m[N], cp[N], cs[N];
    bool left[N];
 #  define GA_N _Pragma( "unroll" ) for (int n=0; n<N; n++)
    GA_N { wl[n] = vmin( L[n].u - L[n].cs, Q[n].u - Q[n].cs );  wr[n] = vmax( L[n].u + L[n].cs, Q[n].u + Q[n].cs ); }
    GA_N { tl[n] = L[n].d*( L[n].u - wl[n] );  tr[n] = Q[n].d*( wr[n] - Q[n].u ); }
-   GA_N x[n]  = rcp( tl[n] + tr[n] )*fmad( tr[n], Q[n].u - L[n].u, L[n].p - Q[n].p );
-   GA_N vs[n] = L[n].u + x[n];
-   GA_N ps[n] = vmax( fmad( -tl[n], x[n], L[n].p ), pmin );           // a NaN here is a NaN in vs too
+   GA_N r[n]  = rcp( tl[n] + tr[n] );
+   GA_N vs[n] = r[n]*fmad( tl[n], L[n].u, fmad( tr[n], Q[n].u, L[n].p - Q[n].p ) );
+   GA_N ps[n] = floor_nan( r[n]*fmad( tl[n], fmad( tr[n], L[n].u - Q[n].u, Q[n].p ), tr[n]*L[n].p ), pmin );
    GA_N left[n] = ( vs[n] >= Z );
    GA_N sp[n] = left[n] ? vmin( wl[n], Z ) : vmax( wr[n], Z );
    GA_N t[n]  = rcp( vs[n] - sp[n] );
