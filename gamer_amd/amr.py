@@ -121,7 +121,7 @@ def time_launch(torch, fn, reps=5, warmup=1):
 
 def launch_kwargs(torch, config, device):
     """solve_batch keyword arguments of an autotuner configuration name: "grid[:w]" or "persistent:g:k[:w]", with
-    w the workgroup shape in waves (absent: the library default)."""
+    w the ``waves_per_group`` to pass (absent: 0; every accepted value runs the scheme's one workgroup shape)."""
     parts = config.split(":")
     kw = {}
     if parts[0] == "grid":
@@ -142,10 +142,10 @@ def autotune(torch, batch: LevelBatch, groups=(1, 2, 3, 4), tickets=(1, 2, 4), w
 
     Configurations: one workgroup per patch group ("grid:w"), and the persistent work queue ("persistent:g:k:w")
     with g workgroups per compute unit for g in ``groups``, each taking k consecutive patch groups per queue
-    ticket for k in ``tickets`` (fewer queue atomics and barriers against a coarser tail); each with every value w of
-    ``waves`` as ``waves_per_group`` (accepted values; each scheme has one workgroup shape).  The configurations are timed in ``rounds`` interleaved rounds of
-    ``reps`` launches and each keeps its best round, so that a clock or thermal drift during the sweep does not
-    pick the winner.  Results are cached in ``cache`` (a JSON path) keyed by the batch shape and precision when
+    ticket for k in ``tickets`` (fewer queue atomics and barriers against a coarser tail).  The launches are timed in
+    ``rounds`` interleaved rounds of ``reps`` and each keeps its best round, so that a clock or thermal drift during the
+    sweep does not pick the winner.  w runs over ``waves``, values of ``waves_per_group`` that the scheme accepts: all of
+    them run its one workgroup shape, so the configurations that differ in w only share one time.  Results are cached in ``cache`` (a JSON path) keyed by the batch shape and precision when
     given."""
     npg = batch.u.shape[0]
     if waves is None:
@@ -163,19 +163,20 @@ def autotune(torch, batch: LevelBatch, groups=(1, 2, 3, 4), tickets=(1, 2, 4), w
     out = torch.empty((npg, 5, 16, 16, 16), dtype=batch.u.dtype, device=batch.u.device)
     flux = torch.empty((npg, 9, 5, 16, 16), dtype=batch.u.dtype, device=batch.u.device)
     counter = torch.zeros(1, dtype=torch.int32, device=batch.u.device)
-    configs = {}
-    for w in waves:
-        configs[f"grid:{w}"] = (lambda w=w: hydro.solve_batch(batch.u, batch.pg_dt_dh, out=out, flux=flux,
-                                                              waves_per_group=w, **kw))
-        for g in groups:
-            for k in tickets:
-                configs[f"persistent:{g}:{k}:{w}"] = (lambda g=g, k=k, w=w: hydro.solve_batch(
-                    batch.u, batch.pg_dt_dh, out=out, flux=flux, queue_counter=counter, groups_per_cu=g,
-                    pgs_per_ticket=k, waves_per_group=w, **kw))
-    trials = {name: float("inf") for name in configs}
+    def launch(w, **mode):
+        hydro.solve_batch(batch.u, batch.pg_dt_dh, out=out, flux=flux, waves_per_group=w, **mode, **kw)
+
+    launches = {"grid": {}}
+    for g in groups:
+        for k in tickets:
+            launches[f"persistent:{g}:{k}"] = dict(queue_counter=counter, groups_per_cu=g, pgs_per_ticket=k)
+    for w in waves:                                          # a value that the scheme does not accept raises here
+        launch(w)
+    ms = {name: float("inf") for name in launches}
     for _ in range(max(1, rounds)):
-        for name, fn in configs.items():
-            trials[name] = min(trials[name], time_launch(torch, fn, reps))
+        for name, mode in launches.items():
+            ms[name] = min(ms[name], time_launch(torch, lambda mode=mode: launch(waves[0], **mode), reps))
+    trials = {f"{name}:{w}": ms[name] for w in waves for name in launches}
     best = min(trials, key=trials.get)
     res = {"best": best, "ms": trials[best], "trials_ms": trials, "measured_at": time.time()}
     if cache:
