@@ -477,10 +477,14 @@ gather_boxes_kernel( const IO *__restrict__ patch, const IO *__restrict__ patch2
 
 } // namespace
 
+// Boxes of one launch: 512 lanes each, and a grid dimension holds less than 2^32 lanes (a launch of more runs the number
+// modulo 2^32, without an error)
+constexpr long BOX_GRID = ( 1L << 23 ) - 1;
+static unsigned boxes_from( long q0, long nbox ) { return (unsigned)( nbox - q0 < BOX_GRID ? nbox - q0 : BOX_GRID ); }
+
 template <typename T>
-int launch_interpolate( T *cdata, T *fdata, int nbox, const InterpPrm &p, int *nfail, hipStream_t stream )
+static int interpolate_boxes( T *cdata, T *fdata, int nbox, const InterpPrm &p, int *nfail, hipStream_t stream )
 {
-   if ( nbox <= 0 ) return 0;
    const bool plain = ( p.mono & 0x1F ) == 0x1F && !p.opp0;
 #  define GA_INT( S ) { if ( plain ) GA_LAUNCH( S, true ); else GA_LAUNCH( S, false ); }
 #  define GA_LAUNCH( S, PLAIN_ ) hipLaunchKernelGGL( ( interpolate_kernel<T, S, PLAIN_> ), dim3( nbox ), dim3( interp_lanes<T>( S ) ), 0, stream, \
@@ -501,6 +505,20 @@ int launch_interpolate( T *cdata, T *fdata, int nbox, const InterpPrm &p, int *n
    return ( hipGetLastError() == hipSuccess ) ? 0 : -2;
 }
 
+template <typename T>
+int launch_interpolate( T *cdata, T *fdata, int nbox, const InterpPrm &p, int *nfail, hipStream_t stream )
+{
+   const long C3 = (long)p.cs[0]*p.cs[1]*p.cs[2], F3 = (long)p.fs[0]*p.fs[1]*p.fs[2], ncell = (long)p.cr[0]*p.cr[1]*p.cr[2];
+   int rc = 0;
+   for (long q0 = 0; q0 < nbox && rc == 0; q0 += BOX_GRID)
+   {
+      InterpPrm part = p;
+      if ( p.need ) part.need = p.need + q0*ncell;
+      rc = interpolate_boxes( cdata + q0*NV*C3, fdata + q0*NV*F3, (int)boxes_from( q0, nbox ), part, nfail, stream );
+   }
+   return rc;
+}
+
 template <typename IO>
 int launch_prepare_patches( const IO *patch, IO *pg_in, int npg, const int *slot, int ghost, hipStream_t stream )
 {
@@ -511,10 +529,14 @@ template <typename IO>
 int launch_gather_boxes( const IO *patch, const IO *patch2, IO *box, int nbox, const BoxGeom &g, const int *slot, hipStream_t stream )
 {
    if ( nbox <= 0 ) return 0;
-   const long n = (long)g.size[0]*g.size[1]*g.size[2], chunks = ( n + GB_N - 1 )/GB_N;
-#  define GA_GB( SMALL_ ) hipLaunchKernelGGL( ( gather_boxes_kernel<IO, SMALL_> ), dim3( nbox, NV, (unsigned)chunks ), dim3( GB_NT ), 0, \
-                                              stream, patch, patch2, box, g, slot, (unsigned)chunks )
-   if ( n <= GB_SMALL ) GA_GB( true ); else GA_GB( false );
+   const long n = (long)g.size[0]*g.size[1]*g.size[2], chunks = ( n + GB_N - 1 )/GB_N, nslot = (long)g.tdim[0]*g.tdim[1]*g.tdim[2];
+#  define GA_GB( SMALL_ ) hipLaunchKernelGGL( ( gather_boxes_kernel<IO, SMALL_> ), dim3( nb, NV, (unsigned)chunks ), dim3( GB_NT ), 0, stream, \
+                                              patch, patch2, box + q0*NV*n, g, slot + q0*nslot, (unsigned)chunks )
+   for (long q0 = 0; q0 < nbox; q0 += BOX_GRID)
+   {
+      const unsigned nb = boxes_from( q0, nbox );
+      if ( n <= GB_SMALL ) GA_GB( true ); else GA_GB( false );
+   }
 #  undef GA_GB
    return ( hipGetLastError() == hipSuccess ) ? 0 : -2;
 }
