@@ -34,16 +34,18 @@ template <typename T> constexpr int interp_lanes( int scheme ) { return ( scheme
 template <typename T> __device__ __forceinline__ T sgn( T a ) { return ( a < (T)0 ) ? (T)-1 : (T)+1; }
 
 template <typename T>
-__device__ __forceinline__ T cquad_slope( T L, T C, T R, bool mono, T coeff, bool opp0 )
+__device__ __forceinline__ T cquad_slope( T L, T C, T R, bool mono, T coeff, bool opp0, bool turn )
 {
    #pragma clang fp contract(off)
    T s = (T)0.125*( R - L );
    if ( mono )
    {
       const T l = (T)0.25*( C - L ), r = (T)0.25*( R - C );
-      // of one sign where it matters, so that R - L has it too: the smallest magnitude, the smaller side scaled
+      // of one sign where it matters, so that R - L has it too: the smallest magnitude, the smaller side scaled.  A negative
+      // coefficient (turn) turns the slope around
       const T m = vmin( vmin( vmin( vabs( l ), vabs( r ) )*coeff, vmax( vabs( l ), vabs( r ) ) ), vabs( s ) );
       s = ( l*r > (T)0 ) ? __builtin_copysign( m, l ) : (T)0;
+      if ( turn ) s = -s;
    }
    if ( opp0 && L*R < (T)0 ) s = (T)0;
    return s;
@@ -53,7 +55,7 @@ __device__ __forceinline__ T cquad_slope( T L, T C, T R, bool mono, T coeff, boo
 // (lo, hi) of the centre cell (x passes of Int_MinMod3D.cpp:93-103, Int_vanLeer.cpp:93-105, Int_CQuadratic.cpp,
 // Int_Quadratic.cpp:104-160, Int_CQuartic.cpp:100-140, Int_Quartic.cpp:100-165; their y and z passes repeat them)
 template <typename T, int SCHEME>
-__device__ __forceinline__ void pass1d( const T u[5], bool mono, T coeff, bool opp0, T &lo, T &hi )
+__device__ __forceinline__ void pass1d( const T u[5], bool mono, T coeff, bool opp0, bool turn, T &lo, T &hi )
 {
    #pragma clang fp contract(off)
    const T L2 = u[0], L1 = u[1], C = u[2], R1 = u[3], R2 = u[4];
@@ -68,7 +70,7 @@ __device__ __forceinline__ void pass1d( const T u[5], bool mono, T coeff, bool o
    }
    else if ( SCHEME == 4 )                         // conservative quadratic
    {
-      s = cquad_slope( L1, C, R1, mono, coeff, opp0 );
+      s = cquad_slope( L1, C, R1, mono, coeff, opp0, turn );
       lo = C - s;  hi = C + s;
    }
    else if ( SCHEME == 6 )                         // conservative quartic
@@ -136,7 +138,7 @@ __device__ __forceinline__ void pass1d( const T u[5], bool mono, T coeff, bool o
 // the 2x2x2 fine values of coarse cell i of one field: f[(k*2 + j)*2 + i]
 template <typename T, int SCHEME>
 __device__ __forceinline__ void interp_cell( const T *__restrict__ c, int i, int dy, int dz, bool mono, T coeff,
-                                             bool opp0, T f[8] )
+                                             bool opp0, bool turn, T f[8] )
 {
    #pragma clang fp contract(off)
    if ( SCHEME != 2 )
@@ -151,7 +153,7 @@ __device__ __forceinline__ void interp_cell( const T *__restrict__ c, int i, int
             const int q = i + ( a - G )*dz + ( b - G )*dy;
 #           pragma unroll
             for (int k=0; k<5; k++) u[k] = ( k - 2 >= -G && k - 2 <= G ) ? c[q + k - 2] : (T)0;
-            pass1d<T, SCHEME>( u, mono, coeff, opp0, X[a][b][0], X[a][b][1] );
+            pass1d<T, SCHEME>( u, mono, coeff, opp0, turn, X[a][b][0], X[a][b][1] );
          }
 #     pragma unroll
       for (int a=0; a<W; a++)
@@ -160,7 +162,7 @@ __device__ __forceinline__ void interp_cell( const T *__restrict__ c, int i, int
          {
 #           pragma unroll
             for (int k=0; k<5; k++) u[k] = ( k - 2 >= -G && k - 2 <= G ) ? X[a][k - 2 + G][x] : (T)0;
-            pass1d<T, SCHEME>( u, mono, coeff, opp0, Y[a][0][x], Y[a][1][x] );
+            pass1d<T, SCHEME>( u, mono, coeff, opp0, turn, Y[a][0][x], Y[a][1][x] );
          }
 #     pragma unroll
       for (int y=0; y<2; y++)
@@ -169,7 +171,7 @@ __device__ __forceinline__ void interp_cell( const T *__restrict__ c, int i, int
          {
 #           pragma unroll
             for (int k=0; k<5; k++) u[k] = ( k - 2 >= -G && k - 2 <= G ) ? Y[k - 2 + G][y][x] : (T)0;
-            pass1d<T, SCHEME>( u, mono, coeff, opp0, f[( 0*2 + y )*2 + x], f[( 1*2 + y )*2 + x] );
+            pass1d<T, SCHEME>( u, mono, coeff, opp0, turn, f[( 0*2 + y )*2 + x], f[( 1*2 + y )*2 + x] );
          }
    }
    else
@@ -273,7 +275,7 @@ __device__ __forceinline__ bool store_fine( T f[NV][8], bool iterate, bool prim,
 
 // One lane per asked-for coarse cell, from a list: a box next to a patch of its own level needs two layers of its 12^3 cells,
 // and a lane's chain of 95 one-dimensional passes (19 a field) is the time, so the lanes must all have cells.  PLAIN: all
-// fields monotonic and no clipping across 0 (the default); with these as run-time bits every pass had branches of its own,
+// fields monotonic, their coefficient not negative, and no clipping across 0 (the default); with these as run-time bits every pass had branches of its own,
 // which kept the passes from overlapping.  512 boxes of the AMR step (216 ask for nothing, most others for 288 cells), CQUAD:
 // FP32 118 -> 34 us, FP64 155 -> 48; every cell asked for 130 -> 65 and 217 -> 150; one box 95 -> 26.  The first form marched
 // a lane per column through the box: 9 passes a cell and field in place of 19, but 24 lanes of 144 at work beside an x face,
@@ -355,7 +357,8 @@ interpolate_kernel( T *__restrict__ g_c, T *__restrict__ g_f, int nbox, InterpPr
          const int ic = ( p.c0[2] + z )*dz + ( p.c0[1] + y )*dy + p.c0[0] + x;
          T f[NV][8];
 #        pragma unroll
-         for (int v=0; v<NV; v++) interp_cell<T, SCHEME>( C + (size_t)v*C3, ic, dy, dz, PLAIN || ( ( p.mono >> v ) & 1 ), coeff, !PLAIN && p.opp0, f[v] );
+         for (int v=0; v<NV; v++) interp_cell<T, SCHEME>( C + (size_t)v*C3, ic, dy, dz, PLAIN || ( ( p.mono >> v ) & 1 ), coeff,
+                                                             !PLAIN && p.opp0, !PLAIN && p.mono_coeff < 0.0, f[v] );
          const int fo = ( p.f0[2] + 2*z )*fdz + ( p.f0[1] + 2*y )*fdy + p.f0[0] + 2*x;
          if ( store_fine( f, iterate, prim, p, F, F3, fo, fdy, fdz ) ) s_done[c] = 1; else s_fail = 1;
       }
@@ -485,7 +488,7 @@ static unsigned boxes_from( long q0, long nbox ) { return (unsigned)( nbox - q0 
 template <typename T>
 static int interpolate_boxes( T *cdata, T *fdata, int nbox, const InterpPrm &p, int *nfail, hipStream_t stream )
 {
-   const bool plain = ( p.mono & 0x1F ) == 0x1F && !p.opp0;
+   const bool plain = ( p.mono & 0x1F ) == 0x1F && !p.opp0 && !( p.mono_coeff < 0.0 );
 #  define GA_INT( S ) { if ( plain ) GA_LAUNCH( S, true ); else GA_LAUNCH( S, false ); }
 #  define GA_LAUNCH( S, PLAIN_ ) hipLaunchKernelGGL( ( interpolate_kernel<T, S, PLAIN_> ), dim3( nbox ), dim3( interp_lanes<T>( S ) ), 0, stream, \
                                                     cdata, fdata, nbox, p, nfail )
