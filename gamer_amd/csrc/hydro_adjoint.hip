@@ -252,48 +252,58 @@ template <> struct Store< Dual<1> >
 
 constexpr size_t NIN = (size_t)NV*N3, NOUT = (size_t)NV*PS*PS*PS;
 
-// F1 + F2: a workgroup takes F12_JR rows (y) of F12_KS planes (z), plane by plane.  The half-step fluxes of the plane's x
+// F1 + F2: a workgroup takes JR rows (y) of KS planes (z), plane by plane.  The half-step fluxes of the plane's x
 // and y faces and of the z faces above it (Hydro_RiemannPredict_Flux) go to LDS, where the z faces below it are from the
 // plane before (solved first for the first plane), then the cells take the half-step update (x and y flux differences,
 // then z, as the production kernel), the floors and the primitive conversion (Hydro_RiemannPredict).  The fluxes never
 // reach memory; the price is that faces between workgroups are solved by both.  h_off >= 0 (FP64 only): the half-step state h
 // is stored too, for R2.  With one whole plane per workgroup every z face was solved twice: 512 patch groups 264 us, this
 // takes 238; half as many rows 240, five planes 242.  What the cell contributes to its six faces (pressure, 1/rho, sound
-// speed) kept in LDS instead of recomputed took 265: the solves wait, the vector units do not bound it.
-constexpr int F12_JR = 10, F12_KS = 4, F12_NT = 256;
-constexpr int F12_RB = 20/F12_JR, F12_KB = 20/F12_KS, F12_BPP = F12_RB*F12_KB;
-constexpr int F12_NXF = 21*F12_JR, F12_NYF = 20*( F12_JR + 1 ), F12_NZF = 20*F12_JR;
-static_assert( 20 % F12_JR == 0 && 20 % F12_KS == 0, "the blocks must tile the 20 x 20 half-step rows and planes" );
+// speed) kept in LDS instead of recomputed took 265: the solves wait, the vector units do not bound it.  Calls of few patch
+// groups take blocks of one plane (few_blocks()).
+template <int JR_, int KS_>
+struct F12
+{
+   static constexpr int JR = JR_, KS = KS_, RB = 20/JR, KB = 20/KS, BPP = RB*KB;
+   static constexpr int NXF = 21*JR, NYF = 20*( JR + 1 ), NZF = 20*JR;
+   static_assert( 20 % JR == 0 && 20 % KS == 0, "the blocks must tile the 20 x 20 half-step rows and planes" );
+};
+constexpr int F12_NT = 256;
+typedef F12<10, 4> F12Large;
+typedef F12<5, 1>  F12Small;
 
-template <int RS, typename T>
+template <int RS, typename T, typename B>
 __global__ void __launch_bounds__( F12_NT )
 f12_kernel( const double *__restrict__ g_in, const double *__restrict__ g_tin, double *__restrict__ g_ws, int h_off,
             Prm<double> P0, double minmod_coeff )
 {
-   __shared__ double s_raw[NV*( F12_NXF + F12_NYF + 2*F12_NZF )*( sizeof( T )/sizeof( double ) )];
-   T *sX = reinterpret_cast<T*>( s_raw ), *sY = sX + NV*F12_NXF, *sZ = sY + NV*F12_NYF;      // [v][face]; sZ [k % 2][v][face]
-   const int tid = threadIdx.x, lb = (int)xcd_block(), rb = lb % F12_RB, kb = ( lb / F12_RB ) % F12_KB, pg = lb / F12_BPP;
-   const int j0 = rb*F12_JR, ka = 1 + kb*F12_KS;                 // rows j0 + 1 .. j0 + F12_JR, planes ka .. ka + F12_KS - 1
+   __shared__ double s_raw[NV*( B::NXF + B::NYF + 2*B::NZF )*( sizeof( T )/sizeof( double ) )];
+   T *sX = reinterpret_cast<T*>( s_raw ), *sY = sX + NV*B::NXF, *sZ = sY + NV*B::NYF;      // [v][face]; sZ [k % 2][v][face]
+   const int tid = threadIdx.x, lb = (int)xcd_block(), rb = lb % B::RB, kb = ( lb / B::RB ) % B::KB, pg = lb / B::BPP;
+   const int j0 = rb*B::JR, ka = 1 + kb*B::KS;                 // rows j0 + 1 .. j0 + JR, planes ka .. ka + KS - 1
    const Prm<T> P = phase_prm<T>( P0, minmod_coeff );
    const double *in = g_in + pg*NIN, *tin = g_tin ? g_tin + pg*NIN : nullptr;
    Fwd<T> F( reinterpret_cast<T*>( g_ws + (size_t)pg*WS_ADJ*N3 ) );
+   constexpr bool ONE = ( B::KS == 1 );                          // one plane: the z faces below it come with its own
 #  pragma unroll 1
-   for (int k = ka - 1; k < ka + F12_KS; k++)
+   for (int k = ONE ? ka : ka - 1; k < ka + B::KS; k++)
    {
-      // faces, stored at their low cell: x (normal i = 0..20), y (normal j0 .. j0 + F12_JR), then the z faces with low cell
-      // in plane k; lanes run along x
-      const int f0 = ( k < ka ) ? F12_NXF + F12_NYF : 0;
-      for (int f = f0 + tid; f < F12_NXF + F12_NYF + F12_NZF; f += F12_NT)
+      // faces, stored at their low cell: x (normal i = 0..20), y (normal j0 .. j0 + JR), then the z faces with low cell
+      // in plane k (ONE: and those in plane k - 1); lanes run along x
+      const int f0 = ( !ONE && k < ka ) ? B::NXF + B::NYF : 0;
+      for (int f = f0 + tid; f < B::NXF + B::NYF + ( ONE ? 2 : 1 )*B::NZF; f += F12_NT)
       {
-         int d, i, j, r = f, n = F12_NXF;
+         int d, i, j, kf = k, r = f, n = B::NXF;
          T *dst = sX;
-         if ( f < F12_NXF )                 { d = 0;  i = r % 21;  j = j0 + 1 + r / 21; }
-         else if ( f < F12_NXF + F12_NYF )  { d = 1;  r = f - F12_NXF;  i = 1 + r % 20;  j = j0 + r / 20;  dst = sY;  n = F12_NYF; }
+         if ( f < B::NXF )                 { d = 0;  i = r % 21;  j = j0 + 1 + r / 21; }
+         else if ( f < B::NXF + B::NYF )  { d = 1;  r = f - B::NXF;  i = 1 + r % 20;  j = j0 + r / 20;  dst = sY;  n = B::NYF; }
          else
          {
-            d = 2;  r = f - F12_NXF - F12_NYF;  i = 1 + r % 20;  j = j0 + 1 + r / 20;  dst = sZ + ( k & 1 )*NV*F12_NZF;  n = F12_NZF;
+            d = 2;  r = f - B::NXF - B::NYF;
+            if ( ONE && r >= B::NZF ) { r -= B::NZF;  kf = k - 1; }
+            i = 1 + r % 20;  j = j0 + 1 + r / 20;  dst = sZ + ( kf & 1 )*NV*B::NZF;  n = B::NZF;
          }
-         const int c = i + NX*j + N2*k;
+         const int c = i + NX*j + N2*kf;
          T uL[NV], uR[NV], fl[NV];
          Load<T>::cell( in, tin, c, uL );
          Load<T>::cell( in, tin, c + ( d == 0 ? 1 : d == 1 ? NX : N2 ), uR );
@@ -303,19 +313,19 @@ f12_kernel( const double *__restrict__ g_in, const double *__restrict__ g_tin, d
       }
       __syncthreads();
       if ( k >= ka )
-      for (int e = tid; e < F12_NZF; e += F12_NT)
+      for (int e = tid; e < B::NZF; e += F12_NT)
       {
          const int i = 1 + e % 20, jr = e / 20, c = i + NX*( j0 + 1 + jr ) + N2*k;
          const int xh = i + 21*jr, yh = ( i - 1 ) + 20*( jr + 1 );
-         const T *zu = sZ + ( k & 1 )*NV*F12_NZF + e, *zl = sZ + ( ( k - 1 ) & 1 )*NV*F12_NZF + e;
+         const T *zu = sZ + ( k & 1 )*NV*B::NZF + e, *zl = sZ + ( ( k - 1 ) & 1 )*NV*B::NZF + e;
          T u[NV], h[NV], w[NV];
          Load<T>::cell( in, tin, c, u );
 #        pragma unroll
          for (int v=0; v<NV; v++)
          {
-            const T *fx = sX + v*F12_NXF + xh, *fy = sY + v*F12_NYF + yh;
+            const T *fx = sX + v*B::NXF + xh, *fy = sY + v*B::NYF + yh;
             const T dxy = ( fx[0] - fx[-1] ) + ( fy[0] - fy[-20] );
-            h[v] = u[v] - P.dt_dh2*( dxy + ( zu[v*F12_NZF] - zl[v*F12_NZF] ) );
+            h[v] = u[v] - P.dt_dh2*( dxy + ( zu[v*B::NZF] - zl[v*B::NZF] ) );
          }
          con2pri_floor( h, P, w );
 #        pragma unroll
@@ -591,48 +601,63 @@ r32_kernel( double *__restrict__ g_ws, Prm<double> P0, double minmod_coeff )
    }
 }
 
-// R1 + R0: a workgroup takes R10_JR rows (y) of about 22/R10_KB planes (z), plane by plane.  R1: lambda_Fh = dt/(2dh)
+// R1 + R0: a workgroup takes JR rows (y) of about 22/KB planes (z), plane by plane.  R1: lambda_Fh = dt/(2dh)
 // (lambda_U(c+e_d) - lambda_U(c)) of every half-step face, then J_RS^T per side; the side contributions of the plane's x
 // and y faces and of the z face above it (normal k) stay in LDS.  R0: lambda_in of the plane's cells = lambda_out (output
 // cells) + lambda_U_half (half-step cells) + the face contributions in the order x low, x high, y low, y high, z low, z high,
 // the last one from the plane before (solved first for the first plane).  Faces between workgroups are solved by both.
 // 3 waves per SIMD (<= 170 VGPRs); Roe's reverse solve needs about 230, 2 waves.  512 patch groups 514 us; one whole plane of
 // 768 lanes, with the z faces' high sides added by a kernel of their own through memory, 525 + 95.  192 lanes against 256
-// (610) and 128 (608); Roe 128 lanes against 256: 1724 and 1917 us for the whole adjoint.
-constexpr int R10_JR = 5, R10_KB = 4;
-constexpr int r10_nt( int rs ) { return rs == 2 ? 128 : 192; }
-constexpr int R10_RB = 20/R10_JR, R10_BPP = R10_RB*R10_KB;
-constexpr int R10_NXF = 21*R10_JR, R10_NYF = 20*( R10_JR + 1 ), R10_NZF = 20*R10_JR;
-static_assert( 20 % R10_JR == 0, "the blocks must tile the 20 half-step rows" );
+// (610) and 128 (608); Roe 128 lanes against 256: 1724 and 1917 us for the whole adjoint.  Calls of few patch groups take
+// blocks of one plane (few_blocks()).
+template <int JR_, int KB_>
+struct R10
+{
+   static constexpr int JR = JR_, KB = KB_, RB = 20/JR, BPP = RB*KB;
+   static constexpr int NXF = 21*JR, NYF = 20*( JR + 1 ), NZF = 20*JR;
+   static constexpr bool ONE = ( KB == NX );            // one plane: the z faces below it come with its own
+   static constexpr int nt( int rs ) { return ( rs == 2 && !ONE ) ? 128 : 192; }
+   static_assert( 20 % JR == 0, "the blocks must tile the 20 half-step rows" );
+};
+typedef R10<5, 4>  R10Large;
+typedef R10<5, NX> R10Small;
 
-template <int RS>
-__global__ void __launch_bounds__( r10_nt( RS ) )
+template <int RS, typename B>
+__global__ void __launch_bounds__( B::nt( RS ) )
 r10_kernel( const double *__restrict__ g_in, const double *__restrict__ g_lout, double *__restrict__ g_lin,
             double *__restrict__ g_ws, Prm<double> P0, double minmod_coeff )
 {
-   constexpr int R10_NT = r10_nt( RS );
+   constexpr int R10_NT = B::nt( RS );
+   constexpr bool ONE = B::ONE;
    // [low/high side][v][face]; sZh [k % 2][v][face]: the z faces' high sides, read one plane later
-   __shared__ double sX[2][NV][R10_NXF], sY[2][NV][R10_NYF], sZ[NV][R10_NZF], sZh[2][NV][R10_NZF];
-   const int tid = threadIdx.x, lb = (int)xcd_block(), rb = lb % R10_RB, kb = ( lb / R10_RB ) % R10_KB, pg = lb / R10_BPP;
-   const int j0 = rb*R10_JR, ka = 22*kb/R10_KB, ke = 22*( kb + 1 )/R10_KB;      // half-step rows j0 + 1 .. j0 + R10_JR, planes [ka, ke)
-   const int ja = ( rb == 0 ) ? 0 : j0 + 1, je = ( rb == R10_RB - 1 ) ? NX : j0 + R10_JR + 1;      // rows of lambda_in [ja, je)
+   __shared__ double sX[2][NV][B::NXF], sY[2][NV][B::NYF], sZ[NV][B::NZF], sZh[2][NV][B::NZF];
+   const int tid = threadIdx.x, lb = (int)xcd_block(), rb = lb % B::RB, kb = ( lb / B::RB ) % B::KB, pg = lb / B::BPP;
+   const int j0 = rb*B::JR, ka = 22*kb/B::KB, ke = 22*( kb + 1 )/B::KB;      // half-step rows j0 + 1 .. j0 + JR, planes [ka, ke)
+   const int ja = ( rb == 0 ) ? 0 : j0 + 1, je = ( rb == B::RB - 1 ) ? NX : j0 + B::JR + 1;      // rows of lambda_in [ja, je)
    const Prm<double> P = phase_prm<double>( P0, minmod_coeff );
    const double *in = g_in + pg*NIN, *lout = g_lout + pg*NOUT;
    double *lin = g_lin + pg*NIN;
    Adj A( g_ws + (size_t)pg*WS_ADJ*N3 );
 #  pragma unroll 1
-   for (int k = ( ka > 0 ) ? ka - 1 : 0; k < ke; k++)
+   for (int k = ( !ONE && ka > 0 ) ? ka - 1 : ka; k < ke; k++)
    {
-      // faces with low cell in plane k: x (normal i = 0..20), y (normal j0 .. j0 + R10_JR), z; plane 0 and the plane
-      // before the first have only their z faces, plane 21 none
-      const int f0 = ( k == 0 || k < ka ) ? R10_NXF + R10_NYF : 0, f1 = ( k <= 20 ) ? R10_NXF + R10_NYF + R10_NZF : 0;
+      // faces with low cell in plane k: x (normal i = 0..20), y (normal j0 .. j0 + JR), z; plane 0 and the plane
+      // before the first have only their z faces, plane 21 none (ONE: and those with low cell in plane k - 1)
+      const int nxy = B::NXF + B::NYF;
+      const int f0 = ( k == 0 || k < ka ) ? nxy : ( ONE && k == NX - 1 ) ? nxy + B::NZF : 0;
+      const int f1 = ( ONE && k > 0 ) ? nxy + 2*B::NZF : ( k <= 20 ) ? nxy + B::NZF : 0;
       for (int f = f0 + tid; f < f1; f += R10_NT)
       {
-         int d, i, j, r = f, n;
-         if ( f < R10_NXF )                 { d = 0;  i = r % 21;  j = j0 + 1 + r / 21;  n = i; }
-         else if ( f < R10_NXF + R10_NYF )  { d = 1;  r = f - R10_NXF;  i = 1 + r % 20;  j = j0 + r / 20;  n = j; }
-         else                               { d = 2;  r = f - R10_NXF - R10_NYF;  i = 1 + r % 20;  j = j0 + 1 + r / 20;  n = k; }
-         const int c = i + NX*j + N2*k, s = ( d == 0 ? 1 : d == 1 ? NX : N2 );
+         int d, i, j, kf = k, r = f, n;
+         if ( f < B::NXF )                 { d = 0;  i = r % 21;  j = j0 + 1 + r / 21;  n = i; }
+         else if ( f < B::NXF + B::NYF )  { d = 1;  r = f - B::NXF;  i = 1 + r % 20;  j = j0 + r / 20;  n = j; }
+         else
+         {
+            d = 2;  r = f - nxy;
+            if ( ONE && r >= B::NZF ) { r -= B::NZF;  kf = k - 1; }
+            i = 1 + r % 20;  j = j0 + 1 + r / 20;  n = kf;
+         }
+         const int c = i + NX*j + N2*kf, s = ( d == 0 ? 1 : d == 1 ? NX : N2 );
          const bool lo = in_rng( n, 1, 20 ), hi = in_rng( n + 1, 1, 20 );   // tangential range is 1..20 already
          double lf[NV];
 #        pragma unroll
@@ -643,10 +668,14 @@ r10_kernel( const double *__restrict__ g_in, const double *__restrict__ g_lout, 
          double gl[NV] = { 0.0, 0.0, 0.0, 0.0, 0.0 }, gr[NV] = { 0.0, 0.0, 0.0, 0.0, 0.0 };
          half_flux_rev<RS>( d, uL, uR, P, lf, gl, gr );
          double *pl = ( d == 0 ) ? &sX[0][0][r] : ( d == 1 ) ? &sY[0][0][r] : &sZ[0][r];
-         double *ph = ( d == 0 ) ? &sX[1][0][r] : ( d == 1 ) ? &sY[1][0][r] : &sZh[k & 1][0][r];
-         const int m = ( d == 0 ) ? R10_NXF : ( d == 1 ) ? R10_NYF : R10_NZF;
+         double *ph = ( d == 0 ) ? &sX[1][0][r] : ( d == 1 ) ? &sY[1][0][r] : &sZh[kf & 1][0][r];
+         const int m = ( d == 0 ) ? B::NXF : ( d == 1 ) ? B::NYF : B::NZF;
 #        pragma unroll
-         for (int v=0; v<NV; v++) { pl[ v*m ] = gl[v];  ph[ v*m ] = gr[v]; }
+         for (int v=0; v<NV; v++)
+         {
+            if ( !ONE || kf == k ) pl[ v*m ] = gl[v];
+            ph[ v*m ] = gr[v];
+         }
       }
       __syncthreads();
       if ( k >= ka )
@@ -739,7 +768,32 @@ namespace {
 void phase_grid( int npg, int count, dim3 &grid ) { grid = dim3( (unsigned)( (long)npg*bpp( count ) ) ); }
 // whether every phase's grid of npg patch groups fits one launch (R4 has the most lanes)
 bool grids_fit( int npg ) { return (long)npg*bpp( N_R4 )*NT < ( 1L << 32 ); }
-static_assert( F12_BPP*F12_NT <= bpp( N_R4 )*NT && R10_BPP*r10_nt( 4 ) <= bpp( N_R4 )*NT && R32_BPP*R32_NT <= bpp( N_R4 )*NT, "R4 has the most lanes" );
+static_assert( F12Large::BPP*F12_NT <= bpp( N_R4 )*NT && R10Large::BPP*R10Large::nt( 4 ) <= bpp( N_R4 )*NT && R32_BPP*R32_NT <= bpp( N_R4 )*NT,
+               "R4 has the most lanes" );
+
+// Whether a phase of `blocks` marching workgroups leaves the chip idle, most of them per compute unit
+bool few_blocks( long blocks, double most ) { return (double)blocks <= most*device_cus(); }
+
+// The marching blocks for calls that fill the chip with them, blocks of one plane for those that do not: a march of four to
+// six planes takes its time however few patch groups there are.  us of the whole call, marching -> one plane, adjoint HLLC 1
+// patch group 84 -> 45, 16 97 -> 70, 64 183 -> 171, 128 372 -> 360, 256 702 -> 711; Roe 8 121 -> 62, 48 207 -> 192, 64 249
+// -> 257 (its blocks of one plane alone 263), 128 480 -> 530; tangent HLLC 4 38 -> 21, 64 126 -> 120, 96 175 -> 182; Roe 4 60 -> 27, 64 218 -> 209,
+// 96 310 -> 317.  So the lines: 2.5 marching blocks of F1 + F2 per compute unit, of R1 + R0 eight, with Roe three.
+template <int RS, typename T>
+void launch_f12( const double *in, const double *tin, double *ws, int h_off, int npg, double minmod_coeff, const Prm<double> &P, hipStream_t stream )
+{
+#  define GA_F12( B ) hipLaunchKernelGGL( ( f12_kernel<RS, T, B> ), dim3( (unsigned)( B::BPP*npg ) ), dim3( F12_NT ), 0, stream, in, tin, ws, h_off, P, minmod_coeff )
+   if ( few_blocks( (long)F12Large::BPP*npg, 2.5 ) ) GA_F12( F12Small ); else GA_F12( F12Large );
+#  undef GA_F12
+}
+
+template <int RS>
+void launch_r10( const double *in, const double *lam_out, double *lam_in, double *ws, int npg, double minmod_coeff, const Prm<double> &P, hipStream_t stream )
+{
+#  define GA_R10( B ) hipLaunchKernelGGL( ( r10_kernel<RS, B> ), dim3( (unsigned)( B::BPP*npg ) ), dim3( B::nt( RS ) ), 0, stream, in, lam_out, lam_in, ws, P, minmod_coeff )
+   if ( few_blocks( (long)R10Large::BPP*npg, RS == 2 ? 3.0 : 8.0 ) ) GA_R10( R10Small ); else GA_R10( R10Large );
+#  undef GA_R10
+}
 
 template <int RS, int LIM>
 int adjoint_phases( const double *in, const double *lam_out, double *lam_in, double *ws, int npg, double minmod_coeff,
@@ -749,12 +803,12 @@ int adjoint_phases( const double *in, const double *lam_out, double *lam_in, dou
    dim3 g;
    // forward: F1 + F2 (the PLM faces are recomputed where they are needed instead of stored)
    if ( !grids_fit( npg ) ) return -3;
-   hipLaunchKernelGGL( ( f12_kernel<RS, double> ), dim3( (unsigned)( F12_BPP*npg ) ), dim3( F12_NT ), 0, stream, in, nullptr, ws, WS_H, P, minmod_coeff );
+   launch_f12<RS, double>( in, nullptr, ws, WS_H, npg, minmod_coeff, P, stream );
    // reverse: R4, R3 + R2, R1 + R0
    phase_grid( npg, N_R4, g );
    hipLaunchKernelGGL( ( r4_kernel<RS, LIM> ), g, block, 0, stream, lam_out, ws, P, minmod_coeff );
    hipLaunchKernelGGL( ( r32_kernel<LIM> ), dim3( (unsigned)( npg*R32_BPP ) ), dim3( R32_NT ), 0, stream, ws, P, minmod_coeff );
-   hipLaunchKernelGGL( ( r10_kernel<RS> ), dim3( (unsigned)( R10_BPP*npg ) ), dim3( r10_nt( RS ) ), 0, stream, in, lam_out, lam_in, ws, P, minmod_coeff );
+   launch_r10<RS>( in, lam_out, lam_in, ws, npg, minmod_coeff, P, stream );
    return ( hipGetLastError() == hipSuccess ) ? 0 : -2;
 }
 
@@ -765,7 +819,7 @@ int tangent_phases( const double *in, const double *tin, double *out, double *to
    const dim3 block( NT );
    dim3 g;
    if ( !grids_fit( npg ) ) return -3;
-   hipLaunchKernelGGL( ( f12_kernel<RS, T> ), dim3( (unsigned)( F12_BPP*npg ) ), dim3( F12_NT ), 0, stream, in, tin, ws, -1, P, minmod_coeff );
+   launch_f12<RS, T>( in, tin, ws, -1, npg, minmod_coeff, P, stream );
    phase_grid( npg, 3*NFF, g );
    hipLaunchKernelGGL( ( f4_face_kernel<RS, LIM, T> ), g, block, 0, stream, ws, P, minmod_coeff );
    phase_grid( npg, N_F4, g );
