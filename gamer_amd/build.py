@@ -10,7 +10,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libgamer_amd_hydro.so")
 SOURCES = ["hydro_api.hip", "hydro_mhm_rp.hip", "hydro_mhm.hip:32", "hydro_mhm.hip:64", "hydro_grid.hip",
-           "hydro_adjoint.hip", "hydro_sync.hip", "hydro_interp.hip"]     # "file:NN": the file for one precision only
+           "hydro_adjoint.hip", "hydro_sync.hip", "hydro_interp.hip:32", "hydro_interp.hip:64"]     # "file:NN": the file for one precision only
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
@@ -23,7 +23,8 @@ FLAGS = [
 # kernels run fastest with the default scheduler in FP32 (532 against 538 us on 4096 patch groups) and the same with
 # both in FP64; the adjoint, interpolation and sync sources crash the compiler under these strategies.
 EXTRA = {"hydro_mhm.hip:32": ["-DMHM_PRECISION=32", "-mllvm", "-amdgpu-sched-strategy=max-ilp"],
-         "hydro_mhm.hip:64": ["-DMHM_PRECISION=64", "-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]}
+         "hydro_mhm.hip:64": ["-DMHM_PRECISION=64", "-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
+         "hydro_interp.hip:32": ["-DINTERP_PRECISION=32"], "hydro_interp.hip:64": ["-DINTERP_PRECISION=64"]}
 
 
 def build(verbose: bool = False) -> str:

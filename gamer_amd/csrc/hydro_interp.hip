@@ -195,6 +195,28 @@ __device__ __forceinline__ void interp_cell( const T *__restrict__ c, int i, int
    }
 }
 
+// x pass of the rows y-1, y, y+1 of coarse plane z' around index q, then the y pass: Y[y-lo/hi][x-lo/hi] of that
+// plane, exactly as interp_cell computes its Y[a] (3-point schemes)
+template <typename T, int SCHEME>
+__device__ __forceinline__ void xy_pass( const T *__restrict__ c, int q, int dy, bool mono, T coeff, bool opp0, T Y[2][2] )
+{
+   #pragma clang fp contract(off)
+   T X[3][2], u[5];
+#  pragma unroll
+   for (int b=0; b<3; b++)
+   {
+      const int qq = q + ( b - 1 )*dy;
+      u[0] = (T)0;  u[1] = c[qq - 1];  u[2] = c[qq];  u[3] = c[qq + 1];  u[4] = (T)0;
+      pass1d<T, SCHEME>( u, mono, coeff, opp0, false, X[b][0], X[b][1] );
+   }
+#  pragma unroll
+   for (int x=0; x<2; x++)
+   {
+      u[0] = (T)0;  u[1] = X[0][x];  u[2] = X[1][x];  u[3] = X[2][x];  u[4] = (T)0;
+      pass1d<T, SCHEME>( u, mono, coeff, opp0, false, Y[0][x], Y[1][x] );
+   }
+}
+
 template <typename T> struct Huge;
 template <> struct Huge<double> { static constexpr double v = 1.7976931348623157e308; static constexpr double eps = 2.2204460492503131e-16; };
 template <> struct Huge<float>  { static constexpr float  v = 3.40282346638528859812e+38f; static constexpr float eps = 1.1920928955078125e-07f; };
@@ -280,16 +302,19 @@ __device__ __forceinline__ bool store_fine( T f[NV][8], bool iterate, bool prim,
 // FP32 118 -> 34 us, FP64 155 -> 48; every cell asked for 130 -> 65 and 217 -> 150; one box 95 -> 26.  The first form marched
 // a lane per column through the box: 9 passes a cell and field in place of 19, but 24 lanes of 144 at work beside an x face,
 // twelve planes in sequence; the list with the branches took 90.
-template <typename T, int SCHEME, bool PLAIN>
-__global__ void __launch_bounds__( interp_lanes<T>( SCHEME ) )
+// MARCH: no list, and the first pass (not of MINMOD1D) with a lane per column, marching along z with the y-pass results of planes z-1, z, z+1 in registers:
+// 9 passes a cell and field in place of 19, with interp_cell's operations in its order, so the same bits.  interp_launch()
+// says where that is the faster one, and how many lanes (NT) a block has and waves per SIMD (EU) its registers leave room
+// for (0: as the compiler finds).
+template <typename T, int SCHEME, bool PLAIN, bool MARCH, int NT, int EU>
+__global__ void __launch_bounds__( NT ) __attribute__(( amdgpu_waves_per_eu( EU ) ))
 interpolate_kernel( T *__restrict__ g_c, T *__restrict__ g_f, int nbox, InterpPrm p, int *__restrict__ nfail )
 {
    #pragma clang fp contract(off)
-   constexpr int NT = interp_lanes<T>( SCHEME );
    __shared__ int s_fail;
    __shared__ int s_n;
    __shared__ unsigned char s_done[INTERP_MAX_CELLS];
-   __shared__ unsigned short s_todo[INTERP_MAX_CELLS];
+   __shared__ unsigned short s_todo[MARCH ? 1 : INTERP_MAX_CELLS];
    const int q = blockIdx.x, tid = threadIdx.x;
    if ( q >= nbox ) return;
    const int dy = p.cs[0], dz = p.cs[0]*p.cs[1], C3 = dz*p.cs[2];
@@ -301,22 +326,31 @@ interpolate_kernel( T *__restrict__ g_c, T *__restrict__ g_f, int nbox, InterpPr
    const int mono_max = p.reduce ? p.mono_max_iter : 0, max_iter = p.int_prim ? mono_max + 1 : mono_max;
 
    // the cells that are asked for, listed (in any order: they are independent)
-   if ( tid == 0 ) s_n = 0;
-   __syncthreads();
-   for (int c = tid; c < ncell; c += NT)
+   int ntodo = ncell;
+   if constexpr ( MARCH )
    {
-      const bool todo = !p.need || p.need[ (size_t)q*ncell + c ];
-      s_done[c] = !todo;
-      const unsigned long long m = __ballot( todo );
-      const int lane = tid & 63, first = __ffsll( (long long)__ballot( true ) ) - 1;
-      int at = 0;
-      if ( lane == first ) at = atomicAdd( &s_n, __popcll( m ) );
-      at = __shfl( at, first, 64 );
-      if ( todo ) s_todo[ at + __popcll( m & ( ( 1ULL << lane ) - 1 ) ) ] = (unsigned short)c;
+      for (int c = tid; c < ncell; c += NT) s_done[c] = p.need ? !p.need[ (size_t)q*ncell + c ] : 0;
+      __syncthreads();
    }
-   __syncthreads();
-   const int ntodo = s_n;
-   if ( ntodo == 0 ) return;
+   else
+   {
+      if ( tid == 0 ) s_n = 0;
+      __syncthreads();
+      for (int c = tid; c < ncell; c += NT)
+      {
+         const bool todo = !p.need || p.need[ (size_t)q*ncell + c ];
+         s_done[c] = !todo;
+         const unsigned long long m = __ballot( todo );
+         const int lane = tid & 63, first = __ffsll( (long long)__ballot( true ) ) - 1;
+         int at = 0;
+         if ( lane == first ) at = atomicAdd( &s_n, __popcll( m ) );
+         at = __shfl( at, first, 64 );
+         if ( todo ) s_todo[ at + __popcll( m & ( ( 1ULL << lane ) - 1 ) ) ] = (unsigned short)c;
+      }
+      __syncthreads();
+      ntodo = s_n;
+      if ( ntodo == 0 ) return;
+   }
    T coeff = (T)p.mono_coeff;
    bool prim = false;
    for (int it = 0; ; it++)
@@ -349,9 +383,52 @@ interpolate_kernel( T *__restrict__ g_c, T *__restrict__ g_f, int nbox, InterpPr
       if ( tid == 0 ) s_fail = 0;
       __syncthreads();
 
+      if ( MARCH && SCHEME != 2 && it == 0 )
+      {
+         const int ncol = p.cr[0]*p.cr[1];
+         for (int col = tid; col < ncol; col += NT)
+         {
+            const int x = col % p.cr[0], y = col / p.cr[0];
+            const int q0 = p.c0[2]*dz + ( p.c0[1] + y )*dy + p.c0[0] + x;      // coarse index of (x, y, z = 0)
+            T Yw[NV][3][2][2];
+#           pragma unroll
+            for (int v=0; v<NV; v++)
+            {
+               xy_pass<T, SCHEME>( C + (size_t)v*C3, q0 - dz, dy, ( p.mono >> v ) & 1, coeff, p.opp0, Yw[v][0] );
+               xy_pass<T, SCHEME>( C + (size_t)v*C3, q0,      dy, ( p.mono >> v ) & 1, coeff, p.opp0, Yw[v][1] );
+            }
+            for (int z = 0; z < p.cr[2]; z++)
+            {
+               T f[NV][8], u[5];
+#              pragma unroll
+               for (int v=0; v<NV; v++)
+               {
+                  xy_pass<T, SCHEME>( C + (size_t)v*C3, q0 + ( z + 1 )*dz, dy, ( p.mono >> v ) & 1, coeff, p.opp0, Yw[v][2] );
+#                 pragma unroll
+                  for (int yy=0; yy<2; yy++)
+#                    pragma unroll
+                     for (int xx=0; xx<2; xx++)
+                     {
+                        u[0] = (T)0;  u[1] = Yw[v][0][yy][xx];  u[2] = Yw[v][1][yy][xx];  u[3] = Yw[v][2][yy][xx];  u[4] = (T)0;
+                        pass1d<T, SCHEME>( u, ( p.mono >> v ) & 1, coeff, p.opp0, false, f[v][( 0*2 + yy )*2 + xx],
+                                           f[v][( 1*2 + yy )*2 + xx] );
+                     }
+               }
+               const int fo = ( p.f0[2] + 2*z )*fdz + ( p.f0[1] + 2*y )*fdy + p.f0[0] + 2*x;
+               if ( store_fine( f, iterate, prim, p, F, F3, fo, fdy, fdz ) ) s_done[ col + z*ncol ] = 1; else s_fail = 1;
+#              pragma unroll
+               for (int v=0; v<NV; v++)
+#                 pragma unroll
+                  for (int yy=0; yy<2; yy++)
+#                    pragma unroll
+                     for (int xx=0; xx<2; xx++) { Yw[v][0][yy][xx] = Yw[v][1][yy][xx];  Yw[v][1][yy][xx] = Yw[v][2][yy][xx]; }
+            }
+         }
+      }
+      else
       for (int k = tid; k < ntodo; k += NT)
       {
-         const int c = s_todo[k];
+         const int c = MARCH ? k : s_todo[k];
          if ( s_done[c] ) continue;
          const int x = c % p.cr[0], y = ( c/p.cr[0] ) % p.cr[1], z = c/( p.cr[0]*p.cr[1] );
          const int ic = ( p.c0[2] + z )*dz + ( p.c0[1] + y )*dy + p.c0[0] + x;
@@ -485,26 +562,65 @@ gather_boxes_kernel( const IO *__restrict__ patch, const IO *__restrict__ patch2
 constexpr long BOX_GRID = ( 1L << 23 ) - 1;
 static unsigned boxes_from( long q0, long nbox ) { return (unsigned)( nbox - q0 < BOX_GRID ? nbox - q0 : BOX_GRID ); }
 
+// Which form a call takes; us before -> now, for boxes of n^3 cells.
+//   * 64 lanes for boxes of up to 64 cells (CQUAD with clipping FP32, 2048 boxes of 2^3: 95 -> 11; CQUAR of 4^3: 287 -> 53).
+//     Small boxes of the wide FP32 stencil in large numbers take 256 lanes, large ones four waves per SIMD with some
+//     registers in scratch (512 of 12^3: 373 -> 280) or, with options, 256 lanes.
+//   * the march where the lists' second pass of the same rows costs more than its idle lanes: every cell asked for, more
+//     than one box per resident block, and options in the kernel (whose registers leave room for one block per unit) or
+//     divisions in the passes, or boxes of more columns than a block has lanes (512 boxes of 12^3, CQUAD with clipping
+//     FP32: 138 -> 131, 2048: 679 -> 520; VANLEER FP64 512 of 16^3 497 -> 338).  Below 1,200 cells the lists win (QUAD with
+//     clipping, 512 of 10^3: 104, march 139).
+//   * MINMOD1D has one pass a cell: cell by cell, without a list, where the list takes as long as the passes.
+template <typename T, int S>
+static void interp_launch( T *cdata, T *fdata, int nbox, const InterpPrm &p, int *nfail, hipStream_t stream )
+{
+   constexpr bool F64 = ( sizeof( T ) == 8 );
+   const bool plain = ( p.mono & 0x1F ) == 0x1F && !p.opp0 && !( p.mono_coeff < 0.0 );
+   const int  ncell = p.cr[0]*p.cr[1]*p.cr[2];
+   const bool many  = nbox >= 2*device_cus(), big = ncell >= 2048;
+#  define GA_LAUNCH( PLAIN_, MARCH_, NT_, EU_ ) hipLaunchKernelGGL( ( interpolate_kernel<T, S, PLAIN_, MARCH_, NT_, EU_> ), dim3( nbox ), dim3( NT_ ), \
+                                                              0, stream, cdata, fdata, nbox, p, nfail )
+#  define GA_BOTH( NT_ ) { if ( plain ) GA_LAUNCH( true, false, NT_, 0 ); else GA_LAUNCH( false, false, NT_, 0 );  return; }
+   if constexpr ( S == 1 || S == 3 || S == 4 || S == 5 )
+      if ( !p.need )
+      {
+         const bool march = plain ? many && ( ( S == 1 && big ) || ( S != 5 && S != 4 && F64 && ncell >= 1200 ) )
+                                  : ( many && ( S == 1 ? big || ( F64 && ncell >= 1200 ) : ncell >= 1200 ) ) || ( F64 && S != 4 && big );
+         if ( march ) { GA_LAUNCH( false, true, 256, 0 );  return; }
+      }
+   if ( ncell <= 64 ) GA_BOTH( 64 );
+   if constexpr ( S == 2 )
+      if ( many && ( ncell <= 256 || ( p.need && !F64 && nbox >= 4*device_cus() && ncell <= 600 ) ) ) { GA_LAUNCH( false, true, 256, 0 );  return; }
+   if constexpr ( S == 6 && !F64 )
+      if ( many && ncell <= 256 ) GA_BOTH( 256 );
+   if constexpr ( S == 6 && !F64 )
+      if ( many )
+      {
+         if ( plain ) GA_LAUNCH( true, false, 512, 4 ); else GA_LAUNCH( false, false, 256, 0 );
+         return;
+      }
+   if constexpr ( S == 5 && F64 )
+      if ( plain && !many && big ) { GA_LAUNCH( true, false, 512, 0 );  return; }
+   GA_BOTH( interp_lanes<T>( S ) );
+#  undef GA_BOTH
+#  undef GA_LAUNCH
+}
+
 template <typename T>
 static int interpolate_boxes( T *cdata, T *fdata, int nbox, const InterpPrm &p, int *nfail, hipStream_t stream )
 {
-   const bool plain = ( p.mono & 0x1F ) == 0x1F && !p.opp0 && !( p.mono_coeff < 0.0 );
-#  define GA_INT( S ) { if ( plain ) GA_LAUNCH( S, true ); else GA_LAUNCH( S, false ); }
-#  define GA_LAUNCH( S, PLAIN_ ) hipLaunchKernelGGL( ( interpolate_kernel<T, S, PLAIN_> ), dim3( nbox ), dim3( interp_lanes<T>( S ) ), 0, stream, \
-                                                    cdata, fdata, nbox, p, nfail )
    switch ( p.scheme )
    {
-      case 1: GA_INT( 1 ); break;
-      case 2: GA_INT( 2 ); break;
-      case 3: GA_INT( 3 ); break;
-      case 4: GA_INT( 4 ); break;
-      case 5: GA_INT( 5 ); break;
-      case 6: GA_INT( 6 ); break;
-      case 7: GA_INT( 7 ); break;
+      case 1: interp_launch<T, 1>( cdata, fdata, nbox, p, nfail, stream ); break;
+      case 2: interp_launch<T, 2>( cdata, fdata, nbox, p, nfail, stream ); break;
+      case 3: interp_launch<T, 3>( cdata, fdata, nbox, p, nfail, stream ); break;
+      case 4: interp_launch<T, 4>( cdata, fdata, nbox, p, nfail, stream ); break;
+      case 5: interp_launch<T, 5>( cdata, fdata, nbox, p, nfail, stream ); break;
+      case 6: interp_launch<T, 6>( cdata, fdata, nbox, p, nfail, stream ); break;
+      case 7: interp_launch<T, 7>( cdata, fdata, nbox, p, nfail, stream ); break;
       default: return -1;
    }
-#  undef GA_INT
-#  undef GA_LAUNCH
    return ( hipGetLastError() == hipSuccess ) ? 0 : -2;
 }
 
@@ -555,13 +671,18 @@ int launch_assemble( const IO *patch, const IO *fbox, IO *pg_in, int npg, const 
    return ( hipGetLastError() == hipSuccess ) ? 0 : -2;
 }
 
-template int launch_gather_boxes<double>( const double*, const double*, double*, int, const BoxGeom&, const int*, hipStream_t );
-template int launch_gather_boxes<float> ( const float*,  const float*,  float*,  int, const BoxGeom&, const int*, hipStream_t );
-template int launch_assemble<double>( const double*, const double*, double*, int, const int*, int, const BoxGeom&, hipStream_t );
-template int launch_assemble<float> ( const float*,  const float*,  float*,  int, const int*, int, const BoxGeom&, hipStream_t );
-template int launch_interpolate<double>( double*, double*, int, const InterpPrm&, int*, hipStream_t );
-template int launch_interpolate<float> ( float*,  float*,  int, const InterpPrm&, int*, hipStream_t );
-template int launch_prepare_patches<double>( const double*, double*, int, const int*, int, hipStream_t );
-template int launch_prepare_patches<float> ( const float*,  float*,  int, const int*, int, hipStream_t );
+#define GA_INSTANTIATE( T ) \
+template int launch_gather_boxes<T>( const T*, const T*, T*, int, const BoxGeom&, const int*, hipStream_t ); \
+template int launch_assemble<T>( const T*, const T*, T*, int, const int*, int, const BoxGeom&, hipStream_t ); \
+template int launch_interpolate<T>( T*, T*, int, const InterpPrm&, int*, hipStream_t ); \
+template int launch_prepare_patches<T>( const T*, T*, int, const int*, int, hipStream_t );
+// INTERP_PRECISION (32 or 64; both if undefined): the build compiles the two precisions as two objects at the same time
+#if !defined( INTERP_PRECISION ) || INTERP_PRECISION == 64
+GA_INSTANTIATE( double )
+#endif
+#if !defined( INTERP_PRECISION ) || INTERP_PRECISION == 32
+GA_INSTANTIATE( float )
+#endif
+#undef GA_INSTANTIATE
 
 } // namespace gamer_amd
