@@ -726,21 +726,26 @@ __device__ __forceinline__ int copies( int x, int G, int ghost, int pl[2], int i
 
 // one level cell per lane, a row of cells per (y, z, field), neighbouring rows on one XCD: at most 8 copies, most cells
 // have one.  Element index divisions and a search over candidate patch groups took 34 us for 64 FP64 patch groups and
-// 397 us for 960 FP32 ones, this takes 12.9 and 133 us; lanes over 16 x 16 cells took 16 and 134 us.
-template <typename IO>
+// 397 us for 960 FP32 ones, this takes 12.9 and 133 us; lanes over 16 x 16 cells took 16 and 134 us.  THIN, for rows of less than
+// 64 cells and for few rows: lx lanes a row, and the rows in xs pieces (1 x 1 x 32 patch groups with ghost 8 22 -> 9.8 us, 32 x 1
+// x 1 FP64 27 -> 12; as run-time values for all levels they cost 5 to 15% of the others).
+template <typename IO, bool THIN>
 __global__ void __launch_bounds__( 256 )
-prepare_adjoint_kernel( const IO *__restrict__ pg_lam, IO *__restrict__ lam, int nx, int ny, int nz, int ghost, long rows )
+prepare_adjoint_kernel( const IO *__restrict__ pg_lam, IO *__restrict__ lam, int nx, int ny, int nz, int ghost, long rows, int lx_, int xs_ )
 {
+   const int lx = THIN ? lx_ : 64, xs = THIN ? xs_ : 1;
    const int n = PS + 2*ghost, n3 = n*n*n, gx = nx/PS, gy = ny/PS;
-   const int tx = threadIdx.x & 63, lr = threadIdx.x >> 6;            // 64 cells of 4 rows per pass
-   for (long row = xcd_block()*4 + lr; row < rows; row += (long)gridDim.x*4)
+   const int tx = threadIdx.x & ( lx - 1 ), lr = (unsigned)threadIdx.x / (unsigned)lx, nr = 256 / lx;      // lx cells of nr rows per pass
+   const long lb = xcd_block(), rb = THIN ? lb / xs : lb;
+   const int  xc = THIN ? (int)( lb - rb*xs )*lx : 0;
+   for (long row = rb*nr + lr; row < rows; row += (long)( gridDim.x/xs )*nr)
    {
       const int  y = (int)( row % ny );
       const long vz = row / ny;
       const int  z = (int)( vz % nz ), v = (int)( vz / nz );
       int py[2], iy[2], pz[2], iz[2];
       const int my = copies( y, gy, ghost, py, iy ), mz = copies( z, nz/PS, ghost, pz, iz );
-      for (int x = tx; x < nx; x += 64)
+      for (int x = xc + tx; x < nx; x += lx*xs)
       {
          int px[2], ix[2];
          const int mx = copies( x, gx, ghost, px, ix );
@@ -868,9 +873,14 @@ int launch_prepare_adjoint( const IO *pg_lam, IO *lam, int nx, int ny, int nz, i
 {
    const long rows = (long)NV*ny*nz;
    if ( rows <= 0 || nx <= 0 ) return 0;
-   const long b = ( rows + 3 )/4;
-   hipLaunchKernelGGL( prepare_adjoint_kernel<IO>, dim3( (unsigned)( b < 65536 ? b : 65536 ) ), dim3( 256 ), 0, stream, pg_lam, lam, nx, ny, nz,
-                       ghost, rows );
+   const int  lx = ( nx < 32 ) ? 16 : ( nx < 64 ) ? 32 : 64, nr = 256/lx;
+   const long b = ( rows + nr - 1 )/nr, blocks = b < 65536 ? b : 65536;
+   int xs = 1;
+   while ( xs*lx < nx && blocks*xs < 4L*device_cus() ) xs *= 2;
+   if ( lx < 64 || xs > 1 ) hipLaunchKernelGGL( ( prepare_adjoint_kernel<IO, true> ), dim3( (unsigned)( blocks*xs ) ), dim3( 256 ), 0, stream, pg_lam, lam,
+                                                nx, ny, nz, ghost, rows, lx, xs );
+   else hipLaunchKernelGGL( ( prepare_adjoint_kernel<IO, false> ), dim3( (unsigned)blocks ), dim3( 256 ), 0, stream, pg_lam, lam, nx, ny, nz, ghost,
+                            rows, lx, xs );
    return ( hipGetLastError() == hipSuccess ) ? 0 : -2;
 }
 
