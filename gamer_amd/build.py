@@ -22,6 +22,7 @@ FLAGS = [
 # scheduler (2.3% ahead of iterative ILP), its FP64 kernels with iterative ILP (4.1% ahead of the default).  The MHM_RP
 # kernels run fastest with the default scheduler in FP32 (532 against 538 us on 4096 patch groups) and the same with
 # both in FP64; the adjoint, interpolation and sync sources crash the compiler under these strategies.
+# The interpolation file is two objects as well, so that its kernels compile at the same time.
 EXTRA = {"hydro_mhm.hip:32": ["-DMHM_PRECISION=32", "-mllvm", "-amdgpu-sched-strategy=max-ilp"],
          "hydro_mhm.hip:64": ["-DMHM_PRECISION=64", "-mllvm", "-amdgpu-sched-strategy=iterative-ilp"],
          "hydro_interp.hip:32": ["-DINTERP_PRECISION=32"], "hydro_interp.hip:64": ["-DINTERP_PRECISION=64"]}

@@ -23,18 +23,20 @@
 // limiter, with the limited slope's two partials from a two-direction dual evaluation (written out for VL_GMINMOD).  The half-step conversion
 // with floors takes its local Jacobian from forward-mode dual numbers (hydro_dual.hpp) pushed through the same
 // templated device function, one input direction at a time.  All forms take exactly the branches of the forward
-// evaluation.
+// evaluation of this file (F12, F4), which solves the interfaces by rs_hllc(), rs_hlle() and rs_roe().  The marching
+// kernels solve them by hllc_flux() and its twins of hydro_math.hpp: the same functions rounded differently, so that a
+// face within rounding of a kink (a floor, a wave speed of 0) may be on the other side of it there.
 // The reverse phases are gathers: every workspace entry has one writer, so there are no atomics and the result
 // is deterministic.
 //
 // Scope: MHM_RP, FP64, any Riemann solver and limiter of the forward path.  The MinMod retry is not
 // differentiated (the first-iteration coefficient is used); dt and dh are constants.
 //
-// No floating-point contraction in this translation unit (it holds only the derivative kernels, and the
+// No floating-point contraction of values in this translation unit (it holds only the derivative kernels, and the
 // pragma comes before the solver headers it instantiates).  Every value is then the rounded result of its own
 // source expression, with fused multiply-adds only where fmad() is written, so the dual-number evaluation, the
 // plain recomputation inside the reverse sweeps and the forward phases all produce bitwise equal values and
-// split ties the same way.  Ties are common: a uniform floored region puts the HLLC star pressure on the
+// split ties the same way.  hydro_reverse.hpp turns contraction on for the adjoints alone, from which no branch depends.  Ties are common: a uniform floored region puts the HLLC star pressure on the
 // pressure floor up to rounding, and the floor decides whether its derivative passes.
 
 #pragma clang fp contract(off)

@@ -4,7 +4,8 @@
 //
 //   interpolate_kernel   Interpolate() with Interpolate_Iterate (Interpolate.cpp:90-330) for INT_MINMOD3D, INT_MINMOD1D,
 //                        INT_VANLEER, INT_CQUAD, INT_QUAD, INT_CQUAR and INT_QUAR (src/Interpolation/Int_*.cpp): one
-//                        workgroup per coarse box, one lane per asked-for coarse cell producing its 2x2x2 fine cells.  For the
+//                        workgroup per coarse box, one lane per asked-for coarse cell (listed, or a column of a box
+//                        marched along z: interp_launch) producing its 2x2x2 fine cells.  For the
 //                        tensor-product schemes (all but INT_MINMOD1D) the lane evaluates the x pass on the
 //                        (2G+1)x(2G+1) coarse (y,z) neighbourhood (G = 1, or 2 for the quartic schemes), then the y
 //                        pass, then the z pass: the same operations in the same order as the reference's split
@@ -12,13 +13,12 @@
 //                        variables, then primitive variables, then lower monotonic coefficients) redo only coarse
 //                        cells whose fine cells failed the physicality test: the INTERP_MASK rule (include/Macro.h:947)
 //                        at the granularity of 2x2x2 fine blocks.
-//   prepare_patches_kernel  the same-level copies: window cell (x,y,z) of a patch group from the patch in its
-//                        4x4x4 slot table (-1: no patch at this level, the cell keeps the interpolated value)
+//   prepare_patches_kernel, prepare_patches_vec_kernel  the same-level copies: window cell (x,y,z) of a patch group from
+//                        the patch in its 4x4x4 slot table; a cell without a patch (-1) comes from the interpolated fine
+//                        box, or keeps its value if there is none.  The second takes four cells a lane (FP32)
 //   gather_boxes_kernel  the coarse data of InterpolateGhostZone (src/Main/InterpolateGhostZone.cpp): box cell (x,y,z)
 //                        from the patch covering cell origin + (x,y,z) of the box's slot table (e.g. the father patch
-//                        and its 26 siblings)
-//   assemble_kernel      prepare_patches_kernel with the interpolated fine box as the source of the cells that have no
-//                        patch at this level
+//                        and its 26 siblings); gather_small_boxes_kernel runs across the boxes, gather_planes_kernel by planes
 
 #include "hydro_math.hpp"
 #include "hydro_kernels.hpp"

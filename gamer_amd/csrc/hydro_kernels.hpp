@@ -30,7 +30,11 @@ __device__ __forceinline__ long xcd_block()
 // which is decided over the whole patch group; with the fused dt only into halves, whose patches do not straddle slabs.
 // Measured (us, whole -> split), MHM_RP: FP32 8 patch groups 51.7 -> 14.5, 32 with dt 54.7 -> 35.5, 100 53 -> 31.7, 256
 // 53.7 -> 46.3; FP64 16 73 -> 20, 64 73.8 -> 33.4, 700 224 -> 222.6, 1331 464 -> 433; FP64 Roe 300 264 -> 192.  MHM:
-// FP32 8 103 -> 17, 64 102 -> 31, 200 with dt 106 -> 81; FP64 8 122 -> 20, 64 123 -> 44, Roe 300 338 -> 219.
+// FP32 8 103 -> 17, 64 102 -> 31, 200 with dt 106 -> 81; FP64 8 122 -> 20, 64 123 -> 44, Roe 300 338 -> 219.  The 0.78 holds
+// for MHM as well: of 336 launches of 1 to 1100 patch groups none was slower than whole ones (least gain 1.03).
+// The rule takes the chip as free: a library cannot see what other streams run.  With 1 to 8 streams of the same launches at
+// once, 160 of 168 combinations were as fast as whole patch groups or faster; the others lose their extra halo planes
+// (FP32 4 streams of 128: 98 -> 106 us; FP64 8 of 64: 214 -> 246; MHM FP32 8 of 128: 284 -> 314, FP64 8 of 64 282 -> 319).
 int device_cus();                    // compute units of the current device, 0 if unknown
 inline void slab_split( int npg, int halo, int per_cu, int minmod_maxiter, bool with_dt, Batch &B )
 {

@@ -481,7 +481,10 @@ __device__ __forceinline__ St<R> cons_state( const R c[NV], const Prm<R> &P )
 // Contraction is off and fused multiply-adds are written out, so that every code path that solves a face gets the
 // same bits.  Roe and HLLE follow the same layout.  With the PLM below and the third-order reciprocals, on 4096 patch
 // groups FP32 HLLC went from 0.696 to 0.654 ms, on 1331 FP64 HLLC from 0.594 to 0.516 ms, on 300 FP64 Roe from 0.445
-// to 0.325 ms, on 1000 FP32 MHM HLLE from 0.264 to 0.257 ms, with the same error against 64 bits.
+// to 0.325 ms, on 1000 FP32 MHM HLLE from 0.264 to 0.257 ms (the kernels as they were then; the weighted means of HLLC's
+// contact and the Newton steps of the FP64 sound speed cost 1.2% and gain 1.8% of that).  Against 80-bit arithmetic (L1 of
+// five kinds of data) the outputs of a step are as far off as with rs_*(): FP64 Roe 0.993, FP32 HLLE 0.99 of it.  HLLE's
+// FP32 mass flux has 1.08 times the error in a flow and half of it in static gas, where the sides cancel exactly.
 template <typename R>
 struct Side { R d, u, a, b, p, cs, e, mn; };
 

@@ -30,10 +30,13 @@
 // and more for an LDS read) is most of that at any occupancy; the vector units issue half of the time (FP64) or three
 // quarters (FP32).  So the work is split for the longest wave of each interval, by clock readings at the barriers:
 // [A] columns 2,600, arms 2,500, side waves 2-3 2,500; [H] 2,700 to 3,000.  The previous layout, with all x work on the
-// column waves and four barriers a plane, left the side waves waiting.  Nothing may spill in the loops: a reload, also
-// one placed in front of the loop, makes its first use wait for all outstanding prefetches and stores on every plane
-// (the same kernel with 80 instead of 16 bytes of scratch: 563 against 532 us).  On 4096 patch groups FP32 654 -> 528 us
-// (HLLE on 2048: 389 -> 249 before the cheaper solves of both), on 1331 FP64 516 -> 463 us.
+// column waves and four barriers a plane, left the side waves waiting.  A spill costs more here than its instructions: a
+// reload, also one placed in front of the loop, makes its first use wait for all outstanding prefetches and stores on
+// every plane (the default kernel with 80 instead of 16 bytes of scratch a lane: 563 against 532 us).  FP64 HLLC and HLLE
+// and FP32 HLLE with VL_GMINMOD run without scratch; FP32 HLLC holds 20 bytes (queue 40), Roe 88 (FP64 64 to 76), the
+// kernels with a run-time limiter 40 to 92 (FP64 72 to 88), where 128 (FP64 256) registers do not hold the limiter's or
+// Roe's temporaries beside the z history.  On 4096 patch groups FP32 654 -> 528 us (HLLE on 2048: 389 -> 249 before the
+// cheaper solves of both), on 1331 FP64 516 -> 463 us; with HLLC's contact as weighted means 543 and 438 (with dt).
 
 #include "hydro_math.hpp"
 #include "hydro_kernels.hpp"
