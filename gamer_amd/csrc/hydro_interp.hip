@@ -690,6 +690,7 @@ static unsigned boxes_from( long q0, long nbox ) { return (unsigned)( nbox - q0 
 //     divisions in the passes, or boxes of more columns than a block has lanes (512 boxes of 12^3, CQUAD with clipping
 //     FP32: 138 -> 131, 2048: 679 -> 520; VANLEER FP64 512 of 16^3 497 -> 338).  Below 1,200 cells the lists win (QUAD with
 //     clipping, 512 of 10^3: 104, march 139).
+//   * CQUAD with a negative coefficient never takes the march, whose passes do not turn slopes around.
 //   * MINMOD1D has one pass a cell: cell by cell, without a list, where the list takes as long as the passes.
 template <typename T, int S>
 static void interp_launch( T *cdata, T *fdata, int nbox, const InterpPrm &p, int *nfail, hipStream_t stream )
@@ -702,7 +703,7 @@ static void interp_launch( T *cdata, T *fdata, int nbox, const InterpPrm &p, int
                                                               0, stream, cdata, fdata, nbox, p, nfail )
 #  define GA_BOTH( NT_ ) { if ( plain ) GA_LAUNCH( true, false, NT_, 0 ); else GA_LAUNCH( false, false, NT_, 0 );  return; }
    if constexpr ( S == 1 || S == 3 || S == 4 || S == 5 )
-      if ( !p.need )
+      if ( !p.need && !( S == 4 && p.mono_coeff < 0.0 ) )
       {
          const bool march = plain ? many && ( ( S == 1 && big ) || ( S != 5 && S != 4 && F64 && ncell >= 1200 ) )
                                   : ( many && ( S == 1 ? big || ( F64 && ncell >= 1200 ) : ncell >= 1200 ) ) || ( F64 && S != 4 && big );
