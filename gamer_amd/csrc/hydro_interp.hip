@@ -28,8 +28,6 @@ namespace gamer_amd {
 namespace {
 
 constexpr int PS = 16, H = 8, P3 = H*H*H;
-// Lanes of an interpolation block: the wide stencils need more registers than 512 lanes leave.
-template <typename T> constexpr int interp_lanes( int scheme ) { return ( scheme == 7 || ( sizeof( T ) == 8 && scheme >= 5 ) ) ? 256 : 512; }
 
 template <typename T> __device__ __forceinline__ T sgn( T a ) { return ( a < (T)0 ) ? (T)-1 : (T)+1; }
 
@@ -681,49 +679,68 @@ gather_planes_kernel( const IO *__restrict__ patch, const IO *__restrict__ patch
 constexpr long BOX_GRID = ( 1L << 23 ) - 1;
 static unsigned boxes_from( long q0, long nbox ) { return (unsigned)( nbox - q0 < BOX_GRID ? nbox - q0 : BOX_GRID ); }
 
-// Which form a call takes; us before -> now, for boxes of n^3 cells.
-//   * 64 lanes for boxes of up to 64 cells (CQUAD with clipping FP32, 2048 boxes of 2^3: 95 -> 11; CQUAR of 4^3: 287 -> 53).
-//     Small boxes of the wide FP32 stencil in large numbers take 256 lanes, large ones four waves per SIMD with some
-//     registers in scratch (512 of 12^3: 373 -> 280) or, with options, 256 lanes.
-//   * the march where the lists' second pass of the same rows costs more than its idle lanes: every cell asked for, more
-//     than one box per resident block, and options in the kernel (whose registers leave room for one block per unit) or
-//     divisions in the passes, or boxes of more columns than a block has lanes (512 boxes of 12^3, CQUAD with clipping
-//     FP32: 138 -> 131, 2048: 679 -> 520; VANLEER FP64 512 of 16^3 497 -> 338).  Below 1,200 cells the lists win (QUAD with
-//     clipping, 512 of 10^3: 104, march 139).
+// Which form a call takes.  A list takes 19 one-dimensional passes a cell and field, a march 9 and 10 more a column, but the
+// march's registers leave room for fewer waves and its planes are in sequence; and a block holds the registers of all its
+// waves, busy or not, so that with many boxes idle lanes cost what busy ones would.  us, against a march of 256 lanes for all:
+//   * few boxes: a list of as many lanes as cells, up to 512 (256 for the wide stencils in FP64 and QUAR).
+//   * many boxes of up to 128 cells: a list of 64 or 128 lanes (CQUAD with clipping FP32, 2048 boxes of 2^3: 95 -> 11; VANLEER
+//     FP64, 4096 of 8 x 8 x 2: 240 -> 87, with 512 lanes 300); of up to 256 cells 256 lanes.
+//   * many boxes with a mask, of which few cells may be asked for: 128 lanes up to 512 cells (CQUAD with clipping FP32, 4096 of
+//     8 x 8 x 2: 134 -> 48, with 512 lanes 193), 256 up to 1331; MINMOD3D and CQUAD without options in FP32, whose lists are short
+//     of nothing but lanes, 512 from 257 on (MINMOD3D, 2048 of 8^3: 45, 128 lanes 54).
+//   * the march for many boxes where options are in the kernel or the passes hold divisions in FP64 (`heavy`: there lists get
+//     two waves per SIMD at most too): from three boxes per unit on, 128 lanes for 65 to 128 columns (QUAD with clipping FP32,
+//     1024 of 10^3: 272 -> 150, list 203), 256 for more; 64 lanes for 33 to 64 columns from eight boxes per unit on (VANLEER with
+//     clipping FP32, 4096 of 8 x 8 x 2: 163 -> 71, list 78).  Without options, in FP32, only for thin boxes of more than 128
+//     columns (VANLEER, 1400 of 16 x 16 x 3: 94, list 123).
 //   * CQUAD with a negative coefficient never takes the march, whose passes do not turn slopes around.
-//   * MINMOD1D has one pass a cell: cell by cell, without a list, where the list takes as long as the passes.
+//   * CQUAR in FP32, many boxes: 256 lanes, or 128 where those hold all boxes at once; without options large boxes take four waves
+//     per SIMD with some registers in scratch (512 of 12^3: 373 -> 280).
+//   * MINMOD1D has one pass a cell: cell by cell, without a list, where the list takes as long as the passes, or where 256 lanes
+//     hold all boxes at once and 512 do not (masked FP32, 1024 of 10^3: 31, list 41).
 template <typename T, int S>
 static void interp_launch( T *cdata, T *fdata, int nbox, const InterpPrm &p, int *nfail, hipStream_t stream )
 {
-   constexpr bool F64 = ( sizeof( T ) == 8 );
+   constexpr bool F64 = ( sizeof( T ) == 8 ), WIDE = ( S == 6 || S == 7 );
    const bool plain = ( p.mono & 0x1F ) == 0x1F && !p.opp0 && !( p.mono_coeff < 0.0 );
-   const int  ncell = p.cr[0]*p.cr[1]*p.cr[2];
-   const bool many  = nbox >= 2*device_cus(), big = ncell >= 2048;
-#  define GA_LAUNCH( PLAIN_, MARCH_, NT_, EU_ ) hipLaunchKernelGGL( ( interpolate_kernel<T, S, PLAIN_, MARCH_, NT_, EU_> ), dim3( nbox ), dim3( NT_ ), \
-                                                              0, stream, cdata, fdata, nbox, p, nfail )
-#  define GA_BOTH( NT_ ) { if ( plain ) GA_LAUNCH( true, false, NT_, 0 ); else GA_LAUNCH( false, false, NT_, 0 );  return; }
-   if constexpr ( S == 1 || S == 3 || S == 4 || S == 5 )
-      if ( !p.need && !( S == 4 && p.mono_coeff < 0.0 ) )
-      {
-         const bool march = plain ? many && ( ( S == 1 && big ) || ( S != 5 && S != 4 && F64 && ncell >= 1200 ) )
-                                  : ( many && ( S == 1 ? big || ( F64 && ncell >= 1200 ) : ncell >= 1200 ) ) || ( F64 && S != 4 && big );
-         if ( march ) { GA_LAUNCH( false, true, 256, 0 );  return; }
-      }
-   if ( ncell <= 64 ) GA_BOTH( 64 );
+   const int  ncell = p.cr[0]*p.cr[1]*p.cr[2], ncol = p.cr[0]*p.cr[1], cus = device_cus();
+   const bool many  = nbox >= 2*cus, full = nbox >= 3*cus, one_round = ( full && nbox <= 6*cus ), big = ncell >= 2048;
+#  define GA_LAUNCH( PLAIN_, MARCH_, NT_, EU_ ) { hipLaunchKernelGGL( ( interpolate_kernel<T, S, PLAIN_, MARCH_, NT_, EU_> ), dim3( nbox ), dim3( NT_ ), \
+                                                                0, stream, cdata, fdata, nbox, p, nfail );  return; }
+#  define GA_LIST( NT_ ) { if ( plain ) GA_LAUNCH( true, false, NT_, 0 ) else GA_LAUNCH( false, false, NT_, 0 ) }
    if constexpr ( S == 2 )
-      if ( many && ( ncell <= 256 || ( p.need && !F64 && nbox >= 4*device_cus() && ncell <= 600 ) ) ) { GA_LAUNCH( false, true, 256, 0 );  return; }
-   if constexpr ( S == 6 && !F64 )
-      if ( many && ncell <= 256 ) GA_BOTH( 256 );
-   if constexpr ( S == 6 && !F64 )
-      if ( many )
-      {
-         if ( plain ) GA_LAUNCH( true, false, 512, 4 ); else GA_LAUNCH( false, false, 256, 0 );
-         return;
-      }
-   if constexpr ( S == 5 && F64 )
-      if ( plain && !many && big ) { GA_LAUNCH( true, false, 512, 0 );  return; }
-   GA_BOTH( interp_lanes<T>( S ) );
-#  undef GA_BOTH
+   {
+      if ( many && ( ncell <= 256 || ( p.need && ncell <= 600 && ( F64 || nbox >= 4*cus ) ) || ( p.need && !F64 && one_round && ncell <= 2000 ) ) )
+         GA_LAUNCH( false, true, 256, 0 )
+      if ( ncell <= 64 ) GA_LIST( 64 )
+      GA_LIST( 512 )
+   }
+   else
+   {
+      if constexpr ( !WIDE )
+         if ( !p.need && ncell > 64 && !( S == 4 && p.mono_coeff < 0.0 ) )
+         {
+            const bool heavy = !plain || ( F64 && ( S == 1 || S == 3 ) );
+            if ( heavy && full && ncol > 64 && ncol <= 128 && ncell >= ( F64 && S == 1 ? 300 : 200 ) ) GA_LAUNCH( false, true, 128, 0 )
+            if ( heavy && nbox >= 8*cus && ncol > 32 && ncol <= 64 && ncell >= 128 ) GA_LAUNCH( false, true, 64, 0 )
+            if ( ( heavy && many && ( ( ncol > 128 && ncell > 256 ) || ncell >= 1200 ) ) || ( !plain && F64 && S != 4 && big ) ||
+                 ( plain && !F64 && S != 4 && full && ncol > 128 && ncell >= 512 && p.cr[2] <= 4 ) || ( plain && S == 1 && many && big ) )
+               GA_LAUNCH( false, true, 256, 0 )
+         }
+      const bool light = plain && !F64 && ( S == 1 || S == 4 );
+      if ( ncell <= 64 ) GA_LIST( 64 )
+      if ( ncell <= 128 || ( p.need && many && ncell <= ( light ? 256 : 512 ) ) || ( S == 6 && !F64 && plain && one_round && ncell <= 256 ) ) GA_LIST( 128 )
+      if constexpr ( S == 6 && !F64 )
+         if ( many && !p.need )
+         {
+            if ( !plain || ncell <= 256 ) GA_LIST( 256 )
+            GA_LAUNCH( true, false, 512, 4 )
+         }
+      if ( S == 7 || ( S == 6 && F64 ) || ncell <= 256 || ( p.need && many && !light && ( ncell <= 1331 || WIDE ) ) || ( full && ncell <= 512 && !p.need ) ||
+           ( S == 5 && F64 && many ) ) GA_LIST( 256 )
+      if constexpr ( S != 7 && !( S == 6 && F64 ) ) GA_LIST( 512 )
+   }
+#  undef GA_LIST
 #  undef GA_LAUNCH
 }
 
