@@ -18,8 +18,9 @@
 //                        box, or keeps its value if there is none.  The second takes four cells a lane (FP32)
 //   gather_boxes_kernel  the coarse data of InterpolateGhostZone (src/Main/InterpolateGhostZone.cpp): box cell (x,y,z)
 //                        from the patch covering cell origin + (x,y,z) of the box's slot table (e.g. the father patch
-//                        and its 26 siblings); gather_small_boxes_kernel runs across the boxes, gather_planes_kernel by planes
+//                        and its 26 siblings); gather_planes_kernel does the same plane by plane
 
+#include <type_traits>
 #include "hydro_math.hpp"
 #include "hydro_kernels.hpp"
 
@@ -558,101 +559,56 @@ prepare_patches_vec_kernel( const IO *__restrict__ patch, const IO *__restrict__
 }
 
 // box[q][v][z][y][x] (size) = patch[ slot[q][Z/8][Y/8][X/8] ][v][Z%8][Y%8][X%8], (X,Y,Z) = origin + (x,y,z);
-// slot -1 keeps the box value.  Block (box, field, GB_N cells of the box in linear order), as above; the sizes are general,
-// so the cell's coordinates take two integer divisions.  With patch2, half the sum of the cells of both: coarse data halfway
-// between two times, where two passes over the whole level made them first (20 + 23 us of a two-level step of 4096 patches). 
-// One block per plane took 24 us where the same with divisions takes 22.
-// SMALL: boxes of at most GB_SMALL cells take the coordinates from float reciprocals instead, which is most of the instructions
-// otherwise: (e + 0.5)/nxy lies at least 1/(2 nxy) from an integer and its float error is below nz/2^22, less than that for
-// nxy*nz < 2^21.  512 boxes of 14^3 FP32 cells: 18 us with them, 23 with the divisions (the half sum 24.6 and 27.5).
-constexpr int GB_NT = 512, GB_Q = 6, GB_N = GB_NT*GB_Q, GB_SMALL = 1 << 20;
+// slot -1 keeps the box value.  Blocks of GB_N consecutive cells across boxes and fields, a thread copies the cells t, t + 256, ...,
+// as above, with GB_Q loads in flight.  With patch2, half the sum of the cells of both: coarse data halfway between two times, where
+// two passes over the whole level made them first (20 + 23 us of a two-level step of 4096 patches).  A cell's coordinates come from
+// reciprocals instead of integer divisions, which are most of the instructions otherwise (512 boxes of 14^3 FP32 cells 18 us and
+// 23): (e + 0.5)/nxy lies at least 1/(2 nxy) from an integer, and its error is below nz/2^22 in float, less than that for
+// nxy*nz < 2^21 (SMALL: boxes of at most GB_SMALL cells), and far below it in double for the others.
+// Bound by memory.  Blocks of one box and field each, of 512 x 6 cells, leave what a box does not fill: us, FP32, 4096 boxes: 1^3
+// cells 49 -> 9.2, 8^3 52 -> 27, 9 x 9 x 9 51 -> 37, 16^3 252 -> 193; 512 of 14^3 the same 20.
+constexpr int GB_NT = 256, GB_Q = 4, GB_N = GB_NT*GB_Q, GB_SMALL = 1 << 20;
 template <typename IO, bool SMALL>
 __global__ void __launch_bounds__( GB_NT )
 gather_boxes_kernel( const IO *__restrict__ patch, const IO *__restrict__ patch2, IO *__restrict__ box, BoxGeom g,
-                     const int *__restrict__ slot, unsigned chunks )
+                     const int *__restrict__ slot, long first, long total )
 {
-   const long lb = xcd_block();
-   const long w = lb / chunks, q = w / NV, v = w - q*NV;                          // chunk fastest, then field, then box
-   const unsigned nx = g.size[0], nxy = nx*g.size[1];
-   const long n = (long)nxy*g.size[2], e0 = ( lb - w*chunks )*GB_N + threadIdx.x;
-   const int *sl = slot + (size_t)q*g.tdim[0]*g.tdim[1]*g.tdim[2];
-   const IO *pv = patch + (size_t)v*P3;
-   IO *dst = box + w*n;
-   const IO *src[GB_Q];
+   using R = std::conditional_t<SMALL, float, double>;
+   using I = std::conditional_t<SMALL, unsigned, unsigned long>;
+   const I nx = g.size[0], nxy = nx*g.size[1], n = nxy*g.size[2];
+   const size_t nt = (size_t)g.tdim[0]*g.tdim[1]*g.tdim[2];
+   const R rx = (R)1/(R)nx, rxy = (R)1/(R)nxy;
    const ptrdiff_t other = patch2 ? patch2 - patch : 0;
-   const float rx = 1.0f/(float)nx, rxy = 1.0f/(float)nxy;
+   const IO *src[GB_Q];
+   IO val[GB_Q];
+   const long e0 = first + (long)blockIdx.x*GB_N + threadIdx.x;
 #  pragma unroll
    for (int k=0; k<GB_Q; k++)
    {
       const long e = e0 + k*GB_NT;
       src[k] = nullptr;
-      if ( e >= n ) continue;
-      unsigned z, r, y;
-      if ( SMALL )
-      {
-         z = (unsigned)( ( (float)(int)e + 0.5f )*rxy );  r = (unsigned)e - z*nxy;
-         y = (unsigned)( ( (float)(int)r + 0.5f )*rx );
-      }
-      else
-      {
-         z = ( n >> 32 ) ? (unsigned)( e / nxy ) : (unsigned)e / nxy;  r = (unsigned)( e - (long)z*nxy );
-         y = r / nx;
-      }
-      const unsigned x = r - y*nx;
+      if ( e >= total ) continue;
+      const unsigned long w = ( total >> 32 ) ? (unsigned long)e / n : (unsigned)e / (unsigned)n;
+      const unsigned long q = ( total >> 32 ) ? w / NV : (unsigned)w / NV;
+      const int v = (int)( w - q*NV );
+      const I c = (I)( e - (long)( w*n ) );
+      const I z = (I)( ( (R)c + (R)0.5 )*rxy ), r = c - z*nxy, y = (I)( ( (R)r + (R)0.5 )*rx ), x = r - y*nx;
       const int X = (int)x + g.origin[0], Y = (int)y + g.origin[1], Z = (int)z + g.origin[2];
-      const int s = sl[ ( (size_t)( Z >> 3 )*g.tdim[1] + ( Y >> 3 ) )*g.tdim[0] + ( X >> 3 ) ];
-      if ( s >= 0 ) src[k] = pv + ( (size_t)s*NV*P3 + ( Z & 7 )*H*H + ( Y & 7 )*H + ( X & 7 ) );
+      const int s = slot[ q*nt + ( (size_t)( Z >> 3 )*g.tdim[1] + ( Y >> 3 ) )*g.tdim[0] + ( X >> 3 ) ];
+      if ( s >= 0 ) src[k] = patch + ( ( (size_t)s*NV + v )*P3 + ( Z & 7 )*H*H + ( Y & 7 )*H + ( X & 7 ) );
    }
-   IO val[GB_Q];
 #  pragma unroll
    for (int k=0; k<GB_Q; k++) if ( src[k] ) val[k] = *src[k];
    if ( patch2 )
 #     pragma unroll
       for (int k=0; k<GB_Q; k++) if ( src[k] ) val[k] = ( val[k] + src[k][other] )*(IO)0.5;
 #  pragma unroll
-   for (int k=0; k<GB_Q; k++) if ( src[k] ) dst[ e0 + k*GB_NT ] = val[k];
+   for (int k=0; k<GB_Q; k++) if ( src[k] ) box[ e0 + k*GB_NT ] = val[k];
 }
 
-// The same for boxes of up to GF_MAX cells: blocks of consecutive cells across boxes and fields, where a block of their own would
-// leave most of its lanes without a cell.  us, FP32, 4096 boxes: 1^3 cells 49 -> 9.2, 4^3 50 -> 9.3, 8^3 52 -> 27 (with a block
-// per plane 9.1, 23 and 46); from 10^3 on as fast as the blocks of their own.
-constexpr int GF_NT = 256, GF_Q = 4, GF_MAX = 512;
-template <typename IO>
-__global__ void __launch_bounds__( GF_NT )
-gather_small_boxes_kernel( const IO *__restrict__ patch, const IO *__restrict__ patch2, IO *__restrict__ box, BoxGeom g,
-                           const int *__restrict__ slot, long total )
-{
-   const unsigned nx = g.size[0], nxy = nx*g.size[1], n = nxy*g.size[2], nt = g.tdim[0]*g.tdim[1]*g.tdim[2];
-   const float rx = 1.0f/(float)nx, rxy = 1.0f/(float)nxy;
-   const ptrdiff_t other = patch2 ? patch2 - patch : 0;
-   const IO *src[GF_Q];
-   IO val[GF_Q];
-   const long e0 = (long)blockIdx.x*( GF_NT*GF_Q ) + threadIdx.x;
-#  pragma unroll
-   for (int k=0; k<GF_Q; k++)
-   {
-      const long e = e0 + k*GF_NT;
-      src[k] = nullptr;
-      if ( e >= total ) continue;
-      const unsigned w = ( total >> 32 ) ? (unsigned)( e / n ) : (unsigned)e / n, q = w / NV, v = w - q*NV, c = (unsigned)( e - (long)w*n );
-      const unsigned z = (unsigned)( ( (float)(int)c + 0.5f )*rxy ), r = c - z*nxy, y = (unsigned)( ( (float)(int)r + 0.5f )*rx ), x = r - y*nx;
-      const int X = (int)x + g.origin[0], Y = (int)y + g.origin[1], Z = (int)z + g.origin[2];
-      const int s = slot[ (size_t)q*nt + ( (size_t)( Z >> 3 )*g.tdim[1] + ( Y >> 3 ) )*g.tdim[0] + ( X >> 3 ) ];
-      if ( s >= 0 ) src[k] = patch + ( ( (size_t)s*NV + v )*P3 + ( Z & 7 )*H*H + ( Y & 7 )*H + ( X & 7 ) );
-   }
-#  pragma unroll
-   for (int k=0; k<GF_Q; k++) if ( src[k] ) val[k] = *src[k];
-   if ( patch2 )
-#     pragma unroll
-      for (int k=0; k<GF_Q; k++) if ( src[k] ) val[k] = ( val[k] + src[k][other] )*(IO)0.5;
-#  pragma unroll
-   for (int k=0; k<GF_Q; k++) if ( src[k] ) box[ e0 + k*GF_NT ] = val[k];
-}
-
-// The same, a block per (box, field, z plane) whose lanes take the plane's cells in linear order: the faster one for large boxes
-// where many planes keep the memory streams long (us, FP32: 64 boxes of 64^3 cells 172 -> 151, 8 of 128^3 186 -> 166, 64 of 24^3
-// 15.4 -> 13.1), and the slower one where the planes do not fill the chip (one box of 128^3 28 -> 47) or, in FP64, in calls past
-// the caches (64 of 64^3 247 -> 280).
+// The same, a block per (box, field, z plane) whose lanes take the plane's cells in linear order: the faster one for planes of many
+// cells if there are enough of them, which keep the memory streams long (us, FP32: 64 boxes of 64^3 cells 172 -> 151, 8 of 128^3 186
+// -> 166, 4096 of 256 x 16 x 1 150 -> 125), in FP64 only for thin boxes (2048 of 64 x 64 x 2 211 -> 202; 64 of 64^3 247 -> 280).
 constexpr int GP_NT = 256;
 template <typename IO>
 __global__ void __launch_bounds__( GP_NT )
@@ -785,33 +741,20 @@ template <typename IO>
 int launch_gather_boxes( const IO *patch, const IO *patch2, IO *box, int nbox, const BoxGeom &g, const int *slot, hipStream_t stream )
 {
    if ( nbox <= 0 ) return 0;
-   const long n = (long)g.size[0]*g.size[1]*g.size[2], chunks = ( n + GB_N - 1 )/GB_N, nslot = (long)g.tdim[0]*g.tdim[1]*g.tdim[2];
-   if ( n <= GF_MAX )
-   {
-      const long most = ( 1L << 33 )/( NV*n ), per = BOX_GRID < most ? BOX_GRID : most;      // blocks of one launch, as BOX_GRID
-      for (long q0 = 0; q0 < nbox; q0 += per)
-      {
-         const long total = ( nbox - q0 < per ? nbox - q0 : per )*NV*n;
-         hipLaunchKernelGGL( gather_small_boxes_kernel<IO>, dim3( (unsigned)( ( total + GF_NT*GF_Q - 1 )/( GF_NT*GF_Q ) ) ), dim3( GF_NT ), 0, stream,
-                             patch, patch2, box + q0*NV*n, g, slot + q0*nslot, total );
-      }
-      return ( hipGetLastError() == hipSuccess ) ? 0 : -2;
-   }
-   const long planes = (long)nbox*NV*g.size[2];
-   if ( n >= 13824 && (long)g.size[0]*g.size[1] < ( 1L << 30 ) &&
-        ( sizeof( IO ) == 4 ? planes >= 4000 : planes >= 1600 && n <= 64000 && nbox*NV*n <= 8000000 ) )
+   const long nxy = (long)g.size[0]*g.size[1], n = nxy*g.size[2], total = (long)nbox*NV*n, planes = (long)nbox*NV*g.size[2];
+   if ( nxy >= ( sizeof( IO ) == 4 ? 512 : 1024 ) && ( sizeof( IO ) == 4 || g.size[2] <= 4 ) && planes >= 1900 && nxy < ( 1L << 30 ) && nbox <= BOX_GRID )
    {
       hipLaunchKernelGGL( gather_planes_kernel<IO>, dim3( nbox, NV, g.size[2] ), dim3( GP_NT ), 0, stream, patch, patch2, box, g, slot );
       return ( hipGetLastError() == hipSuccess ) ? 0 : -2;
    }
-#  define GA_GB( SMALL_ ) hipLaunchKernelGGL( ( gather_boxes_kernel<IO, SMALL_> ), dim3( nb, NV, (unsigned)chunks ), dim3( GB_NT ), 0, stream, \
-                                              patch, patch2, box + q0*NV*n, g, slot + q0*nslot, (unsigned)chunks )
-   for (long q0 = 0; q0 < nbox; q0 += BOX_GRID)
+   constexpr long most = BOX_GRID*GB_N;                                     // cells of one launch
+   for (long first = 0; first < total; first += most)
    {
-      const unsigned nb = boxes_from( q0, nbox );
-      if ( n <= GB_SMALL ) GA_GB( true ); else GA_GB( false );
+      const long left = total - first, part = left < most ? left : most;
+      const dim3 grid( (unsigned)( ( part + GB_N - 1 )/GB_N ) );
+      if ( n <= GB_SMALL ) hipLaunchKernelGGL( ( gather_boxes_kernel<IO, true> ), grid, dim3( GB_NT ), 0, stream, patch, patch2, box, g, slot, first, total );
+      else hipLaunchKernelGGL( ( gather_boxes_kernel<IO, false> ), grid, dim3( GB_NT ), 0, stream, patch, patch2, box, g, slot, first, total );
    }
-#  undef GA_GB
    return ( hipGetLastError() == hipSuccess ) ? 0 : -2;
 }
 
