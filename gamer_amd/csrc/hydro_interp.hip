@@ -500,9 +500,9 @@ prepare_patches_kernel( const IO *__restrict__ patch, const IO *__restrict__ fbo
 
 // The same with four consecutive cells a lane, put as one vector where all are copied and the destination is aligned (N^3 is a
 // multiple of 8, so a group never straddles two windows).  More blocks in flight for less work each: the faster one in FP32 for
-// narrow windows and for few patch groups without fine boxes (us, caches cold / warm, against the form above: 512 patch groups
-// without ghost zones 28 / 14.6 and 31 / 19, 64 with ghost 3 11.6 / 8 and 12.9 / 10), the slower one else (1024 with ghost 3 123
-// and 119, in FP64 265 and 177).
+// narrow windows and for few patch groups (us, caches warm / cold, against the form above: 512 patch groups without ghost zones
+// 14.6 / 28 and 19 / 31; with ghost 3 64 8.6 / 11.7 and 11 / 13, 729 58 / 89 and 68 / 87, 216 with fine boxes 21 / 30 and 24 / 32),
+// the slower one else (2000 with ghost 3 226 / 251 and 216 / 224; 512 with fine boxes in an AMR step 78 and 62; FP64 1024 265 and 177).
 constexpr int PV_NT = 256, PV_N = 4;
 template <typename IO> struct Vec4;
 template <> struct Vec4<float>  { typedef float  type __attribute__(( ext_vector_type( 4 ) )); };
@@ -765,7 +765,7 @@ int launch_assemble( const IO *patch, const IO *fbox, IO *pg_in, int npg, const 
    if ( npg <= 0 ) return 0;
    const int n = PS + 2*ghost;
    if constexpr ( sizeof( IO ) == 4 )
-      if ( ghost <= 2 || ( !fbox && npg <= 2*device_cus() ) )
+      if ( ghost <= 2 || npg <= ( fbox ? 1 : 3 )*device_cus() )
       {
          hipLaunchKernelGGL( prepare_patches_vec_kernel<IO>, dim3( npg, NV, ( n*n*n + PV_NT*PV_N - 1 )/( PV_NT*PV_N ) ), dim3( PV_NT ), 0, stream,
                              patch, fbox, pg_in, slot, ghost, fb );
